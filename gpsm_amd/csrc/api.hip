@@ -943,9 +943,15 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // ---------------- host: join orders ----------------
   std::vector<CetDesc> jdesc;
   std::vector<JoinPlan> plans;
-  std::vector<JoinTask> tasks, tasks_cyc;
+  std::vector<JoinTask> tasks;
   std::vector<uint32_t> plan_of_q(nq, ~0u);
   uint64_t off_words = fwd_words, list_words = 0, term_words = 0;  // reversed tables' regions follow the forward ones
+  // Only tuples need the last levels enumerated; otherwise the tables of the
+  // last one or two positions without back positions become records.
+  const uint64_t emit_cap = o.want_tuples && nq == 1 ? o.tuple_cap : 0;
+  uint64_t agg_words = 0;         // records of those tables
+  std::vector<uint32_t> wtab;     // last positions' tables (no list is written)
+  std::vector<AggDesc> adesc;     // tables of the positions before them
   std::vector<uint32_t> recount;  // tables of reversed plan edges (count again)
   std::vector<uint32_t> term_desc;   // tables of last join levels
   std::vector<uint64_t> term_start;  // their term ranges, back to back (+ total)
@@ -1029,13 +1035,20 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     JoinPlan jp{};
     jp.q = S.hq.n;
     jp.vbase = S.vbase;
-    auto add_desc = [&](uint32_t xq, uint32_t wq, uint32_t edge) {
+    const OrderPlan& pl = S.plan;
+    if (!emit_cap && S.hq.n >= 3 && pl.backs[S.hq.n - 1].empty())
+      jp.agg = S.hq.n >= 4 && pl.backs[S.hq.n - 2].empty() ? 2 : 1;
+    // list: the table's list is written (else its candidates get records only)
+    auto add_desc = [&](uint32_t xq, uint32_t wq, uint32_t edge, bool list) {
       CetDesc d{};
       d.x_slot = S.vbase + xq;
       d.w_slot = S.vbase + wq;
       d.ncand = counts[d.x_slot];
       d.clist_off = coff[d.x_slot];
-      if (xq == S.hq.ef[edge]) {
+      d.agg_base = ~0ull;
+      if (!list) {
+        d.off_base = 0;
+      } else if (xq == S.hq.ef[edge]) {
         d.off_base = fdesc[fdesc_of_q[b] + edge].off_base;  // its counts are there since phase B
       } else {
         d.off_base = off_words;
@@ -1046,12 +1059,11 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       d.list_cap = (uint32_t)S.cet_size[edge];
       d.term_base = ~0ull;
       key_range(S.hq, st, wq, d.w_lo, d.w_hi);
-      list_words += S.cet_size[edge];
+      if (list) list_words += S.cet_size[edge];
       jdesc.push_back(d);
       return (uint32_t)jdesc.size() - 1;
     };
-    const OrderPlan& pl = S.plan;
-    jp.first_cet = add_desc(pl.order[0], pl.order[1], pl.first_edge);
+    jp.first_cet = add_desc(pl.order[0], pl.order[1], pl.first_edge, true);
     S.first_desc = jp.first_cet;
     uint32_t nb = 0;
     for (uint32_t k = 0; k < S.hq.n; ++k) {
@@ -1059,11 +1071,16 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       jp.back_off[k] = nb;
       if (k >= 2) {
         jp.par[k] = pl.par_pos[k];
-        jp.cet[k] = add_desc(pl.order[pl.par_pos[k]], pl.order[k], pl.par_edge[k]);
-        if (k + 1 == S.hq.n) {
-          CetDesc& d = jdesc.back();
+        const bool last = k + 1 == S.hq.n;
+        jp.cet[k] = add_desc(pl.order[pl.par_pos[k]], pl.order[k], pl.par_edge[k], !(last && jp.agg));
+        CetDesc& d = jdesc.back();
+        d.term_qid = pl.order[k];
+        if (jp.agg && k + jp.agg >= S.hq.n) {
+          d.agg_base = agg_words;
+          agg_words += d.ncand;
+          if (last) wtab.push_back(jp.cet[k]);
+        } else if (last) {
           d.term_base = term_words;
-          d.term_qid = pl.order[k];
           term_desc.push_back(jp.cet[k]);
           term_start.push_back(term_words);
           term_words += S.cet_size[pl.par_edge[k]];
@@ -1079,6 +1096,27 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     }
     jp.back_off[S.hq.n] = nb;
     jp.nback_total = nb;
+    if (jp.agg == 2) {
+      const uint32_t w = S.hq.n - 1, y = w - 1;
+      const CetDesc &dy = jdesc[jp.cet[y]], &dw = jdesc[jp.cet[w]];
+      AggDesc ad{};
+      ad.off_base = dy.off_base;
+      ad.list_base = dy.list_base;
+      ad.agg_base = dy.agg_base;
+      ad.w_agg_base = dw.agg_base;
+      ad.ncand = dy.ncand;
+      // pairs of y's and w's lists of one candidate matter only when both
+      // carry one label
+      ad.mode = jp.par[w] == y ? AGG_CHAIN
+                               : jp.par[w] == jp.par[y] && ((jp.inj[w] >> y) & 1) ? AGG_SIBLING : AGG_SUM;
+      ad.y_slot = dy.w_slot;
+      ad.y_qid = pl.order[y];
+      ad.w_slot = dw.w_slot;
+      ad.w_qid = pl.order[w];
+      adesc.push_back(ad);
+    }
+    // what the join enumerates of it sizes its tasks
+    if (jp.agg) est[b] = analytic_cost_upto(pcs[b], pl, S.hq.n - 1 - jp.agg);
     plan_of_q[b] = (uint32_t)plans.size();
     plans.push_back(jp);
   }
@@ -1090,8 +1128,15 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // the grid is idle.  The persistent grid holds at most as many workgroups
   // as are resident at once: a workgroup beyond that would start only once
   // the task counter has run out.
-  const uint32_t nwg = std::max<uint32_t>(1, c->ncu * std::min(wg_per_cu, join_resident_per_cu(qmax, false)));
-  const uint32_t nwg_cyc = std::max<uint32_t>(1, c->ncu * std::min(wg_per_cu, join_resident_per_cu(qmax, true)));
+  // The launches, by plan: tree plans (counted from records, or enumerated
+  // when tuples are wanted), cyclic plans counted from records, other cyclic
+  // plans.
+  constexpr int NJOIN = 3;
+  const JoinKind kinds[NJOIN] = {emit_cap ? JOIN_TREE_ENUM : JOIN_TREE, JOIN_CYCLIC, JOIN_CYCLIC_ENUM};
+  uint32_t resident[NJOIN];
+  for (int i = 0; i < NJOIN; ++i)
+    resident[i] = std::max<uint32_t>(1, c->ncu * std::min(wg_per_cu, join_resident_per_cu(qmax, kinds[i])));
+  const uint32_t nwg = resident[0];
   const uint64_t tpw = std::max<uint32_t>(1, c->tune.tasks_per_wg);
   uint64_t rows_total = 0;
   double est_total = 0;
@@ -1103,18 +1148,30 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   const uint64_t tsize =
       std::min<uint64_t>(std::max<uint64_t>(rows_total / ((uint64_t)nwg * tpw) + 1, c->tune.task_min), 1u << 20);
   const double target = est_total / ((double)nwg * tpw);
+  std::vector<JoinTask> ltasks[NJOIN];  // by launch
   for (uint32_t b = 0; b < nq; ++b) {
     if (plan_of_q[b] == ~0u) continue;
     const uint64_t R1 = Q[b].cet_size[Q[b].plan.first_edge];
     uint64_t T = (R1 + tsize - 1) / tsize;
     if (target > 0 && est[b] > target) T = std::max<uint64_t>(T, (uint64_t)std::min(est[b] / target + 1.0, 1e9));
-    T = std::min<uint64_t>(std::max<uint64_t>(T, 1), R1);
-    // tree plans' tasks first, the cyclic plans' after them (two launches)
-    std::vector<JoinTask>& dst = plans[plan_of_q[b]].nback_total ? tasks_cyc : tasks;
-    for (uint64_t t = 0; t < T; ++t) dst.push_back({plan_of_q[b], (uint32_t)T, t, (R1 - t + T - 1) / T});
+    const JoinPlan& jp = plans[plan_of_q[b]];
+    // first-table rows counted from records cost about the same each: 64
+    // consecutive ones per chunk, so that their loads are coalesced
+    const uint32_t shift = jp.agg && jp.agg + 2 == jp.q ? 6 : 0;
+    const uint64_t NC = (R1 + (1ull << shift) - 1) >> shift;  // chunks
+    T = std::min<uint64_t>(std::max<uint64_t>(T, 1), NC);
+    std::vector<JoinTask>& dst = ltasks[!jp.nback_total ? 0 : jp.agg ? 1 : 2];
+    for (uint64_t t = 0; t < T; ++t) {
+      uint64_t rows = ((NC - t + T - 1) / T) << shift;
+      if ((NC - 1) % T == t) rows -= (NC << shift) - R1;  // the last chunk may be short
+      dst.push_back({plan_of_q[b], (uint32_t)T, shift, 0, t, rows});
+    }
   }
-  const uint32_t ntree = (uint32_t)tasks.size(), ncyc = (uint32_t)tasks_cyc.size();
-  tasks.insert(tasks.end(), tasks_cyc.begin(), tasks_cyc.end());
+  uint32_t ltask0[NJOIN];  // each launch's first task
+  for (int i = 0; i < NJOIN; ++i) {
+    ltask0[i] = (uint32_t)tasks.size();
+    tasks.insert(tasks.end(), ltasks[i].begin(), ltasks[i].end());
+  }
 
   // ---------------- phase C: candidate-edge tables ----------------
   wall(K_WALL_PLAN);
@@ -1125,6 +1182,23 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if ((rc = c->bufs[B_TERMS].ensure(sizeof(uint64_t) * std::max<uint64_t>(term_words, 1)))) return rc;
   std::vector<CetDesc> cdesc;
   for (uint32_t i : recount) cdesc.push_back(jdesc[i]);
+  // the tables with lists, those of the last positions and those before
+  // them, each with the chunks of 64 candidates before every table
+  std::vector<CetDesc> ldesc, wdesc;
+  std::vector<uint8_t> no_list(jdesc.size(), 0);
+  for (uint32_t i : wtab) no_list[i] = 1, wdesc.push_back(jdesc[i]);
+  for (size_t i = 0; i < jdesc.size(); ++i)
+    if (!no_list[i]) ldesc.push_back(jdesc[i]);
+  auto chunks_before = [](const auto& v) {
+    std::vector<uint32_t> base(1, 0);
+    for (const auto& d : v) base.push_back(base.back() + (d.ncand + 63) / 64);
+    return base;
+  };
+  if ((rc = upload(c, B_LDESC, ldesc)) || (rc = upload(c, B_WDESC, wdesc)) || (rc = upload(c, B_ADESC, adesc)) ||
+      (!wdesc.empty() && (rc = upload(c, B_WCHUNK, chunks_before(wdesc)))) ||
+      (!adesc.empty() && (rc = upload(c, B_ACHUNK, chunks_before(adesc)))) ||
+      (rc = c->bufs[B_AGGS].ensure(sizeof(CetAgg) * std::max<uint64_t>(agg_words, 1))))
+    return rc;
   if (off_words > off_capacity) return GPSM_EINVAL;  // cannot happen: rev_bound covers every reversed table
   if ((rc = upload(c, B_CDESC, cdesc)) ||
       (rc = c->bufs[B_LISTS].ensure(sizeof(uint32_t) * std::max<uint64_t>(list_words, 1))) ||
@@ -1135,35 +1209,37 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       (rc = c->h_stage[2].ensure(sizeof(JoinOut) * std::max<uint32_t>(nplans, 1))))
     return rc;
   if ((rc = c->bufs[B_CTR].ensure(256))) return rc;
-  // Level buffers of the workgroups launched (the tree plans' launch, then
-  // the cyclic plans', which run at the same time), within kLevelBytes: rows
-  // per level halve (to 2048) and then workgroups are dropped, from both
-  // launches in proportion, until they fit.
-  uint32_t gt = ntree ? std::min<uint32_t>(nwg, ntree) : 0, gc = ncyc ? std::min<uint32_t>(nwg_cyc, ncyc) : 0;
+  // Level buffers of the workgroups launched, a region per launch (they may
+  // run at the same time), within kLevelBytes: rows per level halve (to 2048)
+  // and then workgroups are dropped, from every launch in proportion, until
+  // they fit.
+  uint32_t lwg[NJOIN];
+  uint64_t gsum = 0;
+  for (int i = 0; i < NJOIN; ++i) gsum += lwg[i] = (uint32_t)std::min<uint64_t>(resident[i], ltasks[i].size());
   uint32_t lcap = cap;
-  const uint64_t gsum = std::max<uint64_t>(1, (uint64_t)gt + gc);
   while (lcap > 2048 && (double)join_level_words(qmax, lcap) * 4.0 * gsum > kLevelBytes) lcap /= 2;
   const uint64_t lw = join_level_words(qmax, lcap);
   if (lw && (double)lw * 4.0 * gsum > kLevelBytes) {
-    const uint64_t fit = std::max<uint64_t>(2, (uint64_t)(kLevelBytes / (4.0 * lw)));
-    if (gt) gt = (uint32_t)std::max<uint64_t>(1, (uint64_t)gt * fit / gsum);
-    if (gc) gc = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((uint64_t)gc * fit / gsum + 1, fit - gt));
+    const uint64_t fit = std::max<uint64_t>(NJOIN, (uint64_t)(kLevelBytes / (4.0 * lw)));
+    const uint64_t all = gsum;
+    gsum = 0;
+    for (uint32_t& n : lwg) {
+      if (n) n = (uint32_t)std::max<uint64_t>(1, (uint64_t)n * fit / all);
+      gsum += n;
+    }
   }
-  if ((rc = c->bufs[B_LEVELS].ensure(sizeof(uint32_t) * std::max<uint64_t>(lw * ((uint64_t)gt + gc), 1)))) return rc;
-  uint64_t emit_cap = 0;
-  if (o.want_tuples && nq == 1) {
-    emit_cap = o.tuple_cap;
-    if ((rc = c->bufs[B_EMIT].ensure(sizeof(uint32_t) * std::max<uint64_t>(emit_cap * qmax, 1)))) return rc;
-  }
+  if ((rc = c->bufs[B_LEVELS].ensure(sizeof(uint32_t) * std::max<uint64_t>(lw * gsum, 1)))) return rc;
+  if (emit_cap && (rc = c->bufs[B_EMIT].ensure(sizeof(uint32_t) * emit_cap * qmax))) return rc;
   PhaseSig sig_c;
   if (o.use_graph) {
     sig_c.add(uint64_t{1});
     sig_c.add_graph(dg);
     for (int i : {B_BITMAPS, B_CLIST, B_CDESC, B_OFFSETS, B_CHUNKS, B_JDESC, B_LISTS, B_TERM_DESC, B_TERM_START,
-                  B_TERMS, B_JOUT, B_CTR})
+                  B_TERMS, B_JOUT, B_CTR, B_LDESC, B_WDESC, B_WCHUNK, B_ADESC, B_ACHUNK, B_AGGS, B_BPREFIX})
       sig_c.add(c->bufs[i].ptr);
     for (uint64_t v : {(uint64_t)cdesc.size(), (uint64_t)cgrid, (uint64_t)jdesc.size(), (uint64_t)term_desc.size(),
-                       (uint64_t)term_words, (uint64_t)nplans})
+                       (uint64_t)term_words, (uint64_t)nplans, (uint64_t)ldesc.size(), (uint64_t)wdesc.size(),
+                       (uint64_t)adesc.size()})
       sig_c.add(v);
   }
   bool replayed_c = o.use_graph && replay_cached(c, 1, sig_c.w, s, &rc);
@@ -1177,11 +1253,17 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
                        dptr<uint32_t>(c, B_OFFSETS), 1, dptr<uint32_t>(c, B_CHUNKS), cgrid, s,
                        counters ? fstats + fstat_step * slot_cet_c : nullptr);
     pend(K_CET_COUNT, pa, 0.0, counters ? slot_cet_c : -1);
-    launch_cet_offsets(dptr<CetDesc>(c, B_JDESC), (uint32_t)jdesc.size(), dptr<uint32_t>(c, B_OFFSETS), s);
+    launch_cet_offsets(dptr<CetDesc>(c, B_LDESC), (uint32_t)ldesc.size(), dptr<uint32_t>(c, B_OFFSETS), s);
     pa = pbegin(K_CET_WRITE);
-    launch_cet_write(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_JDESC), (uint32_t)jdesc.size(),
+    launch_cet_write(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_LDESC), (uint32_t)ldesc.size(),
                      dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_LISTS), dptr<uint32_t>(c, B_CHUNKS), cgrid, s,
                      counters ? fstats + fstat_step * slot_cet_w : nullptr);
+    launch_cet_sums(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_WDESC), (uint32_t)wdesc.size(),
+                    dptr<uint32_t>(c, B_WCHUNK), dptr<CetAgg>(c, B_AGGS), cgrid, s,
+                    counters ? fstats + fstat_step * slot_cet_w : nullptr);
+    launch_cet_aggs(bitmaps, dptr<uint32_t>(c, B_BPREFIX), W, NB, dptr<AggDesc>(c, B_ADESC), (uint32_t)adesc.size(),
+                    dptr<uint32_t>(c, B_ACHUNK), dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_LISTS),
+                    dptr<CetAgg>(c, B_AGGS), cgrid, s);
     launch_cet_terms(dptr<uint32_t>(c, B_LISTS), dptr<CetDesc>(c, B_JDESC), dptr<uint32_t>(c, B_TERM_DESC),
                      dptr<uint64_t>(c, B_TERM_START), (uint32_t)term_desc.size(), term_words,
                      dptr<unsigned long long>(c, B_TERMS), s);
@@ -1205,17 +1287,14 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     ja.offsets = dptr<uint32_t>(c, B_OFFSETS);
     ja.lists = dptr<uint32_t>(c, B_LISTS);
     ja.terms = dptr<unsigned long long>(c, B_TERMS);
+    ja.aggs = dptr<CetAgg>(c, B_AGGS);
     ja.cets = dptr<CetDesc>(c, B_JDESC);
     ja.plans = dptr<JoinPlan>(c, B_PLANS);
-    ja.tasks = dptr<JoinTask>(c, B_TASKS);
-    ja.ntasks = (uint32_t)tasks.size();
     ja.W = W;
     ja.NB = NB;
     ja.cap = lcap;
     ja.qmax = qmax;
-    ja.levels = dptr<uint32_t>(c, B_LEVELS);
     ja.level_stride = lw;
-    ja.task_counter = dptr<unsigned int>(c, B_CTR);
     ja.out = dptr<JoinOut>(c, B_JOUT);
     if (emit_cap) {
       ja.emit = dptr<uint32_t>(c, B_EMIT);
@@ -1224,31 +1303,31 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     }
     ja.budget = o.work_budget;
     ja.count_bytes = counters ? 1u : 0u;
-    // tree plans and cyclic plans: one launch each, its own task counter;
-    // timed together as one join
+    // one launch per kind of plan, each with its own task counter and level
+    // buffers; timed together as one join.  The enumerated cyclic plans run on
+    // stream2, forked after everything before on stream and joined back before
+    // what follows, the others one after the other on stream.
     hipEvent_t pa = pbegin(K_JOIN);
-    // the cyclic plans on stream2 (own task counter and level buffers),
-    // forked after everything before on stream and joined back before what
-    // follows; the tree plans on stream
-    if (ncyc) {
-      JoinArgs jc = ja;
-      jc.tasks = dptr<JoinTask>(c, B_TASKS) + ntree;
-      jc.ntasks = ncyc;
-      jc.task_counter = dptr<unsigned int>(c, B_CTR) + 1;
-      jc.levels = dptr<uint32_t>(c, B_LEVELS) + lw * gt;
-      hipStream_t s2 = ntree ? c->stream2 : s;
-      if (ntree) {
+    const bool fork = !ltasks[2].empty() && (!ltasks[0].empty() || !ltasks[1].empty());
+    uint64_t level0 = 0;
+    for (int i : {2, 1, 0}) {
+      if (ltasks[i].empty()) continue;
+      JoinArgs jl = ja;
+      jl.tasks = dptr<JoinTask>(c, B_TASKS) + ltask0[i];
+      jl.ntasks = (uint32_t)ltasks[i].size();
+      jl.task_counter = dptr<unsigned int>(c, B_CTR) + i;
+      jl.levels = dptr<uint32_t>(c, B_LEVELS) + lw * level0;
+      level0 += lwg[i];
+      if (i == 2 && fork) {
         HIPCHK(hipEventRecord(c->ev_fork, s));
-        HIPCHK(hipStreamWaitEvent(s2, c->ev_fork, 0));
+        HIPCHK(hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
+        launch_join(jl, lwg[i], kinds[i], c->stream2);
+        HIPCHK(hipEventRecord(c->ev_join, c->stream2));
+      } else {
+        launch_join(jl, lwg[i], kinds[i], s);
       }
-      launch_join(jc, gc, true, s2);
-      if (ntree) HIPCHK(hipEventRecord(c->ev_join, s2));
     }
-    if (ntree) {
-      ja.ntasks = ntree;
-      launch_join(ja, gt, false, s);
-    }
-    if (ncyc && ntree) HIPCHK(hipStreamWaitEvent(s, c->ev_join, 0));
+    if (fork) HIPCHK(hipStreamWaitEvent(s, c->ev_join, 0));
     pend(K_JOIN, pa, 0.0, -1);
     HIPCHK(hipGetLastError());
     std::vector<JoinOut> jo(std::max<uint32_t>(nplans, 1));

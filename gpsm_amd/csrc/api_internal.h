@@ -80,6 +80,12 @@ enum BufId {
   B_FITEMS,      // filter superstep: (op, vertex range) pairs with candidates
   B_FNITEMS,     // ... their number, one counter per superstep
   B_CDESC,       // candidate-edge tables of reversed plan edges (counted again)
+  B_LDESC,       // candidate-edge tables whose lists are written
+  B_WDESC,       // last levels' tables counted from records
+  B_WCHUNK,      // ... chunks of 64 candidates before each
+  B_ADESC,       // tables of the level before (AggDesc)
+  B_ACHUNK,      // ... chunks before each
+  B_AGGS,        // their candidates' records (CetAgg)
   B_RFLAGS,      // refine rounds that removed a candidate, 4 per query
   B_COUNT_
 };

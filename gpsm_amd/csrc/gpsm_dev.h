@@ -67,6 +67,31 @@ struct CetDesc {
   // means no range is known (every entry is probed)
   uint32_t w_lo, w_hi;
   uint32_t pad;
+  // records of the last two levels' tables (CetAgg of candidate j at
+  // agg_base + j); ~0 for the other tables
+  uint64_t agg_base;
+};
+
+// What the join's last two levels need of one candidate's list, so that a
+// row counts and hashes its embeddings without walking the list.  term_u(v)
+// is tuple_term(u, v), L(j) the candidate's list.
+//   last level's table (bound vertex w):   s = sum over L(j) of term_w(v)
+//   the level before (bound vertex y, list L_y(j)): s the same with term_y and
+//     w's parent is y:          a = sum of |L_w(v)|,  b = sum of term_y(v) * s_w(v)
+//     w's parent is y's parent: a = |L_y(j) in C(w)|, b = sum of term_y(v) * term_w(v) over them
+struct CetAgg {
+  unsigned long long s, a, b;
+  uint32_t off, len;  // the list inside its table (off: tables with lists only)
+};
+
+enum AggMode : uint32_t { AGG_SUM = 0, AGG_SIBLING = 1, AGG_CHAIN = 2 };
+
+// One table of the level before the last: the inputs of its records.
+struct AggDesc {
+  uint64_t off_base, list_base, agg_base;  // the table's
+  uint64_t w_agg_base;                     // the last table's records (AGG_CHAIN)
+  uint32_t ncand, mode;
+  uint32_t y_slot, y_qid, w_slot, w_qid;
 };
 
 // Join plan of one query: vertex order and, per level, how to extend.
@@ -75,6 +100,9 @@ struct JoinPlan {
   uint32_t vbase;             // slot of query vertex 0
   uint32_t first_cet;         // CetDesc index of the first table (pi0 -> pi1)
   uint32_t nback_total;
+  // levels the join counts from CetAgg records instead of enumerating them:
+  // the last agg levels (0, 1 or 2), none of which has a back position
+  uint32_t agg;
   // injectivity checks of level k: positions c < k whose query vertex has
   // the label of position k's, other than the parent and the back
   // positions.  A candidate of another label cannot equal the vertex bound
@@ -87,14 +115,16 @@ struct JoinPlan {
   uint8_t backs[MAXQ * MAXQ / 2];  // back positions (excluding the parent)
 };
 
-// A slice of the first table of one query: rows [lo, hi).
-// Rows first, first + stride, ..., (count of them) of one query's first
-// table.  A query's tasks interleave its rows, so the rows of hub
-// candidates (the table's first rows on a power-law graph) are spread over
-// all of its tasks instead of making the first task the longest.
+// A slice of one query's first table: chunks first, first + stride, ... of
+// 2^shift consecutive rows, count rows in all.  A query's tasks interleave
+// its chunks, so the rows of hub candidates (the table's first rows on a
+// power-law graph) are spread over all of its tasks instead of making the
+// first task the longest.  Row r of the task is row task_row(t, r) of the
+// table.
 struct JoinTask {
   uint32_t query;
   uint32_t stride;
+  uint32_t shift, pad;
   uint64_t first, count;
 };
 

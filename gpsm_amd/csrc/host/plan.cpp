@@ -637,6 +637,22 @@ double analytic_cost(const PlanContext& c, const OrderPlan& plan) {
   return s.cost;
 }
 
+double analytic_cost_upto(const PlanContext& c, const OrderPlan& plan, uint32_t last) {
+  PlanCost s;
+  if (!cost_start(c, plan.order.data(), s)) return 0.0;
+  double cost = (double)(*c.cet_size)[s.plan.first_edge];
+  std::vector<float> f;
+  while (s.k <= last && s.k < c.q->n) {
+    cost += s.rows * examine_factor(s, s.k);
+    if (s.done) break;
+    f.clear();
+    cost_emit(s, f);
+    const float y = f[27];
+    cost_consume(s, &y);
+  }
+  return cost;
+}
+
 int learned_plans(const std::vector<const PlanContext*>& qs, PredictFn predict, void* user, uint64_t big,
                   std::vector<OrderPlan>& out, std::vector<uint32_t>* chosen, std::vector<double>* cost,
                   const std::vector<uint8_t>* rank) {

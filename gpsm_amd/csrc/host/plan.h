@@ -190,5 +190,9 @@ int learned_plans(const std::vector<const PlanContext*>& qs, PredictFn predict, 
 // the expand edge / |C(parent)|) + the log densities of its back edges
 // (feature 27 of step_features).  Used to size the join's tasks.
 double analytic_cost(const PlanContext& c, const OrderPlan& plan);
+// The part of it up to position last: the first table's rows and the
+// candidates examined for positions 2 .. last (what the join enumerates of a
+// plan whose later levels are counted from records).
+double analytic_cost_upto(const PlanContext& c, const OrderPlan& plan, uint32_t last);
 
 }  // namespace gpsm

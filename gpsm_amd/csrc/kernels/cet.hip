@@ -268,6 +268,208 @@ __global__ void __launch_bounds__(256) cet_write_kernel(const uint32_t* __restri
   if (stats) flush_tally(tl, stats);
 }
 
+// cell[seg] += x for every lane, lanes of one seg consecutive (seg
+// non-decreasing over the wave's lanes, all active): one wave scan, then two
+// LDS atomics per segment boundary, whatever the segments' lengths.
+__device__ __forceinline__ void seg_add(unsigned long long* cell, uint32_t seg, bool tail, uint32_t next,
+                                        unsigned long long x) {
+  const unsigned long long incl = wave_incl_scan64(x);
+  if (tail) {
+    atomicAdd(&cell[seg], incl);
+    if (next != WAVE) atomicAdd(&cell[next], 0ull - incl);
+  }
+}
+
+// Records of the last join levels' tables: one wave per 64 candidates of
+// C(x) with a stride, flattened over their adjacency as in cet_count, but an
+// entry in C(w) adds its hash term (computed here, about 30 VALU
+// instructions, only in lanes with a hit) to its candidate's sum and is not
+// written: the join reads 32 bytes per candidate instead of 12 per list
+// entry.  Bound by the random probes of C(w), like cet_count.
+struct SumLds {
+  CetLds c;
+  unsigned long long s[WAVE];
+};
+
+__global__ void __launch_bounds__(256) cet_sum_kernel(const uint32_t* __restrict__ row,
+                                                      const uint32_t* __restrict__ col,
+                                                      const uint32_t* __restrict__ ckey,
+                                                      const uint32_t* __restrict__ bitmaps, uint32_t W,
+                                                      const uint32_t* __restrict__ clist,
+                                                      const CetDesc* __restrict__ descs,
+                                                      const uint32_t* __restrict__ chunk_base, uint32_t ndesc,
+                                                      CetAgg* __restrict__ aggs,
+                                                      unsigned long long* __restrict__ stats) {
+  __shared__ SumLds lds[4];
+  CetTally tl;
+  SumLds& L = lds[threadIdx.x / WAVE];
+  const uint32_t lane = lane_id();
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  const uint32_t nwaves = (gridDim.x * blockDim.x) / WAVE;
+  const uint32_t nitems = chunk_base[ndesc];
+  for (uint32_t it = wave; it < nitems; it += nwaves) {
+    const uint32_t di = uniform(seg_search(chunk_base, ndesc + 1, it));
+    const CetDesc d = descs[di];
+    const uint32_t j = it - chunk_base[di], nch = chunk_base[di + 1] - chunk_base[di];
+    bool mine;
+    uint32_t D;
+    L.s[lane] = 0;
+    load_chunk(row, clist, d, j, nch, L.c, mine, D);
+    tl.cand += mine;
+    const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
+    const uint32_t wlo = d.w_hi ? d.w_lo : 0u, whi = d.w_hi ? d.w_hi : ~0u;
+    for (uint32_t f = 0; f < D; f += WAVE * CET_UNROLL) {
+      uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], ks[CET_UNROLL], pw[CET_UNROLL];
+#pragma unroll
+      for (int u = 0; u < CET_UNROLL; ++u) cis[u] = f + u * WAVE + lane;
+      halving_search<CET_UNROLL>(L.c.pre, WAVE, cis);  // an index past D falls in the last candidate
+#pragma unroll
+      for (int u = 0; u < CET_UNROLL; ++u) {
+        const uint32_t g = f + u * WAVE + lane;
+        const uint32_t e = L.c.off[cis[u]] + (g - L.c.pre[cis[u]]);
+        mvs[u] = g < D ? col[e] : 0u;
+        ks[u] = g < D ? ckey[e] : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < CET_UNROLL; ++u) {
+        const bool in = f + u * WAVE + lane < D && ks[u] >= wlo && ks[u] <= whi;
+        pw[u] = in ? bm_w[mvs[u] >> 5] >> (mvs[u] & 31) : 0u;
+        if (stats) {
+          tl.ent += f + u * WAVE + lane < D;
+          tl.probe += in;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < CET_UNROLL; ++u) {
+        const bool hit = (pw[u] & 1u) != 0;
+        const unsigned long long hm = __ballot(hit);
+        if (!hm) continue;  // the whole wave
+        const uint32_t fu = f + u * WAVE, ci = cis[u];
+        const uint32_t next = __shfl_down(ci, 1, WAVE);
+        const bool tail = lane == WAVE - 1 || next != ci;
+        seg_add(L.s, ci, tail, lane == WAVE - 1 ? (uint32_t)WAVE : next, hit ? tuple_term(d.term_qid, mvs[u]) : 0ull);
+        if (tail) {
+          const uint32_t seg_lo = L.c.pre[ci] > fu ? L.c.pre[ci] - fu : 0u;
+          if (seg_lo < WAVE) {
+            const unsigned long long seg = (~0ULL << seg_lo) & (~0ULL >> (WAVE - 1 - lane));
+            atomicAdd(&L.c.cnt[ci], (uint32_t)__popcll(hm & seg));
+          }
+        }
+      }
+    }
+    wave_sync();
+    if (mine) {
+      CetAgg r;
+      r.s = L.s[lane];
+      r.a = r.b = 0;
+      r.off = 0;
+      r.len = L.c.cnt[lane];
+      aggs[d.agg_base + cand_index(j, nch, lane)] = r;
+    }
+    wave_sync();
+  }
+  if (stats) flush_tally(tl, stats);
+}
+
+// Records of the level before the last: one wave per 64 candidates with a
+// stride, flattened over their lists.  A list entry costs its hash term and,
+// where w's parent is the entry itself (AGG_CHAIN), its rank in C(y) and its
+// 32-byte record of the last table.
+constexpr int AGG_UNROLL = 2;  // list entries in flight per lane
+
+struct AggLds {
+  uint32_t pre[WAVE];
+  uint32_t off[WAVE];
+  unsigned long long s[WAVE], a[WAVE], b[WAVE];
+};
+
+__global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict__ bitmaps,
+                                                      const uint32_t* __restrict__ bprefix, uint32_t W, uint32_t NB,
+                                                      const AggDesc* __restrict__ descs, uint32_t ndesc,
+                                                      const uint32_t* __restrict__ chunk_base,
+                                                      const uint32_t* __restrict__ offsets,
+                                                      const uint32_t* __restrict__ lists, CetAgg* aggs) {
+  __shared__ AggLds lds[4];
+  AggLds& L = lds[threadIdx.x / WAVE];
+  const uint32_t lane = lane_id();
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  const uint32_t nwaves = (gridDim.x * blockDim.x) / WAVE;
+  const uint32_t nitems = chunk_base[ndesc];
+  for (uint32_t it = wave; it < nitems; it += nwaves) {
+    const uint32_t di = uniform(seg_search(chunk_base, ndesc + 1, it));
+    const AggDesc d = descs[di];
+    const uint32_t j = it - chunk_base[di], nch = chunk_base[di + 1] - chunk_base[di];
+    const uint32_t ci = cand_index(j, nch, lane);
+    const bool mine = ci < d.ncand;
+    const uint32_t off = mine ? offsets[d.off_base + ci] : 0u;
+    const uint32_t len = mine ? offsets[d.off_base + ci + 1] - off : 0u;
+    const uint32_t incl = wave_incl_scan(len);
+    const uint32_t D = uniform(__shfl(incl, WAVE - 1, WAVE));
+    L.pre[lane] = incl - len;
+    L.off[lane] = off;
+    L.s[lane] = L.a[lane] = L.b[lane] = 0;
+    wave_sync();
+    const uint32_t* bm_y = bitmaps + (size_t)d.y_slot * W;
+    const uint32_t* bp_y = bprefix + (size_t)d.y_slot * NB;
+    const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
+    const uint32_t* lst = lists + d.list_base;
+    for (uint32_t f = 0; f < D; f += WAVE * AGG_UNROLL) {
+      uint32_t cis[AGG_UNROLL], v[AGG_UNROLL];
+      unsigned long long t[AGG_UNROLL], xa[AGG_UNROLL], xb[AGG_UNROLL];
+#pragma unroll
+      for (int u = 0; u < AGG_UNROLL; ++u) cis[u] = f + u * WAVE + lane;
+      halving_search<AGG_UNROLL>(L.pre, WAVE, cis);
+#pragma unroll
+      for (int u = 0; u < AGG_UNROLL; ++u) {
+        // an index past D (in the last candidate) reads no entry and adds
+        // nothing; vertex 0 stands in for it (C(y) is not empty, so rank 0
+        // has a record)
+        const uint32_t g = f + u * WAVE + lane;
+        v[u] = g < D ? lst[L.off[cis[u]] + (g - L.pre[cis[u]])] : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < AGG_UNROLL; ++u) {
+        const bool in = f + u * WAVE + lane < D;
+        xa[u] = xb[u] = 0;
+        if (d.mode == AGG_CHAIN) {  // uniform
+          const CetAgg r = aggs[d.w_agg_base + rank_of(bm_y, bp_y, v[u])];
+          xa[u] = in ? r.len : 0u;
+          xb[u] = in ? r.s : 0ull;
+        } else if (d.mode == AGG_SIBLING) {
+          const bool hit = in && bit_of(bm_w, v[u]);
+          xa[u] = hit;
+          xb[u] = hit ? tuple_term(d.w_qid, v[u]) : 0ull;
+        }
+        t[u] = in ? tuple_term(d.y_qid, v[u]) : 0ull;
+        xb[u] *= t[u];
+      }
+#pragma unroll
+      for (int u = 0; u < AGG_UNROLL; ++u) {
+        if (f + u * WAVE >= D) continue;  // uniform
+        const uint32_t next = __shfl_down(cis[u], 1, WAVE);
+        const bool tail = lane == WAVE - 1 || next != cis[u];
+        const uint32_t nx = lane == WAVE - 1 ? (uint32_t)WAVE : next;
+        seg_add(L.s, cis[u], tail, nx, t[u]);
+        if (d.mode != AGG_SUM) {
+          seg_add(L.a, cis[u], tail, nx, xa[u]);
+          seg_add(L.b, cis[u], tail, nx, xb[u]);
+        }
+      }
+    }
+    wave_sync();
+    if (mine) {
+      CetAgg r;
+      r.s = L.s[lane];
+      r.a = L.a[lane];
+      r.b = L.b[lane];
+      r.off = off;
+      r.len = len;
+      aggs[d.agg_base + ci] = r;
+    }
+    wave_sync();
+  }
+}
+
 // One thread per term: the table by a binary search over the term ranges.
 __global__ void __launch_bounds__(256) cet_terms_kernel(const uint32_t* __restrict__ lists,
                                                         const CetDesc* __restrict__ descs,
@@ -329,6 +531,22 @@ void launch_cet_terms(const uint32_t* lists, const CetDesc* descs, const uint32_
   if (grid > 16384) grid = 16384;
   hipLaunchKernelGGL(cet_terms_kernel, dim3((uint32_t)grid), dim3(256), 0, s, lists, descs, term_desc, term_start,
                      nterm_desc, nterms, terms);
+}
+
+void launch_cet_sums(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, const CetDesc* descs,
+                     uint32_t ndesc, const uint32_t* chunk_base, CetAgg* aggs, uint32_t grid, hipStream_t s,
+                     unsigned long long* stats) {
+  if (!ndesc) return;
+  hipLaunchKernelGGL(cet_sum_kernel, dim3(grid), dim3(256), 0, s, g.row, g.col, g.ckey, bitmaps, g.W, clist, descs,
+                     chunk_base, ndesc, aggs, stats);
+}
+
+void launch_cet_aggs(const uint32_t* bitmaps, const uint32_t* bprefix, uint32_t W, uint32_t NB, const AggDesc* descs,
+                     uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
+                     CetAgg* aggs, uint32_t grid, hipStream_t s) {
+  if (!ndesc) return;
+  hipLaunchKernelGGL(cet_agg_kernel, dim3(grid), dim3(256), 0, s, bitmaps, bprefix, W, NB, descs, ndesc, chunk_base,
+                     offsets, lists, aggs);
 }
 
 void launch_cet_write(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, const CetDesc* descs,

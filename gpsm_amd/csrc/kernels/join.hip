@@ -16,12 +16,20 @@
 //    consecutive (row, candidate) pairs, so rows of any fan-out share lanes;
 //  * join-mode edges become edge-membership checks (binary search in the
 //    shorter adjacency) and injectivity is checked in the same pass;
-//  * the last level is never written: each embedding adds its tuple hash
-//    and 1 to the counters.  The tuple hash is a product of one factor per
-//    (query vertex, image) pair, so a row carries the product of its
-//    factors and an embedding costs one multiply by its last factor
-//    (precomputed per list entry); a wave expanding one long row sums the
-//    factors of its valid candidates and multiplies once per row.
+//  * the tuple hash is a product of one factor per (query vertex, image)
+//    pair, so a row carries the product of its factors, and the embeddings
+//    that extend a row hash to that product times a sum of last factors;
+//  * where the last one or two vertices have no back edges and no tuples are
+//    wanted, their levels are not enumerated: a row's embeddings are counted
+//    and hashed from sums kept per candidate (CetAgg), with the injectivity
+//    checks as exact corrections (count_last_level, count_last_two).  On the
+//    245-query mix on the 1M Chung-Lu graph (4.57e11 candidates of the last
+//    levels) the join went from 437 to 9.0 ms and the batch from 467 to 32.6
+//    ms, on one 4-vertex walk of 7e8 embeddings from 3.2 to 0.06 ms;
+//  * otherwise the last level is enumerated but never written: an embedding
+//    costs one multiply by its last factor (precomputed per list entry); a
+//    wave expanding one long row sums the factors of its valid candidates
+//    and multiplies once per row.
 #include <algorithm>
 #include <type_traits>
 
@@ -45,15 +53,6 @@ constexpr int TREE_UNROLL = 3;
 // faster on the R-MAT 22 shapes; 192 is 2% slower on the mix.
 constexpr uint32_t LONG_ROW = 96;
 static_assert((uint64_t)WROWS * LONG_ROW < (1u << 23) && WROWS < 512, "packed scan of short spans and long flags");
-
-__device__ __forceinline__ uint32_t rank_of(const uint32_t* __restrict__ bm, const uint32_t* __restrict__ bp,
-                                            uint32_t x) {
-  const uint32_t blk = x >> 8;
-  uint32_t r = bp[blk];
-  const uint32_t w0 = blk * 8, wx = x >> 5;
-  for (uint32_t w = w0; w < wx; ++w) r += __popc(bm[w]);
-  return r + __popc(bm[wx] & ((1u << (x & 31)) - 1u));
-}
 
 // Edge {a, b}: one bit of a hub's adjacency bitmap when either end is a hub,
 // else a binary search in the shorter of the two (short) adjacency lists.
@@ -123,6 +122,11 @@ __device__ __forceinline__ void back_edges_of_row(const JoinArgs& a, const JoinP
   }
 }
 
+// Row r of a task as a row of its query's first table.
+__device__ __forceinline__ uint64_t task_row(const JoinTask& t, uint64_t r) {
+  return (((r >> t.shift) * t.stride + t.first) << t.shift) | (r & ((1u << t.shift) - 1u));
+}
+
 struct JoinShared {
   uint32_t pre[WROWS + 1];
   uint32_t delta[WROWS];  // list position of a row's candidate g is delta[row] + g
@@ -132,7 +136,7 @@ struct JoinShared {
   unsigned long long lrows[MAXQ];
   unsigned long long lwork[MAXQ];
   uint32_t task, k, abort;
-  unsigned long long red[4];
+  unsigned long long red[4], agg[4][3];
   // last level: the window's long rows (row, list start, candidates) and
   // the candidates they hold
   uint32_t lrow[WROWS], lst[WROWS], lub[WROWS];
@@ -140,16 +144,248 @@ struct JoinShared {
   // followed by the row window: val[c * WROWS + r], c < qmax
 };
 
+// A thread's share of the work and rows of the levels counted from records
+// (counted, not enumerated): examined candidates and valid rows of the level
+// before the last (two levels from records only), candidates of the last.
+struct AggWork {
+  unsigned long long work_y, rows_y, work_w;
+};
+
+// Adds the workgroup's shares to the task's and the query's counters and
+// clears them; checks the work budget.  Contains __syncthreads.
+__device__ __forceinline__ void flush_agg_work(const JoinArgs& a, const JoinPlan& P, JoinShared& S, uint32_t query,
+                                               AggWork& aw) {
+  const uint32_t w = threadIdx.x / WAVE;
+  const unsigned long long v[3] = {wave_sum64(aw.work_y), wave_sum64(aw.rows_y), wave_sum64(aw.work_w)};
+  aw = {0, 0, 0};
+  __syncthreads();
+  if (lane_id() == 0)
+    for (int i = 0; i < 3; ++i) S.agg[w][i] = v[i];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t[3] = {0, 0, 0};
+    for (uint32_t x = 0; x < WROWS / WAVE; ++x)
+      for (int i = 0; i < 3; ++i) t[i] += S.agg[x][i];
+    const uint32_t wl = P.q - 1;
+    if (P.agg == 2) {
+      S.lwork[wl - 1] += t[0];
+      S.lrows[wl - 1] += t[1];
+    }
+    S.lwork[wl] += t[2];
+    const unsigned long long done = t[0] + t[2];
+    if (done) {
+      const unsigned long long before = atomicAdd(&a.out[query].work, done);
+      if (a.budget && before + done > a.budget) {
+        a.out[query].aborted = 1;
+        S.abort = 1;
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ CetAgg agg_of(const JoinArgs& a, const CetDesc& d, uint32_t x) {
+  return a.aggs[d.agg_base + rank_of(a.bitmaps + (size_t)d.x_slot * a.W, a.bprefix + (size_t)d.x_slot * a.NB, x)];
+}
+
+// Whether u is in the candidate-edge list of mu in a table whose bound
+// vertex has candidate set `slot`: u in C(slot) and {mu, u} an edge.
+template <bool BYTES>
+__device__ __forceinline__ bool in_list(const JoinArgs& a, uint32_t slot, uint32_t mu, uint32_t u,
+                                        unsigned long long& bytes) {
+  if (!bit_of(a.bitmaps + (size_t)slot * a.W, u)) return false;
+  return has_edge<BYTES>(a.row, a.col, a.hub_of, a.hub_bits, a.W, mu, u, bytes);
+}
+
+// The embeddings of a window of rows that bind all but the last vertex w
+// (which has no back position): a row has |L| of them, and their hash is the
+// row's product times the sum of the list's terms, less the bound vertices
+// that sit in the list (the injectivity checks of w).  One 32-byte record
+// per row stands for its whole list.
+template <bool BYTES>
+__device__ __forceinline__ void count_last_level(const JoinArgs& a, const JoinPlan& P, const JoinShared& S,
+                                                 const uint32_t* val, uint32_t nw, unsigned long long& my_cnt,
+                                                 unsigned long long& my_hash, unsigned long long& bytes,
+                                                 AggWork& aw) {
+  const uint32_t tid = threadIdx.x, w = P.q - 1;
+  if (tid >= nw) return;
+  const CetDesc& d = a.cets[P.cet[w]];
+  const uint32_t qid = P.order[w];
+  const uint32_t mu = val[P.par[w] * WROWS + tid];
+  const CetAgg r = agg_of(a, d, mu);
+  if (BYTES) bytes += 4 + 4 * (((mu >> 5) & 7) + 1) + sizeof(CetAgg);
+  unsigned long long len = r.len, s = r.s;
+  for (uint64_t m = P.inj[w]; m; m &= m - 1) {
+    const uint32_t u = val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + tid];
+    if (in_list<BYTES>(a, d.w_slot, mu, u, bytes)) {
+      --len;
+      s -= tuple_term(qid, u);
+    }
+  }
+  my_cnt += len;
+  my_hash += S.srow[tid] * s;
+  aw.work_w += r.len;
+}
+
+// The embeddings of a window of rows that bind all but the last two
+// vertices y (position q - 2) and w, neither with a back position.  For a
+// row, with L_y the list of y's parent and L_w(v) that of w's:
+//   w's parent is y:  sum over v in L_y of |L_w(v)| (CetAgg a, b)
+//   otherwise:        |L_y| * |L_w|
+// less, by injectivity (vertices of one label only), exactly:
+//   bound vertices in L_y (one record of the last table each in the first
+//   case), bound vertices in L_w (in the first case y's parent is in every
+//   L_w(v); another bound vertex u is in those of the v adjacent to u), and
+//   pairs v = w of L_y and L_w (a record where the parents are the same).
+// Only the v of L_y adjacent to one other vertex (u, or w's parent) have no
+// record: they are enumerated from the shorter of L_y and that vertex's
+// adjacency.  A row costs O(1) records instead of |L_y| * |L_w| candidates.
+template <bool BYTES>
+__device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan& P, JoinShared& S,
+                                               const uint32_t* val, uint32_t nw, unsigned long long& my_cnt,
+                                               unsigned long long& my_hash, unsigned long long& bytes, AggWork& aw) {
+  const uint32_t tid = threadIdx.x, lane = lane_id();
+  const uint32_t w = P.q - 1, y = w - 1, py = P.par[y], pw = P.par[w];
+  const CetDesc& dy = a.cets[P.cet[y]];
+  const CetDesc& dw = a.cets[P.cet[w]];
+  const uint32_t qy = P.order[y], qw = P.order[w];
+  const uint64_t iy = P.inj[y], iw = P.inj[w];
+  const bool chain = pw == y, sibling = pw == py;
+  const uint32_t* bm_w = a.bitmaps + (size_t)dw.w_slot * a.W;
+  uint32_t mu = 0, st_y = 0, len_y = 0;
+  if (tid < nw) {
+    mu = val[py * WROWS + tid];
+    const CetAgg r = agg_of(a, dy, mu);
+    if (BYTES) bytes += 4 + 4 * (((mu >> 5) & 7) + 1) + sizeof(CetAgg);
+    st_y = r.off;
+    len_y = r.len;
+    unsigned long long n = r.len, ty = r.s, ra = r.a, rb = r.b;
+    for (uint64_t m = iy; m; m &= m - 1) {
+      const uint32_t u = val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + tid];
+      if (!in_list<BYTES>(a, dy.w_slot, mu, u, bytes)) continue;
+      const unsigned long long t = tuple_term(qy, u);
+      --n;
+      ty -= t;
+      if (chain) {
+        const CetAgg x = agg_of(a, dw, u);
+        if (BYTES) bytes += 4 + 4 * (((u >> 5) & 7) + 1) + sizeof(CetAgg);
+        ra -= x.len;
+        rb -= t * x.s;
+      } else if (sibling && bit_of(bm_w, u)) {
+        --ra;
+        rb -= t * tuple_term(qw, u);
+      }
+    }
+    unsigned long long cnt, hash;
+    if (chain) {
+      aw.work_w += ra;
+      cnt = ra;
+      hash = rb;
+      if (((iw >> py) & 1) && bit_of(bm_w, mu)) {  // y's parent is in every list
+        cnt -= n;
+        hash -= tuple_term(qw, mu) * ty;
+      }
+    } else {
+      const uint32_t mw = val[pw * WROWS + tid];
+      const CetAgg x = agg_of(a, dw, mw);
+      if (BYTES) bytes += 4 + 4 * (((mw >> 5) & 7) + 1) + sizeof(CetAgg);
+      aw.work_w += n * x.len;
+      unsigned long long lw = x.len, sw = x.s;
+      for (uint64_t m = iw & ~(1ull << y); m; m &= m - 1) {
+        const uint32_t u = val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + tid];
+        if (in_list<BYTES>(a, dw.w_slot, mw, u, bytes)) {
+          --lw;
+          sw -= tuple_term(qw, u);
+        }
+      }
+      cnt = n * lw;
+      hash = ty * sw;
+      if (sibling && ((iw >> y) & 1)) {
+        cnt -= ra;
+        hash -= rb;
+      }
+    }
+    aw.work_y += len_y;
+    aw.rows_y += n;
+    my_cnt += cnt;
+    my_hash += S.srow[tid] * hash;
+  }
+  // The v of L_y adjacent to one other vertex o per row: in the first case
+  // the bound vertices of w's label except y's parent, one position at a
+  // time, else w's parent (v also in C(w)) when y has w's label.
+  uint64_t pos = chain ? iw & ~(1ull << py) : !sibling && ((iw >> y) & 1) ? 1ull << pw : 0ull;
+  for (; pos; pos &= pos - 1) {  // uniform
+    const uint32_t c = (uint32_t)(__ffsll((long long)pos) - 1);
+    uint32_t o = 0, len = 0, st = 0, side = 0;
+    if (tid < nw && len_y) {
+      o = val[c * WROWS + tid];
+      if (!chain || bit_of(bm_w, o)) {
+        // the cheaper side: L_y against o's hub bitmap or adjacency, or o's
+        // adjacency against C(y) and the edge to y's parent (a bit test about
+        // 2, a binary search about 8 list reads)
+        const uint32_t o0 = a.row[o], od = a.row[o + 1] - o0;
+        const uint64_t c0 = (uint64_t)len_y * (a.hub_of[o] != ~0u ? 2 : 8);
+        const uint64_t c1 = (uint64_t)od * (a.hub_of[mu] != ~0u ? 2 : 8);
+        side = c1 < c0;
+        len = side ? od : len_y;
+        st = side ? o0 : st_y;
+        if (BYTES) bytes += 16;
+      }
+    }
+    __syncthreads();  // the previous position's reads of S are done
+    uint32_t T;
+    const uint32_t ex = block_excl_scan(len, S.tmp, &T);
+    S.pre[tid] = tid < nw ? ex : T;
+    S.delta[tid] = st - ex;
+    S.lst[tid] = o;
+    S.lub[tid] = mu;
+    S.lrow[tid] = side;
+    __syncthreads();
+    constexpr int U = 2;
+    for (uint32_t f = 0; f < T; f += WROWS * U) {
+      const uint32_t g0 = f + (tid / WAVE) * (WAVE * U);
+      if (g0 >= T) break;  // the whole wave; no barrier below
+      uint32_t is[U], v[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) is[u] = min(g0 + u * WAVE + lane, T - 1);
+      halving_search<U>(S.pre, uniform(nw), is);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t e = S.delta[is[u]] + min(g0 + u * WAVE + lane, T - 1);
+        v[u] = S.lrow[is[u]] ? a.col[e] : a.lists[dy.list_base + e];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t i = is[u];
+        bool ok = g0 + u * WAVE + lane < T;
+        if (BYTES && ok) bytes += 4;
+        for (uint64_t m = iy; m; m &= m - 1) ok &= val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + i] != v[u];
+        if (ok && !chain) ok = bit_of(bm_w, v[u]);
+        if (ok) {
+          const bool sd = S.lrow[i] != 0;
+          if (sd) ok = bit_of(a.bitmaps + (size_t)dy.w_slot * a.W, v[u]);
+          if (ok) ok = has_edge<BYTES>(a.row, a.col, a.hub_of, a.hub_bits, a.W, v[u], sd ? S.lub[i] : S.lst[i], bytes);
+        }
+        if (ok) {
+          --my_cnt;
+          my_hash -= S.srow[i] * tuple_term(qy, v[u]) * tuple_term(qw, chain ? S.lst[i] : v[u]);
+        }
+      }
+    }
+  }
+}
+
 // BYTES: account the algorithmic bytes read and written (JoinOut::bytes);
-// the kernel without it is the one timed.  CYCLIC: the plans of the launch
-// have back edges (join-mode edges); a tree plan has none, and its kernel
-// holds no back-edge code.  The two are separate kernels with their own
-// register budgets (join_tree_kernel, join_cyclic_kernel below): the
-// cyclic one's batched back-edge tests need more registers, and sharing
-// them made the tree plans' join 1.2-1.6x slower (spills at seven waves
-// per SIMD, or fewer waves).
-template <bool BYTES, bool CYCLIC>
+// the kernel without it is the one timed.  KIND: the plans of the launch, each
+// kind a kernel with its own register budget.  Tree plans have no back edges
+// (join-mode edges) and their kernels no back-edge code: sharing the cyclic
+// kernel's registers made them 1.2-1.6x slower.  The kernels that count the
+// last levels from records hold no code that enumerates them: one cyclic
+// kernel with both spilled 40 registers and ran R-MAT 18 cycles and cliques
+// 1.2x slower than the two apart.
+template <bool BYTES, JoinKind KIND>
 __device__ __forceinline__ void join_body(const JoinArgs& a) {
+  constexpr bool CYCLIC = KIND == JOIN_CYCLIC || KIND == JOIN_CYCLIC_ENUM;
+  constexpr bool COUNTED = KIND == JOIN_TREE || KIND == JOIN_CYCLIC;  // every plan of the launch has agg > 0 (or q = 2)
   constexpr int XU = CYCLIC ? EXP_UNROLL : TREE_UNROLL;
   extern __shared__ unsigned char lds_raw[];
   JoinShared& S = *reinterpret_cast<JoinShared*>(lds_raw);
@@ -171,6 +407,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
     const uint32_t* ls0 = a.lists + d0.list_base;
     unsigned long long my_cnt = 0, my_hash = 0, my_bytes = 0;
     unsigned long long wave_cnt = 0;  // last-level embeddings of this wave (uniform)
+    AggWork aw = {0, 0, 0};           // this thread's share of the levels counted from records
 
     if (tid < MAXQ) {
       S.lrows[tid] = 0;
@@ -206,7 +443,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
     if (q == 2) {
       // the first table is the embedding set
       for (uint64_t i = tid; i < task.count && !S.abort; i += blockDim.x) {
-        const uint64_t e = task.first + i * task.stride;
+        const uint64_t e = task_row(task, i);
         const uint32_t j = seg_search(off0, d0.ncand + 1, (uint32_t)e);
         const uint32_t mu = cl0[j], mv = ls0[e];
         my_hash += tuple_term(P.order[0], mu) * tuple_term(P.order[1], mv);
@@ -233,7 +470,9 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
         const uint32_t r0 = S.cur_row[k];
         const uint32_t nw = min(WROWS, S.fill[k] - r0);
         const uint32_t nk = k + 1;              // level being produced
-        const bool final = nk == q - 1;
+        // this window's embeddings come from the records of the last levels
+        const bool agg = COUNTED && nk + P.agg == q;
+        const bool final = !COUNTED && nk == q - 1;
         const uint32_t p = P.par[nk];
         const CetDesc dn = a.cets[P.cet[nk]];
         const uint32_t* bm_x = a.bitmaps + (size_t)dn.x_slot * a.W;
@@ -252,7 +491,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
         if (tid < nw) {
           const uint32_t r = r0 + tid;
           if (k == 1) {
-            const uint64_t e = task.first + (uint64_t)r * task.stride;
+            const uint64_t e = task_row(task, r);
             const uint32_t j = seg_search(off0, d0.ncand + 1, (uint32_t)e);
             val[0 * WROWS + tid] = cl0[j];
             val[1 * WROWS + tid] = ls0[e];
@@ -262,6 +501,25 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
           unsigned long long s = 1;
           for (uint32_t c = 0; c <= k; ++c) s *= tuple_term(P.order[c], val[c * WROWS + tid]);
           S.srow[tid] = s;
+          if (BYTES && agg) my_bytes += k == 1 ? 8 : 4 * (k + 1);
+        }
+        if constexpr (COUNTED) {
+          if (agg) {  // uniform
+            if (P.agg == 1) count_last_level<BYTES>(a, P, S, val, nw, my_cnt, my_hash, my_bytes, aw);
+            else count_last_two<BYTES>(a, P, S, val, nw, my_cnt, my_hash, my_bytes, aw);
+            // with a budget every window's work is checked, without one the
+            // task's work is added once at its end
+            if (a.budget) flush_agg_work(a, P, S, task.query, aw);
+            __syncthreads();
+            if (tid == 0) {
+              S.cur_row[k] = r0 + nw;
+              S.cur_cand[k] = 0;
+            }
+            __syncthreads();
+            continue;
+          }
+        }
+        if (tid < nw) {
           // row values, rank index (prefix + words) and the offset pair
           if (BYTES) my_bytes += (k == 1 ? 8 : 4 * (k + 1)) + 4 + 4 * (((val[p * WROWS + tid] >> 5) & 7) + 1) + 8;
           const uint32_t j = rank_of(bm_x, bp_x, val[p * WROWS + tid]);
@@ -433,7 +691,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
           }
           return f;
         };
-        if (final && nlong) {
+        if (!COUNTED && final && nlong) {
           // wave-per-row pass over the window's long rows: lanes take
           // consecutive list entries of one row, whose values are uniform
           const unsigned long long* trm_n = a.terms + dn.term_base;
@@ -495,7 +753,9 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
             my_hash += srow * rsum;
           }
         }
-        const uint32_t f = final ? expand(std::true_type{}) : expand(std::false_type{});
+        uint32_t f;
+        if constexpr (COUNTED) f = expand(std::false_type{});
+        else f = final ? expand(std::true_type{}) : expand(std::false_type{});
         if (final) __syncthreads();  // long_cands complete
         if (!final && tid == 0) S.lrows[nk] += S.fill[nk];
         // advance level k's cursor past what was expanded
@@ -529,6 +789,10 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
     }
 
     // flush this task's counters
+    if (COUNTED && P.agg) {  // uniform
+      flush_agg_work(a, P, S, task.query, aw);
+      __syncthreads();
+    }
     my_cnt = wave_sum64(my_cnt) + wave_cnt;
     my_hash = wave_sum64(my_hash);
     __syncthreads();
@@ -565,29 +829,48 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
   }
 }
 
-// Eight waves per SIMD for tree plans, three candidates per thread: 64
-// VGPRs with 4 spilled.  On the 1M Chung-Lu mix (join per batch, learned
-// order) 438 ms, against 445 ms with four candidates at eight waves (7
-// spilled), 457 ms with four at seven waves (no spill), 452 ms with two at
-// eight and 483-571 ms with six or eight candidates at five to seven waves:
-// the waves in flight hide the list loads better than more loads per wave.
+// Plans counted from records: six waves per SIMD for tree plans (80 VGPRs, 10
+// spilled), five for cyclic ones (no spill).
+// Tree plans whose embeddings are enumerated: eight waves per SIMD, three
+// candidates per thread, 64 VGPRs with 4 spilled.  Enumerating the 1M
+// Chung-Lu mix (join per batch, learned order) took 438 ms, against 445 ms
+// with four candidates at eight waves (7 spilled), 457 ms with four at seven
+// waves (no spill), 452 ms with two at eight and 483-571 ms with six or eight
+// candidates at five to seven waves: the waves in flight hide the list loads
+// better than more loads per wave.
 // Five waves for cyclic plans, whose batched back-edge tests spill heavily
 // beyond (R-MAT 22 cycles and cliques 2.05 s per batch at five, 2.07 s at
 // six, 2.33 s at eight).
 template <bool BYTES>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) join_tree_kernel(JoinArgs a) {
-  join_body<BYTES, false>(a);
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) join_tree_kernel(JoinArgs a) {
+  join_body<BYTES, JOIN_TREE>(a);
+}
+
+template <bool BYTES>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) join_tree_enum_kernel(JoinArgs a) {
+  join_body<BYTES, JOIN_TREE_ENUM>(a);
 }
 
 template <bool BYTES>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) join_cyclic_kernel(JoinArgs a) {
-  join_body<BYTES, true>(a);
+  join_body<BYTES, JOIN_CYCLIC>(a);
 }
 
 template <bool BYTES>
-const void* join_fn(bool cyclic) {
-  return cyclic ? reinterpret_cast<const void*>(join_cyclic_kernel<BYTES>)
-                : reinterpret_cast<const void*>(join_tree_kernel<BYTES>);
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) join_cyclic_enum_kernel(JoinArgs a) {
+  join_body<BYTES, JOIN_CYCLIC_ENUM>(a);
+}
+
+typedef void (*JoinFn)(JoinArgs);
+
+template <bool BYTES>
+JoinFn join_fn(JoinKind kind) {
+  switch (kind) {
+    case JOIN_TREE: return join_tree_kernel<BYTES>;
+    case JOIN_TREE_ENUM: return join_tree_enum_kernel<BYTES>;
+    case JOIN_CYCLIC: return join_cyclic_kernel<BYTES>;
+    default: return join_cyclic_enum_kernel<BYTES>;
+  }
 }
 
 }  // namespace
@@ -605,9 +888,9 @@ size_t join_lds_bytes(uint32_t qmax) {
 }
 }  // namespace
 
-uint32_t join_resident_per_cu(uint32_t qmax, bool cyclic) {
+uint32_t join_resident_per_cu(uint32_t qmax, JoinKind kind) {
   const size_t lds = join_lds_bytes(std::max<uint32_t>(qmax, 2));
-  const void* fn = join_fn<false>(cyclic);
+  const void* fn = reinterpret_cast<const void*>(join_fn<false>(kind));
   if (lds > 65536) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, (int)WROWS, lds) != hipSuccess || per_cu < 1) {
@@ -617,17 +900,12 @@ uint32_t join_resident_per_cu(uint32_t qmax, bool cyclic) {
   return (uint32_t)per_cu;
 }
 
-void launch_join(const JoinArgs& a, uint32_t nwg, bool cyclic, hipStream_t s) {
+void launch_join(const JoinArgs& a, uint32_t nwg, JoinKind kind, hipStream_t s) {
   const size_t lds = join_lds_bytes(a.qmax);
-  const void* fn = a.count_bytes ? join_fn<true>(cyclic) : join_fn<false>(cyclic);
-  if (lds > 65536) (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (a.count_bytes) {
-    if (cyclic) hipLaunchKernelGGL(join_cyclic_kernel<true>, dim3(nwg), dim3(WROWS), lds, s, a);
-    else hipLaunchKernelGGL(join_tree_kernel<true>, dim3(nwg), dim3(WROWS), lds, s, a);
-  } else {
-    if (cyclic) hipLaunchKernelGGL(join_cyclic_kernel<false>, dim3(nwg), dim3(WROWS), lds, s, a);
-    else hipLaunchKernelGGL(join_tree_kernel<false>, dim3(nwg), dim3(WROWS), lds, s, a);
-  }
+  const JoinFn fn = a.count_bytes ? join_fn<true>(kind) : join_fn<false>(kind);
+  if (lds > 65536)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  hipLaunchKernelGGL(fn, dim3(nwg), dim3(WROWS), lds, s, a);
 }
 
 }  // namespace gpsm

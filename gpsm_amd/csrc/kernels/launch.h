@@ -125,6 +125,17 @@ void launch_cet_count(const DevGraph& g, const uint32_t* bitmaps, const uint32_t
                       hipStream_t s, unsigned long long* stats = nullptr);
 // Segmented exclusive scan of the per-candidate counts of every desc.
 void launch_cet_offsets(CetDesc* descs, uint32_t ndesc, uint32_t* offsets, hipStream_t s);
+// Records of the last join levels' tables (CetAgg::s and len of every
+// candidate): one pass over the adjacency, no lists written.  chunk_base[d]:
+// chunks of 64 candidates in the tables before d (ndesc + 1 entries).
+void launch_cet_sums(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, const CetDesc* descs,
+                     uint32_t ndesc, const uint32_t* chunk_base, CetAgg* aggs, uint32_t grid, hipStream_t s,
+                     unsigned long long* stats = nullptr);
+// Records of the tables of the level before the last, from their lists and
+// the last tables' records.
+void launch_cet_aggs(const uint32_t* bitmaps, const uint32_t* bprefix, uint32_t W, uint32_t NB, const AggDesc* descs,
+                     uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
+                     CetAgg* aggs, uint32_t grid, hipStream_t s);
 // Hash terms of the last join levels' lists: for table term_desc[i] (terms
 // [term_start[i], term_start[i+1]) of terms), tuple_term(term_qid, list[e]).
 void launch_cet_terms(const uint32_t* lists, const CetDesc* descs, const uint32_t* term_desc,
@@ -147,6 +158,7 @@ struct JoinArgs {
   const uint32_t* offsets;
   const uint32_t* lists;
   const unsigned long long* terms;  // hash terms of the last level's lists (CetDesc::term_base)
+  const CetAgg* aggs;  // records of the last two levels' tables (CetDesc::agg_base)
   const CetDesc* cets;
   const JoinPlan* plans;
   const JoinTask* tasks;
@@ -167,14 +179,18 @@ struct JoinArgs {
   // nonzero: account algorithmic bytes in JoinOut::bytes (a slower variant)
   uint32_t count_bytes;
 };
-// One persistent join launch over tasks [0, ntasks) of a.tasks; cyclic: the
-// plans of those tasks have back edges (join_cyclic_kernel), else none
-// (join_tree_kernel, which holds no back-edge tests).
-void launch_join(const JoinArgs& a, uint32_t nwg, bool cyclic, hipStream_t s);
+// Kernel of a join launch: tree plans (no back edges) whose last levels are
+// counted from records, tree plans whose embeddings are enumerated (tuples
+// wanted), plans with back edges whose last levels are counted from records,
+// plans with back edges at the last position (or tuples wanted).
+enum JoinKind { JOIN_TREE = 0, JOIN_TREE_ENUM = 1, JOIN_CYCLIC = 2, JOIN_CYCLIC_ENUM = 3 };
+// One persistent join launch over tasks [0, ntasks) of a.tasks, all of them
+// of plans of that kind.
+void launch_join(const JoinArgs& a, uint32_t nwg, JoinKind kind, hipStream_t s);
 uint64_t join_level_words(uint32_t qmax, uint32_t cap);
-// Join workgroups (of the timed variant of the tree or cyclic kernel) that
-// are resident on one CU at once for a batch whose widest query has qmax
+// Join workgroups (of the timed variant of the kind's kernel) that are
+// resident on one CU at once for a batch whose widest query has qmax
 // vertices (LDS and registers); a persistent grid gains nothing from more.
-uint32_t join_resident_per_cu(uint32_t qmax, bool cyclic);
+uint32_t join_resident_per_cu(uint32_t qmax, JoinKind kind);
 
 }  // namespace gpsm
