@@ -583,6 +583,15 @@ namespace {
 // workgroup, so the bound matters only for very wide queries.
 constexpr double kLevelBytes = 16.0 * (1ull << 30);
 
+// First-table rows of the plans joined breadth-first at a time (1 GB of rows).
+constexpr uint64_t kBfsRows = 1ull << 25;
+
+// Words of B_CTR: 0 .. 2 the launches' task counters, 16 .. 17 the tuples
+// emitted, and of the breadth-first join, per level, two row counts and the
+// waves that stopped at a full buffer.
+constexpr uint32_t kCtrRows = 64, kCtrPending = kCtrRows + 2 * (BFS_MAXQ + 2), kCtrWords = 128;
+static_assert(kCtrPending + BFS_MAXQ <= kCtrWords, "levels 0 .. BFS_MAXQ - 1");
+
 template <typename T>
 T* dptr(gpsm_ctx* c, int b) {
   return reinterpret_cast<T*>(c->bufs[b].ptr);
@@ -943,7 +952,6 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // ---------------- host: join orders ----------------
   std::vector<CetDesc> jdesc;
   std::vector<JoinPlan> plans;
-  std::vector<JoinTask> tasks;
   std::vector<uint32_t> plan_of_q(nq, ~0u);
   uint64_t off_words = fwd_words, list_words = 0, term_words = 0;  // reversed tables' regions follow the forward ones
   // Only tuples need the last levels enumerated; otherwise the tables of the
@@ -1117,7 +1125,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     }
     // what the join enumerates of it sizes its tasks
     if (jp.agg) est[b] = analytic_cost_upto(pcs[b], pl, S.hq.n - 1 - jp.agg);
-    plan_of_q[b] = (uint32_t)plans.size();
+    plan_of_q[b] = jp.out = (uint32_t)plans.size();
     plans.push_back(jp);
   }
   // tasks: interleaved row sets of the first tables.  A query gets tasks in
@@ -1138,19 +1146,32 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     resident[i] = std::max<uint32_t>(1, c->ncu * std::min(wg_per_cu, join_resident_per_cu(qmax, kinds[i])));
   const uint32_t nwg = resident[0];
   const uint64_t tpw = std::max<uint32_t>(1, c->tune.tasks_per_wg);
+  // Plans with back edges at their last position are joined breadth-first
+  // (join_bfs.hip), unless tuples are wanted, the join's bytes are counted,
+  // the query is wider than BFS_MAXQ (its levels' buffers would be large) or
+  // its first table has more than kBfsRows rows (they are all in memory, and
+  // the depth-first tasks share them well).
+  // Depth-first, a cycle or clique of an R-MAT graph has a few thousand
+  // first-table rows and most of its work under a few of them.
+  std::vector<uint32_t> bfs_q;
   uint64_t rows_total = 0;
   double est_total = 0;
-  for (uint32_t b = 0; b < nq; ++b)
-    if (plan_of_q[b] != ~0u) {
-      rows_total += Q[b].cet_size[Q[b].plan.first_edge];
-      est_total += est[b];
-    }
-  const uint64_t tsize =
-      std::min<uint64_t>(std::max<uint64_t>(rows_total / ((uint64_t)nwg * tpw) + 1, c->tune.task_min), 1u << 20);
-  const double target = est_total / ((double)nwg * tpw);
-  std::vector<JoinTask> ltasks[NJOIN];  // by launch
   for (uint32_t b = 0; b < nq; ++b) {
     if (plan_of_q[b] == ~0u) continue;
+    const JoinPlan& jp = plans[plan_of_q[b]];
+    if (jp.nback_total && !jp.agg && !emit_cap && !counters && jp.q <= BFS_MAXQ &&
+        Q[b].cet_size[Q[b].plan.first_edge] <= kBfsRows) {
+      bfs_q.push_back(b);
+      continue;
+    }
+    rows_total += Q[b].cet_size[Q[b].plan.first_edge];
+    est_total += est[b];
+  }
+  std::vector<JoinTask> ltasks[NJOIN];  // by launch
+  auto add_tasks = [&](uint32_t b) {
+    const uint64_t tsize =
+        std::min<uint64_t>(std::max<uint64_t>(rows_total / ((uint64_t)nwg * tpw) + 1, c->tune.task_min), 1u << 20);
+    const double target = est_total / ((double)nwg * tpw);
     const uint64_t R1 = Q[b].cet_size[Q[b].plan.first_edge];
     uint64_t T = (R1 + tsize - 1) / tsize;
     if (target > 0 && est[b] > target) T = std::max<uint64_t>(T, (uint64_t)std::min(est[b] / target + 1.0, 1e9));
@@ -1166,18 +1187,19 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       if ((NC - 1) % T == t) rows -= (NC << shift) - R1;  // the last chunk may be short
       dst.push_back({plan_of_q[b], (uint32_t)T, shift, 0, t, rows});
     }
-  }
-  uint32_t ltask0[NJOIN];  // each launch's first task
-  for (int i = 0; i < NJOIN; ++i) {
-    ltask0[i] = (uint32_t)tasks.size();
-    tasks.insert(tasks.end(), ltasks[i].begin(), ltasks[i].end());
+  };
+  {
+    size_t i = 0;
+    for (uint32_t b = 0; b < nq; ++b) {
+      if (i < bfs_q.size() && bfs_q[i] == b) ++i;
+      else if (plan_of_q[b] != ~0u) add_tasks(b);
+    }
   }
 
   // ---------------- phase C: candidate-edge tables ----------------
   wall(K_WALL_PLAN);
   term_start.push_back(term_words);
-  if ((rc = upload(c, B_JDESC, jdesc)) || (rc = upload(c, B_PLANS, plans)) || (rc = upload(c, B_TASKS, tasks)) ||
-      (rc = upload(c, B_TERM_DESC, term_desc)) || (rc = upload(c, B_TERM_START, term_start)))
+  if ((rc = upload(c, B_JDESC, jdesc)) || (rc = upload(c, B_PLANS, plans)) || (rc = upload(c, B_TERM_DESC, term_desc)) || (rc = upload(c, B_TERM_START, term_start)))
     return rc;
   if ((rc = c->bufs[B_TERMS].ensure(sizeof(uint64_t) * std::max<uint64_t>(term_words, 1)))) return rc;
   std::vector<CetDesc> cdesc;
@@ -1208,27 +1230,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if ((rc = c->bufs[B_JOUT].ensure(sizeof(JoinOut) * std::max<uint32_t>(nplans, 1))) ||
       (rc = c->h_stage[2].ensure(sizeof(JoinOut) * std::max<uint32_t>(nplans, 1))))
     return rc;
-  if ((rc = c->bufs[B_CTR].ensure(256))) return rc;
-  // Level buffers of the workgroups launched, a region per launch (they may
-  // run at the same time), within kLevelBytes: rows per level halve (to 2048)
-  // and then workgroups are dropped, from every launch in proportion, until
-  // they fit.
-  uint32_t lwg[NJOIN];
-  uint64_t gsum = 0;
-  for (int i = 0; i < NJOIN; ++i) gsum += lwg[i] = (uint32_t)std::min<uint64_t>(resident[i], ltasks[i].size());
-  uint32_t lcap = cap;
-  while (lcap > 2048 && (double)join_level_words(qmax, lcap) * 4.0 * gsum > kLevelBytes) lcap /= 2;
-  const uint64_t lw = join_level_words(qmax, lcap);
-  if (lw && (double)lw * 4.0 * gsum > kLevelBytes) {
-    const uint64_t fit = std::max<uint64_t>(NJOIN, (uint64_t)(kLevelBytes / (4.0 * lw)));
-    const uint64_t all = gsum;
-    gsum = 0;
-    for (uint32_t& n : lwg) {
-      if (n) n = (uint32_t)std::max<uint64_t>(1, (uint64_t)n * fit / all);
-      gsum += n;
-    }
-  }
-  if ((rc = c->bufs[B_LEVELS].ensure(sizeof(uint32_t) * std::max<uint64_t>(lw * gsum, 1)))) return rc;
+  if ((rc = c->bufs[B_CTR].ensure(4 * kCtrWords))) return rc;
   if (emit_cap && (rc = c->bufs[B_EMIT].ensure(sizeof(uint32_t) * emit_cap * qmax))) return rc;
   PhaseSig sig_c;
   if (o.use_graph) {
@@ -1269,7 +1271,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
                      dptr<unsigned long long>(c, B_TERMS), s);
     pend(K_CET_WRITE, pa, 0.0, counters ? slot_cet_w : -1);
     launch_fill_u32(dptr<uint32_t>(c, B_JOUT), 0u, sizeof(JoinOut) / 4 * (uint64_t)std::max<uint32_t>(nplans, 1), s);
-    launch_fill_u32(dptr<uint32_t>(c, B_CTR), 0u, 64, s);
+    launch_fill_u32(dptr<uint32_t>(c, B_CTR), 0u, kCtrWords, s);
     if (captured && (rc = launch_captured(c, 1, s, sig_c.w))) return rc;
   }
   // ---------------- phase D: join ----------------
@@ -1292,9 +1294,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     ja.plans = dptr<JoinPlan>(c, B_PLANS);
     ja.W = W;
     ja.NB = NB;
-    ja.cap = lcap;
     ja.qmax = qmax;
-    ja.level_stride = lw;
     ja.out = dptr<JoinOut>(c, B_JOUT);
     if (emit_cap) {
       ja.emit = dptr<uint32_t>(c, B_EMIT);
@@ -1303,39 +1303,177 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     }
     ja.budget = o.work_budget;
     ja.count_bytes = counters ? 1u : 0u;
-    // one launch per kind of plan, each with its own task counter and level
-    // buffers; timed together as one join.  The enumerated cyclic plans run on
-    // stream2, forked after everything before on stream and joined back before
-    // what follows, the others one after the other on stream.
-    hipEvent_t pa = pbegin(K_JOIN);
-    const bool fork = !ltasks[2].empty() && (!ltasks[0].empty() || !ltasks[1].empty());
-    uint64_t level0 = 0;
-    for (int i : {2, 1, 0}) {
-      if (ltasks[i].empty()) continue;
-      JoinArgs jl = ja;
-      jl.tasks = dptr<JoinTask>(c, B_TASKS) + ltask0[i];
-      jl.ntasks = (uint32_t)ltasks[i].size();
-      jl.task_counter = dptr<unsigned int>(c, B_CTR) + i;
-      jl.levels = dptr<uint32_t>(c, B_LEVELS) + lw * level0;
-      level0 += lwg[i];
-      if (i == 2 && fork) {
-        HIPCHK(hipEventRecord(c->ev_fork, s));
-        HIPCHK(hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
-        launch_join(jl, lwg[i], kinds[i], c->stream2);
-        HIPCHK(hipEventRecord(c->ev_join, c->stream2));
-      } else {
-        launch_join(jl, lwg[i], kinds[i], s);
+    // Depth-first launches, one per kind of plan, each with its own task
+    // counter and level buffers (a region per launch, within kLevelBytes: rows
+    // per level halve, to 2048, and then workgroups are dropped, from every
+    // launch in proportion, until they fit); the enumerated cyclic plans on
+    // stream2, forked after everything before on stream and joined back
+    // before what follows, the others one after the other on stream.
+    auto depth_first = [&]() -> int {
+      std::vector<JoinTask> tasks;
+      uint32_t task0[NJOIN], lwg[NJOIN];
+      uint64_t gsum = 0;
+      for (int i = 0; i < NJOIN; ++i) {
+        task0[i] = (uint32_t)tasks.size();
+        tasks.insert(tasks.end(), ltasks[i].begin(), ltasks[i].end());
+        gsum += lwg[i] = (uint32_t)std::min<uint64_t>(resident[i], ltasks[i].size());
       }
-    }
-    if (fork) HIPCHK(hipStreamWaitEvent(s, c->ev_join, 0));
+      if (tasks.empty()) return GPSM_OK;
+      ja.cap = cap;
+      while (ja.cap > 2048 && (double)join_level_words(qmax, ja.cap) * 4.0 * gsum > kLevelBytes) ja.cap /= 2;
+      const uint64_t lw = join_level_words(qmax, ja.cap);
+      if (lw && (double)lw * 4.0 * gsum > kLevelBytes) {
+        const uint64_t fit = std::max<uint64_t>(NJOIN, (uint64_t)(kLevelBytes / (4.0 * lw)));
+        const uint64_t all = gsum;
+        gsum = 0;
+        for (uint32_t& n : lwg) {
+          if (n) n = (uint32_t)std::max<uint64_t>(1, (uint64_t)n * fit / all);
+          gsum += n;
+        }
+      }
+      int rc;
+      if ((rc = c->bufs[B_LEVELS].ensure(sizeof(uint32_t) * std::max<uint64_t>(lw * gsum, 1))) ||
+          (rc = upload(c, B_TASKS, tasks)))
+        return rc;
+      ja.level_stride = lw;
+      const bool fork = lwg[2] && (lwg[0] || lwg[1]);
+      uint64_t level0 = 0;
+      for (int i : {2, 1, 0}) {
+        if (!lwg[i]) continue;
+        JoinArgs jl = ja;
+        jl.tasks = dptr<JoinTask>(c, B_TASKS) + task0[i];
+        jl.ntasks = (uint32_t)ltasks[i].size();
+        jl.task_counter = dptr<unsigned int>(c, B_CTR) + i;
+        jl.levels = dptr<uint32_t>(c, B_LEVELS) + lw * level0;
+        level0 += lwg[i];
+        if (i == 2 && fork) {
+          HIPCHK(hipEventRecord(c->ev_fork, s));
+          HIPCHK(hipStreamWaitEvent(c->stream2, c->ev_fork, 0));
+          launch_join(jl, lwg[i], kinds[i], c->stream2);
+          HIPCHK(hipEventRecord(c->ev_join, c->stream2));
+        } else {
+          launch_join(jl, lwg[i], kinds[i], s);
+        }
+      }
+      if (fork) HIPCHK(hipStreamWaitEvent(s, c->ev_join, 0));
+      return GPSM_OK;
+    };
+    // Breadth-first launches, BFS_PLANS plans at a time: a buffer per level,
+    // for sixteen times the rows expected at the busiest level (the estimate
+    // is rough), 2^18 to 2^24 rows within kLevelBytes.  After a pass over the
+    // levels the host reads which of them stopped at a full buffer; the
+    // deepest one goes on first, into buffers emptied by then.
+    auto breadth_first = [&]() -> int {
+      uint32_t* ctr = dptr<uint32_t>(c, B_CTR);
+      for (size_t q0 = 0, q1; q0 < bfs_q.size(); q0 = q1) {
+        uint64_t first_rows = 0;
+        for (q1 = q0; q1 < bfs_q.size() && q1 < q0 + BFS_PLANS; ++q1) {
+          const QState& S = Q[bfs_q[q1]];
+          if (q1 > q0 && first_rows + S.cet_size[S.plan.first_edge] > kBfsRows) break;
+          first_rows += S.cet_size[S.plan.first_edge];
+        }
+        std::vector<JoinPlan> bp;
+        std::vector<uint64_t> first(1, 0);
+        uint32_t widest = 3;
+        double rows = 0;
+        for (size_t i = q0; i < q1; ++i) {
+          const uint32_t b = bfs_q[i];
+          bp.push_back(plans[plan_of_q[b]]);
+          first.push_back(first.back() + Q[b].cet_size[Q[b].plan.first_edge]);
+          widest = std::max(widest, bp.back().q);
+          rows += analytic_rows_max(pcs[b], Q[b].plan);
+        }
+        const uint32_t nwg_b = std::max<uint32_t>(1, c->ncu * bfs_resident_per_cu());
+        const uint64_t nwave = (uint64_t)nwg_b * 4;
+        const uint32_t block = (uint32_t)std::min(64.0, std::max(4.0, rows / (4.0 * nwave)));
+        uint64_t words_per_row = 1;
+        for (uint32_t l = 2; l + 1 < widest; ++l) words_per_row += bfs_row_words(l);
+        const uint64_t slack = nwave * block;  // slots of blocks not filled
+        const uint64_t most = std::max<uint64_t>((uint64_t)(kLevelBytes / (4.5 * words_per_row)), 1u << 18);
+        const uint64_t rcap =
+            slack + std::min<uint64_t>(most, (uint64_t)std::min(std::max(16.0 * rows, 262144.0), 16777216.0));
+        const uint64_t cap1 = first.back() + slack;  // every level-1 row
+        auto cap_of = [&](uint32_t l) { return l == 1 ? cap1 : rcap; };
+        auto long_of = [&](uint32_t l) { return l == 1 ? first.back() : rcap / 16; };
+        uint64_t at[BFS_MAXQ] = {0}, words = 0;  // each level's short rows, its long rows after them
+        for (uint32_t l = 1; l + 1 < widest; ++l) {
+          at[l] = words;
+          words += (cap_of(l) + long_of(l)) * bfs_row_words(l);
+        }
+        int rc;
+        if ((rc = c->bufs[B_BROWS].ensure(sizeof(uint32_t) * words)) || (rc = upload(c, B_BPLANS, bp)) ||
+            (rc = upload(c, B_BFIRST, first)) ||
+            (rc = c->bufs[B_BCURS].ensure(sizeof(BfsCursor) * 2 * nwave * BFS_MAXQ)))
+          return rc;
+        if (q0) launch_fill_u32(ctr + kCtrRows, 0u, kCtrWords - kCtrRows, s);
+        BfsArgs a{};
+        a.j = ja;
+        a.j.plans = dptr<JoinPlan>(c, B_BPLANS);
+        a.nplans = (uint32_t)bp.size();
+        a.block = block;
+        a.any_source = learned;
+        a.first_row = dptr<uint64_t>(c, B_BFIRST);
+        uint32_t* rows_base = dptr<uint32_t>(c, B_BROWS);
+        auto out_level = [&](uint32_t l) {
+          const bool kept = l + 1 < widest;
+          a.rows_out = kept ? rows_base + at[l] : nullptr;
+          a.long_out = kept ? a.rows_out + cap_of(l) * bfs_row_words(l) : nullptr;
+          a.cap = kept ? (uint32_t)cap_of(l) : 0;
+          a.long_cap = kept ? (uint32_t)long_of(l) : 0;
+          a.stride_out = bfs_row_words(l);
+          a.cout = ctr + kCtrRows + 2 * l;
+        };
+        // level l's rows to level l + 1
+        auto expand = [&](uint32_t l, bool resume) {
+          out_level(l);
+          a.rows_in = a.rows_out;
+          a.long_in = a.long_out;
+          a.cap_in = a.cap;
+          a.long_cap_in = a.long_cap;
+          a.stride_in = a.stride_out;
+          a.cin = a.cout;
+          out_level(l + 1);
+          a.level = l;
+          a.cursors = dptr<BfsCursor>(c, B_BCURS) + 2 * nwave * l;
+          a.resume = resume;
+          a.pending = ctr + kCtrPending + l;
+          launch_bfs_expand(a, nwg_b, s);
+        };
+        out_level(1);
+        a.level = 0;
+        launch_bfs_first(a, (uint32_t)std::min<uint64_t>(nwg_b, (first.back() + 255) / 256), s);
+        for (uint32_t l = 1; l + 1 < widest; ++l) expand(l, false);
+        if (widest == 3) continue;  // level 1 writes no rows
+        if ((rc = c->h_stage[3].ensure(sizeof(uint32_t) * BFS_MAXQ))) return rc;
+        const uint32_t* pending = static_cast<const uint32_t*>(c->h_stage[3].ptr);
+        for (;;) {
+          HIPCHK(hipMemcpyAsync(c->h_stage[3].ptr, ctr + kCtrPending, sizeof(uint32_t) * BFS_MAXQ,
+                                hipMemcpyDeviceToHost, s));
+          HIPCHK(hipStreamSynchronize(s));
+          uint32_t l = 0;
+          for (uint32_t x = 1; x + 2 < widest; ++x)
+            if (pending[x]) l = x;
+          if (!l) break;
+          launch_fill_u32(ctr + kCtrPending + l, 0u, BFS_MAXQ - l, s);
+          launch_fill_u32(ctr + kCtrRows + 2 * (l + 1), 0u, 2 * (BFS_MAXQ - l), s);
+          expand(l, true);
+          for (++l; l + 1 < widest; ++l) expand(l, false);
+        }
+      }
+      return GPSM_OK;
+    };
+    // timed together as one join
+    hipEvent_t pa = pbegin(K_JOIN);
+    if (!bfs_q.empty() && (rc = breadth_first())) return rc;
+    if ((rc = depth_first())) return rc;
     pend(K_JOIN, pa, 0.0, -1);
     HIPCHK(hipGetLastError());
     std::vector<JoinOut> jo(std::max<uint32_t>(nplans, 1));
-    HIPCHK(hipMemcpyAsync(c->h_stage[2].ptr, dptr<JoinOut>(c, B_JOUT), sizeof(JoinOut) * nplans,
-                          hipMemcpyDeviceToHost, s));
     unsigned long long emitted = 0;
     if (emit_cap)
       HIPCHK(hipMemcpyAsync(&emitted, dptr<uint32_t>(c, B_CTR) + 16, sizeof(emitted), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(c->h_stage[2].ptr, dptr<JoinOut>(c, B_JOUT), sizeof(JoinOut) * nplans,
+                          hipMemcpyDeviceToHost, s));
     hipEventRecord(c->ev1, s);
     HIPCHK(hipStreamSynchronize(s));
     if (nplans) std::memcpy(jo.data(), c->h_stage[2].ptr, sizeof(JoinOut) * nplans);

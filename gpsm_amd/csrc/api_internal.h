@@ -86,6 +86,10 @@ enum BufId {
   B_ADESC,       // tables of the level before (AggDesc)
   B_ACHUNK,      // ... chunks before each
   B_AGGS,        // their candidates' records (CetAgg)
+  B_BPLANS,      // plans joined breadth-first
+  B_BFIRST,      // ... first-table rows before each
+  B_BROWS,       // ... rows of their levels
+  B_BCURS,       // ... where each wave of a level stands
   B_RFLAGS,      // refine rounds that removed a candidate, 4 per query
   B_COUNT_
 };
@@ -180,7 +184,8 @@ struct gpsm_ctx {
   gpsm::Tuning tune;
   gpsm_mlp* planner = nullptr;
   std::vector<uint32_t> h_counts;
-  gpsm::HostBuf h_stage[3];  // pinned readbacks of a batch: counts, |CET| descriptors, join results
+  // pinned readbacks of a batch: counts, |CET| descriptors, join results, join flag
+  gpsm::HostBuf h_stage[4];
   gpsm::PinnedArena arena;   // pinned sources of a batch's uploads
   // Instantiated hipGraphs of a batch's two captured phases (filter;
   // candidate-edge tables), kept across batches: a batch whose launches

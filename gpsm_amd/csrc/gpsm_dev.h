@@ -103,6 +103,7 @@ struct JoinPlan {
   // levels the join counts from CetAgg records instead of enumerating them:
   // the last agg levels (0, 1 or 2), none of which has a back position
   uint32_t agg;
+  uint32_t out;  // index of the query's JoinOut
   // injectivity checks of level k: positions c < k whose query vertex has
   // the label of position k's, other than the parent and the back
   // positions.  A candidate of another label cannot equal the vertex bound

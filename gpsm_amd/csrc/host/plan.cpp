@@ -637,6 +637,21 @@ double analytic_cost(const PlanContext& c, const OrderPlan& plan) {
   return s.cost;
 }
 
+double analytic_rows_max(const PlanContext& c, const OrderPlan& plan) {
+  PlanCost s;
+  if (!cost_start(c, plan.order.data(), s)) return 0.0;
+  double most = s.rows;
+  std::vector<float> f;
+  while (!s.done) {
+    f.clear();
+    cost_emit(s, f);
+    const float y = f[27];
+    cost_consume(s, &y);
+    most = std::max(most, s.rows);
+  }
+  return most;
+}
+
 double analytic_cost_upto(const PlanContext& c, const OrderPlan& plan, uint32_t last) {
   PlanCost s;
   if (!cost_start(c, plan.order.data(), s)) return 0.0;

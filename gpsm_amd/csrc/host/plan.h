@@ -190,6 +190,8 @@ int learned_plans(const std::vector<const PlanContext*>& qs, PredictFn predict, 
 // the expand edge / |C(parent)|) + the log densities of its back edges
 // (feature 27 of step_features).  Used to size the join's tasks.
 double analytic_cost(const PlanContext& c, const OrderPlan& plan);
+// The most rows it expects at a level 1 .. n-2 (the levels a join keeps).
+double analytic_rows_max(const PlanContext& c, const OrderPlan& plan);
 // The part of it up to position last: the first table's rows and the
 // candidates examined for positions 2 .. last (what the join enumerates of a
 // plan whose later levels are counted from records).

@@ -188,6 +188,39 @@ enum JoinKind { JOIN_TREE = 0, JOIN_TREE_ENUM = 1, JOIN_CYCLIC = 2, JOIN_CYCLIC_
 // of plans of that kind.
 void launch_join(const JoinArgs& a, uint32_t nwg, JoinKind kind, hipStream_t s);
 uint64_t join_level_words(uint32_t qmax, uint32_t cap);
+
+// join_bfs.hip -------------------------------------------------------------------
+// Breadth-first join of up to BFS_PLANS plans with back edges and at most
+// BFS_MAXQ positions: launch_bfs_first writes the level-1 rows, launch_bfs_expand
+// takes level to level + 1: all its rows, or (resume) those that an earlier
+// launch left when the next level's buffer was full.  j: plans (nplans of them, JoinPlan::out their
+// results), cets, lists, budget and out as for launch_join.
+constexpr uint32_t BFS_PLANS = 256, BFS_MAXQ = 8;
+struct BfsCursor {
+  uint32_t idx, pos, skip;
+};
+struct BfsArgs {
+  JoinArgs j;
+  uint32_t nplans, level;
+  uint32_t block;             // row slots a wave reserves at a time
+  uint32_t any_source;        // a row's candidates may come from any of its bound neighbours
+  const uint64_t* first_row;  // first-table rows of the plans before each (nplans + 1)
+  // rows of `level` and `level + 1`: records of stride_* words; short lists,
+  // long lists, and their counts (2 words each, zeroed by the caller)
+  const uint32_t *rows_in, *long_in;
+  uint32_t cap_in, long_cap_in, stride_in;
+  const uint32_t* cin;
+  uint32_t *rows_out, *long_out;  // null at the last level
+  uint32_t cap, long_cap, stride_out;
+  uint32_t* cout;
+  BfsCursor* cursors;  // two per wave of the level's launches (the same grid each time)
+  uint32_t resume;
+  uint32_t* pending;   // waves that stopped at a full buffer (zeroed by the caller)
+};
+uint32_t bfs_row_words(uint32_t level);
+void launch_bfs_first(const BfsArgs& a, uint32_t nwg, hipStream_t s);
+void launch_bfs_expand(const BfsArgs& a, uint32_t nwg, hipStream_t s);
+uint32_t bfs_resident_per_cu();
 // Join workgroups (of the timed variant of the kind's kernel) that are
 // resident on one CU at once for a batch whose widest query has qmax
 // vertices (LDS and registers); a persistent grid gains nothing from more.
