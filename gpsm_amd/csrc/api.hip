@@ -12,6 +12,7 @@
 // Phases A and C may be captured in hipGraphs (opts->use_graph); the join
 // (D) is launched directly, its two launches side by side on two streams.
 #include <hip/hip_runtime.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <chrono>
@@ -694,6 +695,44 @@ bool replay_cached(gpsm_ctx* c, int phase, const std::vector<uint64_t>& sig, hip
     ++c->graph_replays;
   }
   return true;
+}
+
+// Host memory of a tuple list (released with free()): large ones in huge
+// pages where the system has them, whose first touch costs one fault per 2 MB
+// instead of one per 4 KB.
+uint32_t* alloc_result(size_t bytes) {
+  constexpr size_t kHuge = 2u << 20;
+  if (bytes < 2 * kHuge) return static_cast<uint32_t*>(std::malloc(bytes));
+  void* p = std::aligned_alloc(kHuge, (bytes + kHuge - 1) / kHuge * kHuge);
+  if (p) (void)madvise(p, bytes, MADV_HUGEPAGE);
+  return static_cast<uint32_t*>(p);
+}
+
+// Rows of the emitted tuples (any number) to host memory in lexicographic
+// order: sorted on the device, or on the host when the device has no room for
+// the sort or there are 2^32 rows or more.
+int sort_emitted(gpsm_ctx* c, const uint32_t* emit, uint64_t n, uint32_t q, uint32_t bits, uint32_t* host) {
+  const size_t bytes = sizeof(uint32_t) * n * q;
+  hipStream_t s = c->stream;
+  const uint64_t words = n < (1ull << 32) ? tuple_sort_words(n) : 0;
+  if (words && c->bufs[B_EMIT_SORT].ensure(sizeof(uint32_t) * (words + n * q)) == GPSM_OK) {
+    uint32_t* scratch = dptr<uint32_t>(c, B_EMIT_SORT);
+    launch_sort_tuples(emit, n, q, bits, scratch, scratch + words, s);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(host, scratch + words, bytes, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    return GPSM_OK;
+  }
+  std::vector<uint32_t> tup(n * q);
+  HIPCHK(hipMemcpy(tup.data(), emit, bytes, hipMemcpyDeviceToHost));
+  std::vector<uint64_t> idx(n);
+  std::iota(idx.begin(), idx.end(), 0);
+  std::sort(idx.begin(), idx.end(), [&](uint64_t x, uint64_t y) {
+    return std::lexicographical_compare(tup.begin() + x * q, tup.begin() + (x + 1) * q, tup.begin() + y * q,
+                                        tup.begin() + (y + 1) * q);
+  });
+  for (uint64_t i = 0; i < n; ++i) std::memcpy(host + i * q, tup.data() + idx[i] * q, sizeof(uint32_t) * q);
+  return GPSM_OK;
 }
 
 int predict_with_ctx(void* user, const float* x, uint32_t B, float* y) {
@@ -1469,6 +1508,14 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     pend(K_JOIN, pa, 0.0, -1);
     HIPCHK(hipGetLastError());
     std::vector<JoinOut> jo(std::max<uint32_t>(nplans, 1));
+    // the tuples sorted behind the join, if they turn out to be few enough
+    const uint32_t id_bits = std::max(1, 32 - __builtin_clz(std::max<uint32_t>(dg.n - 1, 1)));
+    const uint64_t rank_cap = std::min<uint64_t>(emit_cap, TUPLE_RANK);
+    if (emit_cap) {
+      if ((rc = c->h_stage[4].ensure(sizeof(uint32_t) * rank_cap * qmax))) return rc;
+      launch_rank_tuples(ja.emit, Q[0].hq.n, id_bits, ja.emit_ctr, (uint32_t)rank_cap,
+                         static_cast<uint32_t*>(c->h_stage[4].ptr), s);
+    }
     unsigned long long emitted = 0;
     if (emit_cap)
       HIPCHK(hipMemcpyAsync(&emitted, dptr<uint32_t>(c, B_CTR) + 16, sizeof(emitted), hipMemcpyDeviceToHost, s));
@@ -1541,20 +1588,17 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       if (emitted > emit_cap) {
         out[0].status = GPSM_EOVERFLOW;
       } else {
-        std::vector<uint32_t> tup(emitted * qn);
-        if (emitted)
-          HIPCHK(hipMemcpy(tup.data(), dptr<uint32_t>(c, B_EMIT), sizeof(uint32_t) * tup.size(),
-                           hipMemcpyDeviceToHost));
-        std::vector<uint64_t> idx(emitted);
-        std::iota(idx.begin(), idx.end(), 0);
-        std::sort(idx.begin(), idx.end(), [&](uint64_t x, uint64_t y) {
-          return std::lexicographical_compare(tup.begin() + x * qn, tup.begin() + (x + 1) * qn, tup.begin() + y * qn,
-                                              tup.begin() + (y + 1) * qn);
-        });
-        out[0].tuples = (uint32_t*)std::malloc(sizeof(uint32_t) * std::max<uint64_t>(emitted * qn, 1));
+        // few rows were sorted behind the join (launch_rank_tuples); more are
+        // sorted on the device now and copied once
+        const size_t bytes = sizeof(uint32_t) * emitted * qn;
+        out[0].tuples = alloc_result(std::max<size_t>(bytes, 1));
         if (!out[0].tuples) return GPSM_ENOMEM;
-        for (uint64_t i = 0; i < emitted; ++i)
-          std::memcpy(out[0].tuples + i * qn, tup.data() + idx[i] * qn, sizeof(uint32_t) * qn);
+        if (emitted <= rank_cap) {
+          std::memcpy(out[0].tuples, c->h_stage[4].ptr, bytes);
+        } else if ((rc = sort_emitted(c, dptr<uint32_t>(c, B_EMIT), emitted, qn, id_bits, out[0].tuples))) {
+          gpsm_result_free(&out[0]);
+          return rc;
+        }
         out[0].n_tuples = emitted;
       }
     }

@@ -67,6 +67,7 @@ enum BufId {
   B_CTR,
   B_LEVELS,
   B_EMIT,
+  B_EMIT_SORT,   // sorting the emitted tuples: scratch, then the sorted rows
   B_MLP,
   B_FSTATS,
   B_TERMS,       // hash terms of the last join level's lists (u64)
@@ -184,8 +185,9 @@ struct gpsm_ctx {
   gpsm::Tuning tune;
   gpsm_mlp* planner = nullptr;
   std::vector<uint32_t> h_counts;
-  // pinned readbacks of a batch: counts, |CET| descriptors, join results, join flag
-  gpsm::HostBuf h_stage[4];
+  // pinned readbacks of a batch: counts, |CET| descriptors, join results, join
+  // flag, few sorted tuples
+  gpsm::HostBuf h_stage[5];
   gpsm::PinnedArena arena;   // pinned sources of a batch's uploads
   // Instantiated hipGraphs of a batch's two captured phases (filter;
   // candidate-edge tables), kept across batches: a batch whose launches

@@ -7,14 +7,6 @@
 // flags drops duplicates, and the row offsets are lower bounds of v<<32.
 // Self-loops become the key n<<32, which sorts after every real row and is
 // left out of the offsets.
-//
-// One radix pass: each workgroup counts the digits of its tile of
-// RADIX_TILE keys (LDS histogram), an exclusive scan of the counts in
-// digit-major order gives every (digit, tile) its output start, and each
-// workgroup scatters its tile stably: 256 keys at a time, in index order,
-// a key's place among the equal digits of its wave comes from eight
-// ballots (one per digit bit), the waves before it from per-wave digit
-// counts in LDS, the chunks before it from a running count per digit.
 #include <algorithm>
 
 #include "gpsm.h"
@@ -62,62 +54,6 @@ __global__ void columns_kernel(const unsigned long long* __restrict__ keys, uint
   const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
   for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < adj; i += stride)
     col[i] = (uint32_t)keys[i];
-}
-
-constexpr uint32_t RADIX_ITEMS = 16;                  // keys per thread and tile
-constexpr uint32_t RADIX_TILE = 256 * RADIX_ITEMS;     // keys per workgroup
-
-__global__ void __launch_bounds__(256) radix_hist_kernel(const unsigned long long* __restrict__ keys, uint64_t n,
-                                                         uint32_t shift, uint32_t ntiles,
-                                                         uint32_t* __restrict__ hist) {
-  __shared__ uint32_t cnt[256];
-  cnt[threadIdx.x] = 0;
-  __syncthreads();
-  const uint64_t base = (uint64_t)blockIdx.x * RADIX_TILE;
-  for (uint32_t j = 0; j < RADIX_ITEMS; ++j) {
-    const uint64_t i = base + (uint64_t)j * 256 + threadIdx.x;
-    if (i < n) atomicAdd(&cnt[(uint32_t)(keys[i] >> shift) & 255u], 1u);
-  }
-  __syncthreads();
-  hist[(size_t)threadIdx.x * ntiles + blockIdx.x] = cnt[threadIdx.x];  // digit-major
-}
-
-__global__ void __launch_bounds__(256) radix_scatter_kernel(const unsigned long long* __restrict__ in,
-                                                            unsigned long long* __restrict__ out, uint64_t n,
-                                                            uint32_t shift, uint32_t ntiles,
-                                                            const uint32_t* __restrict__ start) {
-  __shared__ uint32_t run[256];     // output position of the next key of each digit
-  __shared__ uint32_t wc[4][256];   // this chunk's keys per (wave, digit)
-  const uint32_t lane = lane_id(), w = threadIdx.x / WAVE;
-  const unsigned long long below = lane ? (~0ULL >> (WAVE - lane)) : 0ULL;
-  run[threadIdx.x] = start[(size_t)threadIdx.x * ntiles + blockIdx.x];
-  const uint64_t base = (uint64_t)blockIdx.x * RADIX_TILE;
-  for (uint32_t j = 0; j < RADIX_ITEMS; ++j) {
-    const uint64_t i = base + (uint64_t)j * 256 + threadIdx.x;
-    const bool valid = i < n;
-    const unsigned long long key = valid ? in[i] : 0ULL;
-    const uint32_t d = (uint32_t)(key >> shift) & 255u;
-    // the lanes of this wave holding the same digit
-    unsigned long long same = __ballot(valid);
-#pragma unroll
-    for (uint32_t b = 0; b < 8; ++b) {
-      const unsigned long long ones = __ballot(valid && ((d >> b) & 1u));
-      same &= ((d >> b) & 1u) ? ones : ~ones;
-    }
-    const uint32_t rank = (uint32_t)__popcll(same & below);
-#pragma unroll
-    for (uint32_t k = 0; k < 4; ++k) wc[w][lane + 64 * k] = 0;
-    if (valid && rank == 0) wc[w][d] = (uint32_t)__popcll(same);
-    __syncthreads();  // also publishes run (first chunk) and the previous chunk's counts
-    if (valid) {
-      uint32_t pos = run[d] + rank;
-      for (uint32_t x = 0; x < w; ++x) pos += wc[x][d];
-      out[pos] = key;
-    }
-    __syncthreads();
-    run[threadIdx.x] += wc[0][threadIdx.x] + wc[1][threadIdx.x] + wc[2][threadIdx.x] + wc[3][threadIdx.x];
-    __syncthreads();
-  }
 }
 
 // flags[i] = 1 where key i starts a run of equal keys (the keys sorted)
@@ -170,8 +106,7 @@ int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint
   unsigned rbits = 1;
   while (rbits < 32 && ((uint64_t)n >> rbits)) ++rbits;
   const unsigned end_bit = 32 + rbits;
-  const uint32_t ntiles = (uint32_t)std::max<uint64_t>(1, (M2 + RADIX_TILE - 1) / RADIX_TILE);
-  const uint64_t nhist = 256ull * ntiles;
+  const uint64_t nhist = radix_hist_words(M2);
   const uint64_t sw = scan_scratch_words(std::max<uint64_t>(nhist, M2)) + 2;
   if (hipMalloc(&d_bad, sizeof(uint32_t)) != hipSuccess ||
       hipMalloc(&d_count, sizeof(unsigned long long)) != hipSuccess ||
@@ -204,9 +139,7 @@ int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint
       hipLaunchKernelGGL(edge_keys_kernel, dim3(grid_for(m)), dim3(256), 0, s, d_src, d_dst, m, n, keys, d_bad);
       unsigned long long *a = keys, *b = sorted;
       for (uint32_t shift = 0; shift < end_bit; shift += 8) {
-        hipLaunchKernelGGL(radix_hist_kernel, dim3(ntiles), dim3(256), 0, s, a, M2, shift, ntiles, hist);
-        launch_exclusive_scan(hist, hstart, nhist, d_count, scratch + 2, sw - 2, s);
-        hipLaunchKernelGGL(radix_scatter_kernel, dim3(ntiles), dim3(256), 0, s, a, b, M2, shift, ntiles, hstart);
+        launch_radix_pass(a, b, nullptr, nullptr, M2, shift, hist, hstart, scratch + 2, sw - 2, s);
         std::swap(a, b);
       }
       // a holds the sorted keys; the first key of each run of equal keys is kept, in order, in b

@@ -102,6 +102,29 @@ uint64_t compact_scratch_words(uint64_t nbits);
 void launch_compact_bitmap(const uint32_t* bits, uint64_t nbits, uint32_t* ids, unsigned long long* count,
                            uint32_t* scratch, hipStream_t s);
 
+// radix.hip --------------------------------------------------------------------
+// One stable pass over the 8 bits of the keys at shift: in to out, with values
+// vin to vout unless null.  hist, hstart: radix_hist_words(n) words each;
+// scratch: scan_scratch_words of that many.  n < 2^32.
+uint64_t radix_hist_words(uint64_t n);
+void launch_radix_pass(const unsigned long long* in, unsigned long long* out, const uint32_t* vin, uint32_t* vout,
+                       uint64_t n, uint32_t shift, uint32_t* hist, uint32_t* hstart, uint32_t* scratch,
+                       uint64_t scratch_words, hipStream_t s);
+
+// tuples.hip -------------------------------------------------------------------
+// Lexicographic order of rows of q u32 values below 2^bits, all distinct.
+// Up to cap <= TUPLE_RANK rows: one launch, the number of rows read from
+// *count on the device (more than cap: nothing is written); out may be host
+// memory the device can write.
+constexpr uint32_t TUPLE_RANK = 8192;
+void launch_rank_tuples(const uint32_t* tuples, uint32_t q, uint32_t bits, const unsigned long long* count,
+                        uint32_t cap, uint32_t* out, hipStream_t s);
+// Any number below 2^32: radix passes over the rows' packed bits, the rows
+// themselves moved once.  scratch: tuple_sort_words(n) words, 8-byte aligned.
+uint64_t tuple_sort_words(uint64_t n);
+void launch_sort_tuples(const uint32_t* tuples, uint64_t n, uint32_t q, uint32_t bits, uint32_t* scratch,
+                        uint32_t* out, hipStream_t s);
+
 // text.hip ---------------------------------------------------------------------
 // Embedding lines "(j, k) ... \n" of IO::output.  R = text_rows_per_wg(q)
 // rows per workgroup; wg_len / wg_off: ceil(rows / R) words.

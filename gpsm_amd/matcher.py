@@ -30,6 +30,10 @@ class MatchResult:
     tuples: np.ndarray = field(default=None)
 
 
+def _free_result(r):
+    _lib.lib().gpsm_result_free(C.byref(r))
+
+
 def _result(r, q):
     return MatchResult(int(r.count), int(r.hash), list(r.order[:q]), [int(x) for x in r.level_rows[:q]],
                        list(r.cand[:q]), float(r.device_ms), int(r.status), int(r.join_work),
@@ -215,9 +219,14 @@ class ResidentGraph:
         res = _result(r, q.n)
         if kw.get("want_tuples"):
             nt = int(r.n_tuples)
-            res.tuples = np.ctypeslib.as_array(r.tuples, shape=(max(nt * q.n, 1),))[:nt * q.n].reshape(
-                nt, q.n).copy() if nt else np.zeros((0, q.n), dtype=np.uint32)
-            _lib.lib().gpsm_result_free(C.byref(r))
+            if nt:
+                # the library's buffer itself, released with the last array over it
+                buf = (C.c_uint32 * (nt * q.n)).from_address(C.addressof(r.tuples.contents))
+                weakref.finalize(buf, _free_result, r).atexit = False
+                res.tuples = np.frombuffer(buf, dtype=np.uint32).reshape(nt, q.n)
+            else:
+                res.tuples = np.zeros((0, q.n), dtype=np.uint32)
+                _free_result(r)
         return res
 
     def match_batch(self, queries, explicit_orders=None, **kw):
