@@ -66,9 +66,13 @@ int DevBuf::ensure(size_t nbytes) {
   bytes = 0;
   size_t want = std::max<size_t>(nbytes + nbytes / 4, 4096);
   if (hipMalloc(&ptr, want) != hipSuccess) {
-    ptr = nullptr;
     (void)hipGetLastError();
-    return GPSM_ENOMEM;
+    if (pool) pool->release();
+    if (!pool || hipMalloc(&ptr, want) != hipSuccess) {
+      ptr = nullptr;
+      (void)hipGetLastError();
+      return GPSM_ENOMEM;
+    }
   }
   bytes = want;
   return GPSM_OK;
@@ -136,69 +140,6 @@ hipEvent_t Prof::get() {
 }
 
 }  // namespace gpsm
-
-namespace {
-
-// Hub adjacency bitmaps of a freshly uploaded graph (see DevGraph::hub_of).
-// Without room for them the graph has no hubs and every edge test searches.
-int build_hubs(gpsm_ctx* c, const uint32_t* row_offset, gpsm_graph* g) {
-  DevGraph& d = g->dg;
-  const uint32_t n = d.n;
-  auto deg = [&](uint32_t v) { return row_offset[v + 1] - row_offset[v]; };
-  auto count_over = [&](uint64_t D) {
-    uint64_t k = 0;
-    for (uint32_t v = 0; v < n; ++v) k += deg(v) > D;
-    return k;
-  };
-  uint64_t D = std::max<uint32_t>(c->hub_min_degree, 1);
-  uint64_t nh = c->hub_max_bytes ? count_over(D) : 0;
-  while (nh && nh * d.W * 4ull > c->hub_max_bytes) nh = count_over(D *= 2);
-  std::vector<uint32_t> hub_of(n, ~0u), hubs, block_base(1, 0);
-  if (nh) {
-    for (uint32_t v = 0; v < n; ++v)
-      if (deg(v) > D) {
-        hub_of[v] = (uint32_t)hubs.size();
-        hubs.push_back(v);
-        block_base.push_back(block_base.back() + (deg(v) + 63) / 64);  // 64-entry blocks, one wave each
-      }
-  }
-  if (hipMalloc(&d.hub_of, sizeof(uint32_t) * n) != hipSuccess) {
-    (void)hipGetLastError();
-    return GPSM_ENOMEM;
-  }
-  uint32_t* tmp = nullptr;
-  if (!hubs.empty()) {
-    if (hipMalloc(&d.hub_bits, sizeof(uint32_t) * (size_t)hubs.size() * d.W) != hipSuccess ||
-        hipMalloc(&tmp, sizeof(uint32_t) * (hubs.size() + block_base.size())) != hipSuccess) {
-      // no room: no hubs
-      (void)hipGetLastError();
-      hipFree(d.hub_bits);
-      d.hub_bits = nullptr;
-      hubs.clear();
-      std::fill(hub_of.begin(), hub_of.end(), ~0u);
-    }
-  }
-  d.nhub = (uint32_t)hubs.size();
-  d.hub_degree = d.nhub ? (uint32_t)D : 0;
-  hipStream_t s = c->stream;
-  if (hipMemcpyAsync(d.hub_of, hub_of.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, s) != hipSuccess)
-    return GPSM_EDEVICE;
-  if (d.nhub) {
-    launch_fill_u32(d.hub_bits, 0u, (uint64_t)d.nhub * d.W, s);
-    if (hipMemcpyAsync(tmp, hubs.data(), sizeof(uint32_t) * hubs.size(), hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(tmp + hubs.size(), block_base.data(), sizeof(uint32_t) * block_base.size(),
-                       hipMemcpyHostToDevice, s) != hipSuccess)
-      return GPSM_EDEVICE;
-    launch_hub_bits(d, tmp, tmp + hubs.size(), block_base.back(), s);
-  }
-  const bool ok = hipStreamSynchronize(s) == hipSuccess && hipGetLastError() == hipSuccess;
-  hipFree(tmp);
-  if (!ok) return GPSM_EDEVICE;
-  g->bytes += sizeof(uint32_t) * ((uint64_t)n + (uint64_t)d.nhub * d.W);
-  return GPSM_OK;
-}
-
-}  // namespace
 
 // ---------------------------------------------------------------------------
 
@@ -323,6 +264,7 @@ void gpsm_shutdown(gpsm_ctx* c) {
   for (auto& b : c->bufs) b.release();
   for (auto& b : c->h_stage) b.release();
   c->arena.release();
+  c->pool.release();
   hipEventDestroy(c->ev0);
   hipEventDestroy(c->ev1);
   hipEventDestroy(c->ev_fork);
@@ -359,76 +301,121 @@ int gpsm_scan_u32_noalloc(gpsm_ctx* c, const uint32_t* d_in, uint32_t* d_out, ui
 
 namespace {
 
-void free_graph_arrays(DevGraph& d) {
-  hipFree(d.row);
-  hipFree(d.col);
-  hipFree(d.key);
-  hipFree(d.ckey);
-  hipFree(d.fchunk);
-  hipFree(d.wrange);
-  hipFree(d.hub_of);
-  hipFree(d.hub_bits);
+// The graph's arrays back to the context's pool (its stream waited for).
+void free_graph_arrays(gpsm_ctx* c, DevGraph& d) {
+  for (uint32_t* p : {d.row, d.col, d.key, d.ckey, d.fchunk, d.wrange, d.hub_of, d.hub_bits}) c->pool.give(p);
   d = DevGraph();
+}
+
+// Distinct labels of a graph and their counts from the device's histogram, or
+// by sorting where a label is LABEL_HIST or more; false if a label is 0 or
+// there are too many.
+bool label_stats(GraphStats& st, const uint32_t* labels, const uint32_t* hist) {
+  if (hist[0]) return false;
+  if (!hist[LABEL_HIST]) {
+    for (uint32_t l = 1; l < LABEL_HIST; ++l)
+      if (hist[l]) {
+        st.label_value.push_back(l);
+        st.label_count.push_back(hist[l]);
+      }
+  } else {
+    std::vector<uint32_t> lv(labels, labels + st.n);
+    std::sort(lv.begin(), lv.end());
+    for (uint32_t i = 0; i < st.n; ++i) {
+      if (i == 0 || lv[i] != lv[i - 1]) {
+        st.label_value.push_back(lv[i]);
+        st.label_count.push_back(0);
+      }
+      st.label_count.back()++;
+    }
+  }
+  return st.label_value.size() <= MAX_LABELS;
 }
 
 // The rest of a resident graph once row/col are on the device: label
 // statistics, the label/degree keys, the filter's vertex ranges and the hub
-// bitmaps.  row_offset and labels are host copies.  On failure g is freed.
-int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* row_offset, const uint32_t* labels) {
+// bitmaps, on the device but for the choice of labels and hubs.  labels: host
+// copy.  check: the rows are the caller's and validated here (GPSM_EINVAL).
+// On failure g is freed.
+int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check) {
   DevGraph& d = g->dg;
   const uint32_t n = d.n;
+  hipStream_t s = c->stream;
+  uint32_t* tmp = nullptr;
   auto fail = [&](int code) {
-    free_graph_arrays(d);
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(s);
+    c->pool.give(tmp);
+    free_graph_arrays(c, d);
     delete g;
     return code;
   };
-  GraphStats& s = g->stats;
-  s.n = n;
-  s.adj = d.adj;
-  std::vector<uint32_t> lv(labels, labels + n);
-  std::sort(lv.begin(), lv.end());
-  if (lv[0] == 0) return fail(GPSM_EINVAL);
-  for (uint32_t i = 0; i < n; ++i) {
-    if (i == 0 || lv[i] != lv[i - 1]) {
-      s.label_value.push_back(lv[i]);
-      s.label_count.push_back(0);
-    }
-    s.label_count.back()++;
-  }
-  if (s.label_value.size() > MAX_LABELS) return fail(GPSM_EINVAL);
-  std::vector<uint32_t> key(n);
-  for (uint32_t v = 0; v < n; ++v) {
-    uint32_t deg = row_offset[v + 1] - row_offset[v];
-    key[v] = (s.dense(labels[v]) << KEY_DEG_BITS) | std::min(deg, KEY_DEG_MASK);
-  }
+  GraphStats& st = g->stats;
+  st.n = n;
+  st.adj = d.adj;
   d.W = words_of(n);
   d.NB = nblocks_of(n);
-  std::vector<uint32_t> fch;
-  filter_chunks(n, row_offset, fch);
-  d.nfchunk = (uint32_t)fch.size() - 1;
-  std::vector<uint32_t> wr(d.W);
-  for (uint32_t w = 0, r = 0; w < d.W; ++w) {
-    while (fch[r + 1] <= 32 * w) ++r;
-    wr[w] = r;
-  }
-  if (hipMalloc(&d.key, sizeof(uint32_t) * n) != hipSuccess ||
-      hipMalloc(&d.ckey, sizeof(uint32_t) * std::max<uint64_t>(d.adj, 1)) != hipSuccess ||
-      hipMalloc(&d.fchunk, sizeof(uint32_t) * fch.size()) != hipSuccess ||
-      hipMalloc(&d.wrange, sizeof(uint32_t) * d.W) != hipSuccess) {
-    (void)hipGetLastError();
-    return fail(GPSM_ENOMEM);
-  }
-  if (hipMemcpyAsync(d.key, key.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-      hipMemcpyAsync(d.fchunk, fch.data(), sizeof(uint32_t) * fch.size(), hipMemcpyHostToDevice, c->stream) !=
-          hipSuccess ||
-      hipMemcpyAsync(d.wrange, wr.data(), sizeof(uint32_t) * d.W, hipMemcpyHostToDevice, c->stream) != hipSuccess) {
-    (void)hipGetLastError();
+  // scratch: what the host reads (row check, number of ranges, label and hub
+  // counts), the labels, the ranges' ends or the hubs' lists
+  constexpr uint32_t kRead = 4 + LABEL_HIST + 1 + HUB_STEPS;
+  const uint64_t head = (kRead + 1) & ~1u, lw = ((uint64_t)n + 1) & ~1ull;
+  if (!c->pool.take(&tmp, head + lw + range_words(n))) return fail(GPSM_ENOMEM);
+  uint32_t* dlab = tmp + head;
+  uint32_t* ends = dlab + lw;
+  launch_fill_u32(tmp, 0u, kRead, s);
+  if (hipMemcpyAsync(dlab, labels, sizeof(uint32_t) * n, hipMemcpyHostToDevice, s) != hipSuccess)
     return fail(GPSM_EDEVICE);
+  const uint32_t min_degree = std::max<uint32_t>(c->hub_min_degree, 1);
+  if (check) launch_check_rows(d.row, d.col, n, tmp, s);
+  launch_vertex_stats(d.row, dlab, n, min_degree, tmp + 4, tmp + 4 + LABEL_HIST + 1, s);
+  launch_range_ends(d.row, n, ends, reinterpret_cast<unsigned long long*>(tmp + 2), s);
+  uint32_t h[kRead];
+  if (hipMemcpyAsync(h, tmp, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipStreamSynchronize(s) != hipSuccess)
+    return fail(GPSM_EDEVICE);
+  if (h[0] || !label_stats(st, labels, h + 4)) return fail(GPSM_EINVAL);
+  d.nfchunk = h[2];
+  // hubs: the degree doubles until their bitmaps fit
+  const uint32_t* over = h + 4 + LABEL_HIST + 1;
+  uint64_t D = min_degree, nh = 0;
+  for (uint32_t k = 1; k < HUB_STEPS; ++k) nh += over[k];
+  if (!c->hub_max_bytes) nh = 0;
+  for (uint32_t k = 1; nh && nh * d.W * 4ull > c->hub_max_bytes; ++k, D *= 2) nh -= over[k];
+  const uint32_t nl = (uint32_t)st.label_value.size();
+  uint32_t* hub_tmp = nullptr;
+  if (!c->pool.take(&d.key, n) || !c->pool.take(&d.ckey, std::max<uint64_t>(d.adj, 1)) ||
+      !c->pool.take(&d.fchunk, (uint64_t)d.nfchunk + 1) || !c->pool.take(&d.wrange, d.W) ||
+      !c->pool.take(&d.hub_of, n))
+    return fail(GPSM_ENOMEM);
+  if (nh && (!c->pool.take(&d.hub_bits, (size_t)nh * d.W) || !c->pool.take(&hub_tmp, hub_words(n, nh)))) {
+    // no room: no hubs, every edge test searches
+    c->pool.give(d.hub_bits);
+    d.hub_bits = nullptr;
+    nh = 0;
   }
-  launch_neighbour_keys(d, c->stream);
-  if (hipStreamSynchronize(c->stream) != hipSuccess || hipGetLastError() != hipSuccess) return fail(GPSM_EDEVICE);
-  g->bytes = sizeof(uint32_t) * ((uint64_t)n + 1 + 2 * d.adj + n + fch.size() + d.W);
-  if (int rc = build_hubs(c, row_offset, g)) return fail(rc);
+  d.nhub = (uint32_t)nh;
+  d.hub_degree = nh ? (uint32_t)D : 0;
+  // the label values over the histogram (it has been read)
+  bool ok = hipMemcpyAsync(tmp + 4, st.label_value.data(), sizeof(uint32_t) * nl, hipMemcpyHostToDevice, s) ==
+            hipSuccess;
+  if (ok) {
+    launch_vertex_keys(d, dlab, tmp + 4, nl, s);
+    launch_ranges(d, ends, s);
+    launch_neighbour_keys(d, s);
+    if (nh) {
+      launch_fill_u32(d.hub_bits, 0u, nh * d.W, s);
+      launch_hubs(d, hub_tmp, s);
+    } else {
+      launch_fill_u32(d.hub_of, ~0u, n, s);
+    }
+    ok = hipGetLastError() == hipSuccess;
+  }
+  ok = hipStreamSynchronize(s) == hipSuccess && ok;
+  c->pool.give(hub_tmp);
+  if (!ok) return fail(GPSM_EDEVICE);
+  c->pool.give(tmp);
+  g->bytes = sizeof(uint32_t) *
+             ((uint64_t)n + 1 + 2 * d.adj + n + d.nfchunk + 1 + d.W + (uint64_t)n + (uint64_t)d.nhub * d.W);
   return GPSM_OK;
 }
 
@@ -442,26 +429,20 @@ int gpsm_graph_upload(gpsm_ctx* c, uint32_t n, const uint32_t* row_offset, const
   *out = nullptr;
   const uint64_t A = row_offset[n];
   if (A && !col) return GPSM_EINVAL;
-  // validate the CSR: monotone offsets, sorted rows, no self-loops/duplicates
+  // monotone offsets here (the device walks them); the rows' order, their
+  // vertices and the labels on the device (finish_graph)
   if (row_offset[0] != 0) return GPSM_EINVAL;
-  for (uint32_t v = 0; v < n; ++v) {
-    if (row_offset[v + 1] < row_offset[v]) return GPSM_EINVAL;
-    for (uint32_t e = row_offset[v]; e < row_offset[v + 1]; ++e) {
-      if (col[e] >= n || col[e] == v) return GPSM_EINVAL;
-      if (e > row_offset[v] && col[e] <= col[e - 1]) return GPSM_EINVAL;
-    }
-    if (labels[v] == 0) return GPSM_EINVAL;
-  }
+  bool monotone = true;
+  for (uint32_t v = 0; v < n; ++v) monotone &= row_offset[v + 1] >= row_offset[v];
+  if (!monotone) return GPSM_EINVAL;
   hipSetDevice(c->device);
   gpsm_graph* g = new gpsm_graph();
   g->ctx = c;
   DevGraph& d = g->dg;
   d.n = n;
   d.adj = A;
-  if (hipMalloc(&d.row, sizeof(uint32_t) * (n + 1)) != hipSuccess ||
-      hipMalloc(&d.col, sizeof(uint32_t) * std::max<uint64_t>(A, 1)) != hipSuccess) {
-    (void)hipGetLastError();
-    free_graph_arrays(d);
+  if (!c->pool.take(&d.row, (size_t)n + 1) || !c->pool.take(&d.col, std::max<uint64_t>(A, 1))) {
+    free_graph_arrays(c, d);
     delete g;
     return GPSM_ENOMEM;
   }
@@ -469,11 +450,12 @@ int gpsm_graph_upload(gpsm_ctx* c, uint32_t n, const uint32_t* row_offset, const
           hipSuccess ||
       (A && hipMemcpyAsync(d.col, col, sizeof(uint32_t) * A, hipMemcpyHostToDevice, c->stream) != hipSuccess)) {
     (void)hipGetLastError();
-    free_graph_arrays(d);
+    (void)hipStreamSynchronize(c->stream);
+    free_graph_arrays(c, d);
     delete g;
     return GPSM_EDEVICE;
   }
-  if (int rc = finish_graph(c, g, row_offset, labels)) return rc;
+  if (int rc = finish_graph(c, g, labels, true)) return rc;
   *out = g;
   return GPSM_OK;
 }
@@ -488,23 +470,14 @@ int gpsm_graph_upload_edges(gpsm_ctx* c, uint32_t n, uint64_t m, const uint32_t*
   DevGraph& d = g->dg;
   d.n = n;
   uint64_t adj = 0;
-  int rc = build_csr_from_edges(n, m, src, dst, c->stream, &d.row, &d.col, &adj);
+  int rc = build_csr_from_edges(n, m, src, dst, c->pool, c->stream, &d.row, &d.col, &adj);
   if (rc) {
-    free_graph_arrays(d);
+    free_graph_arrays(c, d);
     delete g;
     return rc;
   }
   d.adj = adj;
-  std::vector<uint32_t> ro(n + 1);
-  if (hipMemcpyAsync(ro.data(), d.row, sizeof(uint32_t) * (n + 1), hipMemcpyDeviceToHost, c->stream) !=
-          hipSuccess ||
-      hipStreamSynchronize(c->stream) != hipSuccess) {
-    (void)hipGetLastError();
-    free_graph_arrays(d);
-    delete g;
-    return GPSM_EDEVICE;
-  }
-  if ((rc = finish_graph(c, g, ro.data(), labels))) return rc;
+  if ((rc = finish_graph(c, g, labels, false))) return rc;
   *out = g;
   return GPSM_OK;
 }
@@ -535,7 +508,7 @@ int gpsm_graph_free(gpsm_graph* g) {
   if (!g) return GPSM_EINVAL;
   hipSetDevice(g->ctx->device);
   hipStreamSynchronize(g->ctx->stream);
-  free_graph_arrays(g->dg);
+  free_graph_arrays(g->ctx, g->dg);
   g->directed.release();
   delete g;
   return GPSM_OK;

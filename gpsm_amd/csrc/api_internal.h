@@ -8,6 +8,7 @@
 #include "gpsm.h"
 #include "kernels/launch.h"
 #include "plan.h"
+#include "pool.h"
 
 namespace gpsm {
 
@@ -15,6 +16,7 @@ namespace gpsm {
 struct DevBuf {
   void* ptr = nullptr;
   size_t bytes = 0;
+  BlockPool* pool = nullptr;  // asked to return its idle blocks when an allocation fails
   int ensure(size_t nbytes);
   void release();
 };
@@ -181,7 +183,11 @@ struct gpsm_ctx {
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   char name[256] = {0};
+  gpsm::BlockPool pool;  // memory of this context's graphs
   gpsm::DevBuf bufs[gpsm::B_COUNT_];
+  gpsm_ctx() {
+    for (auto& b : bufs) b.pool = &pool;
+  }
   gpsm::Tuning tune;
   gpsm_mlp* planner = nullptr;
   std::vector<uint32_t> h_counts;

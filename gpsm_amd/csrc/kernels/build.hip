@@ -11,6 +11,7 @@
 
 #include "gpsm.h"
 #include "launch.h"
+#include "pool.h"
 #include "wave.h"
 
 namespace gpsm {
@@ -79,8 +80,8 @@ uint32_t grid_for(uint64_t items) {
 
 }  // namespace
 
-int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint32_t* dst, hipStream_t s,
-                         uint32_t** row, uint32_t** col, uint64_t* adj_out) {
+int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint32_t* dst, BlockPool& pool,
+                         hipStream_t s, uint32_t** row, uint32_t** col, uint64_t* adj_out) {
   *row = *col = nullptr;
   *adj_out = 0;
   const uint64_t M2 = 2 * m;
@@ -90,17 +91,17 @@ int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint
   unsigned long long *keys = nullptr, *sorted = nullptr, *d_count = nullptr;
   int rc = GPSM_OK;
   auto cleanup = [&]() {
-    hipFree(d_src);
-    hipFree(d_dst);
-    hipFree(d_bad);
-    hipFree(hist);
-    hipFree(hstart);
-    hipFree(flags);
-    hipFree(fpos);
-    hipFree(scratch);
-    hipFree(keys);
-    hipFree(sorted);
-    hipFree(d_count);
+    pool.give(d_src);
+    pool.give(d_dst);
+    pool.give(d_bad);
+    pool.give(hist);
+    pool.give(hstart);
+    pool.give(flags);
+    pool.give(fpos);
+    pool.give(scratch);
+    pool.give(keys);
+    pool.give(sorted);
+    pool.give(d_count);
   };
   // bits that can differ: the column (32) and the row, up to the sentinel row n
   unsigned rbits = 1;
@@ -108,19 +109,12 @@ int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint
   const unsigned end_bit = 32 + rbits;
   const uint64_t nhist = radix_hist_words(M2);
   const uint64_t sw = scan_scratch_words(std::max<uint64_t>(nhist, M2)) + 2;
-  if (hipMalloc(&d_bad, sizeof(uint32_t)) != hipSuccess ||
-      hipMalloc(&d_count, sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(row, sizeof(uint32_t) * ((size_t)n + 1)) != hipSuccess ||
-      (M2 && (hipMalloc(&d_src, sizeof(uint32_t) * m) != hipSuccess ||
-              hipMalloc(&d_dst, sizeof(uint32_t) * m) != hipSuccess ||
-              hipMalloc(&keys, sizeof(unsigned long long) * M2) != hipSuccess ||
-              hipMalloc(&sorted, sizeof(unsigned long long) * M2) != hipSuccess ||
-              hipMalloc(&hist, sizeof(uint32_t) * nhist) != hipSuccess ||
-              hipMalloc(&hstart, sizeof(uint32_t) * nhist) != hipSuccess ||
-              hipMalloc(&flags, sizeof(uint32_t) * M2) != hipSuccess ||
-              hipMalloc(&fpos, sizeof(uint32_t) * M2) != hipSuccess ||
-              hipMalloc(&scratch, sizeof(uint32_t) * sw) != hipSuccess))) {
-    (void)hipGetLastError();
+  if (!pool.take(&d_bad, 1) || !pool.take(&d_count, 1) || !pool.take(row, (size_t)n + 1) ||
+      (M2 && (!pool.take(&d_src, m) || !pool.take(&d_dst, m) || !pool.take(&keys, M2) || !pool.take(&sorted, M2) ||
+              !pool.take(&hist, nhist) || !pool.take(&hstart, nhist) || !pool.take(&flags, M2) ||
+              !pool.take(&fpos, M2) || !pool.take(&scratch, sw)))) {
+    pool.give(*row);
+    *row = nullptr;
     cleanup();
     return GPSM_ENOMEM;
   }
@@ -163,8 +157,7 @@ int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint
       rc = GPSM_EDEVICE;
     } else {
       *adj_out = adj32;
-      if (hipMalloc(col, sizeof(uint32_t) * std::max<uint64_t>(adj32, 1)) != hipSuccess) {
-        (void)hipGetLastError();
+      if (!pool.take(col, std::max<uint64_t>(adj32, 1))) {
         rc = GPSM_ENOMEM;
       } else {
         if (adj32)
@@ -173,10 +166,11 @@ int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint
       }
     }
   }
+  if (rc) (void)hipStreamSynchronize(s);  // nothing queued still uses what is given back
   cleanup();
   if (rc) {
-    hipFree(*row);
-    hipFree(*col);
+    pool.give(*row);
+    pool.give(*col);
     *row = *col = nullptr;
   }
   return rc;

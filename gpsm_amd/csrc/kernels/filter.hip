@@ -450,21 +450,4 @@ void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, c
                      g.fchunk, items, nitems, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, stats);
 }
 
-void filter_chunks(uint32_t n, const uint32_t* row_offset, std::vector<uint32_t>& bounds) {
-  bounds.assign(1, 0);
-  uint32_t v = 0;
-  while (v < n) {
-    uint32_t end = v + 1;
-    uint64_t entries = row_offset[v + 1] - row_offset[v];
-    while (end < n && end - v < FCHUNK_VERTS) {
-      const uint64_t d = row_offset[end + 1] - row_offset[end];
-      if (entries + d > FCHUNK_ENTRIES) break;
-      entries += d;
-      ++end;
-    }
-    bounds.push_back(end);
-    v = end;
-  }
-}
-
 }  // namespace gpsm

@@ -40,15 +40,36 @@ struct DevGraph {
 constexpr uint32_t FCHUNK_VERTS = 1024;
 constexpr uint32_t FCHUNK_ENTRIES = 4096;
 
-// Boundaries of the filter's work items over a CSR (host side).
-void filter_chunks(uint32_t n, const uint32_t* row_offset, std::vector<uint32_t>& bounds);
+// graph.hip: what a resident graph holds besides its CSR, built from it.
+constexpr uint32_t LABEL_HIST = 4096, HUB_STEPS = 34;
+// hist (LABEL_HIST + 1 words) and hubs (HUB_STEPS), zeroed by the caller: the
+// labels' counts and the vertices by how often min_degree doubles below their
+// degree (vertex_stats_kernel).
+void launch_vertex_stats(const uint32_t* row, const uint32_t* label, uint32_t n, uint32_t min_degree, uint32_t* hist,
+                         uint32_t* hubs, hipStream_t s);
+// Sets *bad (zeroed by the caller) if a row of the CSR (offsets monotone, the
+// last one the length of col) is not strictly ascending, holds its own vertex
+// or one >= n.
+void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uint32_t* bad, hipStream_t s);
+// g.key from the vertices' labels and the nl distinct label values, ascending.
+void launch_vertex_keys(const DevGraph& g, const uint32_t* label, const uint32_t* value, uint32_t nl, hipStream_t s);
+// The filter's vertex ranges: their ends and their number (*total), then, with
+// g.fchunk and g.wrange allocated, those.  scratch: range_words(n) words.
+uint64_t range_words(uint32_t n);
+void launch_range_ends(const uint32_t* row, uint32_t n, uint32_t* scratch, unsigned long long* total, hipStream_t s);
+void launch_ranges(const DevGraph& g, const uint32_t* scratch, hipStream_t s);
+// g.hub_of and, with nhub of them above hub_degree and hub_bits zeroed, their
+// bitmaps.  scratch: hub_words(n, nhub) words, 8-byte aligned.
+uint64_t hub_words(uint32_t n, uint64_t nhub);
+void launch_hubs(const DevGraph& g, uint32_t* scratch, hipStream_t s);
 
 // build.hip: the undirected CSR of an edge list (host arrays src/dst of m
 // edges, either orientation; duplicates and self-loops dropped), built on
-// the device.  *row (n+1) and *col (*adj) are new device allocations.
-// GPSM_EINVAL if an endpoint is >= n.
-int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint32_t* dst, hipStream_t s,
-                         uint32_t** row, uint32_t** col, uint64_t* adj);
+// the device.  *row (n+1) and *col (*adj) are taken from pool, as is what the
+// build itself needs.  GPSM_EINVAL if an endpoint is >= n.
+class BlockPool;
+int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint32_t* dst, BlockPool& pool,
+                         hipStream_t s, uint32_t** row, uint32_t** col, uint64_t* adj);
 
 // Sets the adjacency bitmaps of the hubs: hub_bits (nhub * W words) must be
 // zero; hubs[h] is the vertex of bitmap h; block_base[h] = 64-entry blocks
