@@ -304,6 +304,7 @@ namespace {
 // The graph's arrays back to the context's pool (its stream waited for).
 void free_graph_arrays(gpsm_ctx* c, DevGraph& d) {
   for (uint32_t* p : {d.row, d.col, d.key, d.ckey, d.fchunk, d.wrange, d.hub_of, d.hub_bits}) c->pool.give(p);
+  c->pool.give(d.hparts);
   d = DevGraph();
 }
 
@@ -368,13 +369,14 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   const uint32_t min_degree = std::max<uint32_t>(c->hub_min_degree, 1);
   if (check) launch_check_rows(d.row, d.col, n, tmp, s);
   launch_vertex_stats(d.row, dlab, n, min_degree, tmp + 4, tmp + 4 + LABEL_HIST + 1, s);
-  launch_range_ends(d.row, n, ends, reinterpret_cast<unsigned long long*>(tmp + 2), s);
+  launch_range_ends(d.row, n, ends, reinterpret_cast<unsigned long long*>(tmp + 2), tmp + 1, s);
   uint32_t h[kRead];
   if (hipMemcpyAsync(h, tmp, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return fail(GPSM_EDEVICE);
   if (h[0] || !label_stats(st, labels, h + 4)) return fail(GPSM_EINVAL);
   d.nfchunk = h[2];
+  d.nhparts = h[1];
   // hubs: the degree doubles until their bitmaps fit
   const uint32_t* over = h + 4 + LABEL_HIST + 1;
   uint64_t D = min_degree, nh = 0;
@@ -385,6 +387,7 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   uint32_t* hub_tmp = nullptr;
   if (!c->pool.take(&d.key, n) || !c->pool.take(&d.ckey, std::max<uint64_t>(d.adj, 1)) ||
       !c->pool.take(&d.fchunk, (uint64_t)d.nfchunk + 1) || !c->pool.take(&d.wrange, d.W) ||
+      (d.nhparts && !c->pool.take(&d.hparts, d.nhparts)) ||
       !c->pool.take(&d.hub_of, n))
     return fail(GPSM_ENOMEM);
   if (nh && (!c->pool.take(&d.hub_bits, (size_t)nh * d.W) || !c->pool.take(&hub_tmp, hub_words(n, nh)))) {
@@ -400,7 +403,7 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
             hipSuccess;
   if (ok) {
     launch_vertex_keys(d, dlab, tmp + 4, nl, s);
-    launch_ranges(d, ends, s);
+    launch_ranges(d, ends, tmp, s);  // word 0 is still clear
     launch_neighbour_keys(d, s);
     if (nh) {
       launch_fill_u32(d.hub_bits, 0u, nh * d.W, s);
@@ -415,7 +418,8 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   if (!ok) return fail(GPSM_EDEVICE);
   c->pool.give(tmp);
   g->bytes = sizeof(uint32_t) *
-             ((uint64_t)n + 1 + 2 * d.adj + n + d.nfchunk + 1 + d.W + (uint64_t)n + (uint64_t)d.nhub * d.W);
+             ((uint64_t)n + 1 + 2 * d.adj + n + d.nfchunk + 1 + d.W + (uint64_t)n + 2ull * d.nhparts +
+              (uint64_t)d.nhub * d.W);
   return GPSM_OK;
 }
 
@@ -652,7 +656,7 @@ struct PhaseSig {
   void add(const void* p) { w.push_back((uint64_t)(uintptr_t)p); }
   void add_graph(const DevGraph& g) {
     add(g.n), add(g.adj), add(g.W), add(g.NB), add(g.row), add(g.col), add(g.key), add(g.ckey), add(g.fchunk),
-        add(g.nfchunk), add(g.wrange), add(g.hub_of), add(g.hub_bits), add(g.nhub), add(g.hub_degree);
+        add(g.nfchunk), add(g.wrange), add(g.hparts), add(g.nhparts), add(g.hub_of), add(g.hub_bits), add(g.nhub), add(g.hub_degree);
   }
 };
 
@@ -725,7 +729,10 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   c->arena.reset();
   gpsm_opts o{};
   if (opts) o = *opts;
-  const uint32_t fblock = o.block ? o.block : c->tune.filter_block;
+  uint32_t fblock = o.block ? o.block : c->tune.filter_block;
+  if (fblock != 64 && fblock != 128 && fblock != 256) fblock = 256;
+  uint32_t& fresident = c->filter_resident[fblock / 128];
+  if (!fresident) fresident = filter_resident(fblock);
   // a level buffer must hold at least two expansion steps (2 x 4 x 256 rows)
   const uint32_t cap = std::max<uint32_t>(o.join_cap ? o.join_cap : c->tune.join_cap, 2048);
   const uint32_t wg_per_cu = c->tune.join_wg_per_cu;
@@ -787,6 +794,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   std::vector<InitOp> init;
   std::vector<FilterOp> fops;
   std::vector<uint32_t> step_off(maxsteps + 1, 0), nbr_slot, nbr_lo, nbr_hi;
+  std::vector<uint8_t> explore(maxsteps, 0);  // supersteps with explore ops
   for (uint32_t b = 0; b < nq; ++b)
     if (Q[b].active) init.push_back({Q[b].vbase + Q[b].fs.start, Q[b].fs.start_lo, Q[b].fs.start_hi});
   for (uint32_t sidx = 0; sidx < maxsteps; ++sidx) {
@@ -801,6 +809,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       op.nv = (uint32_t)fsx.v.size();
       op.nbr_off = (uint32_t)nbr_slot.size();
       op.mark = op.need = ~0u;
+      if (fsx.type == OP_EXPLORE) explore[sidx] = 1;
       if (fsx.type == OP_REFINE) {
         op.mark = b * 4 + fsx.round;
         if (fsx.round > 0) op.need = b * 4 + fsx.round - 1;
@@ -824,7 +833,8 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   uint32_t max_ops = 0;  // ops of the largest superstep
   for (uint32_t sidx = 0; sidx < maxsteps; ++sidx) max_ops = std::max(max_ops, step_off[sidx + 1] - step_off[sidx]);
   if ((rc = c->bufs[B_FITEMS].ensure(sizeof(uint2) * std::max<uint64_t>((uint64_t)max_ops * dg.nfchunk, 1))) ||
-      (rc = c->bufs[B_FNITEMS].ensure(sizeof(uint32_t) * std::max<uint32_t>(maxsteps, 1))) ||
+      (rc = c->bufs[B_FDROPS].ensure(sizeof(uint2) * std::max<uint64_t>((uint64_t)max_ops * dg.nhparts, 1))) ||
+      (rc = c->bufs[B_FNITEMS].ensure(sizeof(uint32_t) * 2 * std::max<uint32_t>(maxsteps, 1))) ||
       (rc = c->bufs[B_RFLAGS].ensure(sizeof(uint32_t) * 4 * (uint64_t)std::max<uint32_t>(nq, 1))))
     return rc;
   // work counters (profile mode 2): one slot per filter superstep, then the
@@ -840,11 +850,12 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if (o.use_graph) {
     sig_a.add(uint64_t{0});
     sig_a.add_graph(dg);
-    for (int i : {B_BITMAPS, B_FNITEMS, B_RFLAGS, B_INIT, B_FOPS, B_NBR_SLOT, B_NBR_LO, B_NBR_HI, B_FITEMS, B_SEGC,
+    for (int i : {B_FDROPS, B_BITMAPS, B_FNITEMS, B_RFLAGS, B_INIT, B_FOPS, B_NBR_SLOT, B_NBR_LO, B_NBR_HI, B_FITEMS, B_SEGC,
                   B_COUNTS})
       sig_a.add(c->bufs[i].ptr);
     sig_a.add(nslots), sig_a.add(maxsteps), sig_a.add(nq), sig_a.add(init.size()), sig_a.add(fblock);
     for (uint32_t v : step_off) sig_a.add(v);
+    for (uint8_t v : explore) sig_a.add((uint64_t)v);
   }
   bool replayed = o.use_graph && replay_cached(c, 0, sig_a.w, s, &rc);
   if (replayed && rc) return rc;
@@ -852,7 +863,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     bool captured = false;
     if (o.use_graph && hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) captured = true;
     launch_fill_u32(bitmaps, 0u, (uint64_t)nslots * W, s);
-    if (maxsteps) launch_fill_u32(dptr<uint32_t>(c, B_FNITEMS), 0u, maxsteps, s);
+    if (maxsteps) launch_fill_u32(dptr<uint32_t>(c, B_FNITEMS), 0u, 2 * maxsteps, s);
     launch_fill_u32(dptr<uint32_t>(c, B_RFLAGS), 0u, 4ull * std::max<uint32_t>(nq, 1), s);
     if (counters) launch_fill_u32(reinterpret_cast<uint32_t*>(fstats), 0u, 2ull * fstat_step * nstat_slots, s);
     {
@@ -865,9 +876,9 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       const uint32_t nops_s = step_off[sidx + 1] - step_off[sidx];
       hipEvent_t a = pbegin(K_FILTER);
       launch_filter_step(dg, dptr<FilterOp>(c, B_FOPS) + step_off[sidx], nops_s, dptr<uint32_t>(c, B_NBR_SLOT),
-                         dptr<uint32_t>(c, B_NBR_LO), dptr<uint32_t>(c, B_NBR_HI), bitmaps, fblock,
-                         65536, dptr<uint2>(c, B_FITEMS), dptr<uint32_t>(c, B_FNITEMS) + sidx,
-                         dptr<uint32_t>(c, B_RFLAGS),
+                         dptr<uint32_t>(c, B_NBR_LO), dptr<uint32_t>(c, B_NBR_HI), bitmaps, fblock, fresident,
+                         explore[sidx], dptr<uint2>(c, B_FITEMS), dptr<uint32_t>(c, B_FNITEMS) + 2 * sidx,
+                         dptr<uint2>(c, B_FDROPS), dptr<uint32_t>(c, B_RFLAGS),
                          counters ? fstats + fstat_step * sidx : nullptr, s);
       pend(K_FILTER, a, 4.0 * W * nops_s, counters ? (int)sidx : -1);
     }

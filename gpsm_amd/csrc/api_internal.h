@@ -81,7 +81,8 @@ enum BufId {
   B_TEXT_WG,     // ... scan scratch, per-workgroup lengths and offsets
   B_TEXT_OUT,    // ... the chunk's text
   B_FITEMS,      // filter superstep: (op, vertex range) pairs with candidates
-  B_FNITEMS,     // ... their number, one counter per superstep
+  B_FNITEMS,     // ... their number and that of the dropped hubs, two counters per superstep
+  B_FDROPS,      // ... hubs that leave their op's candidates
   B_CDESC,       // candidate-edge tables of reversed plan edges (counted again)
   B_LDESC,       // candidate-edge tables whose lists are written
   B_WDESC,       // last levels' tables counted from records
@@ -183,6 +184,7 @@ struct gpsm_ctx {
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   char name[256] = {0};
+  uint32_t filter_resident[3] = {0, 0, 0};  // resident superstep workgroups of 64, 128, 256 threads (0: not asked yet)
   gpsm::BlockPool pool;  // memory of this context's graphs
   gpsm::DevBuf bufs[gpsm::B_COUNT_];
   gpsm_ctx() {

@@ -176,12 +176,24 @@ struct WaveLds {
   uint32_t lim[WAVE];
 };
 
+// list null: every (op, range) pair is an item (nops * chunks of them, the ops
+// whose need flag is clear leave theirs).  After the listed or all pairs, nhp
+// hub parts per op: a vertex with more entries than a range holds is not
+// explored with its range but in parts of HUB_PART entries, one wave each
+// (one wave walking the 30,000 entries of a hub of the 1M Chung-Lu graph took
+// 100-360 us, the whole superstep; 25 us in parts).  Every part decides for
+// itself how far the hub meets its op's neighbours, usually in its first
+// steps, so C(u) must not change under them: a hub that leaves C(u) goes to
+// drops, cleared by the next launch.
 __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __restrict__ row,
                                                           const uint32_t* __restrict__ col,
                                                           const uint32_t* __restrict__ ckey, uint32_t W,
                                                           const uint32_t* __restrict__ fchunk,
                                                           const uint2* __restrict__ list,
-                                                          const uint32_t* __restrict__ nlist,
+                                                          const uint32_t* __restrict__ nlist, uint32_t chunks,
+                                                          uint32_t nops, const uint2* __restrict__ hparts,
+                                                          uint32_t nhp, uint2* __restrict__ drops,
+                                                          uint32_t* __restrict__ ndrops,
                                                           const FilterOp* __restrict__ ops,
                                                           const uint32_t* __restrict__ nbr_slot,
                                                           const uint32_t* __restrict__ nbr_lo,
@@ -192,21 +204,34 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
   extern __shared__ unsigned char lds_raw[];
   WaveLds& L = reinterpret_cast<WaveLds*>(lds_raw)[threadIdx.x / WAVE];
   const uint32_t lane = lane_id();
-  const uint32_t items = uniform(*nlist);
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  const uint32_t pairs = list ? uniform(*nlist) : nops * chunks, items = pairs + nops * nhp;
+  const uint32_t wave = uniform((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
   const uint32_t nwaves = (gridDim.x * blockDim.x) / WAVE;
   // per-lane tallies for the optional byte accounting, over all items
   unsigned long long t_cand = 0;
   uint32_t t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
 
   // the next item's list entry is loaded while the current one runs
-  uint2 nxt = wave < items ? list[wave] : make_uint2(0u, 0u);
+  uint2 nxt = list && wave < pairs ? list[wave] : make_uint2(0u, 0u);
   for (uint32_t it = wave; it < items; it += nwaves) {
-    const uint2 item = nxt;
-    if (it + nwaves < items) nxt = list[it + nwaves];
-    const uint32_t o = uniform(item.x);
-    const uint32_t c = uniform(item.y);
+    const bool hub = it >= pairs;
+    uint32_t o, c;
+    if (hub) {
+      o = (it - pairs) / nhp;
+      c = (it - pairs) % nhp;
+    } else if (list) {
+      const uint2 item = nxt;
+      if (it + nwaves < pairs) nxt = list[it + nwaves];
+      o = uniform(item.x);
+      c = uniform(item.y);
+    } else {
+      o = it / chunks;
+      c = it % chunks;
+      const uint32_t need = uniform(ops[o].need);
+      if (need != ~0u && uniform(rflags[need]) == 0) continue;
+    }
     const uint32_t type = uniform(ops[o].type);
+    if (hub && type != OP_EXPLORE) continue;
     const uint32_t nv = uniform(ops[o].nv);
     const uint32_t nb = uniform(ops[o].nbr_off);
     uint32_t* bm_u = bitmaps + (size_t)uniform(ops[o].u_slot) * W;
@@ -214,7 +239,16 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
 
     // collect: candidates of vertex range [v_lo, v_hi), ascending; lane l
     // reads bitmap word w_lo + l and keeps the range's bits of it
-    const uint32_t v_lo = uniform(fchunk[c]), v_hi = uniform(fchunk[c + 1]);
+    uint32_t v_lo, v_hi, part = 0;
+    if (hub) {
+      const uint2 hp = hparts[c];
+      v_lo = uniform(hp.x);
+      v_hi = v_lo + 1;
+      part = uniform(hp.y);
+    } else {
+      v_lo = uniform(fchunk[c]);
+      v_hi = uniform(fchunk[c + 1]);
+    }
     const uint32_t w_lo = v_lo >> 5, nw = ((v_hi - 1) >> 5) - w_lo + 1;
     const uint32_t wi = w_lo + lane;
     uint32_t w = 0;
@@ -226,7 +260,8 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
     const uint32_t pc = __popc(w);
     const uint32_t incl = wave_incl_scan(pc);
     const uint32_t C = uniform(__shfl(incl, WAVE - 1, WAVE));
-    if (lane == 0) t_cand += C;
+    if (C == 0) continue;
+    if (lane == 0 && part == 0) t_cand += C;
     {
       uint32_t pos = incl - pc, x = w;
       while (x) {
@@ -239,10 +274,14 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
 
     for (uint32_t s0 = 0; s0 < C; s0 += WAVE) {
       // lane = one candidate of the sub-chunk
-      const bool mine = s0 + lane < C;
+      bool mine = s0 + lane < C;
       const uint32_t id = mine ? L.cand[s0 + lane] : 0u;
       const uint32_t off = mine ? row[id] : 0u;
-      const uint32_t deg = mine ? row[id + 1] - off : 0u;
+      uint32_t deg = mine ? row[id + 1] - off : 0u;
+      if (!hub && type == OP_EXPLORE && deg > FCHUNK_ENTRIES) {  // explored by its parts
+        mine = false;
+        deg = 0;
+      }
       L.hit[lane] = 0;
       uint32_t cur = 0;  // entries of this candidate already examined
       unsigned long long h = 0;
@@ -330,13 +369,17 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
         // first neighbour without a match: mu leaves C(u); neighbours before
         // it received all of mu's matching data neighbours (match/Match.cu:547-600)
         const uint32_t ff = h == full ? nv : (uint32_t)(__ffsll((long long)~h) - 1);
-        if (mine && ff < nv) clear_bit(bm_u, id);
+        if (mine && ff < nv) {
+          if (!hub) clear_bit(bm_u, id);
+          else if (part == 0) drops[atomicAdd(ndrops, 1u)] = make_uint2(ops[o].u_slot, id);
+        }
         const uint32_t lim = mine ? ff : 0u;
-        const uint32_t len = lim ? deg : 0u;
+        const uint32_t p0 = part * HUB_PART;  // a part's entries; 0 and all of them else
+        const uint32_t len = lim ? (hub ? min(HUB_PART, deg - p0) : deg) : 0u;
         const uint32_t lincl = wave_incl_scan(len);
         const uint32_t T = uniform(__shfl(lincl, WAVE - 1, WAVE));
         L.pre[lane] = lincl - len;
-        L.base[lane] = off;
+        L.base[lane] = off + p0;
         L.lim[lane] = lim;
         wave_sync();
         // pass 2: every matching data neighbour of a surviving prefix enters C(v_i)
@@ -407,6 +450,13 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
   }
 }
 
+// Hubs that leave their op's C(u) (filter_step_kernel's drops).
+__global__ void drop_hubs_kernel(const uint2* __restrict__ drops, const uint32_t* __restrict__ ndrops,
+                                 uint32_t* __restrict__ bitmaps, uint32_t W) {
+  for (uint32_t i = threadIdx.x; i < *ndrops; i += blockDim.x)
+    clear_bit(bitmaps + (size_t)drops[i].x * W, drops[i].y);
+}
+
 }  // namespace
 
 void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* bitmaps, hipStream_t s) {
@@ -418,18 +468,21 @@ void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* 
 
 void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, const uint32_t* nbr_slot,
                         const uint32_t* nbr_lo, const uint32_t* nbr_hi, uint32_t* bitmaps, uint32_t block,
-                        uint32_t max_wg, uint2* items, uint32_t* nitems, uint32_t* rflags,
-                        unsigned long long* stats, hipStream_t s) {
+                        uint32_t resident, bool explore, uint2* items, uint32_t* counters, uint2* drops,
+                        uint32_t* rflags, unsigned long long* stats, hipStream_t s) {
   if (!nops) return;
-  if (block != 64 && block != 128 && block != 256) block = 256;
   const uint64_t pairs = (uint64_t)nops * g.nfchunk;
-  const uint32_t wgs_per_op = ((g.nfchunk + AR_GROUP - 1) / AR_GROUP + 3) / 4;
-  // four waves per workgroup: the kernel's LDS and its per-workgroup append assume 256 threads
-  hipLaunchKernelGGL(active_ranges_kernel, dim3(nops * wgs_per_op), dim3(256), 0, s, g.fchunk, g.wrange, g.nfchunk,
-                     ops, nops, bitmaps, g.W, rflags, items, nitems);
+  const uint32_t nhp = explore ? g.nhparts : 0;
+  const bool direct = pairs <= FILTER_DIRECT;
+  if (!direct) {
+    const uint32_t wgs_per_op = ((g.nfchunk + AR_GROUP - 1) / AR_GROUP + 3) / 4;
+    // four waves per workgroup: the kernel's LDS and its per-workgroup append assume 256 threads
+    hipLaunchKernelGGL(active_ranges_kernel, dim3(nops * wgs_per_op), dim3(256), 0, s, g.fchunk, g.wrange, g.nfchunk,
+                       ops, nops, bitmaps, g.W, rflags, items, counters);
+  }
   // the list's length is known on the device only: a grid of at most
-  // max_wg workgroups, and at most FILTER_OVERSUB times as many as are
-  // resident at once, strides over it (waves past its end leave at once).
+  // FILTER_OVERSUB times as many workgroups as are resident at once strides
+  // over it (waves past its end leave at once).
   // Workgroups beyond the resident ones start as earlier ones finish, which
   // evens out uneven items (R-MAT hub ranges); with far more, the waves in
   // flight touch more bitmaps at a time.  Measured per batch: 1x resident
@@ -437,17 +490,26 @@ void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, c
   // 65,536 workgroups 13.3 / 19.5; items taken from a shared counter (16
   // per atomic) 14.1 / 28.4, the atomics serialising across the XCDs.
   const uint32_t wpb = block / WAVE;
-  const size_t lds = sizeof(WaveLds) * wpb;
-  uint64_t grid = (pairs + wpb - 1) / wpb;
-  if (grid > max_wg) grid = max_wg;
+  const uint64_t grid =
+      std::min<uint64_t>((pairs + (uint64_t)nops * nhp + wpb - 1) / wpb, (uint64_t)resident * FILTER_OVERSUB);
+  hipLaunchKernelGGL(filter_step_kernel, dim3((uint32_t)grid), dim3(block), sizeof(WaveLds) * wpb, s, g.row, g.col,
+                     g.ckey, g.W, g.fchunk, direct ? nullptr : items, counters, g.nfchunk, nops, g.hparts, nhp, drops,
+                     counters + 1, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, stats);
+  if (nhp)
+    hipLaunchKernelGGL(drop_hubs_kernel, dim3(1), dim3(256), 0, s, drops, counters + 1, bitmaps, g.W);
+}
+
+uint32_t filter_resident(uint32_t block) {
   int dev = 0, ncu = 0, per_cu = 0;
-  if (hipGetDevice(&dev) == hipSuccess &&
-      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, filter_step_kernel, (int)block, lds) == hipSuccess &&
-      ncu > 0 && per_cu > 0)
-    grid = std::min<uint64_t>(grid, (uint64_t)ncu * per_cu * FILTER_OVERSUB);
-  hipLaunchKernelGGL(filter_step_kernel, dim3((uint32_t)grid), dim3(block), lds, s, g.row, g.col, g.ckey, g.W,
-                     g.fchunk, items, nitems, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, stats);
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, filter_step_kernel, (int)block,
+                                                   sizeof(WaveLds) * (block / WAVE)) != hipSuccess ||
+      ncu < 1 || per_cu < 1) {
+    (void)hipGetLastError();
+    return 8192;
+  }
+  return (uint32_t)ncu * (uint32_t)per_cu;
 }
 
 }  // namespace gpsm

@@ -103,7 +103,8 @@ __global__ void vertex_keys_kernel(const uint32_t* __restrict__ row, const uint3
 // with more is a range of its own).  ends[b * FCHUNK_VERTS + i]: end of range i
 // of block b; count[b]: its ranges.
 __global__ void __launch_bounds__(256) range_ends_kernel(const uint32_t* __restrict__ row, uint32_t n,
-                                                         uint32_t* __restrict__ ends, uint32_t* __restrict__ count) {
+                                                         uint32_t* __restrict__ ends, uint32_t* __restrict__ count,
+                                                         uint32_t* __restrict__ parts) {
   __shared__ uint32_t off[FCHUNK_VERTS + 1];
   const uint32_t v0 = blockIdx.x * FCHUNK_VERTS, nv = min(FCHUNK_VERTS, n - v0);
   for (uint32_t i = threadIdx.x; i <= nv; i += blockDim.x) off[i] = row[v0 + i];
@@ -118,6 +119,8 @@ __global__ void __launch_bounds__(256) range_ends_kernel(const uint32_t* __restr
       else hi = mid - 1;
     }
     ends[(size_t)v0 + k] = v0 + lo;
+    const uint32_t entries = off[lo] - off[v];  // over the limit: one vertex
+    if (entries > FCHUNK_ENTRIES) atomicAdd(parts, (entries + HUB_PART - 1) / HUB_PART);
     v = lo;
   }
   count[blockIdx.x] = k;
@@ -126,11 +129,20 @@ __global__ void __launch_bounds__(256) range_ends_kernel(const uint32_t* __restr
 // fchunk and wrange from the blocks' ranges; base[b]: ranges before block b.
 __global__ void __launch_bounds__(256) ranges_kernel(const uint32_t* __restrict__ ends,
                                                      const uint32_t* __restrict__ count,
-                                                     const uint32_t* __restrict__ base, uint32_t n,
-                                                     uint32_t* __restrict__ fchunk, uint32_t* __restrict__ wrange) {
+                                                     const uint32_t* __restrict__ base,
+                                                     const uint32_t* __restrict__ row, uint32_t n,
+                                                     uint32_t* __restrict__ fchunk, uint32_t* __restrict__ wrange,
+                                                     uint2* __restrict__ hparts, uint32_t* __restrict__ next) {
   const uint32_t b = blockIdx.x, v0 = b * FCHUNK_VERTS, c = count[b], r0 = base[b];
   const uint32_t* e = ends + v0;
-  for (uint32_t i = threadIdx.x; i < c; i += blockDim.x) fchunk[r0 + i + 1] = e[i];
+  for (uint32_t i = threadIdx.x; i < c; i += blockDim.x) {
+    fchunk[r0 + i + 1] = e[i];
+    const uint32_t v = e[i] - 1, entries = row[v + 1] - row[v];
+    if (entries > FCHUNK_ENTRIES) {
+      const uint32_t np = (entries + HUB_PART - 1) / HUB_PART, at = atomicAdd(next, np);
+      for (uint32_t k = 0; k < np; ++k) hparts[at + k] = make_uint2(v, k);
+    }
+  }
   if (b == 0 && threadIdx.x == 0) fchunk[0] = 0;
   for (uint32_t i = threadIdx.x; i < FCHUNK_VERTS / 32; i += blockDim.x) {
     const uint32_t v = v0 + 32 * i;
@@ -204,19 +216,20 @@ uint64_t range_words(uint32_t n) {
   return nb * FCHUNK_VERTS + 2 * ((nb + 1) & ~1ull) + scan_scratch_words(nb);
 }
 
-void launch_range_ends(const uint32_t* row, uint32_t n, uint32_t* scratch, unsigned long long* total, hipStream_t s) {
+void launch_range_ends(const uint32_t* row, uint32_t n, uint32_t* scratch, unsigned long long* total, uint32_t* parts,
+                       hipStream_t s) {
   const uint32_t nb = range_blocks(n);
   const uint64_t ne = ((uint64_t)nb + 1) & ~1ull;
   uint32_t* count = scratch + (uint64_t)nb * FCHUNK_VERTS;
-  hipLaunchKernelGGL(range_ends_kernel, dim3(nb), dim3(256), 0, s, row, n, scratch, count);
+  hipLaunchKernelGGL(range_ends_kernel, dim3(nb), dim3(256), 0, s, row, n, scratch, count, parts);
   launch_exclusive_scan(count, count + ne, nb, total, count + 2 * ne, scan_scratch_words(nb), s);
 }
 
-void launch_ranges(const DevGraph& g, const uint32_t* scratch, hipStream_t s) {
+void launch_ranges(const DevGraph& g, const uint32_t* scratch, uint32_t* next, hipStream_t s) {
   const uint32_t nb = range_blocks(g.n);
   const uint32_t* count = scratch + (uint64_t)nb * FCHUNK_VERTS;
   hipLaunchKernelGGL(ranges_kernel, dim3(nb), dim3(256), 0, s, scratch, count, count + (((uint64_t)nb + 1) & ~1ull),
-                     g.n, g.fchunk, g.wrange);
+                     g.row, g.n, g.fchunk, g.wrange, g.hparts, next);
 }
 
 uint64_t hub_words(uint32_t n, uint64_t nhub) {

@@ -26,6 +26,10 @@ struct DevGraph {
   // walks far more adjacency than the others (power-law hubs)
   uint32_t* fchunk = nullptr;
   uint32_t nfchunk = 0;
+  // the vertices with more than FCHUNK_ENTRIES entries in parts of HUB_PART:
+  // (vertex, part) pairs
+  uint2* hparts = nullptr;
+  uint32_t nhparts = 0;
   // wrange[w]: the vertex range holding vertex 32w (one per bitmap word)
   uint32_t* wrange = nullptr;
   // hubs (degree above hub_degree): hub_of[v] = index of v's adjacency
@@ -39,6 +43,7 @@ struct DevGraph {
 
 constexpr uint32_t FCHUNK_VERTS = 1024;
 constexpr uint32_t FCHUNK_ENTRIES = 4096;
+constexpr uint32_t HUB_PART = 2048;
 
 // graph.hip: what a resident graph holds besides its CSR, built from it.
 constexpr uint32_t LABEL_HIST = 4096, HUB_STEPS = 34;
@@ -55,9 +60,13 @@ void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uin
 void launch_vertex_keys(const DevGraph& g, const uint32_t* label, const uint32_t* value, uint32_t nl, hipStream_t s);
 // The filter's vertex ranges: their ends and their number (*total), then, with
 // g.fchunk and g.wrange allocated, those.  scratch: range_words(n) words.
+// *parts (zeroed by the caller): the parts of all vertices with more than
+// FCHUNK_ENTRIES entries; launch_ranges also writes g.hparts (in any order,
+// *next zeroed by the caller).
 uint64_t range_words(uint32_t n);
-void launch_range_ends(const uint32_t* row, uint32_t n, uint32_t* scratch, unsigned long long* total, hipStream_t s);
-void launch_ranges(const DevGraph& g, const uint32_t* scratch, hipStream_t s);
+void launch_range_ends(const uint32_t* row, uint32_t n, uint32_t* scratch, unsigned long long* total, uint32_t* parts,
+                       hipStream_t s);
+void launch_ranges(const DevGraph& g, const uint32_t* scratch, uint32_t* next, hipStream_t s);
 // g.hub_of and, with nhub of them above hub_degree and hub_bits zeroed, their
 // bitmaps.  scratch: hub_words(n, nhub) words, 8-byte aligned.
 uint64_t hub_words(uint32_t n, uint64_t nhub);
@@ -86,19 +95,27 @@ void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* 
 // copy c, entries 0..4 = candidates, adjacency entries read, key gathers,
 // bitmap probes, bits set, added by the workgroups with blockIdx % copies
 // == c (the sum over copies is the launch's total).
-// The superstep visits only the (op, vertex range) pairs whose range holds a
-// candidate of C(u): a first kernel lists them in items (nops x g.nfchunk
-// capacity) and counts them in *nitems (zeroed by the caller), the second
-// processes the list with at most max_wg workgroups, and at most
-// FILTER_OVERSUB times as many as are resident.  rflags: the refine
-// rounds' change flags (FilterOp::mark / need), zeroed by the caller once
-// per batch; an op whose need flag is clear lists no range.
+// Of more than FILTER_DIRECT (op, vertex range) pairs the superstep visits
+// only those whose range holds a candidate of C(u): a first kernel lists them
+// in items (nops x g.nfchunk capacity) and counts them in counters[0], the
+// second processes the list.  Fewer are all visited by one launch, whose waves
+// leave an empty range after reading its bitmap words: listing the pairs of
+// one op on a 1M-vertex graph took 35 us (four workgroups), more than the
+// pass over its 5,000 ranges.  explore: the superstep has explore ops, whose
+// hubs go in parts (drops: nops x the vertices in parts, counted in
+// counters[1]).  counters: two words, zeroed by the caller.  resident:
+// filter_resident(block).  rflags: the refine rounds' change flags
+// (FilterOp::mark / need), zeroed by the caller once per batch; an op whose
+// need flag is clear is left out.
 constexpr uint32_t STAT_COPIES = 32, STAT_STRIDE = 8;
 constexpr uint32_t FILTER_OVERSUB = 8;
+constexpr uint64_t FILTER_DIRECT = 1u << 17;
 void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, const uint32_t* nbr_slot,
                         const uint32_t* nbr_lo, const uint32_t* nbr_hi, uint32_t* bitmaps, uint32_t block,
-                        uint32_t max_wg, uint2* items, uint32_t* nitems, uint32_t* rflags,
-                        unsigned long long* stats, hipStream_t s);
+                        uint32_t resident, bool explore, uint2* items, uint32_t* counters, uint2* drops,
+                        uint32_t* rflags, unsigned long long* stats, hipStream_t s);
+// Workgroups of `block` threads of the superstep's kernel that are resident at once.
+uint32_t filter_resident(uint32_t block);
 
 // scan.hip ---------------------------------------------------------------------
 // Bitmap rows are compacted in segments of SEG_WORDS words, one workgroup
