@@ -794,11 +794,16 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   std::vector<InitOp> init;
   std::vector<FilterOp> fops;
   std::vector<uint32_t> step_off(maxsteps + 1, 0), nbr_slot, nbr_lo, nbr_hi;
-  std::vector<uint8_t> explore(maxsteps, 0);  // supersteps with explore ops
+  // explore ops: their neighbours' fills, and bitmap rows for the candidates
+  // that leave C(u) part of the way (after the slots')
+  std::vector<FillOp> fills;
+  std::vector<uint32_t> fill_off(maxsteps + 1, 0);
+  uint32_t nexplore = 0, erows = nslots;
   for (uint32_t b = 0; b < nq; ++b)
     if (Q[b].active) init.push_back({Q[b].vbase + Q[b].fs.start, Q[b].fs.start_lo, Q[b].fs.start_hi});
   for (uint32_t sidx = 0; sidx < maxsteps; ++sidx) {
     step_off[sidx] = (uint32_t)fops.size();
+    fill_off[sidx] = (uint32_t)fills.size();
     for (uint32_t b = 0; b < nq; ++b) {
       const QState& S = Q[b];
       if (!S.active || sidx >= S.fs.steps.size()) continue;
@@ -809,7 +814,15 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       op.nv = (uint32_t)fsx.v.size();
       op.nbr_off = (uint32_t)nbr_slot.size();
       op.mark = op.need = ~0u;
-      if (fsx.type == OP_EXPLORE) explore[sidx] = 1;
+      op.e_slot = op.cnt = ~0u;
+      if (fsx.type == OP_EXPLORE) {
+        op.cnt = nexplore++;
+        op.e_slot = erows;
+        for (uint32_t i = 0; i < op.nv; ++i)
+          fills.push_back({op.u_slot, i + 1 < op.nv ? op.e_slot + i : ~0u, S.vbase + fsx.v[i], fsx.lo[i], fsx.hi[i],
+                           op.cnt, st.count(S.hq.lab[fsx.v[i]])});
+        erows += op.nv - 1;
+      }
       if (fsx.type == OP_REFINE) {
         op.mark = b * 4 + fsx.round;
         if (fsx.round > 0) op.need = b * 4 + fsx.round - 1;
@@ -823,7 +836,11 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     }
   }
   step_off[maxsteps] = (uint32_t)fops.size();
-  if ((rc = c->bufs[B_BITMAPS].ensure(sizeof(uint32_t) * (size_t)std::max<uint32_t>(nslots, 1) * W))) return rc;
+  fill_off[maxsteps] = (uint32_t)fills.size();
+  const size_t ncounters = (size_t)maxsteps + nexplore;  // listed items per superstep, candidates per explore op
+  if ((rc = c->bufs[B_BITMAPS].ensure(sizeof(uint32_t) * (size_t)std::max<uint32_t>(erows, 1) * W)) ||
+      (rc = upload(c, B_FILLS, fills)))
+    return rc;
   if ((rc = upload(c, B_INIT, init)) || (rc = upload(c, B_FOPS, fops)) || (rc = upload(c, B_NBR_SLOT, nbr_slot)) ||
       (rc = upload(c, B_NBR_LO, nbr_lo)) || (rc = upload(c, B_NBR_HI, nbr_hi)))
     return rc;
@@ -833,8 +850,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   uint32_t max_ops = 0;  // ops of the largest superstep
   for (uint32_t sidx = 0; sidx < maxsteps; ++sidx) max_ops = std::max(max_ops, step_off[sidx + 1] - step_off[sidx]);
   if ((rc = c->bufs[B_FITEMS].ensure(sizeof(uint2) * std::max<uint64_t>((uint64_t)max_ops * dg.nfchunk, 1))) ||
-      (rc = c->bufs[B_FDROPS].ensure(sizeof(uint2) * std::max<uint64_t>((uint64_t)max_ops * dg.nhparts, 1))) ||
-      (rc = c->bufs[B_FNITEMS].ensure(sizeof(uint32_t) * 2 * std::max<uint32_t>(maxsteps, 1))) ||
+      (rc = c->bufs[B_FNITEMS].ensure(sizeof(uint32_t) * std::max<size_t>(ncounters, 1))) ||
       (rc = c->bufs[B_RFLAGS].ensure(sizeof(uint32_t) * 4 * (uint64_t)std::max<uint32_t>(nq, 1))))
     return rc;
   // work counters (profile mode 2): one slot per filter superstep, then the
@@ -850,20 +866,21 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if (o.use_graph) {
     sig_a.add(uint64_t{0});
     sig_a.add_graph(dg);
-    for (int i : {B_FDROPS, B_BITMAPS, B_FNITEMS, B_RFLAGS, B_INIT, B_FOPS, B_NBR_SLOT, B_NBR_LO, B_NBR_HI, B_FITEMS, B_SEGC,
+    for (int i : {B_FILLS, B_BITMAPS, B_FNITEMS, B_RFLAGS, B_INIT, B_FOPS, B_NBR_SLOT, B_NBR_LO, B_NBR_HI, B_FITEMS, B_SEGC,
                   B_COUNTS})
       sig_a.add(c->bufs[i].ptr);
     sig_a.add(nslots), sig_a.add(maxsteps), sig_a.add(nq), sig_a.add(init.size()), sig_a.add(fblock);
     for (uint32_t v : step_off) sig_a.add(v);
-    for (uint8_t v : explore) sig_a.add((uint64_t)v);
+    for (uint32_t v : fill_off) sig_a.add(v);
+    sig_a.add(erows), sig_a.add(ncounters);
   }
   bool replayed = o.use_graph && replay_cached(c, 0, sig_a.w, s, &rc);
   if (replayed && rc) return rc;
   if (!replayed) {
     bool captured = false;
     if (o.use_graph && hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) captured = true;
-    launch_fill_u32(bitmaps, 0u, (uint64_t)nslots * W, s);
-    if (maxsteps) launch_fill_u32(dptr<uint32_t>(c, B_FNITEMS), 0u, 2 * maxsteps, s);
+    launch_fill_u32(bitmaps, 0u, (uint64_t)erows * W, s);
+    if (ncounters) launch_fill_u32(dptr<uint32_t>(c, B_FNITEMS), 0u, ncounters, s);
     launch_fill_u32(dptr<uint32_t>(c, B_RFLAGS), 0u, 4ull * std::max<uint32_t>(nq, 1), s);
     if (counters) launch_fill_u32(reinterpret_cast<uint32_t*>(fstats), 0u, 2ull * fstat_step * nstat_slots, s);
     {
@@ -876,9 +893,10 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       const uint32_t nops_s = step_off[sidx + 1] - step_off[sidx];
       hipEvent_t a = pbegin(K_FILTER);
       launch_filter_step(dg, dptr<FilterOp>(c, B_FOPS) + step_off[sidx], nops_s, dptr<uint32_t>(c, B_NBR_SLOT),
-                         dptr<uint32_t>(c, B_NBR_LO), dptr<uint32_t>(c, B_NBR_HI), bitmaps, fblock, fresident,
-                         explore[sidx], dptr<uint2>(c, B_FITEMS), dptr<uint32_t>(c, B_FNITEMS) + 2 * sidx,
-                         dptr<uint2>(c, B_FDROPS), dptr<uint32_t>(c, B_RFLAGS),
+                         dptr<uint32_t>(c, B_NBR_LO), dptr<uint32_t>(c, B_NBR_HI),
+                         dptr<FillOp>(c, B_FILLS) + fill_off[sidx], fill_off[sidx + 1] - fill_off[sidx], bitmaps,
+                         fblock, fresident, dptr<uint2>(c, B_FITEMS), dptr<uint32_t>(c, B_FNITEMS) + sidx,
+                         dptr<uint32_t>(c, B_RFLAGS), dptr<uint32_t>(c, B_FNITEMS) + maxsteps,
                          counters ? fstats + fstat_step * sidx : nullptr, s);
       pend(K_FILTER, a, 4.0 * W * nops_s, counters ? (int)sidx : -1);
     }

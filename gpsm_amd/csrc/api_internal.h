@@ -81,8 +81,8 @@ enum BufId {
   B_TEXT_WG,     // ... scan scratch, per-workgroup lengths and offsets
   B_TEXT_OUT,    // ... the chunk's text
   B_FITEMS,      // filter superstep: (op, vertex range) pairs with candidates
-  B_FNITEMS,     // ... their number and that of the dropped hubs, two counters per superstep
-  B_FDROPS,      // ... hubs that leave their op's candidates
+  B_FNITEMS,     // ... their number, one counter per superstep, then the explore ops' candidate counts
+  B_FILLS,       // explore ops' neighbours (FillOp)
   B_CDESC,       // candidate-edge tables of reversed plan edges (counted again)
   B_LDESC,       // candidate-edge tables whose lists are written
   B_WDESC,       // last levels' tables counted from records

@@ -41,6 +41,19 @@ struct FilterOp {
   // this op to run (~0u: always runs).
   uint32_t mark;
   uint32_t need;
+  // explore: bitmap rows (nv - 1 of them) of the candidates that leave C(u)
+  // but hand on matches of v_0, v_1, ...; index of the op's candidate count
+  uint32_t e_slot;
+  uint32_t cnt;
+};
+
+// One neighbour v_i of an explore op: C(v_i) receives the vertices with key in
+// [lo, hi] that have a neighbour in C(u) or (e_slot != ~0) in e_slot's row.
+struct FillOp {
+  uint32_t u_slot, e_slot, v_slot;
+  uint32_t lo, hi;
+  uint32_t cnt;     // the op's candidate count
+  uint32_t nlabel;  // vertices of v_i's label
 };
 
 // Initial label/degree check of a query's start vertex.

@@ -176,35 +176,39 @@ struct WaveLds {
   uint32_t lim[WAVE];
 };
 
-// list null: every (op, range) pair is an item (nops * chunks of them, the ops
-// whose need flag is clear leave theirs).  After the listed or all pairs, nhp
-// hub parts per op: a vertex with more entries than a range holds is not
-// explored with its range but in parts of HUB_PART entries, one wave each
-// (one wave walking the 30,000 entries of a hub of the 1M Chung-Lu graph took
-// 100-360 us, the whole superstep; 25 us in parts).  Every part decides for
-// itself how far the hub meets its op's neighbours, usually in its first
-// steps, so C(u) must not change under them: a hub that leaves C(u) goes to
-// drops, cleared by the next launch.
+// Which candidates meet their op's neighbours.  list null: every (op, range)
+// pair is an item (nops * chunks of them, the ops whose need flag is clear
+// leave theirs).  A refine op drops the others.  An explore op drops them too
+// and leaves behind what the neighbours' sets are filled from (fill_kernel):
+// a candidate that meets v_0 .. v_{i-1} but not v_i still hands its matches
+// to those before v_i (match/Match.cu:547-600), so its bit goes to their
+// bitmaps at e_slot (v_0 .. v_{nv-2}: no candidate that fails has met all);
+// counts[cnt] counts the candidates that meet v_0.
+// PUSH: an explore op sets its neighbours' bits itself, in a second pass over
+// the adjacency just read, and leaves only its hubs to fill_kernel.  With
+// hundreds of ops in flight the atomics of one bitmap no longer bound the
+// launch and the pass over adjacency still in the caches is the cheaper one:
+// all supersteps of 245 queries on the 1M Chung-Lu graph 9.9 ms, 12.3 ms with
+// their fills launched apart.
+template <bool PUSH>
 __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __restrict__ row,
                                                           const uint32_t* __restrict__ col,
                                                           const uint32_t* __restrict__ ckey, uint32_t W,
                                                           const uint32_t* __restrict__ fchunk,
                                                           const uint2* __restrict__ list,
                                                           const uint32_t* __restrict__ nlist, uint32_t chunks,
-                                                          uint32_t nops, const uint2* __restrict__ hparts,
-                                                          uint32_t nhp, uint2* __restrict__ drops,
-                                                          uint32_t* __restrict__ ndrops,
-                                                          const FilterOp* __restrict__ ops,
+                                                          uint32_t nops, const FilterOp* __restrict__ ops,
                                                           const uint32_t* __restrict__ nbr_slot,
                                                           const uint32_t* __restrict__ nbr_lo,
                                                           const uint32_t* __restrict__ nbr_hi,
                                                           uint32_t* __restrict__ bitmaps,
                                                           uint32_t* __restrict__ rflags,
+                                                          uint32_t* __restrict__ counts,
                                                           unsigned long long* __restrict__ stats) {
   extern __shared__ unsigned char lds_raw[];
   WaveLds& L = reinterpret_cast<WaveLds*>(lds_raw)[threadIdx.x / WAVE];
   const uint32_t lane = lane_id();
-  const uint32_t pairs = list ? uniform(*nlist) : nops * chunks, items = pairs + nops * nhp;
+  const uint32_t items = list ? uniform(*nlist) : nops * chunks;
   const uint32_t wave = uniform((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
   const uint32_t nwaves = (gridDim.x * blockDim.x) / WAVE;
   // per-lane tallies for the optional byte accounting, over all items
@@ -212,16 +216,12 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
   uint32_t t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
 
   // the next item's list entry is loaded while the current one runs
-  uint2 nxt = list && wave < pairs ? list[wave] : make_uint2(0u, 0u);
+  uint2 nxt = list && wave < items ? list[wave] : make_uint2(0u, 0u);
   for (uint32_t it = wave; it < items; it += nwaves) {
-    const bool hub = it >= pairs;
     uint32_t o, c;
-    if (hub) {
-      o = (it - pairs) / nhp;
-      c = (it - pairs) % nhp;
-    } else if (list) {
+    if (list) {
       const uint2 item = nxt;
-      if (it + nwaves < pairs) nxt = list[it + nwaves];
+      if (it + nwaves < items) nxt = list[it + nwaves];
       o = uniform(item.x);
       c = uniform(item.y);
     } else {
@@ -231,7 +231,6 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
       if (need != ~0u && uniform(rflags[need]) == 0) continue;
     }
     const uint32_t type = uniform(ops[o].type);
-    if (hub && type != OP_EXPLORE) continue;
     const uint32_t nv = uniform(ops[o].nv);
     const uint32_t nb = uniform(ops[o].nbr_off);
     uint32_t* bm_u = bitmaps + (size_t)uniform(ops[o].u_slot) * W;
@@ -239,16 +238,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
 
     // collect: candidates of vertex range [v_lo, v_hi), ascending; lane l
     // reads bitmap word w_lo + l and keeps the range's bits of it
-    uint32_t v_lo, v_hi, part = 0;
-    if (hub) {
-      const uint2 hp = hparts[c];
-      v_lo = uniform(hp.x);
-      v_hi = v_lo + 1;
-      part = uniform(hp.y);
-    } else {
-      v_lo = uniform(fchunk[c]);
-      v_hi = uniform(fchunk[c + 1]);
-    }
+    const uint32_t v_lo = uniform(fchunk[c]), v_hi = uniform(fchunk[c + 1]);
     const uint32_t w_lo = v_lo >> 5, nw = ((v_hi - 1) >> 5) - w_lo + 1;
     const uint32_t wi = w_lo + lane;
     uint32_t w = 0;
@@ -261,7 +251,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
     const uint32_t incl = wave_incl_scan(pc);
     const uint32_t C = uniform(__shfl(incl, WAVE - 1, WAVE));
     if (C == 0) continue;
-    if (lane == 0 && part == 0) t_cand += C;
+    if (lane == 0) t_cand += C;
     {
       uint32_t pos = incl - pc, x = w;
       while (x) {
@@ -272,16 +262,13 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
     }
     wave_sync();
 
+    uint32_t met = 0;  // explore: candidates that meet v_0
     for (uint32_t s0 = 0; s0 < C; s0 += WAVE) {
       // lane = one candidate of the sub-chunk
-      bool mine = s0 + lane < C;
+      const bool mine = s0 + lane < C;
       const uint32_t id = mine ? L.cand[s0 + lane] : 0u;
       const uint32_t off = mine ? row[id] : 0u;
-      uint32_t deg = mine ? row[id + 1] - off : 0u;
-      if (!hub && type == OP_EXPLORE && deg > FCHUNK_ENTRIES) {  // explored by its parts
-        mine = false;
-        deg = 0;
-      }
+      const uint32_t deg = mine ? row[id + 1] - off : 0u;
       L.hit[lane] = 0;
       uint32_t cur = 0;  // entries of this candidate already examined
       unsigned long long h = 0;
@@ -366,72 +353,69 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
         if (drop) clear_bit(bm_u, id);
         if (__ballot(drop) && lane == 0) rflags[uniform(ops[o].mark)] = 1u;
       } else {
-        // first neighbour without a match: mu leaves C(u); neighbours before
-        // it received all of mu's matching data neighbours (match/Match.cu:547-600)
+        // first neighbour without a match: mu leaves C(u), its matches of the
+        // neighbours before it stay
         const uint32_t ff = h == full ? nv : (uint32_t)(__ffsll((long long)~h) - 1);
-        if (mine && ff < nv) {
-          if (!hub) clear_bit(bm_u, id);
-          else if (part == 0) drops[atomicAdd(ndrops, 1u)] = make_uint2(ops[o].u_slot, id);
+        const bool left = !PUSH || deg > FCHUNK_ENTRIES;  // to fill_kernel
+        if (mine && ff < nv) clear_bit(bm_u, id);
+        if (mine && ff < nv && left) {
+          uint32_t* e = bitmaps + (size_t)ops[o].e_slot * W;
+          for (uint32_t i = 0; i < ff; ++i) set_bit(e + (size_t)i * W, id);  // ff < nv: e_slot has nv - 1 rows
         }
-        const uint32_t lim = mine ? ff : 0u;
-        const uint32_t p0 = part * HUB_PART;  // a part's entries; 0 and all of them else
-        const uint32_t len = lim ? (hub ? min(HUB_PART, deg - p0) : deg) : 0u;
-        const uint32_t lincl = wave_incl_scan(len);
-        const uint32_t T = uniform(__shfl(lincl, WAVE - 1, WAVE));
-        L.pre[lane] = lincl - len;
-        L.base[lane] = off + p0;
-        L.lim[lane] = lim;
-        wave_sync();
-        // pass 2: every matching data neighbour of a surviving prefix enters C(v_i)
-        for (uint32_t f = 0; f < T; f += UNROLL * WAVE) {
-          uint32_t mvs[UNROLL], ks[UNROLL], cis[UNROLL], es[UNROLL], gi[UNROLL];
+        met += (uint32_t)__popcll(__ballot(mine && ff > 0 && left));
+        if constexpr (PUSH) {
+          // every matching neighbour of a surviving prefix enters C(v_i)
+          const uint32_t lim = mine && !left ? ff : 0u;
+          const uint32_t len = lim ? deg : 0u;
+          const uint32_t lincl = wave_incl_scan(len);
+          const uint32_t T = uniform(__shfl(lincl, WAVE - 1, WAVE));
+          L.pre[lane] = lincl - len;
+          L.base[lane] = off;
+          L.lim[lane] = lim;
+          wave_sync();
+          for (uint32_t f = 0; f < T; f += UNROLL * WAVE) {
+            uint32_t mvs[UNROLL], ks[UNROLL], cis[UNROLL], es[UNROLL], gi[UNROLL], lms[UNROLL];
 #pragma unroll
-          for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(f + u * WAVE + lane, T - 1);
-          halving_search<UNROLL>(L.pre, WAVE, cis);
+            for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(f + u * WAVE + lane, T - 1);
+            halving_search<UNROLL>(L.pre, WAVE, cis);
 #pragma unroll
-          for (int u = 0; u < UNROLL; ++u) es[u] = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
-#pragma unroll
-          for (int u = 0; u < UNROLL; ++u) {
-            mvs[u] = col[es[u]];
-            ks[u] = ckey[es[u]];
-            if (f + u * WAVE + lane >= T) cis[u] = WAVE;
-          }
-          // the UNROLL entries of a lane side by side: their prefix limits
-          // read together, then per neighbour v_i the bitmap words of the
-          // entries that enter C(v_i) loaded together, and a bit set (one
-          // atomic) only where it is still clear
-          uint32_t lms[UNROLL];
-#pragma unroll
-          for (int u = 0; u < UNROLL; ++u) {
-            lms[u] = cis[u] != WAVE ? L.lim[cis[u]] : 0u;
-            if (cis[u] != WAVE) {
-              ++t_ent;
-              ++t_key;
-            }
-          }
-          for (uint32_t i = 0; i < nv; ++i) {  // lim <= nv
-            const uint32_t lo = nbr_lo[nb + i], hi = nbr_hi[nb + i];
-            uint32_t* bm = bitmaps + (size_t)nbr_slot[nb + i] * W;
-            bool want[UNROLL];
-            uint32_t cw[UNROLL];
+            for (int u = 0; u < UNROLL; ++u) es[u] = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
 #pragma unroll
             for (int u = 0; u < UNROLL; ++u) {
-              want[u] = i < lms[u] && ks[u] >= lo && ks[u] <= hi;
-              cw[u] = want[u] ? __hip_atomic_load(bm + (mvs[u] >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                              : ~0u;
+              mvs[u] = col[es[u]];
+              ks[u] = ckey[es[u]];
+              const bool in = f + u * WAVE + lane < T;
+              lms[u] = in ? L.lim[cis[u]] : 0u;
+              t_ent += in;
+              t_key += in;
             }
+            // per neighbour v_i the words of the UNROLL entries are loaded
+            // together, and a bit is set (one atomic) only where still clear
+            for (uint32_t i = 0; i < nv; ++i) {  // lim <= nv
+              const uint32_t lo = nbr_lo[nb + i], hi = nbr_hi[nb + i];
+              uint32_t* bm = bitmaps + (size_t)nbr_slot[nb + i] * W;
+              bool want[UNROLL];
+              uint32_t cw[UNROLL];
 #pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
-              if (want[u]) {
-                ++t_set;
-                const uint32_t m = 1u << (mvs[u] & 31);
-                if (!(cw[u] & m)) atomicOr(bm + (mvs[u] >> 5), m);
+              for (int u = 0; u < UNROLL; ++u) {
+                want[u] = i < lms[u] && ks[u] >= lo && ks[u] <= hi;
+                cw[u] = want[u] ? __hip_atomic_load(bm + (mvs[u] >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                                : ~0u;
               }
+#pragma unroll
+              for (int u = 0; u < UNROLL; ++u)
+                if (want[u]) {
+                  ++t_set;
+                  const uint32_t m = 1u << (mvs[u] & 31);
+                  if (!(cw[u] & m)) atomicOr(bm + (mvs[u] >> 5), m);
+                }
+            }
           }
         }
       }
       wave_sync();
     }
+    if (met && lane == 0) atomicAdd(&counts[ops[o].cnt], met);
   }
   if (stats) {
     // one atomic per counter per workgroup, spread over STAT_COPIES copies
@@ -450,11 +434,194 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
   }
 }
 
-// Hubs that leave their op's C(u) (filter_step_kernel's drops).
-__global__ void drop_hubs_kernel(const uint2* __restrict__ drops, const uint32_t* __restrict__ ndrops,
-                                 uint32_t* __restrict__ bitmaps, uint32_t W) {
-  for (uint32_t i = threadIdx.x; i < *ndrops; i += blockDim.x)
-    clear_bit(bitmaps + (size_t)drops[i].x * W, drops[i].y);
+// The vertices an explore op's neighbour v receives: those in v's label and
+// degree range with a neighbour in C(u) (or in e_slot's bitmap).  One wave
+// per (fill, vertex range), whichever way is cheaper for the fill:
+//  pull  the range's vertices of v's label look for a neighbour in C(u) and
+//        stop at the first, as a refine op does; the range's words are
+//        written once;
+//  push  the range's candidates of C(u) set the bits of their matches (read
+//        first, an atomic only where clear); a vertex with more entries than
+//        a range holds goes in parts of HUB_PART, one wave each.
+// Pushing alone took 85-340 us per op on the 1M Chung-Lu graph for some 1e5
+// vertices found, bound by the atomics: the lines of one 125 KB bitmap move
+// between the L2s of eight XCDs.  Pulling them takes 11-28 us.  A vertex of v's
+// label without a neighbour in C(u) is walked to its end, so where v's label
+// has more than FILL_PULL times as many vertices as C(u) they are pushed.
+// hubs_only: only the hubs of C(u) are pushed, in parts (the others' matches
+// are set already).
+struct FillLds {
+  uint32_t cand[MAX_CAND];
+  uint32_t pre[WAVE + 1];
+  uint32_t base[WAVE];
+  uint32_t hit[WAVE];
+  uint32_t word[WAVE];
+};
+
+__global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ row, const uint32_t* __restrict__ col,
+                                                   const uint32_t* __restrict__ key,
+                                                   const uint32_t* __restrict__ ckey, uint32_t W,
+                                                   const uint32_t* __restrict__ fchunk, uint32_t chunks,
+                                                   const uint2* __restrict__ hparts, uint32_t nhp,
+                                                   const FillOp* __restrict__ fills, uint32_t nfill,
+                                                   const uint32_t* __restrict__ counts, bool hubs_only,
+                                                   uint32_t* bitmaps, unsigned long long* __restrict__ stats) {
+  extern __shared__ unsigned char lds_raw[];
+  FillLds& L = reinterpret_cast<FillLds*>(lds_raw)[threadIdx.x / WAVE];
+  const uint32_t lane = lane_id();
+  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
+  const uint64_t pairs = hubs_only ? 0 : (uint64_t)nfill * chunks, items = pairs + (uint64_t)nfill * nhp;
+  uint32_t t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
+  for (uint64_t it = wave; it < items; it += nwaves) {
+    const bool part = it >= pairs;
+    const uint64_t x = part ? it - pairs : it;
+    const uint32_t per = part ? nhp : chunks;
+    const uint32_t f = uniform((uint32_t)(x / per)), c = uniform((uint32_t)(x % per));
+    const FillOp& op = fills[f];
+    const uint32_t lo = uniform(op.lo), hi = uniform(op.hi), met = uniform(counts[op.cnt]);
+    if (met == 0) continue;
+    const bool pull = !hubs_only && (uint64_t)met * FILL_PULL >= uniform(op.nlabel);
+    if (part && pull) continue;
+    const uint32_t* bm_u = bitmaps + (size_t)uniform(op.u_slot) * W;
+    const uint32_t e_slot = uniform(op.e_slot);
+    const uint32_t* bm_e = e_slot != ~0u ? bitmaps + (size_t)e_slot * W : nullptr;
+    uint32_t* bm_v = bitmaps + (size_t)uniform(op.v_slot) * W;
+    uint32_t v_lo, v_hi, first = 0;  // first: where a part's entries start
+    if (part) {
+      const uint2 hp = hparts[c];
+      v_lo = uniform(hp.x);
+      v_hi = v_lo + 1;
+      first = uniform(hp.y) * HUB_PART;
+    } else {
+      v_lo = uniform(fchunk[c]);
+      v_hi = uniform(fchunk[c + 1]);
+    }
+    const uint32_t w_lo = v_lo >> 5, nw = ((v_hi - 1) >> 5) - w_lo + 1;
+    uint32_t C = 0;
+    if (pull) {
+      // the range's vertices with v's label and degree, ascending
+      for (uint32_t v0 = v_lo; v0 < v_hi; v0 += WAVE) {
+        const uint32_t v = v0 + lane, k = v < v_hi ? key[v] : 0u;
+        const unsigned long long m = __ballot(k >= lo && k <= hi && v < v_hi);
+        if ((m >> lane) & 1ULL) L.cand[C + (uint32_t)__popcll(lane ? m & (~0ULL >> (WAVE - lane)) : 0ULL)] = v;
+        C += (uint32_t)__popcll(m);
+      }
+      L.word[lane] = 0;
+    } else {
+      uint32_t w = 0;
+      if (lane < nw) {
+        w = bm_u[w_lo + lane];
+        if (bm_e) w |= bm_e[w_lo + lane];
+        if (lane == 0) w &= ~0u << (v_lo & 31);
+        if (lane == nw - 1 && (v_hi & 31)) w &= (1u << (v_hi & 31)) - 1u;
+      }
+      const uint32_t pc = __popc(w);
+      const uint32_t incl = wave_incl_scan(pc);
+      C = uniform(__shfl(incl, WAVE - 1, WAVE));
+      uint32_t pos = incl - pc;
+      for (; w; w &= w - 1) L.cand[pos++] = (w_lo + lane) * 32 + (uint32_t)(__ffs(w) - 1);
+    }
+    if (C == 0) continue;
+    wave_sync();
+    for (uint32_t s0 = 0; s0 < C; s0 += WAVE) {
+      const bool mine = s0 + lane < C;
+      const uint32_t id = mine ? L.cand[s0 + lane] : 0u;
+      const uint32_t off = mine ? row[id] + first : 0u;
+      uint32_t len = mine ? row[id + 1] - off : 0u;
+      if (part) len = min(len, HUB_PART);
+      else if (!pull && len > FCHUNK_ENTRIES) len = 0;  // pushed by its parts
+      if (pull) {
+        L.hit[lane] = 0;
+        uint32_t cur = 0;
+        bool h = false;
+        wave_sync();
+        for (;;) {
+          const uint32_t rem = h ? 0u : len - cur;
+          const uint32_t rincl = wave_incl_scan(rem);
+          const uint32_t T = uniform(__shfl(rincl, WAVE - 1, WAVE));
+          if (T == 0) break;
+          const uint32_t rpre = rincl - rem;
+          L.pre[lane] = rpre;
+          L.base[lane] = off + cur;
+          wave_sync();
+          uint32_t cis[UNROLL], gi[UNROLL], mvs[UNROLL], wv[UNROLL];
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(u * WAVE + lane, T - 1);
+          halving_search<UNROLL>(L.pre, WAVE, cis);
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) mvs[u] = col[L.base[cis[u]] + (gi[u] - L.pre[cis[u]])];
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) {
+            wv[u] = bm_u[mvs[u] >> 5];
+            if (bm_e) wv[u] |= bm_e[mvs[u] >> 5];
+          }
+          // an index past T repeats entry T - 1: the same answer again
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+            if ((wv[u] >> (mvs[u] & 31)) & 1u) L.hit[cis[u]] = 1;
+          wave_sync();
+          const uint32_t span = UNROLL * WAVE;
+          cur += rpre >= span ? 0u : min(rem, span - rpre);
+          h = L.hit[lane] != 0;
+          if (stats) {
+            t_ent += min((T + WAVE - 1 - lane) / WAVE, (uint32_t)UNROLL);
+            t_probe += min((T + WAVE - 1 - lane) / WAVE, (uint32_t)UNROLL);
+          }
+        }
+        if (h) atomicOr(&L.word[(id >> 5) - w_lo], 1u << (id & 31));
+        t_set += h;
+      } else {
+        const uint32_t incl = wave_incl_scan(len);
+        const uint32_t T = uniform(__shfl(incl, WAVE - 1, WAVE));
+        L.pre[lane] = incl - len;
+        L.base[lane] = off;
+        wave_sync();
+        for (uint32_t f0 = 0; f0 < T; f0 += UNROLL * WAVE) {
+          uint32_t cis[UNROLL], gi[UNROLL], mvs[UNROLL], cw[UNROLL];
+          bool want[UNROLL];
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(f0 + u * WAVE + lane, T - 1);
+          halving_search<UNROLL>(L.pre, WAVE, cis);
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) {
+            const uint32_t e = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
+            mvs[u] = col[e];
+            const uint32_t k = ckey[e];
+            want[u] = f0 + u * WAVE + lane < T && k >= lo && k <= hi;
+          }
+          // a bit is set (one atomic) only where it is still clear
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u)
+            cw[u] = want[u] ? __hip_atomic_load(bm_v + (mvs[u] >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ~0u;
+#pragma unroll
+          for (int u = 0; u < UNROLL; ++u) {
+            const uint32_t m = 1u << (mvs[u] & 31);
+            if (want[u] && !(cw[u] & m)) atomicOr(bm_v + (mvs[u] >> 5), m);
+            if (stats) {
+              const bool in = f0 + u * WAVE + lane < T;
+              t_ent += in;
+              t_key += in;
+              t_set += want[u];
+            }
+          }
+        }
+      }
+      wave_sync();
+    }
+    if (pull) {
+      // two ranges may share a word
+      const uint32_t w = lane < nw ? L.word[lane] : 0u;
+      if (w) atomicOr(bm_v + w_lo + lane, w);
+    }
+    wave_sync();
+  }
+  if (stats) {
+    const unsigned long long v[4] = {wave_sum64(t_ent), wave_sum64(t_key), wave_sum64(t_probe), wave_sum64(t_set)};
+    if (lane == 0)
+      for (int i = 0; i < 4; ++i)
+        if (v[i]) atomicAdd(stats + (blockIdx.x % STAT_COPIES) * STAT_STRIDE + 1 + i, v[i]);
+  }
 }
 
 }  // namespace
@@ -467,18 +634,17 @@ void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* 
 }
 
 void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, const uint32_t* nbr_slot,
-                        const uint32_t* nbr_lo, const uint32_t* nbr_hi, uint32_t* bitmaps, uint32_t block,
-                        uint32_t resident, bool explore, uint2* items, uint32_t* counters, uint2* drops,
-                        uint32_t* rflags, unsigned long long* stats, hipStream_t s) {
+                        const uint32_t* nbr_lo, const uint32_t* nbr_hi, const FillOp* fills, uint32_t nfill,
+                        uint32_t* bitmaps, uint32_t block, uint32_t resident, uint2* items, uint32_t* nitems,
+                        uint32_t* rflags, uint32_t* counts, unsigned long long* stats, hipStream_t s) {
   if (!nops) return;
   const uint64_t pairs = (uint64_t)nops * g.nfchunk;
-  const uint32_t nhp = explore ? g.nhparts : 0;
   const bool direct = pairs <= FILTER_DIRECT;
   if (!direct) {
     const uint32_t wgs_per_op = ((g.nfchunk + AR_GROUP - 1) / AR_GROUP + 3) / 4;
     // four waves per workgroup: the kernel's LDS and its per-workgroup append assume 256 threads
     hipLaunchKernelGGL(active_ranges_kernel, dim3(nops * wgs_per_op), dim3(256), 0, s, g.fchunk, g.wrange, g.nfchunk,
-                       ops, nops, bitmaps, g.W, rflags, items, counters);
+                       ops, nops, bitmaps, g.W, rflags, items, nitems);
   }
   // the list's length is known on the device only: a grid of at most
   // FILTER_OVERSUB times as many workgroups as are resident at once strides
@@ -490,20 +656,22 @@ void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, c
   // 65,536 workgroups 13.3 / 19.5; items taken from a shared counter (16
   // per atomic) 14.1 / 28.4, the atomics serialising across the XCDs.
   const uint32_t wpb = block / WAVE;
-  const uint64_t grid =
-      std::min<uint64_t>((pairs + (uint64_t)nops * nhp + wpb - 1) / wpb, (uint64_t)resident * FILTER_OVERSUB);
-  hipLaunchKernelGGL(filter_step_kernel, dim3((uint32_t)grid), dim3(block), sizeof(WaveLds) * wpb, s, g.row, g.col,
-                     g.ckey, g.W, g.fchunk, direct ? nullptr : items, counters, g.nfchunk, nops, g.hparts, nhp, drops,
-                     counters + 1, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, stats);
-  if (nhp)
-    hipLaunchKernelGGL(drop_hubs_kernel, dim3(1), dim3(256), 0, s, drops, counters + 1, bitmaps, g.W);
+  const uint64_t most = (uint64_t)resident * FILTER_OVERSUB;
+  hipLaunchKernelGGL(direct ? filter_step_kernel<false> : filter_step_kernel<true>, dim3((uint32_t)std::min((pairs + wpb - 1) / wpb, most)), dim3(block),
+                     sizeof(WaveLds) * wpb, s, g.row, g.col, g.ckey, g.W, g.fchunk, direct ? nullptr : items, nitems,
+                     g.nfchunk, nops, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, counts, stats);
+  const uint64_t fwaves = (uint64_t)nfill * ((direct ? (uint64_t)g.nfchunk : 0) + g.nhparts);
+  if (!fwaves) return;
+  hipLaunchKernelGGL(fill_kernel, dim3((uint32_t)std::min((fwaves + wpb - 1) / wpb, most)), dim3(block),
+                     sizeof(FillLds) * wpb, s, g.row, g.col, g.key, g.ckey, g.W, g.fchunk, g.nfchunk, g.hparts,
+                     g.nhparts, fills, nfill, counts, !direct, bitmaps, stats);
 }
 
 uint32_t filter_resident(uint32_t block) {
   int dev = 0, ncu = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, filter_step_kernel, (int)block,
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, filter_step_kernel<true>, (int)block,
                                                    sizeof(WaveLds) * (block / WAVE)) != hipSuccess ||
       ncu < 1 || per_cu < 1) {
     (void)hipGetLastError();

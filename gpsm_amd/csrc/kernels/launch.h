@@ -90,30 +90,37 @@ void launch_hub_bits(const DevGraph& g, const uint32_t* hubs, const uint32_t* bl
 // filter.hip ------------------------------------------------------------------
 // Start-vertex candidates: C(slot) = {v : lo <= key[v] <= hi} (check_kernel).
 void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* bitmaps, hipStream_t s);
-// One superstep: every op (one per query) explores or refines its C(u).
-// stats (optional, STAT_COPIES x STAT_STRIDE u64, zeroed by the caller):
-// copy c, entries 0..4 = candidates, adjacency entries read, key gathers,
-// bitmap probes, bits set, added by the workgroups with blockIdx % copies
-// == c (the sum over copies is the launch's total).
+// One superstep: every op (one per query) explores or refines its C(u); the
+// explore ops' neighbours are filled by a second launch (fills, one per
+// neighbour), but above FILTER_DIRECT pairs by the ops themselves, with only
+// the hubs left to it.  stats (optional, STAT_COPIES x STAT_STRIDE u64, zeroed by the
+// caller): copy c, entries 0..4 = candidates, adjacency entries read, key
+// gathers, bitmap probes, bits set, added by the workgroups with blockIdx %
+// copies == c (the sum over copies is the launch's total).
 // Of more than FILTER_DIRECT (op, vertex range) pairs the superstep visits
 // only those whose range holds a candidate of C(u): a first kernel lists them
-// in items (nops x g.nfchunk capacity) and counts them in counters[0], the
-// second processes the list.  Fewer are all visited by one launch, whose waves
-// leave an empty range after reading its bitmap words: listing the pairs of
-// one op on a 1M-vertex graph took 35 us (four workgroups), more than the
-// pass over its 5,000 ranges.  explore: the superstep has explore ops, whose
-// hubs go in parts (drops: nops x the vertices in parts, counted in
-// counters[1]).  counters: two words, zeroed by the caller.  resident:
-// filter_resident(block).  rflags: the refine rounds' change flags
+// in items (nops x g.nfchunk capacity) and counts them in *nitems (zeroed by
+// the caller), the second processes the list.  Fewer are all visited by one
+// launch, whose waves leave an empty range after reading its bitmap words:
+// listing the pairs of one op on a 1M-vertex graph took 35 us (four
+// workgroups), more than the pass over its 5,000 ranges.
+// resident: filter_resident(block).  rflags: the refine rounds' change flags
 // (FilterOp::mark / need), zeroed by the caller once per batch; an op whose
-// need flag is clear is left out.
+// need flag is clear is left out.  counts: the explore ops' candidates
+// (FilterOp::cnt), zeroed by the caller.
 constexpr uint32_t STAT_COPIES = 32, STAT_STRIDE = 8;
 constexpr uint32_t FILTER_OVERSUB = 8;
 constexpr uint64_t FILTER_DIRECT = 1u << 17;
+// A fill is pulled when FILL_PULL times the op's candidates are at least the
+// vertices of the neighbour's label.  The first three fills of 32 cycles and
+// cliques on an R-MAT 18 graph take 485 us pushed, 219 us by this rule; the
+// explore fills of 245 queries on the 1M graph 7.1 ms pushed, 6.4 / 5.7 / 5.8
+// / 5.9 ms with 4 / 12 / 32 / 100 here, 5.9 ms all pulled.
+constexpr uint32_t FILL_PULL = 32;
 void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, const uint32_t* nbr_slot,
-                        const uint32_t* nbr_lo, const uint32_t* nbr_hi, uint32_t* bitmaps, uint32_t block,
-                        uint32_t resident, bool explore, uint2* items, uint32_t* counters, uint2* drops,
-                        uint32_t* rflags, unsigned long long* stats, hipStream_t s);
+                        const uint32_t* nbr_lo, const uint32_t* nbr_hi, const FillOp* fills, uint32_t nfill,
+                        uint32_t* bitmaps, uint32_t block, uint32_t resident, uint2* items, uint32_t* nitems,
+                        uint32_t* rflags, uint32_t* counts, unsigned long long* stats, hipStream_t s);
 // Workgroups of `block` threads of the superstep's kernel that are resident at once.
 uint32_t filter_resident(uint32_t block);
 
