@@ -303,7 +303,7 @@ namespace {
 
 // The graph's arrays back to the context's pool (its stream waited for).
 void free_graph_arrays(gpsm_ctx* c, DevGraph& d) {
-  for (uint32_t* p : {d.row, d.col, d.key, d.ckey, d.fchunk, d.wrange, d.hub_of, d.hub_bits}) c->pool.give(p);
+  for (uint32_t* p : {d.row0, d.col0, d.ids, d.pos, d.lrow, d.row, d.col, d.key, d.ckey, d.fchunk, d.wrange, d.hub_of, d.hub_bits}) c->pool.give(p);
   c->pool.give(d.hparts);
   d = DevGraph();
 }
@@ -333,9 +333,10 @@ bool label_stats(GraphStats& st, const uint32_t* labels, const uint32_t* hist) {
   return st.label_value.size() <= MAX_LABELS;
 }
 
-// The rest of a resident graph once row/col are on the device: label
-// statistics, the label/degree keys, the filter's vertex ranges and the hub
-// bitmaps, on the device but for the choice of labels and hubs.  labels: host
+// The rest of a resident graph once row0/col0 are on the device: label
+// statistics, the vertices' numbering and its CSR, the label/degree keys, the
+// filter's vertex ranges and the hub bitmaps, on the device but for the choice
+// of labels and hubs.  labels: host
 // copy.  check: the rows are the caller's and validated here (GPSM_EINVAL).
 // On failure g is freed.
 int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check) {
@@ -357,9 +358,10 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   d.W = words_of(n);
   d.NB = nblocks_of(n);
   // scratch: what the host reads (row check, number of ranges, label and hub
-  // counts), the labels, the ranges' ends or the hubs' lists
+  // counts), the labels, the ranges' ends
+  // (the counts' words later take the labels' values, starts and ranges)
   constexpr uint32_t kRead = 4 + LABEL_HIST + 1 + HUB_STEPS;
-  const uint64_t head = (kRead + 1) & ~1u, lw = ((uint64_t)n + 1) & ~1ull;
+  const uint64_t head = (std::max(kRead, 4 + 4 * MAX_LABELS + 1) + 1) & ~1u, lw = ((uint64_t)n + 1) & ~1ull;
   if (!c->pool.take(&tmp, head + lw + range_words(n))) return fail(GPSM_ENOMEM);
   uint32_t* dlab = tmp + head;
   uint32_t* ends = dlab + lw;
@@ -367,30 +369,65 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   if (hipMemcpyAsync(dlab, labels, sizeof(uint32_t) * n, hipMemcpyHostToDevice, s) != hipSuccess)
     return fail(GPSM_EDEVICE);
   const uint32_t min_degree = std::max<uint32_t>(c->hub_min_degree, 1);
-  if (check) launch_check_rows(d.row, d.col, n, tmp, s);
-  launch_vertex_stats(d.row, dlab, n, min_degree, tmp + 4, tmp + 4 + LABEL_HIST + 1, s);
-  launch_range_ends(d.row, n, ends, reinterpret_cast<unsigned long long*>(tmp + 2), tmp + 1, s);
+  if (check) launch_check_rows(d.row0, d.col0, n, tmp, s);
+  launch_vertex_stats(d.row0, dlab, n, min_degree, tmp + 4, tmp + 4 + LABEL_HIST + 1, s);
   uint32_t h[kRead];
   if (hipMemcpyAsync(h, tmp, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return fail(GPSM_EDEVICE);
   if (h[0] || !label_stats(st, labels, h + 4)) return fail(GPSM_EINVAL);
-  d.nfchunk = h[2];
-  d.nhparts = h[1];
+  const uint32_t nl = (uint32_t)st.label_value.size();
+  if (!c->pool.take(&d.ids, n) || !c->pool.take(&d.pos, n) || !c->pool.take(&d.key, n)) return fail(GPSM_ENOMEM);
+  // numbered by label, unless there is one label or no room for the sort
+  uint32_t* sort_tmp = nullptr;
+  const bool grouped = nl > 1 && c->pool.take(&sort_tmp, relabel_words(n, d.adj)) &&
+                       c->pool.take(&d.row, (uint64_t)n + 1) && c->pool.take(&d.col, std::max<uint64_t>(d.adj, 1));
+  if (!grouped) {
+    c->pool.give(d.row);
+    d.row = d.row0;
+    d.col = d.col0;
+    if (!sort_tmp && !c->pool.take(&sort_tmp, relabel_words(n, 0))) return fail(GPSM_ENOMEM);
+  }
+  if (grouped) choose_pieces(d, nl);
+  if (d.ngroup > 1 && !c->pool.take(&d.lrow, (uint64_t)n * d.ngroup + 1)) d.ngroup = 1;
+  if (d.ngroup == 1) {
+    d.lrow = d.row;
+    d.gshift = 31;  // every label
+  }
+  // the labels' values and first vertices over the histogram (it has been read)
+  uint32_t* dvalue = tmp + 4;
+  uint32_t* dstart = dvalue + nl;
+  std::vector<uint32_t> label_words(st.label_value);
+  label_words.push_back(0);
+  for (uint32_t x : st.label_count) label_words.push_back(label_words.back() + x);
+  bool ok = hipMemcpyAsync(dvalue, label_words.data(), sizeof(uint32_t) * label_words.size(), hipMemcpyHostToDevice,
+                           s) == hipSuccess;
+  uint32_t found[2] = {0, 0};  // parts of large vertices, ranges
+  if (ok) {
+    launch_relabel(d, dlab, dvalue, nl, sort_tmp, s);
+    launch_range_ends(d.row, n, ends, reinterpret_cast<unsigned long long*>(tmp + 2), tmp + 1, s);
+    ok = hipGetLastError() == hipSuccess &&
+         hipMemcpyAsync(found, tmp + 1, sizeof(found), hipMemcpyDeviceToHost, s) == hipSuccess;
+  }
+  ok = hipStreamSynchronize(s) == hipSuccess && ok;
+  c->pool.give(sort_tmp);
+  if (!ok) return fail(GPSM_EDEVICE);
+  d.nhparts = found[0];
+  d.nfchunk = found[1];
   // hubs: the degree doubles until their bitmaps fit
   const uint32_t* over = h + 4 + LABEL_HIST + 1;
   uint64_t D = min_degree, nh = 0;
   for (uint32_t k = 1; k < HUB_STEPS; ++k) nh += over[k];
   if (!c->hub_max_bytes) nh = 0;
   for (uint32_t k = 1; nh && nh * d.W * 4ull > c->hub_max_bytes; ++k, D *= 2) nh -= over[k];
-  const uint32_t nl = (uint32_t)st.label_value.size();
   uint32_t* hub_tmp = nullptr;
-  if (!c->pool.take(&d.key, n) || !c->pool.take(&d.ckey, std::max<uint64_t>(d.adj, 1)) ||
+  st.label_range.assign(2 * (size_t)nl, 0);
+  if (!c->pool.take(&d.ckey, std::max<uint64_t>(d.adj, 1)) ||
       !c->pool.take(&d.fchunk, (uint64_t)d.nfchunk + 1) || !c->pool.take(&d.wrange, d.W) ||
       (d.nhparts && !c->pool.take(&d.hparts, d.nhparts)) ||
       !c->pool.take(&d.hub_of, n))
     return fail(GPSM_ENOMEM);
-  if (nh && (!c->pool.take(&d.hub_bits, (size_t)nh * d.W) || !c->pool.take(&hub_tmp, hub_words(n, nh)))) {
+  if (nh && (!c->pool.take(&d.hub_bits, (size_t)nh * d.W) || !c->pool.take(&hub_tmp, hub_words(n)))) {
     // no room: no hubs, every edge test searches
     c->pool.give(d.hub_bits);
     d.hub_bits = nullptr;
@@ -398,28 +435,27 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   }
   d.nhub = (uint32_t)nh;
   d.hub_degree = nh ? (uint32_t)D : 0;
-  // the label values over the histogram (it has been read)
-  bool ok = hipMemcpyAsync(tmp + 4, st.label_value.data(), sizeof(uint32_t) * nl, hipMemcpyHostToDevice, s) ==
-            hipSuccess;
-  if (ok) {
-    launch_vertex_keys(d, dlab, tmp + 4, nl, s);
-    launch_ranges(d, ends, tmp, s);  // word 0 is still clear
-    launch_neighbour_keys(d, s);
-    if (nh) {
-      launch_fill_u32(d.hub_bits, 0u, nh * d.W, s);
-      launch_hubs(d, hub_tmp, s);
-    } else {
-      launch_fill_u32(d.hub_of, ~0u, n, s);
-    }
-    ok = hipGetLastError() == hipSuccess;
+  launch_ranges(d, ends, tmp, s);  // word 0 is still clear
+  launch_neighbour_keys(d, s);
+  if (nh) {
+    launch_fill_u32(d.hub_bits, 0u, nh * d.W, s);
+    launch_hubs(d, hub_tmp, s);
+  } else {
+    launch_fill_u32(d.hub_of, ~0u, n, s);
   }
+  if (grouped) launch_label_ranges(d, dstart, nl, dstart + nl + 1, s);
+  ok = hipGetLastError() == hipSuccess;
+  if (grouped)
+    ok = ok && hipMemcpyAsync(st.label_range.data(), dstart + nl + 1, sizeof(uint32_t) * 2 * nl,
+                              hipMemcpyDeviceToHost, s) == hipSuccess;
   ok = hipStreamSynchronize(s) == hipSuccess && ok;
+  for (uint32_t l = 0; !grouped && l < nl; ++l) st.label_range[2 * l + 1] = d.nfchunk;
   c->pool.give(hub_tmp);
   if (!ok) return fail(GPSM_EDEVICE);
   c->pool.give(tmp);
   g->bytes = sizeof(uint32_t) *
-             ((uint64_t)n + 1 + 2 * d.adj + n + d.nfchunk + 1 + d.W + (uint64_t)n + 2ull * d.nhparts +
-              (uint64_t)d.nhub * d.W);
+             ((d.row == d.row0 ? 1 : 2) * ((uint64_t)n + 1 + d.adj) + d.adj + 4ull * n + d.nfchunk + 1 + d.W +
+              (d.ngroup > 1 ? (uint64_t)n * d.ngroup + 1 : 0) + 2ull * d.nhparts + (uint64_t)d.nhub * d.W);
   return GPSM_OK;
 }
 
@@ -445,14 +481,14 @@ int gpsm_graph_upload(gpsm_ctx* c, uint32_t n, const uint32_t* row_offset, const
   DevGraph& d = g->dg;
   d.n = n;
   d.adj = A;
-  if (!c->pool.take(&d.row, (size_t)n + 1) || !c->pool.take(&d.col, std::max<uint64_t>(A, 1))) {
+  if (!c->pool.take(&d.row0, (size_t)n + 1) || !c->pool.take(&d.col0, std::max<uint64_t>(A, 1))) {
     free_graph_arrays(c, d);
     delete g;
     return GPSM_ENOMEM;
   }
-  if (hipMemcpyAsync(d.row, row_offset, sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice, c->stream) !=
+  if (hipMemcpyAsync(d.row0, row_offset, sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice, c->stream) !=
           hipSuccess ||
-      (A && hipMemcpyAsync(d.col, col, sizeof(uint32_t) * A, hipMemcpyHostToDevice, c->stream) != hipSuccess)) {
+      (A && hipMemcpyAsync(d.col0, col, sizeof(uint32_t) * A, hipMemcpyHostToDevice, c->stream) != hipSuccess)) {
     (void)hipGetLastError();
     (void)hipStreamSynchronize(c->stream);
     free_graph_arrays(c, d);
@@ -474,7 +510,7 @@ int gpsm_graph_upload_edges(gpsm_ctx* c, uint32_t n, uint64_t m, const uint32_t*
   DevGraph& d = g->dg;
   d.n = n;
   uint64_t adj = 0;
-  int rc = build_csr_from_edges(n, m, src, dst, c->pool, c->stream, &d.row, &d.col, &adj);
+  int rc = build_csr_from_edges(n, m, src, dst, c->pool, c->stream, &d.row0, &d.col0, &adj);
   if (rc) {
     free_graph_arrays(c, d);
     delete g;
@@ -497,10 +533,10 @@ int gpsm_graph_csr(const gpsm_graph* g, uint32_t* row_offset, uint32_t* col) {
   if (!g || !row_offset || (g->dg.adj && !col)) return GPSM_EINVAL;
   hipSetDevice(g->ctx->device);
   hipStream_t s = g->ctx->stream;
-  if (hipMemcpyAsync(row_offset, g->dg.row, sizeof(uint32_t) * ((size_t)g->dg.n + 1), hipMemcpyDeviceToHost, s) !=
+  if (hipMemcpyAsync(row_offset, g->dg.row0, sizeof(uint32_t) * ((size_t)g->dg.n + 1), hipMemcpyDeviceToHost, s) !=
           hipSuccess ||
       (g->dg.adj &&
-       hipMemcpyAsync(col, g->dg.col, sizeof(uint32_t) * g->dg.adj, hipMemcpyDeviceToHost, s) != hipSuccess) ||
+       hipMemcpyAsync(col, g->dg.col0, sizeof(uint32_t) * g->dg.adj, hipMemcpyDeviceToHost, s) != hipSuccess) ||
       hipStreamSynchronize(s) != hipSuccess) {
     (void)hipGetLastError();
     return GPSM_EDEVICE;
@@ -655,7 +691,7 @@ struct PhaseSig {
   void add(uint64_t v) { w.push_back(v); }
   void add(const void* p) { w.push_back((uint64_t)(uintptr_t)p); }
   void add_graph(const DevGraph& g) {
-    add(g.n), add(g.adj), add(g.W), add(g.NB), add(g.row), add(g.col), add(g.key), add(g.ckey), add(g.fchunk),
+    add(g.n), add(g.adj), add(g.W), add(g.NB), add(g.ids), add(g.row), add(g.lrow), add(g.ngroup), add(g.gshift), add(g.col), add(g.key), add(g.ckey), add(g.fchunk),
         add(g.nfchunk), add(g.wrange), add(g.hparts), add(g.nhparts), add(g.hub_of), add(g.hub_bits), add(g.nhub), add(g.hub_degree);
   }
 };
@@ -798,6 +834,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // that leave C(u) part of the way (after the slots')
   std::vector<FillOp> fills;
   std::vector<uint32_t> fill_off(maxsteps + 1, 0);
+  std::vector<uint32_t> step_ranges(maxsteps, 0);  // the most vertex ranges an op's or fill's label has
   uint32_t nexplore = 0, erows = nslots;
   for (uint32_t b = 0; b < nq; ++b)
     if (Q[b].active) init.push_back({Q[b].vbase + Q[b].fs.start, Q[b].fs.start_lo, Q[b].fs.start_hi});
@@ -815,12 +852,20 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       op.nbr_off = (uint32_t)nbr_slot.size();
       op.mark = op.need = ~0u;
       op.e_slot = op.cnt = ~0u;
+      const uint32_t ul = st.dense(S.hq.lab[fsx.u]) - 1;
+      op.range0 = st.label_range[2 * ul];
+      op.nrange = st.label_range[2 * ul + 1] - op.range0;
+      step_ranges[sidx] = std::max(step_ranges[sidx], op.nrange);
       if (fsx.type == OP_EXPLORE) {
         op.cnt = nexplore++;
         op.e_slot = erows;
-        for (uint32_t i = 0; i < op.nv; ++i)
+        for (uint32_t i = 0; i < op.nv; ++i) {
+          const uint32_t vl = st.dense(S.hq.lab[fsx.v[i]]) - 1, v0 = st.label_range[2 * vl];
+          const uint32_t nr = st.label_range[2 * vl + 1] - v0;
           fills.push_back({op.u_slot, i + 1 < op.nv ? op.e_slot + i : ~0u, S.vbase + fsx.v[i], fsx.lo[i], fsx.hi[i],
-                           op.cnt, st.count(S.hq.lab[fsx.v[i]])});
+                           (ul + 1) << KEY_DEG_BITS, {op.range0, v0}, {op.nrange, nr}, op.cnt, st.label_count[vl]});
+          step_ranges[sidx] = std::max(step_ranges[sidx], nr);
+        }
         erows += op.nv - 1;
       }
       if (fsx.type == OP_REFINE) {
@@ -829,8 +874,8 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       }
       for (size_t i = 0; i < fsx.v.size(); ++i) {
         nbr_slot.push_back(S.vbase + fsx.v[i]);
-        nbr_lo.push_back(fsx.type == OP_EXPLORE ? fsx.lo[i] : 0);
-        nbr_hi.push_back(fsx.type == OP_EXPLORE ? fsx.hi[i] : 0);
+        nbr_lo.push_back(fsx.lo[i]);
+        nbr_hi.push_back(fsx.hi[i]);
       }
       fops.push_back(op);
     }
@@ -847,9 +892,10 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if ((rc = c->bufs[B_COUNTS].ensure(sizeof(uint32_t) * std::max<uint32_t>(nslots, 1)))) return rc;
   if ((rc = c->bufs[B_SEGC].ensure(sizeof(uint32_t) * std::max<uint64_t>((uint64_t)nslots * segs_of(W), 1))))
     return rc;
-  uint32_t max_ops = 0;  // ops of the largest superstep
-  for (uint32_t sidx = 0; sidx < maxsteps; ++sidx) max_ops = std::max(max_ops, step_off[sidx + 1] - step_off[sidx]);
-  if ((rc = c->bufs[B_FITEMS].ensure(sizeof(uint2) * std::max<uint64_t>((uint64_t)max_ops * dg.nfchunk, 1))) ||
+  uint64_t max_items = 1;  // (op, vertex range) pairs of the largest superstep
+  for (uint32_t sidx = 0; sidx < maxsteps; ++sidx)
+    max_items = std::max(max_items, (uint64_t)(step_off[sidx + 1] - step_off[sidx]) * step_ranges[sidx]);
+  if ((rc = c->bufs[B_FITEMS].ensure(sizeof(uint2) * max_items)) ||
       (rc = c->bufs[B_FNITEMS].ensure(sizeof(uint32_t) * std::max<size_t>(ncounters, 1))) ||
       (rc = c->bufs[B_RFLAGS].ensure(sizeof(uint32_t) * 4 * (uint64_t)std::max<uint32_t>(nq, 1))))
     return rc;
@@ -872,6 +918,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     sig_a.add(nslots), sig_a.add(maxsteps), sig_a.add(nq), sig_a.add(init.size()), sig_a.add(fblock);
     for (uint32_t v : step_off) sig_a.add(v);
     for (uint32_t v : fill_off) sig_a.add(v);
+    for (uint32_t v : step_ranges) sig_a.add(v);
     sig_a.add(erows), sig_a.add(ncounters);
   }
   bool replayed = o.use_graph && replay_cached(c, 0, sig_a.w, s, &rc);
@@ -895,7 +942,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       launch_filter_step(dg, dptr<FilterOp>(c, B_FOPS) + step_off[sidx], nops_s, dptr<uint32_t>(c, B_NBR_SLOT),
                          dptr<uint32_t>(c, B_NBR_LO), dptr<uint32_t>(c, B_NBR_HI),
                          dptr<FillOp>(c, B_FILLS) + fill_off[sidx], fill_off[sidx + 1] - fill_off[sidx], bitmaps,
-                         fblock, fresident, dptr<uint2>(c, B_FITEMS), dptr<uint32_t>(c, B_FNITEMS) + sidx,
+                         step_ranges[sidx], fblock, fresident, dptr<uint2>(c, B_FITEMS), dptr<uint32_t>(c, B_FNITEMS) + sidx,
                          dptr<uint32_t>(c, B_RFLAGS), dptr<uint32_t>(c, B_FNITEMS) + maxsteps,
                          counters ? fstats + fstat_step * sidx : nullptr, s);
       pend(K_FILTER, a, 4.0 * W * nops_s, counters ? (int)sidx : -1);
@@ -1304,10 +1351,10 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     launch_cet_sums(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_WDESC), (uint32_t)wdesc.size(),
                     dptr<uint32_t>(c, B_WCHUNK), dptr<CetAgg>(c, B_AGGS), cgrid, s,
                     counters ? fstats + fstat_step * slot_cet_w : nullptr);
-    launch_cet_aggs(bitmaps, dptr<uint32_t>(c, B_BPREFIX), W, NB, dptr<AggDesc>(c, B_ADESC), (uint32_t)adesc.size(),
+    launch_cet_aggs(dg, bitmaps, dptr<uint32_t>(c, B_BPREFIX), dptr<AggDesc>(c, B_ADESC), (uint32_t)adesc.size(),
                     dptr<uint32_t>(c, B_ACHUNK), dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_LISTS),
                     dptr<CetAgg>(c, B_AGGS), cgrid, s);
-    launch_cet_terms(dptr<uint32_t>(c, B_LISTS), dptr<CetDesc>(c, B_JDESC), dptr<uint32_t>(c, B_TERM_DESC),
+    launch_cet_terms(dg, dptr<uint32_t>(c, B_LISTS), dptr<CetDesc>(c, B_JDESC), dptr<uint32_t>(c, B_TERM_DESC),
                      dptr<uint64_t>(c, B_TERM_START), (uint32_t)term_desc.size(), term_words,
                      dptr<unsigned long long>(c, B_TERMS), s);
     pend(K_CET_WRITE, pa, 0.0, counters ? slot_cet_w : -1);
@@ -1320,8 +1367,9 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // by side on two streams, which a captured graph's replay does not keep
   {
     JoinArgs ja{};
-    ja.row = dg.row;
     ja.col = dg.col;
+    ja.ids = dg.ids;
+    ja.pieces = pieces_of(dg);
     ja.hub_of = dg.hub_of;
     ja.hub_bits = dg.hub_bits;
     ja.bitmaps = bitmaps;

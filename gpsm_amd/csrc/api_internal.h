@@ -124,9 +124,6 @@ struct BatchHooks {
 int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* qs, const gpsm_opts* opts,
               gpsm_result* out, const BatchHooks* hooks);
 
-// scan.hip
-void launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
-
 }  // namespace gpsm
 
 namespace gpsm {

@@ -26,6 +26,12 @@ constexpr uint32_t BLOCK_BITS = 256;  // rank-index block
 inline uint32_t words_of(uint32_t n) { return (n + 31) / 32; }
 inline uint32_t nblocks_of(uint32_t n) { return (words_of(n) + 7) / 8 + 1; }
 
+// A data graph's rows in pieces by the neighbours' label (DevGraph::lrow).
+struct Pieces {
+  const uint32_t* lrow;
+  uint32_t n, gshift;
+};
+
 enum FilterOpType : uint32_t { OP_EXPLORE = 1, OP_REFINE = 2 };
 
 // One filter operation of one query in a superstep.
@@ -45,6 +51,8 @@ struct FilterOp {
   // but hand on matches of v_0, v_1, ...; index of the op's candidate count
   uint32_t e_slot;
   uint32_t cnt;
+  // vertex ranges that hold u's label: [range0, range0 + nrange)
+  uint32_t range0, nrange;
 };
 
 // One neighbour v_i of an explore op: C(v_i) receives the vertices with key in
@@ -52,8 +60,10 @@ struct FilterOp {
 struct FillOp {
   uint32_t u_slot, e_slot, v_slot;
   uint32_t lo, hi;
-  uint32_t cnt;     // the op's candidate count
-  uint32_t nlabel;  // vertices of v_i's label
+  uint32_t u_lo;              // low key of u's label
+  uint32_t range0[2], nrange[2];  // vertex ranges that hold u's label, v's label
+  uint32_t cnt;                   // the op's candidate count
+  uint32_t nlabel;                // vertices of v_i's label
 };
 
 // Initial label/degree check of a query's start vertex.

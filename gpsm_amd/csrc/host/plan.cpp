@@ -156,6 +156,12 @@ void make_filter_schedule(const HostQuery& q, const GraphStats& s, FilterSchedul
         if (valid[id]) st.v.push_back(id);
       for (uint32_t id : q.out[u])
         if (valid[id]) st.v.push_back(id);
+      for (uint32_t v : st.v) {
+        uint32_t lo, hi;
+        key_range(q, s, v, lo, hi);
+        st.lo.push_back(lo);
+        st.hi.push_back(hi);
+      }
       if (!st.v.empty()) out.steps.push_back(std::move(st));
     }
 }

@@ -16,6 +16,7 @@ struct GraphStats {
   uint64_t adj = 0;
   std::vector<uint32_t> label_value;  // distinct labels, ascending
   std::vector<uint32_t> label_count;  // vertices per label
+  std::vector<uint32_t> label_range;  // filter vertex ranges of each label: first, one past the last
   // dense label id (1-based index into label_value) or 0 when absent
   uint32_t dense(uint32_t label) const;
   uint32_t count(uint32_t label) const;
@@ -39,7 +40,7 @@ struct FilterStep {
   uint32_t u;
   uint32_t round = 0;            // refine: round 0..3
   std::vector<uint32_t> v;       // neighbour query ids, in the reference's order
-  std::vector<uint32_t> lo, hi;  // explore: key range of each neighbour
+  std::vector<uint32_t> lo, hi;  // key range of each neighbour
 };
 
 struct FilterSchedule {

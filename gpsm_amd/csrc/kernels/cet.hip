@@ -7,10 +7,9 @@
 // of a table, wave j takes candidates j, j + N, j + 2N, ..., so the hubs of
 // a power-law graph (its lowest ids, the first candidates) land on
 // different waves.  The wave walks the concatenated adjacency of its
-// candidates 64 entries per step (balanced across hub and leaf candidates)
-// and tests C(w) membership in the bitmap, probing it only for entries
-// whose neighbour key (ckey, read beside col) is in w's label/degree range:
-// C(w) holds no vertex outside it.  Outputs are per candidate (its
+// candidates towards w's label (DevGraph::lrow: C(w) holds no vertex of
+// another) 64 entries per step (balanced across hub and leaf candidates) and
+// tests C(w) membership in the bitmap.  Outputs are per candidate (its
 // count, its list at its offset), so the assignment does not change them.
 // The write pass ranks each hit inside its candidate's run with a ballot,
 // so lists stay in adjacency order without a second scan.
@@ -53,15 +52,15 @@ __device__ __forceinline__ void flush_tally(const CetTally& t, unsigned long lon
 // Lane l of chunk j of a table with nch chunks holds candidate j + l * nch.
 __device__ __forceinline__ uint32_t cand_index(uint32_t j, uint32_t nch, uint32_t lane) { return j + lane * nch; }
 
-__device__ __forceinline__ void load_chunk(const uint32_t* __restrict__ row, const uint32_t* __restrict__ clist,
+__device__ __forceinline__ void load_chunk(const Pieces& pieces, const uint32_t* __restrict__ clist,
                                            const CetDesc& d, uint32_t j, uint32_t nch, CetLds& L, bool& mine,
                                            uint32_t& D) {
   const uint32_t lane = lane_id();
   const uint32_t ci = cand_index(j, nch, lane);
   mine = ci < d.ncand;
   const uint32_t id = mine ? clist[d.clist_off + ci] : 0u;
-  const uint32_t off = mine ? row[id] : 0u;
-  const uint32_t deg = mine ? row[id + 1] - off : 0u;
+  uint32_t off = 0, deg = 0;
+  if (mine) piece(pieces, id, d.w_lo, off, deg);
   const uint32_t incl = wave_incl_scan(deg);
   D = uniform(__shfl(incl, WAVE - 1, WAVE));
   L.pre[lane] = incl - deg;
@@ -72,9 +71,7 @@ __device__ __forceinline__ void load_chunk(const uint32_t* __restrict__ row, con
 
 // Eight waves per SIMD (64 VGPRs, no spill; seven at the compiler's own
 // choice): 9-11% faster on the 1M Chung-Lu mix and the R-MAT 22 shapes.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) cet_count_kernel(const uint32_t* __restrict__ row,
-                                                        const uint32_t* __restrict__ col,
-                                                        const uint32_t* __restrict__ ckey,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) cet_count_kernel(Pieces pieces, const uint32_t* __restrict__ col,
                                                         const uint32_t* __restrict__ bitmaps, uint32_t W,
                                                         const uint32_t* __restrict__ clist, CetDesc* descs,
                                                         const uint32_t* __restrict__ chunk_base, uint32_t ndesc,
@@ -93,15 +90,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) c
     const uint32_t j = it - chunk_base[di], nch = chunk_base[di + 1] - chunk_base[di];
     bool mine;
     uint32_t D;
-    load_chunk(row, clist, d, j, nch, L, mine, D);
+    load_chunk(pieces, clist, d, j, nch, L, mine, D);
     tl.cand += mine;
     const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
-    const uint32_t wlo = d.w_hi ? d.w_lo : 0u, whi = d.w_hi ? d.w_hi : ~0u;
     uint32_t tot = 0;
     for (uint32_t f = 0; f < D; f += WAVE * CET_UNROLL) {
       // CET_UNROLL entries per lane: all adjacency and key loads, then the
       // probes of the entries whose key is in range
-      uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], ks[CET_UNROLL], es[CET_UNROLL];
+      uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], es[CET_UNROLL];
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u) cis[u] = f + u * WAVE + lane;
       halving_search<CET_UNROLL>(L.pre, WAVE, cis);
@@ -111,7 +107,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) c
       for (int u = 0; u < CET_UNROLL; ++u) {
         if (f + u * WAVE + lane < D) {
           mvs[u] = col[es[u]];
-          ks[u] = ckey[es[u]];
         } else {
           cis[u] = WAVE;
         }
@@ -120,12 +115,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) c
       uint32_t pw[CET_UNROLL];
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u)
-        pw[u] = cis[u] != WAVE && ks[u] >= wlo && ks[u] <= whi ? bm_w[mvs[u] >> 5] >> (mvs[u] & 31) : 0u;
+        pw[u] = cis[u] != WAVE ? bm_w[mvs[u] >> 5] >> (mvs[u] & 31) : 0u;
       if (stats) {
 #pragma unroll
         for (int u = 0; u < CET_UNROLL; ++u) {
           tl.ent += cis[u] != WAVE;
-          tl.probe += cis[u] != WAVE && ks[u] >= wlo && ks[u] <= whi;
+          tl.probe += cis[u] != WAVE;
         }
       }
 #pragma unroll
@@ -177,9 +172,7 @@ __global__ void __launch_bounds__(256) cet_offsets_kernel(const CetDesc* __restr
   if (threadIdx.x == 0) o[d.ncand] = min(carry, d.list_cap);
 }
 
-__global__ void __launch_bounds__(256) cet_write_kernel(const uint32_t* __restrict__ row,
-                                                        const uint32_t* __restrict__ col,
-                                                        const uint32_t* __restrict__ ckey,
+__global__ void __launch_bounds__(256) cet_write_kernel(Pieces pieces, const uint32_t* __restrict__ col,
                                                         const uint32_t* __restrict__ bitmaps, uint32_t W,
                                                         const uint32_t* __restrict__ clist,
                                                         const CetDesc* __restrict__ descs,
@@ -200,19 +193,18 @@ __global__ void __launch_bounds__(256) cet_write_kernel(const uint32_t* __restri
     const uint32_t j = it - chunk_base[di], nch = chunk_base[di + 1] - chunk_base[di];
     bool mine;
     uint32_t D;
-    load_chunk(row, clist, d, j, nch, L, mine, D);
+    load_chunk(pieces, clist, d, j, nch, L, mine, D);
     tl.cand += mine;
     // each lane's list starts at its candidate's offset; cnt advances it
     L.cnt[lane_id()] = mine ? offsets[d.off_base + cand_index(j, nch, lane_id())] : 0u;
     wave_sync();
     const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
-    const uint32_t wlo = d.w_hi ? d.w_lo : 0u, whi = d.w_hi ? d.w_hi : ~0u;
     uint32_t* out = lists + d.list_base;
     for (uint32_t f = 0; f < D; f += WAVE * CET_UNROLL) {
       // CET_UNROLL sub-steps of 64 entries: all adjacency and key loads, the
       // probes of in-range entries, then the writes sub-step by sub-step
       // (lists stay in adjacency order)
-      uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], ks[CET_UNROLL];
+      uint32_t cis[CET_UNROLL], mvs[CET_UNROLL];
       bool hits[CET_UNROLL];
       uint32_t es[CET_UNROLL];
 #pragma unroll
@@ -223,25 +215,21 @@ __global__ void __launch_bounds__(256) cet_write_kernel(const uint32_t* __restri
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u) {
         mvs[u] = 0;
-        ks[u] = 0;
         hits[u] = false;
-        if (f + u * WAVE + lane < D) {
-          mvs[u] = col[es[u]];
-          ks[u] = ckey[es[u]];
-        }
+        if (f + u * WAVE + lane < D) mvs[u] = col[es[u]];
       }
       // the probes' bitmap words loaded together, then tested
       uint32_t pw[CET_UNROLL];
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u)
-        pw[u] = f + u * WAVE + lane < D && ks[u] >= wlo && ks[u] <= whi ? bm_w[mvs[u] >> 5] >> (mvs[u] & 31) : 0u;
+        pw[u] = f + u * WAVE + lane < D ? bm_w[mvs[u] >> 5] >> (mvs[u] & 31) : 0u;
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u) hits[u] = (pw[u] & 1u) != 0;
       if (stats) {
 #pragma unroll
         for (int u = 0; u < CET_UNROLL; ++u) {
           tl.ent += f + u * WAVE + lane < D;
-          tl.probe += f + u * WAVE + lane < D && ks[u] >= wlo && ks[u] <= whi;
+          tl.probe += f + u * WAVE + lane < D;
         }
       }
 #pragma unroll
@@ -291,9 +279,8 @@ struct SumLds {
   unsigned long long s[WAVE];
 };
 
-__global__ void __launch_bounds__(256) cet_sum_kernel(const uint32_t* __restrict__ row,
-                                                      const uint32_t* __restrict__ col,
-                                                      const uint32_t* __restrict__ ckey,
+__global__ void __launch_bounds__(256) cet_sum_kernel(Pieces pieces, const uint32_t* __restrict__ col,
+                                                      const uint32_t* __restrict__ ids,
                                                       const uint32_t* __restrict__ bitmaps, uint32_t W,
                                                       const uint32_t* __restrict__ clist,
                                                       const CetDesc* __restrict__ descs,
@@ -314,12 +301,11 @@ __global__ void __launch_bounds__(256) cet_sum_kernel(const uint32_t* __restrict
     bool mine;
     uint32_t D;
     L.s[lane] = 0;
-    load_chunk(row, clist, d, j, nch, L.c, mine, D);
+    load_chunk(pieces, clist, d, j, nch, L.c, mine, D);
     tl.cand += mine;
     const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
-    const uint32_t wlo = d.w_hi ? d.w_lo : 0u, whi = d.w_hi ? d.w_hi : ~0u;
     for (uint32_t f = 0; f < D; f += WAVE * CET_UNROLL) {
-      uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], ks[CET_UNROLL], pw[CET_UNROLL];
+      uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], pw[CET_UNROLL];
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u) cis[u] = f + u * WAVE + lane;
       halving_search<CET_UNROLL>(L.c.pre, WAVE, cis);  // an index past D falls in the last candidate
@@ -328,14 +314,13 @@ __global__ void __launch_bounds__(256) cet_sum_kernel(const uint32_t* __restrict
         const uint32_t g = f + u * WAVE + lane;
         const uint32_t e = L.c.off[cis[u]] + (g - L.c.pre[cis[u]]);
         mvs[u] = g < D ? col[e] : 0u;
-        ks[u] = g < D ? ckey[e] : 0u;
       }
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u) {
-        const bool in = f + u * WAVE + lane < D && ks[u] >= wlo && ks[u] <= whi;
+        const bool in = f + u * WAVE + lane < D;
         pw[u] = in ? bm_w[mvs[u] >> 5] >> (mvs[u] & 31) : 0u;
         if (stats) {
-          tl.ent += f + u * WAVE + lane < D;
+          tl.ent += in;
           tl.probe += in;
         }
       }
@@ -347,7 +332,7 @@ __global__ void __launch_bounds__(256) cet_sum_kernel(const uint32_t* __restrict
         const uint32_t fu = f + u * WAVE, ci = cis[u];
         const uint32_t next = __shfl_down(ci, 1, WAVE);
         const bool tail = lane == WAVE - 1 || next != ci;
-        seg_add(L.s, ci, tail, lane == WAVE - 1 ? (uint32_t)WAVE : next, hit ? tuple_term(d.term_qid, mvs[u]) : 0ull);
+        seg_add(L.s, ci, tail, lane == WAVE - 1 ? (uint32_t)WAVE : next, hit ? tuple_term(d.term_qid, ids[mvs[u]]) : 0ull);
         if (tail) {
           const uint32_t seg_lo = L.c.pre[ci] > fu ? L.c.pre[ci] - fu : 0u;
           if (seg_lo < WAVE) {
@@ -383,7 +368,8 @@ struct AggLds {
   unsigned long long s[WAVE], a[WAVE], b[WAVE];
 };
 
-__global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict__ bitmaps,
+__global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict__ ids,
+                                                      const uint32_t* __restrict__ bitmaps,
                                                       const uint32_t* __restrict__ bprefix, uint32_t W, uint32_t NB,
                                                       const AggDesc* __restrict__ descs, uint32_t ndesc,
                                                       const uint32_t* __restrict__ chunk_base,
@@ -430,6 +416,7 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
 #pragma unroll
       for (int u = 0; u < AGG_UNROLL; ++u) {
         const bool in = f + u * WAVE + lane < D;
+        const uint32_t id = ids[v[u]];
         xa[u] = xb[u] = 0;
         if (d.mode == AGG_CHAIN) {  // uniform
           const CetAgg r = aggs[d.w_agg_base + rank_of(bm_y, bp_y, v[u])];
@@ -438,9 +425,9 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
         } else if (d.mode == AGG_SIBLING) {
           const bool hit = in && bit_of(bm_w, v[u]);
           xa[u] = hit;
-          xb[u] = hit ? tuple_term(d.w_qid, v[u]) : 0ull;
+          xb[u] = hit ? tuple_term(d.w_qid, id) : 0ull;
         }
-        t[u] = in ? tuple_term(d.y_qid, v[u]) : 0ull;
+        t[u] = in ? tuple_term(d.y_qid, id) : 0ull;
         xb[u] *= t[u];
       }
 #pragma unroll
@@ -471,7 +458,8 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
 }
 
 // One thread per term: the table by a binary search over the term ranges.
-__global__ void __launch_bounds__(256) cet_terms_kernel(const uint32_t* __restrict__ lists,
+__global__ void __launch_bounds__(256) cet_terms_kernel(const uint32_t* __restrict__ ids,
+                                                        const uint32_t* __restrict__ lists,
                                                         const CetDesc* __restrict__ descs,
                                                         const uint32_t* __restrict__ term_desc,
                                                         const uint64_t* __restrict__ term_start, uint32_t nd,
@@ -486,7 +474,7 @@ __global__ void __launch_bounds__(256) cet_terms_kernel(const uint32_t* __restri
     }
     const CetDesc& d = descs[term_desc[lo]];
     const uint64_t e = t - term_start[lo];
-    terms[t] = e < d.list_cap ? tuple_term(d.term_qid, lists[d.list_base + e]) : 0ull;
+    terms[t] = e < d.list_cap ? tuple_term(d.term_qid, ids[lists[d.list_base + e]]) : 0ull;
   }
 }
 
@@ -514,7 +502,7 @@ void launch_cet_count(const DevGraph& g, const uint32_t* bitmaps, const uint32_t
                       hipStream_t s, unsigned long long* stats) {
   if (!ndesc) return;
   hipLaunchKernelGGL(chunk_base_kernel, dim3(1), dim3(256), 0, s, descs, ndesc, chunk_base);
-  hipLaunchKernelGGL(cet_count_kernel, dim3(grid), dim3(256), 0, s, g.row, g.col, g.ckey, bitmaps, g.W, clist,
+  hipLaunchKernelGGL(cet_count_kernel, dim3(grid), dim3(256), 0, s, pieces_of(g), g.col, bitmaps, g.W, clist,
                      descs, chunk_base, ndesc, offsets, per_cand, stats);
 }
 
@@ -523,13 +511,13 @@ void launch_cet_offsets(CetDesc* descs, uint32_t ndesc, uint32_t* offsets, hipSt
   hipLaunchKernelGGL(cet_offsets_kernel, dim3(ndesc), dim3(256), 0, s, descs, offsets);
 }
 
-void launch_cet_terms(const uint32_t* lists, const CetDesc* descs, const uint32_t* term_desc,
+void launch_cet_terms(const DevGraph& g, const uint32_t* lists, const CetDesc* descs, const uint32_t* term_desc,
                       const uint64_t* term_start, uint32_t nterm_desc, uint64_t nterms, unsigned long long* terms,
                       hipStream_t s) {
   if (!nterm_desc || !nterms) return;
   uint64_t grid = (nterms + 255) / 256;
   if (grid > 16384) grid = 16384;
-  hipLaunchKernelGGL(cet_terms_kernel, dim3((uint32_t)grid), dim3(256), 0, s, lists, descs, term_desc, term_start,
+  hipLaunchKernelGGL(cet_terms_kernel, dim3((uint32_t)grid), dim3(256), 0, s, g.ids, lists, descs, term_desc, term_start,
                      nterm_desc, nterms, terms);
 }
 
@@ -537,16 +525,16 @@ void launch_cet_sums(const DevGraph& g, const uint32_t* bitmaps, const uint32_t*
                      uint32_t ndesc, const uint32_t* chunk_base, CetAgg* aggs, uint32_t grid, hipStream_t s,
                      unsigned long long* stats) {
   if (!ndesc) return;
-  hipLaunchKernelGGL(cet_sum_kernel, dim3(grid), dim3(256), 0, s, g.row, g.col, g.ckey, bitmaps, g.W, clist, descs,
+  hipLaunchKernelGGL(cet_sum_kernel, dim3(grid), dim3(256), 0, s, pieces_of(g), g.col, g.ids, bitmaps, g.W, clist, descs,
                      chunk_base, ndesc, aggs, stats);
 }
 
-void launch_cet_aggs(const uint32_t* bitmaps, const uint32_t* bprefix, uint32_t W, uint32_t NB, const AggDesc* descs,
+void launch_cet_aggs(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* bprefix, const AggDesc* descs,
                      uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
                      CetAgg* aggs, uint32_t grid, hipStream_t s) {
   if (!ndesc) return;
-  hipLaunchKernelGGL(cet_agg_kernel, dim3(grid), dim3(256), 0, s, bitmaps, bprefix, W, NB, descs, ndesc, chunk_base,
-                     offsets, lists, aggs);
+  hipLaunchKernelGGL(cet_agg_kernel, dim3(grid), dim3(256), 0, s, g.ids, bitmaps, bprefix, g.W, g.NB, descs, ndesc,
+                     chunk_base, offsets, lists, aggs);
 }
 
 void launch_cet_write(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, const CetDesc* descs,
@@ -554,7 +542,7 @@ void launch_cet_write(const DevGraph& g, const uint32_t* bitmaps, const uint32_t
                       hipStream_t s, unsigned long long* stats) {
   if (!ndesc) return;
   hipLaunchKernelGGL(chunk_base_kernel, dim3(1), dim3(256), 0, s, descs, ndesc, chunk_base);
-  hipLaunchKernelGGL(cet_write_kernel, dim3(grid), dim3(256), 0, s, g.row, g.col, g.ckey, bitmaps, g.W, clist,
+  hipLaunchKernelGGL(cet_write_kernel, dim3(grid), dim3(256), 0, s, pieces_of(g), g.col, bitmaps, g.W, clist,
                      descs, chunk_base, ndesc, offsets, lists, stats);
 }
 

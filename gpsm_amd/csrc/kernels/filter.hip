@@ -6,14 +6,17 @@
 // Layout: candidate sets are bitmaps (1 bit per data vertex, 32-bit words);
 // the reference used one byte per (query vertex, data vertex).
 // Parallel decomposition: one wave per (op, vertex range).  The ranges are
-// fixed per data graph (DevGraph::fchunk): at most 1024 vertices and 4096
-// adjacency entries each, so a power-law graph's hubs (which a Chung-Lu or
+// fixed per data graph (DevGraph::fchunk): at most FCHUNK_VERTS vertices and
+// FCHUNK_ENTRIES adjacency entries each, so a power-law graph's hubs (which a Chung-Lu or
 // R-MAT generator gives the lowest ids) do not pile onto one wave.  The wave
 // compacts the range's candidates into LDS (the reference's kernel_collect,
-// fused), then walks the concatenated adjacency lists of 64 candidates at a
-// time, 64 adjacency entries per lane step (lane t takes entry t; a binary
-// search in the 64 degree prefix sums finds its candidate), so hub and leaf
-// candidates share lanes evenly instead of one 32-lane warp per candidate.
+// fused), then, neighbour by neighbour of the query vertex, walks the entries
+// of 64 candidates at a time towards that neighbour's label, concatenated,
+// 64 entries per lane step (lane t takes entry t; a binary search in the 64
+// prefix sums finds its candidate), so hub and leaf candidates share lanes
+// evenly instead of one 32-lane warp per candidate.
+#include <type_traits>
+
 #include "launch.h"
 #include "wave.h"
 
@@ -79,7 +82,7 @@ constexpr uint32_t AR_GROUP = 4 * WAVE;  // vertex ranges per wave
 constexpr int AR_UNROLL = 8;             // bitmap words in flight per lane
 
 __global__ void __launch_bounds__(256) active_ranges_kernel(const uint32_t* __restrict__ fchunk,
-                                                             const uint32_t* __restrict__ wrange, uint32_t chunks,
+                                                             const uint32_t* __restrict__ wrange, uint32_t max_ranges,
                                                              const FilterOp* __restrict__ ops, uint32_t nops,
                                                              const uint32_t* __restrict__ bitmaps, uint32_t W,
                                                              const uint32_t* __restrict__ rflags,
@@ -88,7 +91,7 @@ __global__ void __launch_bounds__(256) active_ranges_kernel(const uint32_t* __re
   __shared__ uint32_t s_act[4][AR_GROUP];
   __shared__ uint32_t s_wtot[4], s_wbase[4];
   const uint32_t lane = lane_id(), wv = threadIdx.x / WAVE;
-  const uint32_t groups = (chunks + AR_GROUP - 1) / AR_GROUP;
+  const uint32_t groups = (max_ranges + AR_GROUP - 1) / AR_GROUP;
   const uint32_t wgs_per_op = (groups + 3) / 4;
   const uint32_t o_wg = blockIdx.x / wgs_per_op;  // the workgroup's op
   const uint32_t g = (blockIdx.x % wgs_per_op) * 4 + wv;
@@ -99,10 +102,12 @@ __global__ void __launch_bounds__(256) active_ranges_kernel(const uint32_t* __re
   const uint32_t o = o_wg;
   uint32_t c0 = 0, nc = 0;
   if (o < nops && g < groups) {  // uniform per wave
-    c0 = g * AR_GROUP;
+    const uint32_t nrange = uniform(ops[o].nrange);
+    c0 = uniform(ops[o].range0) + g * AR_GROUP;
     const uint32_t need = uniform(ops[o].need);
     // an op whose previous refine round removed nothing lists no range
-    if (need == ~0u || uniform(rflags[need]) != 0) nc = min(AR_GROUP, chunks - c0);
+    if (g * AR_GROUP < nrange && (need == ~0u || uniform(rflags[need]) != 0))
+      nc = min(AR_GROUP, nrange - g * AR_GROUP);
   }
   if (nc) {
     for (uint32_t j = lane; j <= nc; j += WAVE) lo_b[j] = fchunk[c0 + j];
@@ -172,9 +177,21 @@ struct WaveLds {
   uint32_t cand[MAX_CAND];
   uint32_t pre[WAVE + 1];
   uint32_t base[WAVE];
-  unsigned long long hit[WAVE];
-  uint32_t lim[WAVE];
+  uint32_t hit[WAVE];
 };
+
+// One step over the next entries of T flattened ones: UNROLL in flight per
+// lane, or one where that takes them all (pieces are short: most steps do).
+// The number of entries it covers.
+template <typename Step>
+__device__ __forceinline__ uint32_t step_entries(uint32_t T, Step step) {
+  if (T <= WAVE) {
+    step(std::integral_constant<int, 1>());
+    return WAVE;
+  }
+  step(std::integral_constant<int, UNROLL>());
+  return UNROLL * WAVE;
+}
 
 // Which candidates meet their op's neighbours.  list null: every (op, range)
 // pair is an item (nops * chunks of them, the ops whose need flag is clear
@@ -191,12 +208,12 @@ struct WaveLds {
 // all supersteps of 245 queries on the 1M Chung-Lu graph 9.9 ms, 12.3 ms with
 // their fills launched apart.
 template <bool PUSH>
-__global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __restrict__ row,
+__global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __restrict__ row, Pieces pieces,
                                                           const uint32_t* __restrict__ col,
                                                           const uint32_t* __restrict__ ckey, uint32_t W,
                                                           const uint32_t* __restrict__ fchunk,
                                                           const uint2* __restrict__ list,
-                                                          const uint32_t* __restrict__ nlist, uint32_t chunks,
+                                                          const uint32_t* __restrict__ nlist, uint32_t max_ranges,
                                                           uint32_t nops, const FilterOp* __restrict__ ops,
                                                           const uint32_t* __restrict__ nbr_slot,
                                                           const uint32_t* __restrict__ nbr_lo,
@@ -208,7 +225,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
   extern __shared__ unsigned char lds_raw[];
   WaveLds& L = reinterpret_cast<WaveLds*>(lds_raw)[threadIdx.x / WAVE];
   const uint32_t lane = lane_id();
-  const uint32_t items = list ? uniform(*nlist) : nops * chunks;
+  const uint32_t items = list ? uniform(*nlist) : nops * max_ranges;
   const uint32_t wave = uniform((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
   const uint32_t nwaves = (gridDim.x * blockDim.x) / WAVE;
   // per-lane tallies for the optional byte accounting, over all items
@@ -225,8 +242,10 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
       o = uniform(item.x);
       c = uniform(item.y);
     } else {
-      o = it / chunks;
-      c = it % chunks;
+      o = it / max_ranges;
+      c = it % max_ranges;
+      if (c >= uniform(ops[o].nrange)) continue;
+      c += uniform(ops[o].range0);
       const uint32_t need = uniform(ops[o].need);
       if (need != ~0u && uniform(rflags[need]) == 0) continue;
     }
@@ -234,7 +253,6 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
     const uint32_t nv = uniform(ops[o].nv);
     const uint32_t nb = uniform(ops[o].nbr_off);
     uint32_t* bm_u = bitmaps + (size_t)uniform(ops[o].u_slot) * W;
-    const unsigned long long full = nv >= 64 ? ~0ULL : ((1ULL << nv) - 1);
 
     // collect: candidates of vertex range [v_lo, v_hi), ascending; lane l
     // reads bitmap word w_lo + l and keeps the range's bits of it
@@ -264,144 +282,129 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
 
     uint32_t met = 0;  // explore: candidates that meet v_0
     for (uint32_t s0 = 0; s0 < C; s0 += WAVE) {
-      // lane = one candidate of the sub-chunk
+      // lane = one candidate of the sub-chunk; the neighbours v_i one after
+      // the other, each in the candidates' pieces towards its label
       const bool mine = s0 + lane < C;
       const uint32_t id = mine ? L.cand[s0 + lane] : 0u;
-      const uint32_t off = mine ? row[id] : 0u;
-      const uint32_t deg = mine ? row[id + 1] - off : 0u;
-      L.hit[lane] = 0;
-      uint32_t cur = 0;  // entries of this candidate already examined
-      unsigned long long h = 0;
-      wave_sync();
-
-      // pass 1: constraints met by each candidate.  Every step re-flattens
-      // the remaining adjacency of the candidates not yet satisfying all of
-      // them, so a satisfied candidate stops costing lanes.
-      for (;;) {
-        const uint32_t rem = (mine && h != full) ? deg - cur : 0u;
-        const uint32_t rincl = wave_incl_scan(rem);
-        const uint32_t T = uniform(__shfl(rincl, WAVE - 1, WAVE));
-        if (T == 0) break;
-        const uint32_t rpre = rincl - rem;
-        L.pre[lane] = rpre;
-        L.base[lane] = off + cur;
+      uint32_t ff = mine ? nv : 0u;  // the first neighbour without a match
+      uint32_t off = 0, len = 0;
+      piece(pieces, id, nbr_lo[nb], off, len);
+      for (uint32_t i = 0; i < nv; ++i) {
+        const uint32_t lo = uniform(nbr_lo[nb + i]), hi = uniform(nbr_hi[nb + i]);
+        const uint32_t* bm = bitmaps + (size_t)uniform(nbr_slot[nb + i]) * W;
+        // the next neighbour's pieces load behind this one's entries
+        uint32_t noff = 0, nlen = 0;
+        if (i + 1 < nv) piece(pieces, id, nbr_lo[nb + i + 1], noff, nlen);
+        const bool alive = mine && ff == nv;
+        L.hit[lane] = 0;
+        uint32_t cur = 0;  // entries of this candidate already examined
+        bool h = !alive;
         wave_sync();
-        // refine needs the neighbour ids, explore only their keys
-        const uint32_t* __restrict__ src = type == OP_REFINE ? col : ckey;
-        uint32_t mvs[UNROLL], cis[UNROLL], es[UNROLL];
-        // an entry index past T reads entry T - 1 (in bounds) and is masked
-        // out (cis = WAVE): every lane loads, no branch per entry
-        uint32_t gi[UNROLL];
+        // every step re-flattens the remaining entries of the candidates
+        // without a match, so one that has it stops costing lanes
+        for (;;) {
+          const uint32_t rem = h ? 0u : len - cur;
+          const uint32_t rincl = wave_incl_scan(rem);
+          const uint32_t T = uniform(__shfl(rincl, WAVE - 1, WAVE));
+          if (T == 0) break;
+          const uint32_t rpre = rincl - rem;
+          L.pre[lane] = rpre;
+          L.base[lane] = off + cur;
+          wave_sync();
+          const uint32_t span = step_entries(T, [&](auto U) {
+            constexpr int N = decltype(U)::value;
+            // an entry index past T reads entry T - 1 (in bounds): the same
+            // answer again, and every lane loads, no branch per entry
+            uint32_t cis[N], gi[N], es[N];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(u * WAVE + lane, T - 1);
-        halving_search<UNROLL>(L.pre, WAVE, cis);
+            for (int u = 0; u < N; ++u) cis[u] = gi[u] = min(u * WAVE + lane, T - 1);
+            halving_search<N>(L.pre, WAVE, cis);
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) es[u] = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
+            for (int u = 0; u < N; ++u) es[u] = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
+            if (type == OP_REFINE) {
+              // refine: in C(v_i)
+              uint32_t mvs[N], wv[N];
 #pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-          mvs[u] = src[es[u]];
-          if (u * WAVE + lane >= T) cis[u] = WAVE;
+              for (int u = 0; u < N; ++u) mvs[u] = col[es[u]];
+#pragma unroll
+              for (int u = 0; u < N; ++u) wv[u] = bm[mvs[u] >> 5];
+#pragma unroll
+              for (int u = 0; u < N; ++u)
+                if ((wv[u] >> (mvs[u] & 31)) & 1u) L.hit[cis[u]] = 1;
+              t_probe += min((T + WAVE - 1 - lane) / WAVE, (uint32_t)N);
+            } else {
+              // explore: the entry's key (read in place of the column index:
+              // no extra bytes) in v_i's label/degree range
+              uint32_t ks[N];
+#pragma unroll
+              for (int u = 0; u < N; ++u) ks[u] = ckey[es[u]];
+#pragma unroll
+              for (int u = 0; u < N; ++u)
+                if (ks[u] >= lo && ks[u] <= hi) L.hit[cis[u]] = 1;
+            }
+            t_ent += min((T + WAVE - 1 - lane) / WAVE, (uint32_t)N);
+          });
+          wave_sync();
+          cur += rpre >= span ? 0u : min(rem, span - rpre);
+          h = !alive || L.hit[lane] != 0;
         }
-        // constraints each entry meets, the UNROLL entries of a lane side by
-        // side: their candidates' known bits read together, then per
-        // neighbour v_i one probe (refine) or key comparison (explore) each,
-        // the probes' loads in flight together
-        unsigned long long kn[UNROLL], bits[UNROLL];
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-          kn[u] = cis[u] != WAVE ? L.hit[cis[u]] : ~0ULL;
-          bits[u] = 0;
-        }
-        if (type == OP_REFINE) {
-          for (uint32_t i = 0; i < nv; ++i) {
-            const uint32_t* bm = bitmaps + (size_t)nbr_slot[nb + i] * W;
-            uint32_t wv[UNROLL];
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u) wv[u] = (kn[u] >> i) & 1ULL ? 0u : bm[mvs[u] >> 5];
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
-              if (!((kn[u] >> i) & 1ULL)) {
-                ++t_probe;
-                if ((wv[u] >> (mvs[u] & 31)) & 1u) bits[u] |= 1ULL << i;
-              }
-          }
-        } else {
-          // explore compares the entry's key (read in place of the column
-          // index: no extra bytes) with v_i's label/degree range
-          for (uint32_t i = 0; i < nv; ++i) {
-            const uint32_t lo = nbr_lo[nb + i], hi = nbr_hi[nb + i];
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u)
-              if (mvs[u] >= lo && mvs[u] <= hi) bits[u] |= 1ULL << i;
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < UNROLL; ++u) {
-          if (cis[u] == WAVE) continue;
-          ++t_ent;
-          if (bits[u]) atomicOr(&L.hit[cis[u]], bits[u]);
-        }
-        wave_sync();
-        // entries of this lane's candidate covered by the UNROLL*64 examined
-        const uint32_t span = UNROLL * WAVE;
-        cur += rpre >= span ? 0u : min(rem, span - rpre);
-        h = L.hit[lane];
+        if (alive && !h) ff = i;
+        off = noff;
+        len = nlen;
+        if (!__any(mine && ff == nv)) break;
       }
 
       if (type == OP_REFINE) {
-        const bool drop = mine && h != full;
+        const bool drop = mine && ff < nv;
         if (drop) clear_bit(bm_u, id);
         if (__ballot(drop) && lane == 0) rflags[uniform(ops[o].mark)] = 1u;
       } else {
         // first neighbour without a match: mu leaves C(u), its matches of the
         // neighbours before it stay
-        const uint32_t ff = h == full ? nv : (uint32_t)(__ffsll((long long)~h) - 1);
-        const bool left = !PUSH || deg > FCHUNK_ENTRIES;  // to fill_kernel
+        bool left = mine;  // to fill_kernel
+        if constexpr (PUSH) left = mine && row[id + 1] - row[id] > FCHUNK_ENTRIES;
         if (mine && ff < nv) clear_bit(bm_u, id);
-        if (mine && ff < nv && left) {
+        if (left && ff < nv) {
           uint32_t* e = bitmaps + (size_t)ops[o].e_slot * W;
           for (uint32_t i = 0; i < ff; ++i) set_bit(e + (size_t)i * W, id);  // ff < nv: e_slot has nv - 1 rows
         }
-        met += (uint32_t)__popcll(__ballot(mine && ff > 0 && left));
+        met += (uint32_t)__popcll(__ballot(left && ff > 0));
         if constexpr (PUSH) {
           // every matching neighbour of a surviving prefix enters C(v_i)
           const uint32_t lim = mine && !left ? ff : 0u;
-          const uint32_t len = lim ? deg : 0u;
-          const uint32_t lincl = wave_incl_scan(len);
-          const uint32_t T = uniform(__shfl(lincl, WAVE - 1, WAVE));
-          L.pre[lane] = lincl - len;
-          L.base[lane] = off;
-          L.lim[lane] = lim;
-          wave_sync();
-          for (uint32_t f = 0; f < T; f += UNROLL * WAVE) {
-            uint32_t mvs[UNROLL], ks[UNROLL], cis[UNROLL], es[UNROLL], gi[UNROLL], lms[UNROLL];
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(f + u * WAVE + lane, T - 1);
-            halving_search<UNROLL>(L.pre, WAVE, cis);
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u) es[u] = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
-#pragma unroll
-            for (int u = 0; u < UNROLL; ++u) {
-              mvs[u] = col[es[u]];
-              ks[u] = ckey[es[u]];
-              const bool in = f + u * WAVE + lane < T;
-              lms[u] = in ? L.lim[cis[u]] : 0u;
-              t_ent += in;
-              t_key += in;
-            }
-            // per neighbour v_i the words of the UNROLL entries are loaded
-            // together, and a bit is set (one atomic) only where still clear
-            for (uint32_t i = 0; i < nv; ++i) {  // lim <= nv
-              const uint32_t lo = nbr_lo[nb + i], hi = nbr_hi[nb + i];
-              uint32_t* bm = bitmaps + (size_t)nbr_slot[nb + i] * W;
+          for (uint32_t i = 0; i < nv && __any(i < lim); ++i) {
+            const uint32_t lo = uniform(nbr_lo[nb + i]), hi = uniform(nbr_hi[nb + i]);
+            uint32_t* bm = bitmaps + (size_t)uniform(nbr_slot[nb + i]) * W;
+            piece(pieces, id, lo, off, len);
+            if (i >= lim) len = 0;
+            const uint32_t lincl = wave_incl_scan(len);
+            const uint32_t T = uniform(__shfl(lincl, WAVE - 1, WAVE));
+            L.pre[lane] = lincl - len;
+            L.base[lane] = off;
+            wave_sync();
+            for (uint32_t f = 0; f < T; f += UNROLL * WAVE) {
+              uint32_t mvs[UNROLL], ks[UNROLL], cis[UNROLL], es[UNROLL], gi[UNROLL], cw[UNROLL];
               bool want[UNROLL];
-              uint32_t cw[UNROLL];
+#pragma unroll
+              for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(f + u * WAVE + lane, T - 1);
+              halving_search<UNROLL>(L.pre, WAVE, cis);
+#pragma unroll
+              for (int u = 0; u < UNROLL; ++u) es[u] = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
 #pragma unroll
               for (int u = 0; u < UNROLL; ++u) {
-                want[u] = i < lms[u] && ks[u] >= lo && ks[u] <= hi;
+                mvs[u] = col[es[u]];
+                ks[u] = ckey[es[u]];
+                const bool in = f + u * WAVE + lane < T;
+                want[u] = in && ks[u] >= lo && ks[u] <= hi;
+                t_ent += in;
+                t_key += in;
+              }
+              // the words of the UNROLL entries are loaded together, and a bit
+              // is set (one atomic) only where still clear
+#pragma unroll
+              for (int u = 0; u < UNROLL; ++u)
                 cw[u] = want[u] ? __hip_atomic_load(bm + (mvs[u] >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
                                 : ~0u;
-              }
 #pragma unroll
               for (int u = 0; u < UNROLL; ++u)
                 if (want[u]) {
@@ -410,6 +413,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
                   if (!(cw[u] & m)) atomicOr(bm + (mvs[u] >> 5), m);
                 }
             }
+            wave_sync();
           }
         }
       }
@@ -458,10 +462,11 @@ struct FillLds {
   uint32_t word[WAVE];
 };
 
-__global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ row, const uint32_t* __restrict__ col,
+__global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ row, Pieces pieces,
+                                                   const uint32_t* __restrict__ col,
                                                    const uint32_t* __restrict__ key,
                                                    const uint32_t* __restrict__ ckey, uint32_t W,
-                                                   const uint32_t* __restrict__ fchunk, uint32_t chunks,
+                                                   const uint32_t* __restrict__ fchunk, uint32_t max_ranges,
                                                    const uint2* __restrict__ hparts, uint32_t nhp,
                                                    const FillOp* __restrict__ fills, uint32_t nfill,
                                                    const uint32_t* __restrict__ counts, bool hubs_only,
@@ -471,20 +476,21 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
   const uint32_t lane = lane_id();
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
   const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  const uint64_t pairs = hubs_only ? 0 : (uint64_t)nfill * chunks, items = pairs + (uint64_t)nfill * nhp;
+  const uint64_t pairs = hubs_only ? 0 : (uint64_t)nfill * max_ranges, items = pairs + (uint64_t)nfill * nhp;
   uint32_t t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
   for (uint64_t it = wave; it < items; it += nwaves) {
     const bool part = it >= pairs;
     const uint64_t x = part ? it - pairs : it;
-    const uint32_t per = part ? nhp : chunks;
-    const uint32_t f = uniform((uint32_t)(x / per)), c = uniform((uint32_t)(x % per));
+    const uint32_t per = part ? nhp : max_ranges;
+    const uint32_t f = uniform((uint32_t)(x / per));
+    uint32_t c = uniform((uint32_t)(x % per));
     const FillOp& op = fills[f];
     const uint32_t lo = uniform(op.lo), hi = uniform(op.hi), met = uniform(counts[op.cnt]);
     if (met == 0) continue;
     const bool pull = !hubs_only && (uint64_t)met * FILL_PULL >= uniform(op.nlabel);
     if (part && pull) continue;
     const uint32_t* bm_u = bitmaps + (size_t)uniform(op.u_slot) * W;
-    const uint32_t e_slot = uniform(op.e_slot);
+    const uint32_t e_slot = uniform(op.e_slot), u_lo = uniform(op.u_lo);
     const uint32_t* bm_e = e_slot != ~0u ? bitmaps + (size_t)e_slot * W : nullptr;
     uint32_t* bm_v = bitmaps + (size_t)uniform(op.v_slot) * W;
     uint32_t v_lo, v_hi, first = 0;  // first: where a part's entries start
@@ -494,6 +500,8 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
       v_hi = v_lo + 1;
       first = uniform(hp.y) * HUB_PART;
     } else {
+      if (c >= uniform(op.nrange[pull])) continue;
+      c += uniform(op.range0[pull]);
       v_lo = uniform(fchunk[c]);
       v_hi = uniform(fchunk[c + 1]);
     }
@@ -527,10 +535,13 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
     for (uint32_t s0 = 0; s0 < C; s0 += WAVE) {
       const bool mine = s0 + lane < C;
       const uint32_t id = mine ? L.cand[s0 + lane] : 0u;
-      const uint32_t off = mine ? row[id] + first : 0u;
-      uint32_t len = mine ? row[id + 1] - off : 0u;
-      if (part) len = min(len, HUB_PART);
-      else if (!pull && len > FCHUNK_ENTRIES) len = 0;  // pushed by its parts
+      uint32_t off = 0, len = 0;
+      if (mine) {
+        piece(pieces, id, pull ? u_lo : lo, off, len);
+        off += first;
+        if (part) len = len > first ? min(len - first, HUB_PART) : 0u;
+        else if (!pull && row[id + 1] - row[id] > FCHUNK_ENTRIES) len = 0;  // pushed by its parts
+      }
       if (pull) {
         L.hit[lane] = 0;
         uint32_t cur = 0;
@@ -635,15 +646,16 @@ void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* 
 
 void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, const uint32_t* nbr_slot,
                         const uint32_t* nbr_lo, const uint32_t* nbr_hi, const FillOp* fills, uint32_t nfill,
-                        uint32_t* bitmaps, uint32_t block, uint32_t resident, uint2* items, uint32_t* nitems,
-                        uint32_t* rflags, uint32_t* counts, unsigned long long* stats, hipStream_t s) {
+                        uint32_t* bitmaps, uint32_t max_ranges, uint32_t block, uint32_t resident, uint2* items,
+                        uint32_t* nitems, uint32_t* rflags, uint32_t* counts, unsigned long long* stats,
+                        hipStream_t s) {
   if (!nops) return;
-  const uint64_t pairs = (uint64_t)nops * g.nfchunk;
+  const uint64_t pairs = (uint64_t)nops * max_ranges;
   const bool direct = pairs <= FILTER_DIRECT;
   if (!direct) {
-    const uint32_t wgs_per_op = ((g.nfchunk + AR_GROUP - 1) / AR_GROUP + 3) / 4;
+    const uint32_t wgs_per_op = ((max_ranges + AR_GROUP - 1) / AR_GROUP + 3) / 4;
     // four waves per workgroup: the kernel's LDS and its per-workgroup append assume 256 threads
-    hipLaunchKernelGGL(active_ranges_kernel, dim3(nops * wgs_per_op), dim3(256), 0, s, g.fchunk, g.wrange, g.nfchunk,
+    hipLaunchKernelGGL(active_ranges_kernel, dim3(nops * wgs_per_op), dim3(256), 0, s, g.fchunk, g.wrange, max_ranges,
                        ops, nops, bitmaps, g.W, rflags, items, nitems);
   }
   // the list's length is known on the device only: a grid of at most
@@ -658,13 +670,13 @@ void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, c
   const uint32_t wpb = block / WAVE;
   const uint64_t most = (uint64_t)resident * FILTER_OVERSUB;
   hipLaunchKernelGGL(direct ? filter_step_kernel<false> : filter_step_kernel<true>, dim3((uint32_t)std::min((pairs + wpb - 1) / wpb, most)), dim3(block),
-                     sizeof(WaveLds) * wpb, s, g.row, g.col, g.ckey, g.W, g.fchunk, direct ? nullptr : items, nitems,
-                     g.nfchunk, nops, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, counts, stats);
-  const uint64_t fwaves = (uint64_t)nfill * ((direct ? (uint64_t)g.nfchunk : 0) + g.nhparts);
+                     sizeof(WaveLds) * wpb, s, g.row, pieces_of(g), g.col, g.ckey, g.W, g.fchunk,
+                     direct ? nullptr : items, nitems, max_ranges, nops, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, counts, stats);
+  const uint64_t fwaves = (uint64_t)nfill * ((direct ? (uint64_t)max_ranges : 0) + g.nhparts);
   if (!fwaves) return;
   hipLaunchKernelGGL(fill_kernel, dim3((uint32_t)std::min((fwaves + wpb - 1) / wpb, most)), dim3(block),
-                     sizeof(FillLds) * wpb, s, g.row, g.col, g.key, g.ckey, g.W, g.fchunk, g.nfchunk, g.hparts,
-                     g.nhparts, fills, nfill, counts, !direct, bitmaps, stats);
+                     sizeof(FillLds) * wpb, s, g.row, pieces_of(g), g.col, g.key, g.ckey, g.W, g.fchunk, max_ranges,
+                     g.hparts, g.nhparts, fills, nfill, counts, !direct, bitmaps, stats);
 }
 
 uint32_t filter_resident(uint32_t block) {

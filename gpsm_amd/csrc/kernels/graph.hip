@@ -16,24 +16,22 @@ namespace gpsm {
 
 namespace {
 
-// One wave per (hub, 64-entry block of its adjacency): grid-stride over the
-// blocks of all hubs, found with a binary search over their prefix sums.
-__global__ void __launch_bounds__(256) hub_bits_kernel(const uint32_t* __restrict__ row,
+// One wave per 64 pieces, flattened over their entries; a hub's entry sets its
+// neighbour's bit.
+__global__ void __launch_bounds__(256) hub_bits_kernel(const uint32_t* __restrict__ lrow, uint64_t npieces, uint32_t n,
                                                        const uint32_t* __restrict__ col,
-                                                       const uint32_t* __restrict__ hubs,
-                                                       const uint32_t* __restrict__ block_base, uint32_t nhub,
-                                                       uint32_t W, uint32_t* __restrict__ bits) {
+                                                       const uint32_t* __restrict__ hub_of, uint32_t W,
+                                                       uint32_t* __restrict__ bits) {
   const uint32_t lane = lane_id();
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
   const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  const uint32_t nblocks = block_base[nhub];
-  for (uint64_t it = wave; it < nblocks; it += nwaves) {
-    const uint32_t h = uniform(seg_search(block_base, nhub + 1, (uint32_t)it));
-    const uint32_t v = hubs[h];
-    const uint32_t e = row[v] + ((uint32_t)it - block_base[h]) * WAVE + lane;
-    if (e < row[v + 1]) {
+  for (uint64_t p0 = wave * WAVE; p0 < npieces; p0 += nwaves * WAVE) {
+    const uint32_t np = (uint32_t)min((uint64_t)WAVE, npieces - p0);
+    const uint32_t e1 = lrow[p0 + np];
+    for (uint32_t e = lrow[p0] + lane; e < e1; e += WAVE) {
+      const uint32_t h = hub_of[(uint32_t)((p0 + seg_search(lrow + p0, np, e)) % n)];
       const uint32_t w = col[e];
-      atomicOr(bits + (size_t)h * W + (w >> 5), 1u << (w & 31));
+      if (h != ~0u) atomicOr(bits + (size_t)h * W + (w >> 5), 1u << (w & 31));
     }
   }
 }
@@ -89,13 +87,123 @@ __global__ void check_rows_kernel(const uint32_t* __restrict__ row, const uint32
   if (wrong) atomicOr(bad, 1u);
 }
 
-// key[v] = (dense label << KEY_DEG_BITS) | min(degree, KEY_DEG_MASK): the
-// dense label is 1 + the label's place among the nl distinct ones.
-__global__ void vertex_keys_kernel(const uint32_t* __restrict__ row, const uint32_t* __restrict__ label, uint32_t n,
-                                   const uint32_t* __restrict__ value, uint32_t nl, uint32_t* __restrict__ key) {
+// place[v] = (place of id v's label among the nl distinct ones) << 32 | v, to
+// be sorted by label.
+__global__ void label_places_kernel(const uint32_t* __restrict__ label, uint32_t n, const uint32_t* __restrict__ value,
+                                    uint32_t nl, unsigned long long* __restrict__ place) {
   const uint32_t stride = gridDim.x * blockDim.x;
   for (uint64_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride)
-    key[v] = ((seg_search(value, nl, label[v]) + 1) << KEY_DEG_BITS) | min(row[v + 1] - row[v], KEY_DEG_MASK);
+    place[v] = ((unsigned long long)seg_search(value, nl, label[v]) << 32) | v;
+}
+
+// ids, pos and key of the sorted places; deg[i]: vertex i's degree, deg[n] = 0.
+// key[i] = (dense label << KEY_DEG_BITS) | min(degree, KEY_DEG_MASK): the dense
+// label is 1 + the label's place.
+__global__ void numbering_kernel(const unsigned long long* __restrict__ place, const uint32_t* __restrict__ row0,
+                                 uint32_t n, uint32_t* __restrict__ ids, uint32_t* __restrict__ pos,
+                                 uint32_t* __restrict__ key, uint32_t* __restrict__ deg) {
+  const uint32_t stride = gridDim.x * blockDim.x;
+  for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const unsigned long long p = place[i];
+    const uint32_t v = (uint32_t)p, d = row0[v + 1] - row0[v];
+    ids[i] = v;
+    pos[v] = (uint32_t)i;
+    key[i] = (((uint32_t)(p >> 32) + 1) << KEY_DEG_BITS) | min(d, KEY_DEG_MASK);
+    deg[i] = d;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) deg[n] = 0;
+}
+
+// The entries of vertex 0, 1, ... as (label group, vertex, label, neighbour)
+// keys: the vertex and the neighbour in pb bits, the label in lb (0: left
+// out).  One wave per 64 vertices, flattened over their entries.
+__global__ void row_entries_kernel(const uint32_t* __restrict__ row0, const uint32_t* __restrict__ col0,
+                                   const uint32_t* __restrict__ ids, const uint32_t* __restrict__ pos,
+                                   const uint32_t* __restrict__ key, const uint32_t* __restrict__ row, uint32_t n,
+                                   uint32_t pb, uint32_t lb, uint32_t gshift,
+                                   unsigned long long* __restrict__ entry) {
+  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / WAVE;
+  const uint32_t lane = lane_id();
+  for (uint64_t v0 = wave * WAVE; v0 < n; v0 += nwaves * WAVE) {
+    const uint32_t nv = (uint32_t)min((uint64_t)WAVE, n - v0);
+    const uint32_t e1 = row[v0 + nv];
+    for (uint32_t e = row[v0] + lane; e < e1; e += WAVE) {
+      const uint32_t i = seg_search(row + v0, nv, e);
+      const uint32_t x = pos[col0[row0[ids[v0 + i]] + (e - row[v0 + i])]];
+      const uint32_t l = (key[x] >> KEY_DEG_BITS) - 1;
+      unsigned long long k = ((unsigned long long)(l >> gshift) << pb) | (v0 + i);
+      if (lb) k = (k << lb) | l;
+      entry[e] = (k << pb) | x;
+    }
+  }
+}
+
+// lrow[p] for the pieces p = 256 b .. 256 b + 255 of a workgroup, and the end:
+// entries before the piece, searched between the workgroup's first and last.
+__global__ void __launch_bounds__(256) pieces_kernel(const unsigned long long* __restrict__ entry, uint32_t adj,
+                                                     uint32_t n, uint64_t npieces, uint32_t pb, uint32_t lb,
+                                                     uint32_t* __restrict__ lrow) {
+  __shared__ uint32_t bound[2];
+  // the key of piece p's first possible entry
+  auto first_key = [&](uint64_t p) { return (((p / n) << pb) | (p % n)) << (lb + pb); };
+  auto before = [&](unsigned long long k, uint32_t lo, uint32_t hi) {
+    while (lo < hi) {
+      const uint32_t mid = lo + ((hi - lo) >> 1);
+      if (entry[mid] < k) lo = mid + 1;
+      else hi = mid;
+    }
+    return lo;
+  };
+  for (uint64_t p0 = (uint64_t)blockIdx.x * 256; p0 <= npieces; p0 += (uint64_t)gridDim.x * 256) {
+    if (threadIdx.x < 2) {
+      const uint64_t p = p0 + 256 * threadIdx.x;
+      bound[threadIdx.x] = p >= npieces ? adj : before(first_key(p), 0, adj);
+    }
+    __syncthreads();
+    const uint64_t p = p0 + threadIdx.x;
+    if (p <= npieces) lrow[p] = p == npieces ? adj : before(first_key(p), bound[0], bound[1]);
+    __syncthreads();
+  }
+}
+
+__global__ void entry_columns_kernel(const unsigned long long* __restrict__ entry, uint64_t adj, uint32_t pb,
+                                     uint32_t* __restrict__ col) {
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < adj; e += stride)
+    col[e] = (uint32_t)(entry[e] & ((1ull << pb) - 1));
+}
+
+__global__ void label_ranges_kernel(const uint32_t* __restrict__ fchunk, uint32_t nfchunk,
+                                    const uint32_t* __restrict__ start, uint32_t nl, uint32_t* __restrict__ range) {
+  const uint32_t l = blockIdx.x * blockDim.x + threadIdx.x;
+  if (l >= nl) return;
+  range[2 * l] = seg_search(fchunk, nfchunk + 1, start[l]);
+  range[2 * l + 1] = seg_search(fchunk, nfchunk + 1, start[l + 1] - 1) + 1;
+}
+
+// Two words of every row's bitmap by id per wave: lane l gathers the bit of
+// id 64 p + l, one ballot makes the words.  Within a label the ids are in the
+// vertices' order, so a row's bits, all of one label, are read almost in order.
+__global__ void id_bitmaps_kernel(const uint32_t* __restrict__ pos, const uint32_t* __restrict__ bitmaps, uint32_t n,
+                                  uint32_t W, uint32_t nrows, uint32_t* __restrict__ out) {
+  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / WAVE;
+  const uint32_t lane = lane_id();
+  for (uint64_t p = wave; p < ((uint64_t)n + WAVE - 1) / WAVE; p += nwaves) {
+    const uint64_t id = p * WAVE + lane;
+    const uint32_t v = id < n ? pos[id] : 0u;
+    for (uint32_t r = 0; r < nrows; ++r) {
+      const bool set = id < n && bit_of(bitmaps + (size_t)r * W, v);
+      const unsigned long long m = __ballot(set);
+      if (lane < 2 && 2 * p + lane < W) out[(size_t)r * W + 2 * p + lane] = (uint32_t)(m >> (32 * lane));
+    }
+  }
+}
+
+__global__ void to_ids_kernel(const uint32_t* __restrict__ ids, uint32_t* __restrict__ v, uint64_t n) {
+  const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) v[i] = ids[v[i]];
 }
 
 // The filter's vertex ranges: each block of FCHUNK_VERTS vertices is cut
@@ -164,23 +272,12 @@ __global__ void hub_flags_kernel(const uint32_t* __restrict__ row, uint32_t n, u
     flag[v] = row[v + 1] - row[v] > degree;
 }
 
-// hub_of[v] = pos[v] for hubs (pos: hubs before v), ~0 for others; the hubs and
-// their 64-entry adjacency blocks (one more entry, 0, for a scan's total).
-__global__ void hub_list_kernel(const uint32_t* __restrict__ row, uint32_t n, uint32_t degree, uint32_t nhub,
-                                const uint32_t* __restrict__ pos, uint32_t* __restrict__ hub_of,
-                                uint32_t* __restrict__ hubs, uint32_t* __restrict__ blocks) {
+// hub_of[v] = before[v] (hubs before v) for hubs, ~0 for others.
+__global__ void hub_list_kernel(const uint32_t* __restrict__ row, uint32_t n, uint32_t degree,
+                                const uint32_t* __restrict__ before, uint32_t* __restrict__ hub_of) {
   const uint32_t stride = gridDim.x * blockDim.x;
-  for (uint64_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
-    const uint32_t deg = row[v + 1] - row[v];
-    if (deg > degree) {
-      hub_of[v] = pos[v];
-      hubs[pos[v]] = (uint32_t)v;
-      blocks[pos[v]] = (deg + WAVE - 1) / WAVE;
-    } else {
-      hub_of[v] = ~0u;
-    }
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) blocks[nhub] = 0;
+  for (uint64_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride)
+    hub_of[v] = row[v + 1] - row[v] > degree ? before[v] : ~0u;
 }
 
 __global__ void neighbour_keys_kernel(const uint32_t* __restrict__ col, const uint32_t* __restrict__ key,
@@ -192,6 +289,9 @@ __global__ void neighbour_keys_kernel(const uint32_t* __restrict__ col, const ui
 uint32_t grid_for(uint64_t items) {
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((items + 255) / 256, 16384));
 }
+
+// Bits of x.
+uint32_t bits_of(uint32_t x) { return x ? 32 - (uint32_t)__builtin_clz(x) : 0; }
 
 uint32_t range_blocks(uint32_t n) { return (uint32_t)(((uint64_t)n + FCHUNK_VERTS - 1) / FCHUNK_VERTS); }
 
@@ -207,8 +307,80 @@ void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uin
   hipLaunchKernelGGL(check_rows_kernel, dim3(grid_for(n)), dim3(256), 0, s, row, col, n, bad);
 }
 
-void launch_vertex_keys(const DevGraph& g, const uint32_t* label, const uint32_t* value, uint32_t nl, hipStream_t s) {
-  hipLaunchKernelGGL(vertex_keys_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.row, label, g.n, value, nl, g.key);
+uint64_t relabel_words(uint32_t n, uint64_t adj) {
+  const uint64_t m = std::max<uint64_t>(n, adj);
+  return 4 * m + 2 * radix_hist_words(m) + scan_scratch_words(std::max(radix_hist_words(m), (uint64_t)n + 1)) +
+         (((uint64_t)n + 2) & ~1ull);
+}
+
+void launch_relabel(const DevGraph& g, const uint32_t* label, const uint32_t* value, uint32_t nl, uint32_t* scratch,
+                    hipStream_t s) {
+  // row == row0: the vertices keep their ids, only the keys are made
+  const bool sorted = g.row != g.row0;
+  const uint64_t m = sorted ? std::max<uint64_t>(g.n, g.adj) : g.n, hw = radix_hist_words(m);
+  unsigned long long* a = reinterpret_cast<unsigned long long*>(scratch);
+  unsigned long long* b = a + m;
+  uint32_t* hist = reinterpret_cast<uint32_t*>(b + m);  // hw is even
+  uint32_t* hstart = hist + hw;
+  uint32_t* deg = hstart + hw;
+  uint32_t* scan = deg + (((uint64_t)g.n + 2) & ~1ull);
+  const uint64_t sw = scan_scratch_words(std::max(hw, (uint64_t)g.n + 1));
+  hipLaunchKernelGGL(label_places_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, label, g.n, value, nl, a);
+  for (uint32_t shift = 32; sorted && (uint64_t)(nl - 1) >> (shift - 32); shift += 8) {
+    launch_radix_pass(a, b, nullptr, nullptr, g.n, shift, hist, hstart, scan, sw, s);
+    std::swap(a, b);
+  }
+  hipLaunchKernelGGL(numbering_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, a, g.row0, g.n, g.ids, g.pos, g.key, deg);
+  if (!sorted) return;
+  launch_exclusive_scan(deg, g.row, (uint64_t)g.n + 1, nullptr, scan, sw, s);
+  if (!g.adj) {
+    if (g.ngroup > 1) launch_fill_u32(g.lrow, 0u, (uint64_t)g.n * g.ngroup + 1, s);
+    return;
+  }
+  // A vertex's entries come in the ids' order, in which those of one label
+  // ascend: where every label is a group of its own, a stable sort by the group
+  // is all (one pass for 256 labels).  Else by (group, vertex, label), or by
+  // the whole key where the label's bits do not fit.
+  const uint32_t pb = bits_of(g.n - 1), gb = bits_of(g.ngroup - 1);
+  const bool exact = g.gshift == 0;
+  uint32_t lb = exact ? 0 : bits_of(nl - 1);
+  if (gb + 2 * pb + lb > 64) lb = 0;
+  hipLaunchKernelGGL(row_entries_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.row0, g.col0, g.ids, g.pos, g.key,
+                     g.row, g.n, pb, lb, g.gshift, a);
+  for (uint32_t shift = exact ? 2 * pb : lb ? pb : 0; shift < gb + 2 * pb + lb; shift += 8) {
+    launch_radix_pass(a, b, nullptr, nullptr, g.adj, shift, hist, hstart, scan, sw, s);
+    std::swap(a, b);
+  }
+  if (g.ngroup > 1) {
+    const uint64_t np = (uint64_t)g.n * g.ngroup;
+    hipLaunchKernelGGL(pieces_kernel, dim3(grid_for(np + 1)), dim3(256), 0, s, a, (uint32_t)g.adj, g.n, np, pb, lb,
+                       g.lrow);
+  }
+  hipLaunchKernelGGL(entry_columns_kernel, dim3(grid_for(g.adj)), dim3(256), 0, s, a, g.adj, pb, g.col);
+}
+
+void choose_pieces(DevGraph& g, uint32_t nl) {
+  g.gshift = 0;
+  for (;; ++g.gshift) {
+    g.ngroup = ((nl - 1) >> g.gshift) + 1;
+    if (g.ngroup == 1 || (g.ngroup <= PIECE_GROUPS && (uint64_t)g.ngroup * g.n <= 4 * g.adj + g.n &&
+                          bits_of(g.ngroup - 1) + 2 * bits_of(g.n - 1) <= 64))
+      return;
+  }
+}
+
+void launch_label_ranges(const DevGraph& g, const uint32_t* start, uint32_t nl, uint32_t* range, hipStream_t s) {
+  hipLaunchKernelGGL(label_ranges_kernel, dim3((nl + 255) / 256), dim3(256), 0, s, g.fchunk, g.nfchunk, start, nl,
+                     range);
+}
+
+void launch_id_bitmaps(const DevGraph& g, const uint32_t* bitmaps, uint32_t nrows, uint32_t* out, hipStream_t s) {
+  hipLaunchKernelGGL(id_bitmaps_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.pos, bitmaps, g.n, g.W, nrows, out);
+}
+
+void launch_to_ids(const DevGraph& g, uint32_t* v, uint64_t n, hipStream_t s) {
+  if (!n) return;
+  hipLaunchKernelGGL(to_ids_kernel, dim3(grid_for(n)), dim3(256), 0, s, g.ids, v, n);
 }
 
 uint64_t range_words(uint32_t n) {
@@ -232,26 +404,19 @@ void launch_ranges(const DevGraph& g, const uint32_t* scratch, uint32_t* next, h
                      g.row, g.n, g.fchunk, g.wrange, g.hparts, next);
 }
 
-uint64_t hub_words(uint32_t n, uint64_t nhub) {
-  return 2 * (((uint64_t)n + 1) & ~1ull) + 3 * ((nhub + 2) & ~1ull) +
-         scan_scratch_words(std::max<uint64_t>(n, nhub + 1));
-}
+uint64_t hub_words(uint32_t n) { return 2 * (((uint64_t)n + 1) & ~1ull) + scan_scratch_words(n); }
 
 void launch_hubs(const DevGraph& g, uint32_t* scratch, hipStream_t s) {
-  const uint64_t nv = ((uint64_t)g.n + 1) & ~1ull, nh = ((uint64_t)g.nhub + 2) & ~1ull;
+  const uint64_t nv = ((uint64_t)g.n + 1) & ~1ull;
   uint32_t* flag = scratch;
-  uint32_t* pos = flag + nv;
-  uint32_t* hubs = pos + nv;
-  uint32_t* blocks = hubs + nh;
-  uint32_t* base = blocks + nh;
-  uint32_t* scan = base + nh;
-  const uint64_t sw = scan_scratch_words(std::max<uint64_t>(g.n, (uint64_t)g.nhub + 1));
+  uint32_t* before = flag + nv;
   hipLaunchKernelGGL(hub_flags_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.row, g.n, g.hub_degree, flag);
-  launch_exclusive_scan(flag, pos, g.n, nullptr, scan, sw, s);
-  hipLaunchKernelGGL(hub_list_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.row, g.n, g.hub_degree, g.nhub, pos,
-                     g.hub_of, hubs, blocks);
-  launch_exclusive_scan(blocks, base, (uint64_t)g.nhub + 1, nullptr, scan, sw, s);
-  launch_hub_bits(g, hubs, base, (uint32_t)std::min<uint64_t>(g.adj / WAVE + g.nhub, 0xFFFFFFFFull), s);
+  launch_exclusive_scan(flag, before, g.n, nullptr, before + nv, scan_scratch_words(g.n), s);
+  hipLaunchKernelGGL(hub_list_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.row, g.n, g.hub_degree, before,
+                     g.hub_of);
+  const uint64_t np = (uint64_t)g.n * g.ngroup;
+  hipLaunchKernelGGL(hub_bits_kernel, dim3(grid_for(np)), dim3(256), 0, s, g.lrow, np, g.n, g.col, g.hub_of, g.W,
+                     g.hub_bits);
 }
 
 void launch_neighbour_keys(const DevGraph& g, hipStream_t s) {
@@ -259,16 +424,6 @@ void launch_neighbour_keys(const DevGraph& g, hipStream_t s) {
   uint64_t grid = (g.adj + 255) / 256;
   if (grid > 16384) grid = 16384;
   hipLaunchKernelGGL(neighbour_keys_kernel, dim3((uint32_t)grid), dim3(256), 0, s, g.col, g.key, g.adj, g.ckey);
-}
-
-void launch_hub_bits(const DevGraph& g, const uint32_t* hubs, const uint32_t* block_base, uint32_t nblocks,
-                     hipStream_t s) {
-  if (!g.nhub || !nblocks) return;
-  const uint32_t block = 256;
-  uint64_t grid = ((uint64_t)nblocks * WAVE + block - 1) / block;
-  if (grid > 65536) grid = 65536;
-  hipLaunchKernelGGL(hub_bits_kernel, dim3((uint32_t)grid), dim3(block), 0, s, g.row, g.col, hubs, block_base,
-                     g.nhub, g.W, g.hub_bits);
 }
 
 }  // namespace gpsm

@@ -66,7 +66,7 @@ static_assert((uint64_t)WROWS * LONG_ROW < (1u << 23) && WROWS < 512, "packed sc
 template <bool BYTES, int U>
 __device__ __forceinline__ void back_edges_of_row(const JoinArgs& a, const JoinPlan& P,
                                                   const uint32_t* __restrict__ val, uint32_t bo, uint32_t be,
-                                                  uint32_t i, const uint32_t (&mvs)[U],
+                                                  uint32_t w_lo, uint32_t i, const uint32_t (&mvs)[U],
                                                   bool (&oks)[U], unsigned long long& bytes) {
   for (uint32_t b = bo; b < be; ++b) {
     const uint32_t bv = uniform(val[P.backs[b] * WROWS + i]);
@@ -84,7 +84,7 @@ __device__ __forceinline__ void back_edges_of_row(const JoinArgs& a, const JoinP
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u)
-        if (oks[u]) oks[u] = has_edge<BYTES>(a.row, a.col, a.hub_of, a.hub_bits, a.W, mvs[u], bv, bytes);
+        if (oks[u]) oks[u] = has_edge<BYTES>(a.pieces, a.col, a.hub_of, a.hub_bits, a.W, mvs[u], w_lo, bv, bytes);
     }
   }
 }
@@ -154,13 +154,13 @@ __device__ __forceinline__ CetAgg agg_of(const JoinArgs& a, const CetDesc& d, ui
   return a.aggs[d.agg_base + rank_of(a.bitmaps + (size_t)d.x_slot * a.W, a.bprefix + (size_t)d.x_slot * a.NB, x)];
 }
 
-// Whether u is in the candidate-edge list of mu in a table whose bound
-// vertex has candidate set `slot`: u in C(slot) and {mu, u} an edge.
+// Whether u is in the candidate-edge list of mu in table d: u in C(w) and
+// {mu, u} an edge.
 template <bool BYTES>
-__device__ __forceinline__ bool in_list(const JoinArgs& a, uint32_t slot, uint32_t mu, uint32_t u,
+__device__ __forceinline__ bool in_list(const JoinArgs& a, const CetDesc& d, uint32_t mu, uint32_t u,
                                         unsigned long long& bytes) {
-  if (!bit_of(a.bitmaps + (size_t)slot * a.W, u)) return false;
-  return has_edge<BYTES>(a.row, a.col, a.hub_of, a.hub_bits, a.W, mu, u, bytes);
+  if (!bit_of(a.bitmaps + (size_t)d.w_slot * a.W, u)) return false;
+  return has_edge<BYTES>(a.pieces, a.col, a.hub_of, a.hub_bits, a.W, u, d.w_lo, mu, bytes);
 }
 
 // The embeddings of a window of rows that bind all but the last vertex w
@@ -183,9 +183,9 @@ __device__ __forceinline__ void count_last_level(const JoinArgs& a, const JoinPl
   unsigned long long len = r.len, s = r.s;
   for (uint64_t m = P.inj[w]; m; m &= m - 1) {
     const uint32_t u = val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + tid];
-    if (in_list<BYTES>(a, d.w_slot, mu, u, bytes)) {
+    if (in_list<BYTES>(a, d, mu, u, bytes)) {
       --len;
-      s -= tuple_term(qid, u);
+      s -= tuple_term(qid, a.ids[u]);
     }
   }
   my_cnt += len;
@@ -228,8 +228,8 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
     unsigned long long n = r.len, ty = r.s, ra = r.a, rb = r.b;
     for (uint64_t m = iy; m; m &= m - 1) {
       const uint32_t u = val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + tid];
-      if (!in_list<BYTES>(a, dy.w_slot, mu, u, bytes)) continue;
-      const unsigned long long t = tuple_term(qy, u);
+      if (!in_list<BYTES>(a, dy, mu, u, bytes)) continue;
+      const unsigned long long t = tuple_term(qy, a.ids[u]);
       --n;
       ty -= t;
       if (chain) {
@@ -239,7 +239,7 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
         rb -= t * x.s;
       } else if (sibling && bit_of(bm_w, u)) {
         --ra;
-        rb -= t * tuple_term(qw, u);
+        rb -= t * tuple_term(qw, a.ids[u]);
       }
     }
     unsigned long long cnt, hash;
@@ -249,7 +249,7 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
       hash = rb;
       if (((iw >> py) & 1) && bit_of(bm_w, mu)) {  // y's parent is in every list
         cnt -= n;
-        hash -= tuple_term(qw, mu) * ty;
+        hash -= tuple_term(qw, a.ids[mu]) * ty;
       }
     } else {
       const uint32_t mw = val[pw * WROWS + tid];
@@ -259,9 +259,9 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
       unsigned long long lw = x.len, sw = x.s;
       for (uint64_t m = iw & ~(1ull << y); m; m &= m - 1) {
         const uint32_t u = val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + tid];
-        if (in_list<BYTES>(a, dw.w_slot, mw, u, bytes)) {
+        if (in_list<BYTES>(a, dw, mw, u, bytes)) {
           --lw;
-          sw -= tuple_term(qw, u);
+          sw -= tuple_term(qw, a.ids[u]);
         }
       }
       cnt = n * lw;
@@ -289,7 +289,8 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
         // the cheaper side: L_y against o's hub bitmap or adjacency, or o's
         // adjacency against C(y) and the edge to y's parent (a bit test about
         // 2, a binary search about 8 list reads)
-        const uint32_t o0 = a.row[o], od = a.row[o + 1] - o0;
+        uint32_t o0, od;
+        piece(a.pieces, o, dy.w_lo, o0, od);
         const uint64_t c0 = (uint64_t)len_y * (a.hub_of[o] != ~0u ? 2 : 8);
         const uint64_t c1 = (uint64_t)od * (a.hub_of[mu] != ~0u ? 2 : 8);
         side = c1 < c0;
@@ -330,11 +331,11 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
         if (ok) {
           const bool sd = S.lrow[i] != 0;
           if (sd) ok = bit_of(a.bitmaps + (size_t)dy.w_slot * a.W, v[u]);
-          if (ok) ok = has_edge<BYTES>(a.row, a.col, a.hub_of, a.hub_bits, a.W, v[u], sd ? S.lub[i] : S.lst[i], bytes);
+          if (ok) ok = has_edge<BYTES>(a.pieces, a.col, a.hub_of, a.hub_bits, a.W, v[u], dy.w_lo, sd ? S.lub[i] : S.lst[i], bytes);
         }
         if (ok) {
           --my_cnt;
-          my_hash -= S.srow[i] * tuple_term(qy, v[u]) * tuple_term(qw, chain ? S.lst[i] : v[u]);
+          my_hash -= S.srow[i] * tuple_term(qy, a.ids[v[u]]) * tuple_term(qw, a.ids[chain ? S.lst[i] : v[u]]);
         }
       }
     }
@@ -413,13 +414,13 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
         const uint64_t e = task_row(task, i);
         const uint32_t j = seg_search(off0, d0.ncand + 1, (uint32_t)e);
         const uint32_t mu = cl0[j], mv = ls0[e];
-        my_hash += tuple_term(P.order[0], mu) * tuple_term(P.order[1], mv);
+        my_hash += tuple_term(P.order[0], a.ids[mu]) * tuple_term(P.order[1], a.ids[mv]);
         ++my_cnt;
         if (a.emit) {
           const unsigned long long pos = atomicAdd(a.emit_ctr, 1ULL);
           if (pos < a.emit_cap) {
-            a.emit[pos * 2 + P.order[0]] = mu;
-            a.emit[pos * 2 + P.order[1]] = mv;
+            a.emit[pos * 2 + P.order[0]] = a.ids[mu];
+            a.emit[pos * 2 + P.order[1]] = a.ids[mv];
           }
         }
       }
@@ -466,7 +467,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
             for (uint32_t c = 0; c <= k; ++c) val[c * WROWS + tid] = Lk[(uint64_t)c * cap + r];
           }
           unsigned long long s = 1;
-          for (uint32_t c = 0; c <= k; ++c) s *= tuple_term(P.order[c], val[c * WROWS + tid]);
+          for (uint32_t c = 0; c <= k; ++c) s *= tuple_term(P.order[c], a.ids[val[c * WROWS + tid]]);
           S.srow[tid] = s;
           if (BYTES && agg) my_bytes += k == 1 ? 8 : 4 * (k + 1);
         }
@@ -604,7 +605,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
                 if (oks[u]) {
                   if (BYTES) my_bytes += 4;  // the list entry
                   for (uint32_t b = bo; b < be && oks[u]; ++b)
-                    oks[u] = has_edge<BYTES>(a.row, a.col, a.hub_of, a.hub_bits, a.W, mvs[u],
+                    oks[u] = has_edge<BYTES>(a.pieces, a.col, a.hub_of, a.hub_bits, a.W, mvs[u], dn.w_lo,
                                              val[P.backs[b] * WROWS + is[u]], my_bytes);
                 }
               }
@@ -637,7 +638,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
                 if (ok) {
                   if (BYTES) my_bytes += 4;  // the list entry (its hash term is a derived copy of it)
                   for (uint32_t b = bo; b < be && ok; ++b)
-                    ok = has_edge<BYTES>(a.row, a.col, a.hub_of, a.hub_bits, a.W, mv, val[P.backs[b] * WROWS + i],
+                    ok = has_edge<BYTES>(a.pieces, a.col, a.hub_of, a.hub_bits, a.W, mv, dn.w_lo, val[P.backs[b] * WROWS + i],
                                          my_bytes);
                 }
                 wave_cnt += __popcll(__ballot(ok));
@@ -647,8 +648,8 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
                     const unsigned long long pos = atomicAdd(a.emit_ctr, 1ULL);
                     if (pos < a.emit_cap) {
                       uint32_t* t = a.emit + pos * q;
-                      for (uint32_t c = 0; c <= k; ++c) t[P.order[c]] = val[c * WROWS + i];
-                      t[wn] = mv;
+                      for (uint32_t c = 0; c <= k; ++c) t[P.order[c]] = a.ids[val[c * WROWS + i]];
+                      t[wn] = a.ids[mv];
                     }
                   }
                 }
@@ -695,7 +696,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
               if (CYCLIC && bo != be) {
                 // with back edges: the tests first, then the factors of the
                 // candidates that passed them
-                back_edges_of_row<BYTES, XU>(a, P, val, bo, be, i, mvs, oks, my_bytes);
+                back_edges_of_row<BYTES, XU>(a, P, val, bo, be, dn.w_lo, i, mvs, oks, my_bytes);
 #pragma unroll
                 for (int u = 0; u < XU; ++u)
                   if (oks[u]) trm[u] = trm_n[st_r + g0 + u * WAVE + lane];
@@ -710,8 +711,8 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
                     const unsigned long long pos = atomicAdd(a.emit_ctr, 1ULL);
                     if (pos < a.emit_cap) {
                       uint32_t* t = a.emit + pos * q;
-                      for (uint32_t c = 0; c <= k; ++c) t[P.order[c]] = val[c * WROWS + i];
-                      t[wn] = mvs[u];
+                      for (uint32_t c = 0; c <= k; ++c) t[P.order[c]] = a.ids[val[c * WROWS + i]];
+                      t[wn] = a.ids[mvs[u]];
                     }
                   }
                 }

@@ -110,7 +110,8 @@ __device__ __forceinline__ bool finish_rows(const BfsArgs& a, PlanAcc* acc, Slot
     for (uint32_t b = a.any_source ? P.back_off[n2] : P.back_off[n2 + 1]; b < P.back_off[n2 + 1]; ++b) {
       const uint32_t c = P.backs[b];
       const uint32_t u = c == k + 1 ? mv : vals[c];
-      const uint32_t r0 = a.j.row[u], dg = a.j.row[u + 1] - r0;
+      uint32_t r0, dg;
+      piece(a.j.pieces, u, d.w_lo, r0, dg);
       if (full && 2 * (uint64_t)dg < len) {
         st = r0;
         len = dg;
@@ -216,7 +217,7 @@ __global__ void __launch_bounds__(256) bfs_first_kernel(BfsArgs a) {
       const uint32_t r = (uint32_t)(e - a.first_row[lo]);
       mu = a.j.clist[d0.clist_off + seg_search(a.j.offsets + d0.off_base, d0.ncand + 1, r)];
       mv = a.j.lists[d0.list_base + r];
-      h = tuple_term(P.order[0], mu) * tuple_term(P.order[1], mv);
+      h = tuple_term(P.order[0], a.j.ids[mu]) * tuple_term(P.order[1], a.j.ids[mv]);
     }
     finish_rows(a, acc, slots, has, &mu, 0, plan, mv, h);
   }
@@ -237,7 +238,6 @@ __device__ __forceinline__ void test_candidates(const BfsArgs& a, const JoinPlan
     ok[u] = idx + u * step < len;
     mv[u] = ok[u] ? from[idx + u * step] : 0u;
   }
-  unsigned long long none = 0;
   if (src) {
     // from an adjacency: in C(w), and adjacent to the parent
     const uint32_t* bm_w = a.j.bitmaps + (size_t)d.w_slot * a.j.W;
@@ -266,9 +266,22 @@ __device__ __forceinline__ void test_candidates(const BfsArgs& a, const JoinPlan
 #pragma unroll
       for (int u = 0; u < BFS_UNROLL; ++u) ok[u] = ok[u] && (wd[u] & 1u);
     } else {
+      // a short row: its piece towards the candidates' label is shorter still
+      uint32_t p0, n;
+      piece(a.j.pieces, bv, d.w_lo, p0, n);
+      const uint32_t* e[BFS_UNROLL];
 #pragma unroll
-      for (int u = 0; u < BFS_UNROLL; ++u)
-        if (ok[u]) ok[u] = has_edge<false>(a.j.row, a.j.col, a.j.hub_of, a.j.hub_bits, a.j.W, mv[u], bv, none);
+      for (int u = 0; u < BFS_UNROLL; ++u) {
+        ok[u] = ok[u] && n;
+        e[u] = a.j.col + p0;
+      }
+      for (; n > 1; n -= n >> 1) {  // the last entry <= mv[u], as in has_edge
+#pragma unroll
+        for (int u = 0; u < BFS_UNROLL; ++u)
+          if (ok[u]) e[u] = e[u][n >> 1] <= mv[u] ? e[u] + (n >> 1) : e[u];
+      }
+#pragma unroll
+      for (int u = 0; u < BFS_UNROLL; ++u) ok[u] = ok[u] && *e[u] == mv[u];
     }
   }
 }
@@ -286,7 +299,7 @@ __device__ __forceinline__ uint32_t drain(const BfsArgs& a, PlanAcc* acc, Slots&
     unsigned long long h = 0;
     if (has) {
       plan = row[R_PLAN];
-      h = (((unsigned long long)row[1] << 32) | row[0]) * tuple_term(a.j.plans[plan].order[nk], mv);
+      h = (((unsigned long long)row[1] << 32) | row[0]) * tuple_term(a.j.plans[plan].order[nk], a.j.ids[mv]);
     }
     if (!finish_rows(a, acc, slots, has, row + R_VAL, a.level, plan, mv, h)) return s0;
   }
@@ -373,7 +386,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
           for (int u = 0; u < BFS_UNROLL; ++u)
             if (ok[u]) {
               ++cnt;
-              hsum += tuple_term(qid, mv[u]);
+              hsum += tuple_term(qid, a.j.ids[mv[u]]);
             }
         } else {
           const uint32_t n = stage_step(G, mv, ok, true, 0);
@@ -448,7 +461,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
           for (int u = 0; u < BFS_UNROLL; ++u)
             if (ok[u]) {
               ++cnt;
-              hsum += tuple_term(qid, mv[u]);
+              hsum += tuple_term(qid, a.j.ids[mv[u]]);
             }
         }
       }

@@ -14,8 +14,27 @@ struct DevGraph {
   uint64_t adj = 0;
   uint32_t W = 0;   // bitmap words per query vertex
   uint32_t NB = 0;  // rank-index entries per query vertex
+  // The vertices are numbered by (label, id) on the device, so that a
+  // candidate set, all of one label, is one dense piece of every bitmap and of
+  // every hub's: ids[i] is the id of vertex i, pos its inverse.  row / col and
+  // everything below are in this numbering; what leaves the device (hashes,
+  // tuples, lists, bitmaps) is in ids.  row0 / col0: the CSR in ids (the same
+  // arrays where the numbering is the ids' own).
+  uint32_t* row0 = nullptr;
+  uint32_t* col0 = nullptr;
+  uint32_t* ids = nullptr;
+  uint32_t* pos = nullptr;
+  // The adjacency in pieces by the neighbours' label, the pieces of one label
+  // side by side: the entries of vertex v whose neighbours have a label of
+  // group g (1 << gshift consecutive dense labels) are col[lrow[g * n + v]] ..
+  // col[lrow[g * n + v + 1] - 1], ascending.  A step that looks for one label
+  // among the neighbours of a candidate set (vertices of one label) streams
+  // what it needs and nothing else.  One group: lrow is row.  row: degrees
+  // (row[v + 1] - row[v]).
   uint32_t* row = nullptr;
   uint32_t* col = nullptr;
+  uint32_t* lrow = nullptr;
+  uint32_t ngroup = 1, gshift = 0;
   uint32_t* key = nullptr;
   // ckey[e] = key[col[e]]: the filter's label/degree tests stream the keys
   // of a row's neighbours beside the row instead of gathering them
@@ -41,7 +60,9 @@ struct DevGraph {
   uint32_t hub_degree = 0;
 };
 
-constexpr uint32_t FCHUNK_VERTS = 1024;
+inline Pieces pieces_of(const DevGraph& g) { return Pieces{g.lrow, g.n, g.gshift}; }
+
+constexpr uint32_t FCHUNK_VERTS = 256;
 constexpr uint32_t FCHUNK_ENTRIES = 4096;
 constexpr uint32_t HUB_PART = 2048;
 
@@ -56,8 +77,25 @@ void launch_vertex_stats(const uint32_t* row, const uint32_t* label, uint32_t n,
 // last one the length of col) is not strictly ascending, holds its own vertex
 // or one >= n.
 void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uint32_t* bad, hipStream_t s);
-// g.key from the vertices' labels and the nl distinct label values, ascending.
-void launch_vertex_keys(const DevGraph& g, const uint32_t* label, const uint32_t* value, uint32_t nl, hipStream_t s);
+// From row0 / col0, the vertices' labels (by id) and the nl distinct label
+// values, ascending: ids, pos, row, col and lrow (unless they are row0 / col0:
+// the vertices then keep their ids) and key.  scratch: relabel_words(n, adj)
+// words, 8-byte aligned; relabel_words(n, 0) where the ids are kept.
+uint64_t relabel_words(uint32_t n, uint64_t adj);
+void launch_relabel(const DevGraph& g, const uint32_t* label, const uint32_t* value, uint32_t nl, uint32_t* scratch,
+                    hipStream_t s);
+// The groups of g.lrow for nl labels: at most PIECE_GROUPS, a table of at most
+// four words per adjacency entry, and entries that sort as 64-bit keys.
+constexpr uint32_t PIECE_GROUPS = 64;
+void choose_pieces(DevGraph& g, uint32_t nl);
+// range[2 l], range[2 l + 1]: the first vertex range with a vertex of label l
+// and the one after the last; start[l]: vertices of the labels before l (nl + 1
+// words, device).
+void launch_label_ranges(const DevGraph& g, const uint32_t* start, uint32_t nl, uint32_t* range, hipStream_t s);
+// Bitmap rows of vertices to bitmap rows of ids.
+void launch_id_bitmaps(const DevGraph& g, const uint32_t* bitmaps, uint32_t nrows, uint32_t* out, hipStream_t s);
+// Vertices to ids in place.
+void launch_to_ids(const DevGraph& g, uint32_t* v, uint64_t n, hipStream_t s);
 // The filter's vertex ranges: their ends and their number (*total), then, with
 // g.fchunk and g.wrange allocated, those.  scratch: range_words(n) words.
 // *parts (zeroed by the caller): the parts of all vertices with more than
@@ -68,8 +106,8 @@ void launch_range_ends(const uint32_t* row, uint32_t n, uint32_t* scratch, unsig
                        hipStream_t s);
 void launch_ranges(const DevGraph& g, const uint32_t* scratch, uint32_t* next, hipStream_t s);
 // g.hub_of and, with nhub of them above hub_degree and hub_bits zeroed, their
-// bitmaps.  scratch: hub_words(n, nhub) words, 8-byte aligned.
-uint64_t hub_words(uint32_t n, uint64_t nhub);
+// bitmaps.  scratch: hub_words(n) words, 8-byte aligned.
+uint64_t hub_words(uint32_t n);
 void launch_hubs(const DevGraph& g, uint32_t* scratch, hipStream_t s);
 
 // build.hip: the undirected CSR of an edge list (host arrays src/dst of m
@@ -80,12 +118,7 @@ class BlockPool;
 int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint32_t* dst, BlockPool& pool,
                          hipStream_t s, uint32_t** row, uint32_t** col, uint64_t* adj);
 
-// Sets the adjacency bitmaps of the hubs: hub_bits (nhub * W words) must be
-// zero; hubs[h] is the vertex of bitmap h; block_base[h] = 64-entry blocks
-// of the adjacency of hubs before h (nhub + 1 entries, last = nblocks).
 void launch_neighbour_keys(const DevGraph& g, hipStream_t s);
-void launch_hub_bits(const DevGraph& g, const uint32_t* hubs, const uint32_t* block_base, uint32_t nblocks,
-                     hipStream_t s);
 
 // filter.hip ------------------------------------------------------------------
 // Start-vertex candidates: C(slot) = {v : lo <= key[v] <= hi} (check_kernel).
@@ -104,6 +137,7 @@ void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* 
 // launch, whose waves leave an empty range after reading its bitmap words:
 // listing the pairs of one op on a 1M-vertex graph took 35 us (four
 // workgroups), more than the pass over its 5,000 ranges.
+// max_ranges: the most ranges any of the ops' or fills' labels has.
 // resident: filter_resident(block).  rflags: the refine rounds' change flags
 // (FilterOp::mark / need), zeroed by the caller once per batch; an op whose
 // need flag is clear is left out.  counts: the explore ops' candidates
@@ -119,8 +153,9 @@ constexpr uint64_t FILTER_DIRECT = 1u << 17;
 constexpr uint32_t FILL_PULL = 32;
 void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, const uint32_t* nbr_slot,
                         const uint32_t* nbr_lo, const uint32_t* nbr_hi, const FillOp* fills, uint32_t nfill,
-                        uint32_t* bitmaps, uint32_t block, uint32_t resident, uint2* items, uint32_t* nitems,
-                        uint32_t* rflags, uint32_t* counts, unsigned long long* stats, hipStream_t s);
+                        uint32_t* bitmaps, uint32_t max_ranges, uint32_t block, uint32_t resident, uint2* items,
+                        uint32_t* nitems, uint32_t* rflags, uint32_t* counts, unsigned long long* stats,
+                        hipStream_t s);
 // Workgroups of `block` threads of the superstep's kernel that are resident at once.
 uint32_t filter_resident(uint32_t block);
 
@@ -137,6 +172,7 @@ void launch_row_popcount(const DevGraph& g, const uint32_t* bitmaps, uint32_t nr
 // plus the rank index, from the segment counts of launch_row_popcount.
 void launch_compact_rows(const DevGraph& g, const uint32_t* bitmaps, uint32_t nrows, const uint32_t* segc,
                          const uint64_t* coff, uint32_t* clist, uint32_t* bprefix, hipStream_t s);
+void launch_fill_u32(uint32_t* p, uint32_t v, uint64_t n, hipStream_t s);
 // Exclusive scan of n u32 values; out may alias in.  total (device, u64) optional.
 void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, unsigned long long* total,
                            uint32_t* scratch, uint64_t scratch_words, hipStream_t s);
@@ -201,12 +237,12 @@ void launch_cet_sums(const DevGraph& g, const uint32_t* bitmaps, const uint32_t*
                      unsigned long long* stats = nullptr);
 // Records of the tables of the level before the last, from their lists and
 // the last tables' records.
-void launch_cet_aggs(const uint32_t* bitmaps, const uint32_t* bprefix, uint32_t W, uint32_t NB, const AggDesc* descs,
+void launch_cet_aggs(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* bprefix, const AggDesc* descs,
                      uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
                      CetAgg* aggs, uint32_t grid, hipStream_t s);
 // Hash terms of the last join levels' lists: for table term_desc[i] (terms
-// [term_start[i], term_start[i+1]) of terms), tuple_term(term_qid, list[e]).
-void launch_cet_terms(const uint32_t* lists, const CetDesc* descs, const uint32_t* term_desc,
+// [term_start[i], term_start[i+1]) of terms), tuple_term(term_qid, id of list[e]).
+void launch_cet_terms(const DevGraph& g, const uint32_t* lists, const CetDesc* descs, const uint32_t* term_desc,
                       const uint64_t* term_start, uint32_t nterm_desc, uint64_t nterms, unsigned long long* terms,
                       hipStream_t s);
 // Writes the lists.
@@ -216,8 +252,9 @@ void launch_cet_write(const DevGraph& g, const uint32_t* bitmaps, const uint32_t
 
 // join.hip ---------------------------------------------------------------------
 struct JoinArgs {
-  const uint32_t* row;
   const uint32_t* col;
+  const uint32_t* ids;       // DevGraph::ids
+  Pieces pieces;
   const uint32_t* hub_of;    // DevGraph::hub_of / hub_bits
   const uint32_t* hub_bits;
   const uint32_t* bitmaps;

@@ -22,7 +22,7 @@ namespace gpsm {
 
 class BlockPool {
  public:
-  static constexpr size_t kMost = 4ull << 30;
+  static constexpr size_t kMost = 8ull << 30;
 
   // At least nbytes (nullptr: no memory).
   void* take(size_t nbytes) {

@@ -16,6 +16,7 @@ namespace {
 constexpr int STOP = 1;  // hook asks run_batch to stop (not an error)
 
 struct FilterOut {
+  const gpsm_graph* g;
   uint32_t* bitmaps;
   uint32_t* counts;
   int rc;
@@ -25,6 +26,17 @@ int filter_hook(void* user, gpsm_ctx* c, const uint32_t* bitmaps, const uint32_t
                 uint32_t W) {
   FilterOut* fo = reinterpret_cast<FilterOut*>(user);
   fo->rc = GPSM_OK;
+  const DevGraph& dg = fo->g->dg;
+  if (fo->bitmaps && dg.row != dg.row0) {
+    // by id; the candidate lists' buffer is not in use yet
+    if (c->bufs[B_CLIST].ensure(sizeof(uint32_t) * (size_t)nslots * W)) {
+      fo->rc = GPSM_ENOMEM;
+      return STOP;
+    }
+    uint32_t* out = reinterpret_cast<uint32_t*>(c->bufs[B_CLIST].ptr);
+    launch_id_bitmaps(dg, bitmaps, nslots, out, c->stream);
+    bitmaps = out;
+  }
   if (fo->bitmaps &&
       hipMemcpyAsync(fo->bitmaps, bitmaps, sizeof(uint32_t) * (size_t)nslots * W, hipMemcpyDeviceToHost,
                      c->stream) != hipSuccess)
@@ -76,7 +88,7 @@ int cet_hook(void* user, gpsm_ctx* c, const CetDesc* fdesc, uint32_t nf) {
   CetDesc* dd = reinterpret_cast<CetDesc*>(c->bufs[B_JDESC].ptr);
   uint32_t* offs = reinterpret_cast<uint32_t*>(c->bufs[B_OFFSETS].ptr);
   uint32_t* lists = reinterpret_cast<uint32_t*>(c->bufs[B_LISTS].ptr);
-  const uint32_t* clist = reinterpret_cast<const uint32_t*>(c->bufs[B_CLIST].ptr);
+  uint32_t* clist = reinterpret_cast<uint32_t*>(c->bufs[B_CLIST].ptr);
   const uint32_t* bitmaps = reinterpret_cast<const uint32_t*>(c->bufs[B_BITMAPS].ptr);
   const DevGraph& dg = co->g->dg;
   const uint32_t grid = std::max<uint32_t>(c->ncu * 8, 64);
@@ -85,12 +97,16 @@ int cet_hook(void* user, gpsm_ctx* c, const CetDesc* fdesc, uint32_t nf) {
   launch_cet_offsets(dd, nf, offs, s);
   launch_cet_write(dg, bitmaps, clist, dd, nf, offs, lists, reinterpret_cast<uint32_t*>(c->bufs[B_CHUNKS].ptr), grid,
                    s);
+  uint64_t cmax = 0;
+  for (auto& x : d) cmax = std::max<uint64_t>(cmax, x.clist_off + x.ncand);
+  if (dg.row != dg.row0) {
+    launch_to_ids(dg, lists, listw, s);
+    launch_to_ids(dg, clist, cmax, s);
+  }
   std::vector<uint32_t> h_off(std::max<uint64_t>(offw, 1)), h_list(std::max<uint64_t>(listw, 1));
   hipMemcpyAsync(h_off.data(), offs, sizeof(uint32_t) * offw, hipMemcpyDeviceToHost, s);
   if (listw) hipMemcpyAsync(h_list.data(), lists, sizeof(uint32_t) * listw, hipMemcpyDeviceToHost, s);
   std::vector<uint32_t> h_clist;
-  uint64_t cmax = 0;
-  for (auto& x : d) cmax = std::max<uint64_t>(cmax, x.clist_off + x.ncand);
   h_clist.resize(std::max<uint64_t>(cmax, 1));
   hipMemcpyAsync(h_clist.data(), clist, sizeof(uint32_t) * cmax, hipMemcpyDeviceToHost, s);
   if (hipStreamSynchronize(s) != hipSuccess) {
@@ -116,7 +132,7 @@ int gpsm_filter(gpsm_ctx* c, const gpsm_graph* g, const gpsm_query* q, uint32_t*
   HostQuery hq;
   int vr = hq.build(q);
   if (vr) return vr;
-  FilterOut fo{bitmaps, counts, GPSM_OK};
+  FilterOut fo{g, bitmaps, counts, GPSM_OK};
   BatchHooks h;
   h.user = &fo;
   h.after_filter = filter_hook;
