@@ -49,8 +49,15 @@ __device__ __forceinline__ void flush_tally(const CetTally& t, unsigned long lon
   }
 }
 
-// Lane l of chunk j of a table with nch chunks holds candidate j + l * nch.
-__device__ __forceinline__ uint32_t cand_index(uint32_t j, uint32_t nch, uint32_t lane) { return j + lane * nch; }
+// Chunk j of a table with nch chunks holds every nch-th of the first CET_RUN *
+// nch candidates (the hubs of a graph whose ids descend by degree are among
+// them, and one piece of theirs can hold thousands of entries), and of the rest
+// runs of CET_RUN consecutive ones, whose pieces are next to each other.
+constexpr uint32_t CET_RUN = 16;
+__device__ __forceinline__ uint32_t cand_index(uint32_t j, uint32_t nch, uint32_t lane) {
+  const uint32_t r = lane / CET_RUN;
+  return r == 0 ? j + lane * nch : (CET_RUN + (r - 1) * CET_RUN) * nch + j * CET_RUN + lane % CET_RUN;
+}
 
 __device__ __forceinline__ void load_chunk(const Pieces& pieces, const uint32_t* __restrict__ clist,
                                            const CetDesc& d, uint32_t j, uint32_t nch, CetLds& L, bool& mine,

@@ -201,15 +201,7 @@ __device__ __forceinline__ uint32_t step_entries(uint32_t T, Step step) {
 // to those before v_i (match/Match.cu:547-600), so its bit goes to their
 // bitmaps at e_slot (v_0 .. v_{nv-2}: no candidate that fails has met all);
 // counts[cnt] counts the candidates that meet v_0.
-// PUSH: an explore op sets its neighbours' bits itself, in a second pass over
-// the adjacency just read, and leaves only its hubs to fill_kernel.  With
-// hundreds of ops in flight the atomics of one bitmap no longer bound the
-// launch and the pass over adjacency still in the caches is the cheaper one:
-// all supersteps of 245 queries on the 1M Chung-Lu graph 9.9 ms, 12.3 ms with
-// their fills launched apart.
-template <bool PUSH>
-__global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __restrict__ row, Pieces pieces,
-                                                          const uint32_t* __restrict__ col,
+__global__ void __launch_bounds__(256) filter_step_kernel(Pieces pieces, const uint32_t* __restrict__ col,
                                                           const uint32_t* __restrict__ ckey, uint32_t W,
                                                           const uint32_t* __restrict__ fchunk,
                                                           const uint2* __restrict__ list,
@@ -230,7 +222,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
   const uint32_t nwaves = (gridDim.x * blockDim.x) / WAVE;
   // per-lane tallies for the optional byte accounting, over all items
   unsigned long long t_cand = 0;
-  uint32_t t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
+  uint32_t t_ent = 0, t_probe = 0;
 
   // the next item's list entry is loaded while the current one runs
   uint2 nxt = list && wave < items ? list[wave] : make_uint2(0u, 0u);
@@ -361,61 +353,12 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
       } else {
         // first neighbour without a match: mu leaves C(u), its matches of the
         // neighbours before it stay
-        bool left = mine;  // to fill_kernel
-        if constexpr (PUSH) left = mine && row[id + 1] - row[id] > FCHUNK_ENTRIES;
-        if (mine && ff < nv) clear_bit(bm_u, id);
-        if (left && ff < nv) {
+        if (mine && ff < nv) {
+          clear_bit(bm_u, id);
           uint32_t* e = bitmaps + (size_t)ops[o].e_slot * W;
           for (uint32_t i = 0; i < ff; ++i) set_bit(e + (size_t)i * W, id);  // ff < nv: e_slot has nv - 1 rows
         }
-        met += (uint32_t)__popcll(__ballot(left && ff > 0));
-        if constexpr (PUSH) {
-          // every matching neighbour of a surviving prefix enters C(v_i)
-          const uint32_t lim = mine && !left ? ff : 0u;
-          for (uint32_t i = 0; i < nv && __any(i < lim); ++i) {
-            const uint32_t lo = uniform(nbr_lo[nb + i]), hi = uniform(nbr_hi[nb + i]);
-            uint32_t* bm = bitmaps + (size_t)uniform(nbr_slot[nb + i]) * W;
-            piece(pieces, id, lo, off, len);
-            if (i >= lim) len = 0;
-            const uint32_t lincl = wave_incl_scan(len);
-            const uint32_t T = uniform(__shfl(lincl, WAVE - 1, WAVE));
-            L.pre[lane] = lincl - len;
-            L.base[lane] = off;
-            wave_sync();
-            for (uint32_t f = 0; f < T; f += UNROLL * WAVE) {
-              uint32_t mvs[UNROLL], ks[UNROLL], cis[UNROLL], es[UNROLL], gi[UNROLL], cw[UNROLL];
-              bool want[UNROLL];
-#pragma unroll
-              for (int u = 0; u < UNROLL; ++u) cis[u] = gi[u] = min(f + u * WAVE + lane, T - 1);
-              halving_search<UNROLL>(L.pre, WAVE, cis);
-#pragma unroll
-              for (int u = 0; u < UNROLL; ++u) es[u] = L.base[cis[u]] + (gi[u] - L.pre[cis[u]]);
-#pragma unroll
-              for (int u = 0; u < UNROLL; ++u) {
-                mvs[u] = col[es[u]];
-                ks[u] = ckey[es[u]];
-                const bool in = f + u * WAVE + lane < T;
-                want[u] = in && ks[u] >= lo && ks[u] <= hi;
-                t_ent += in;
-                t_key += in;
-              }
-              // the words of the UNROLL entries are loaded together, and a bit
-              // is set (one atomic) only where still clear
-#pragma unroll
-              for (int u = 0; u < UNROLL; ++u)
-                cw[u] = want[u] ? __hip_atomic_load(bm + (mvs[u] >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                : ~0u;
-#pragma unroll
-              for (int u = 0; u < UNROLL; ++u)
-                if (want[u]) {
-                  ++t_set;
-                  const uint32_t m = 1u << (mvs[u] & 31);
-                  if (!(cw[u] & m)) atomicOr(bm + (mvs[u] >> 5), m);
-                }
-            }
-            wave_sync();
-          }
-        }
+        met += (uint32_t)__popcll(__ballot(mine && ff > 0));
       }
       wave_sync();
     }
@@ -424,8 +367,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
   if (stats) {
     // one atomic per counter per workgroup, spread over STAT_COPIES copies
     __shared__ unsigned long long red[4][5];
-    const unsigned long long v[5] = {t_cand, wave_sum64(t_ent), wave_sum64(t_key), wave_sum64(t_probe),
-                                     wave_sum64(t_set)};
+    const unsigned long long v[5] = {t_cand, wave_sum64(t_ent), 0, wave_sum64(t_probe), 0};
     const uint32_t w = threadIdx.x / WAVE;
     if (lane == 0)
       for (int i = 0; i < 5; ++i) red[w][i] = v[i];
@@ -452,8 +394,6 @@ __global__ void __launch_bounds__(256) filter_step_kernel(const uint32_t* __rest
 // between the L2s of eight XCDs.  Pulling them takes 11-28 us.  A vertex of v's
 // label without a neighbour in C(u) is walked to its end, so where v's label
 // has more than FILL_PULL times as many vertices as C(u) they are pushed.
-// hubs_only: only the hubs of C(u) are pushed, in parts (the others' matches
-// are set already).
 struct FillLds {
   uint32_t cand[MAX_CAND];
   uint32_t pre[WAVE + 1];
@@ -469,14 +409,13 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
                                                    const uint32_t* __restrict__ fchunk, uint32_t max_ranges,
                                                    const uint2* __restrict__ hparts, uint32_t nhp,
                                                    const FillOp* __restrict__ fills, uint32_t nfill,
-                                                   const uint32_t* __restrict__ counts, bool hubs_only,
-                                                   uint32_t* bitmaps, unsigned long long* __restrict__ stats) {
+                                                   const uint32_t* __restrict__ counts, uint32_t* bitmaps, unsigned long long* __restrict__ stats) {
   extern __shared__ unsigned char lds_raw[];
   FillLds& L = reinterpret_cast<FillLds*>(lds_raw)[threadIdx.x / WAVE];
   const uint32_t lane = lane_id();
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
   const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  const uint64_t pairs = hubs_only ? 0 : (uint64_t)nfill * max_ranges, items = pairs + (uint64_t)nfill * nhp;
+  const uint64_t pairs = (uint64_t)nfill * max_ranges, items = pairs + (uint64_t)nfill * nhp;
   uint32_t t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
   for (uint64_t it = wave; it < items; it += nwaves) {
     const bool part = it >= pairs;
@@ -487,7 +426,7 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
     const FillOp& op = fills[f];
     const uint32_t lo = uniform(op.lo), hi = uniform(op.hi), met = uniform(counts[op.cnt]);
     if (met == 0) continue;
-    const bool pull = !hubs_only && (uint64_t)met * FILL_PULL >= uniform(op.nlabel);
+    const bool pull = (uint64_t)met * FILL_PULL >= uniform(op.nlabel);
     if (part && pull) continue;
     const uint32_t* bm_u = bitmaps + (size_t)uniform(op.u_slot) * W;
     const uint32_t e_slot = uniform(op.e_slot), u_lo = uniform(op.u_lo);
@@ -669,21 +608,21 @@ void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, c
   // per atomic) 14.1 / 28.4, the atomics serialising across the XCDs.
   const uint32_t wpb = block / WAVE;
   const uint64_t most = (uint64_t)resident * FILTER_OVERSUB;
-  hipLaunchKernelGGL(direct ? filter_step_kernel<false> : filter_step_kernel<true>, dim3((uint32_t)std::min((pairs + wpb - 1) / wpb, most)), dim3(block),
-                     sizeof(WaveLds) * wpb, s, g.row, pieces_of(g), g.col, g.ckey, g.W, g.fchunk,
+  hipLaunchKernelGGL(filter_step_kernel, dim3((uint32_t)std::min((pairs + wpb - 1) / wpb, most)), dim3(block),
+                     sizeof(WaveLds) * wpb, s, pieces_of(g), g.col, g.ckey, g.W, g.fchunk,
                      direct ? nullptr : items, nitems, max_ranges, nops, ops, nbr_slot, nbr_lo, nbr_hi, bitmaps, rflags, counts, stats);
-  const uint64_t fwaves = (uint64_t)nfill * ((direct ? (uint64_t)max_ranges : 0) + g.nhparts);
+  const uint64_t fwaves = (uint64_t)nfill * (max_ranges + g.nhparts);
   if (!fwaves) return;
   hipLaunchKernelGGL(fill_kernel, dim3((uint32_t)std::min((fwaves + wpb - 1) / wpb, most)), dim3(block),
                      sizeof(FillLds) * wpb, s, g.row, pieces_of(g), g.col, g.key, g.ckey, g.W, g.fchunk, max_ranges,
-                     g.hparts, g.nhparts, fills, nfill, counts, !direct, bitmaps, stats);
+                     g.hparts, g.nhparts, fills, nfill, counts, bitmaps, stats);
 }
 
 uint32_t filter_resident(uint32_t block) {
   int dev = 0, ncu = 0, per_cu = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, filter_step_kernel<true>, (int)block,
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, filter_step_kernel, (int)block,
                                                    sizeof(WaveLds) * (block / WAVE)) != hipSuccess ||
       ncu < 1 || per_cu < 1) {
     (void)hipGetLastError();

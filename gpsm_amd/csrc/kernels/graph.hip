@@ -207,10 +207,11 @@ __global__ void to_ids_kernel(const uint32_t* __restrict__ ids, uint32_t* __rest
 }
 
 // The filter's vertex ranges: each block of FCHUNK_VERTS vertices is cut
-// greedily into ranges of at most FCHUNK_ENTRIES adjacency entries (a vertex
+// greedily into ranges of at most verts vertices and FCHUNK_ENTRIES adjacency
+// entries (a vertex
 // with more is a range of its own).  ends[b * FCHUNK_VERTS + i]: end of range i
 // of block b; count[b]: its ranges.
-__global__ void __launch_bounds__(256) range_ends_kernel(const uint32_t* __restrict__ row, uint32_t n,
+__global__ void __launch_bounds__(256) range_ends_kernel(const uint32_t* __restrict__ row, uint32_t n, uint32_t verts,
                                                          uint32_t* __restrict__ ends, uint32_t* __restrict__ count,
                                                          uint32_t* __restrict__ parts) {
   __shared__ uint32_t off[FCHUNK_VERTS + 1];
@@ -220,7 +221,7 @@ __global__ void __launch_bounds__(256) range_ends_kernel(const uint32_t* __restr
   if (threadIdx.x) return;
   uint32_t k = 0;
   for (uint32_t v = 0; v < nv; ++k) {
-    uint32_t lo = v + 1, hi = nv;  // the last end whose entries fit, at least one vertex
+    uint32_t lo = v + 1, hi = min(nv, v + verts);  // the last end whose entries fit, at least one vertex
     while (lo < hi) {
       const uint32_t mid = (lo + hi + 1) >> 1;
       if (off[mid] - off[v] <= FCHUNK_ENTRIES) lo = mid;
@@ -393,7 +394,7 @@ void launch_range_ends(const uint32_t* row, uint32_t n, uint32_t* scratch, unsig
   const uint32_t nb = range_blocks(n);
   const uint64_t ne = ((uint64_t)nb + 1) & ~1ull;
   uint32_t* count = scratch + (uint64_t)nb * FCHUNK_VERTS;
-  hipLaunchKernelGGL(range_ends_kernel, dim3(nb), dim3(256), 0, s, row, n, scratch, count, parts);
+  hipLaunchKernelGGL(range_ends_kernel, dim3(nb), dim3(256), 0, s, row, n, range_verts(n), scratch, count, parts);
   launch_exclusive_scan(count, count + ne, nb, total, count + 2 * ne, scan_scratch_words(nb), s);
 }
 

@@ -62,7 +62,10 @@ struct DevGraph {
 
 inline Pieces pieces_of(const DevGraph& g) { return Pieces{g.lrow, g.n, g.gshift}; }
 
-constexpr uint32_t FCHUNK_VERTS = 256;
+// Vertices per range: fewer where the graph is small, whose candidate sets
+// (one label's vertices, next to each other) otherwise fill too few waves.
+constexpr uint32_t FCHUNK_VERTS = 256, FCHUNK_VERTS_SMALL = 64;
+inline uint32_t range_verts(uint32_t n) { return n < 1u << 19 ? FCHUNK_VERTS_SMALL : FCHUNK_VERTS; }
 constexpr uint32_t FCHUNK_ENTRIES = 4096;
 constexpr uint32_t HUB_PART = 2048;
 
@@ -125,14 +128,13 @@ void launch_neighbour_keys(const DevGraph& g, hipStream_t s);
 void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* bitmaps, hipStream_t s);
 // One superstep: every op (one per query) explores or refines its C(u); the
 // explore ops' neighbours are filled by a second launch (fills, one per
-// neighbour), but above FILTER_DIRECT pairs by the ops themselves, with only
-// the hubs left to it.  stats (optional, STAT_COPIES x STAT_STRIDE u64, zeroed by the
+// neighbour).  stats (optional, STAT_COPIES x STAT_STRIDE u64, zeroed by the
 // caller): copy c, entries 0..4 = candidates, adjacency entries read, key
 // gathers, bitmap probes, bits set, added by the workgroups with blockIdx %
 // copies == c (the sum over copies is the launch's total).
 // Of more than FILTER_DIRECT (op, vertex range) pairs the superstep visits
 // only those whose range holds a candidate of C(u): a first kernel lists them
-// in items (nops x g.nfchunk capacity) and counts them in *nitems (zeroed by
+// in items (nops x max_ranges capacity) and counts them in *nitems (zeroed by
 // the caller), the second processes the list.  Fewer are all visited by one
 // launch, whose waves leave an empty range after reading its bitmap words:
 // listing the pairs of one op on a 1M-vertex graph took 35 us (four
@@ -146,11 +148,12 @@ constexpr uint32_t STAT_COPIES = 32, STAT_STRIDE = 8;
 constexpr uint32_t FILTER_OVERSUB = 8;
 constexpr uint64_t FILTER_DIRECT = 1u << 17;
 // A fill is pulled when FILL_PULL times the op's candidates are at least the
-// vertices of the neighbour's label.  The first three fills of 32 cycles and
-// cliques on an R-MAT 18 graph take 485 us pushed, 219 us by this rule; the
-// explore fills of 245 queries on the 1M graph 7.1 ms pushed, 6.4 / 5.7 / 5.8
-// / 5.9 ms with 4 / 12 / 32 / 100 here, 5.9 ms all pulled.
-constexpr uint32_t FILL_PULL = 32;
+// vertices of the neighbour's label.  With 8 / 32 / 256 / 1024 here and all
+// pulled: 245 queries on the 1M Chung-Lu graph 22.3 / 19.6 / 19.0 / 19.0 / 19.0
+// ms, a 14-vertex filter on it 1.38 / 1.28 / 1.11 / 1.13 / 1.14 ms, the filter
+// and tables of an 8-vertex query on a 100k graph 1.19 / 1.14 / 1.18 / 1.19 /
+// 1.18 ms (run to run +-0.03).
+constexpr uint32_t FILL_PULL = 256;
 void launch_filter_step(const DevGraph& g, const FilterOp* ops, uint32_t nops, const uint32_t* nbr_slot,
                         const uint32_t* nbr_lo, const uint32_t* nbr_hi, const FillOp* fills, uint32_t nfill,
                         uint32_t* bitmaps, uint32_t max_ranges, uint32_t block, uint32_t resident, uint2* items,
