@@ -1472,7 +1472,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
           widest = std::max(widest, bp.back().q);
           rows += analytic_rows_max(pcs[b], Q[b].plan);
         }
-        const uint32_t nwg_b = std::max<uint32_t>(1, c->ncu * bfs_resident_per_cu());
+        const uint32_t nwg_b = std::max<uint32_t>(1, c->ncu * bfs_resident_per_cu((uint32_t)bp.size()));
         const uint64_t nwave = (uint64_t)nwg_b * 4;
         const uint32_t block = (uint32_t)std::min(64.0, std::max(4.0, rows / (4.0 * nwave)));
         uint64_t words_per_row = 1;

@@ -12,9 +12,9 @@
 //    extends it) is one record; 16 lanes take a row of at most LONG_LIST
 //    candidates, four rows per wave, a workgroup takes a longer one;
 //  * a row's candidates come from its parent's candidate-edge list, or, with
-//    the learned order, from a back edge's bound vertex of shorter adjacency
-//    (tested against C(w) and the parent's edge instead): the order's choice
-//    of the vertex to expand from, made row by row;
+//    the learned order, from a back edge's bound vertex with fewer neighbours of
+//    the label (tested against C(w) and the parent's edge instead): the order's
+//    choice of the vertex to expand from, made row by row;
 //  * survivors are staged in LDS and finished densely, one lane each: their
 //    own next list (rank index, offsets), then one record;
 //  * the last level is counted and hashed, not written.
@@ -50,9 +50,54 @@ struct PlanAcc {
 
 struct WaveStage {
   uint32_t mv[STAGE];
-  uint32_t grp[STAGE];          // group of the wave whose row the survivor extends
-  const uint32_t* row[WAVE / GROUP];
+  uint32_t lane0[STAGE];  // first lane of the group whose row the survivor extends
 };
+
+// What a launch needs of a plan, in LDS: the table its rows' candidates come
+// from (position nk = level + 1 is bound) and the one of the rows written.
+// Read from the plans and tables themselves, a row's first candidate waited
+// for six loads, each with the address of the one before, its first test for
+// four more; most rows have one or two steps of candidates.
+struct PlanLevel {
+  uint64_t list, off;      // list arena: the lists; offsets arena: the next table's offsets
+  uint32_t w_slot, w_lo;   // C(w) of the candidates, a key of their label
+  uint32_t x_slot, w_lo2;  // the next table: C(x) its candidates are ranked in, a key of their label
+  uint32_t inj, qid;
+  uint8_t par, nb, par2, nb2, final, pad[3];
+  uint8_t backs[BFS_MAXQ], backs2[BFS_MAXQ];
+};
+
+__device__ __forceinline__ void load_plans(const BfsArgs& a, PlanLevel* L) {
+  const uint32_t nk = a.level + 1;
+  for (uint32_t i = threadIdx.x; i < a.nplans; i += blockDim.x) {
+    const JoinPlan& P = a.j.plans[i];
+    PlanLevel p = {};
+    if (nk < P.q) {
+      p.qid = P.order[nk];
+      p.final = nk + 1 == P.q;
+      if (nk >= 2) {
+        const CetDesc& d = a.j.cets[P.cet[nk]];
+        p.list = d.list_base;
+        p.w_slot = d.w_slot;
+        p.w_lo = d.w_lo;
+        p.inj = (uint32_t)P.inj[nk];
+        p.par = (uint8_t)P.par[nk];
+        p.nb = (uint8_t)(P.back_off[nk + 1] - P.back_off[nk]);
+        for (uint32_t b = 0; b < p.nb; ++b) p.backs[b] = P.backs[P.back_off[nk] + b];
+      }
+      if (!p.final) {
+        const CetDesc& d = a.j.cets[P.cet[nk + 1]];
+        p.off = d.off_base;
+        p.x_slot = d.x_slot;
+        p.w_lo2 = d.w_lo;
+        p.par2 = (uint8_t)P.par[nk + 1];
+        p.nb2 = (uint8_t)(P.back_off[nk + 2] - P.back_off[nk + 1]);
+        for (uint32_t b = 0; b < p.nb2; ++b) p.backs2[b] = P.backs[P.back_off[nk + 1] + b];
+      }
+    }
+    L[i] = p;
+  }
+}
 
 // A wave's block of reserved row slots of the level being written.
 struct Slots {
@@ -81,41 +126,47 @@ __device__ __forceinline__ void flush_acc(const BfsArgs& a, const PlanAcc* acc) 
   }
 }
 
-// Finishes one new row per lane (has: the lane holds one): vals[0..k] are the
-// vertices of the row it extends, mv the vertex at position nk = k + 1 and
-// hash the row's product.  Finds the list that extends it, counts it, and
-// writes its record unless it has no candidates.  All lanes of the wave call;
-// false, with nothing written or counted, when the level's buffer is full.
-__device__ __forceinline__ bool finish_rows(const BfsArgs& a, PlanAcc* acc, Slots& slots, bool has,
-                                            const uint32_t* vals, uint32_t k, uint32_t plan, uint32_t mv,
+// Finishes one new row per lane (has: the lane holds one): val(c), c <= k, are
+// the vertices of the row it extends (all lanes call it together), mv the
+// vertex at position k + 1 and hash the row's product.  Finds the list that
+// extends it, counts it, and writes its record unless it has no candidates.
+// All lanes of the wave call; false, with nothing written or counted, when the
+// level's buffer is full.
+template <typename Val>
+__device__ __forceinline__ bool finish_rows(const BfsArgs& a, const PlanLevel* plans, PlanAcc* acc, Slots& slots,
+                                            bool has, Val val, uint32_t k, uint32_t plan, uint32_t mv,
                                             unsigned long long hash) {
   const uint32_t lane = lane_id();
   const unsigned long long bh = __ballot(has);
   if (!bh) return true;
+  const PlanLevel& p = plans[plan];
   uint32_t st = 0, len = 0, src = 0, full = 0;
+  const uint32_t pp = has ? p.par2 : 0u;
+  const uint32_t bound = val(min(pp, k));
   if (has) {
-    const JoinPlan& P = a.j.plans[plan];
-    const uint32_t n2 = k + 2;
-    const CetDesc& d = a.j.cets[P.cet[n2]];
-    const uint32_t pp = P.par[n2];
-    const uint32_t x = pp == k + 1 ? mv : vals[pp];
-    const uint32_t j = rank_of(a.j.bitmaps + (size_t)d.x_slot * a.j.W, a.j.bprefix + (size_t)d.x_slot * a.j.NB, x);
-    const uint32_t* off = a.j.offsets + d.off_base;
+    const uint32_t x = pp == k + 1 ? mv : bound;
+    const uint32_t j = rank_of(a.j.bitmaps + (size_t)p.x_slot * a.j.W, a.j.bprefix + (size_t)p.x_slot * a.j.NB, x);
+    const uint32_t* off = a.j.offsets + p.off;
     st = off[j];
     full = off[j + 1] - st;
     len = full;
-    // a back edge's vertex with less than half as many neighbours is the
-    // cheaper source (its candidates take two tests more).  The heuristic
-    // order's plans keep their expand edge, the reference's rule.
-    for (uint32_t b = a.any_source ? P.back_off[n2] : P.back_off[n2 + 1]; b < P.back_off[n2 + 1]; ++b) {
-      const uint32_t c = P.backs[b];
-      const uint32_t u = c == k + 1 ? mv : vals[c];
+  }
+  // A back edge's vertex with fewer neighbours of the label is the cheaper
+  // source, although its candidates take two tests more: 32 cycles and cliques
+  // on an R-MAT 18 graph take 21.6 ms from the parents' lists alone, 16.0 /
+  // 14.2 / 13.6 ms with those less than 1/4, 1/2, 4/5 as long.  The heuristic
+  // order's plans keep their expand edge, the reference's rule.
+  const uint32_t nb = a.any_source && has ? p.nb2 : 0u;
+  for (uint32_t b = 0; __any(b < nb); ++b) {
+    const uint32_t c = b < nb ? p.backs2[b] : 0u;
+    const uint32_t at = val(min(c, k));
+    if (b < nb && full) {
       uint32_t r0, dg;
-      piece(a.j.pieces, u, d.w_lo, r0, dg);
-      if (full && 2 * (uint64_t)dg < len) {
+      piece(a.j.pieces, c == k + 1 ? mv : at, p.w_lo2, r0, dg);
+      if ((uint64_t)dg + dg / 4 < len) {
         st = r0;
         len = dg;
-        src = 1 + b - P.back_off[n2];
+        src = 1 + b;
       }
     }
   }
@@ -167,9 +218,13 @@ __device__ __forceinline__ bool finish_rows(const BfsArgs& a, PlanAcc* acc, Slot
     dst[R_START] = st;
     dst[R_LEN] = len;
     dst[R_SRC] = src;
-    for (uint32_t c = 0; c <= k; ++c) dst[R_VAL + c] = vals[c];
     dst[R_VAL + k + 1] = mv;
   }
+  if (bs | bl)
+    for (uint32_t c = 0; c <= k; ++c) {
+      const uint32_t v = val(c);
+      if (dst) dst[R_VAL + c] = v;
+    }
   // rows and the work they bring, once per wave where one plan has them all
   const uint32_t p0 = (uint32_t)__shfl((int)plan, __ffsll((long long)bh) - 1, WAVE);
   if (__ballot(has && plan != p0) == 0) {
@@ -195,7 +250,9 @@ __device__ __forceinline__ void close_slots(const BfsArgs& a, const Slots& slots
 __global__ void __launch_bounds__(256) bfs_first_kernel(BfsArgs a) {
   extern __shared__ unsigned char lds_raw[];
   PlanAcc* acc = reinterpret_cast<PlanAcc*>(lds_raw);
+  PlanLevel* plans = reinterpret_cast<PlanLevel*>(acc + a.nplans);
   for (uint32_t i = threadIdx.x; i < a.nplans; i += blockDim.x) acc[i] = {0, 0, 0, 0};
+  load_plans(a, plans);
   __syncthreads();
   Slots slots = {0, 0};
   const uint64_t total = a.first_row[a.nplans];
@@ -219,20 +276,42 @@ __global__ void __launch_bounds__(256) bfs_first_kernel(BfsArgs a) {
       mv = a.j.lists[d0.list_base + r];
       h = tuple_term(P.order[0], a.j.ids[mu]) * tuple_term(P.order[1], a.j.ids[mv]);
     }
-    finish_rows(a, acc, slots, has, &mu, 0, plan, mv, h);
+    finish_rows(a, plans, acc, slots, has, [&](uint32_t) { return mu; }, 0, plan, mv, h);
   }
   close_slots(a, slots);
   __syncthreads();
   flush_acc(a, acc);
 }
 
+// A row as its lanes hold it: lane lane0 + i has word i of the record, and lane
+// lane0 + b what the test of back edge b needs (its vertex and hub index, or
+// where it is none its entries towards the candidates' label).
+struct RowRegs {
+  uint32_t lane0, word, hub, p0, n;
+  __device__ __forceinline__ uint32_t get(uint32_t i) const { return __shfl(word, lane0 + i, WAVE); }
+};
+
+// Looks the back edges' vertices up (len: lanes of a row with candidates).
+__device__ __forceinline__ void load_backs(const BfsArgs& a, const PlanLevel& p, RowRegs& r, uint32_t src, bool live) {
+  const uint32_t b = lane_id() - r.lane0;
+  const bool mine = live && b < p.nb;
+  // the source's own edge holds; the parent's is tested in its place
+  const uint32_t c = mine ? (src == 1 + b ? p.par : p.backs[b]) : 0u;
+  const uint32_t bv = r.get(R_VAL + c);
+  r.hub = ~0u;
+  r.p0 = r.n = 0;
+  if (mine) {
+    r.hub = a.j.hub_of[bv];
+    if (r.hub == ~0u) piece(a.j.pieces, bv, p.w_lo, r.p0, r.n);
+  }
+}
+
 // The candidates idx, idx + step, ... (BFS_UNROLL of them, below len) of a
-// row: ok[u] and mv[u].  nk: the position they would bind.
-__device__ __forceinline__ void test_candidates(const BfsArgs& a, const JoinPlan& P, const CetDesc& d,
-                                                const uint32_t* __restrict__ vals, uint32_t nk, uint32_t st,
+// row: ok[u] and mv[u].  All lanes of the wave call (len 0: no row).
+__device__ __forceinline__ void test_candidates(const BfsArgs& a, const PlanLevel& p, const RowRegs& r, uint32_t st,
                                                 uint32_t len, uint32_t src, uint32_t idx, uint32_t step,
                                                 uint32_t (&mv)[BFS_UNROLL], bool (&ok)[BFS_UNROLL]) {
-  const uint32_t* from = src ? a.j.col + st : a.j.lists + d.list_base + st;
+  const uint32_t* from = src ? a.j.col + st : a.j.lists + p.list + st;
 #pragma unroll
   for (int u = 0; u < BFS_UNROLL; ++u) {
     ok[u] = idx + u * step < len;
@@ -240,26 +319,26 @@ __device__ __forceinline__ void test_candidates(const BfsArgs& a, const JoinPlan
   }
   if (src) {
     // from an adjacency: in C(w), and adjacent to the parent
-    const uint32_t* bm_w = a.j.bitmaps + (size_t)d.w_slot * a.j.W;
+    const uint32_t* bm_w = a.j.bitmaps + (size_t)p.w_slot * a.j.W;
     uint32_t wd[BFS_UNROLL];
 #pragma unroll
     for (int u = 0; u < BFS_UNROLL; ++u) wd[u] = ok[u] ? bm_w[mv[u] >> 5] >> (mv[u] & 31) : 0u;
 #pragma unroll
     for (int u = 0; u < BFS_UNROLL; ++u) ok[u] = ok[u] && (wd[u] & 1u);
   }
-  for (uint64_t m = len ? P.inj[nk] : 0; m; m &= m - 1) {
-    const uint32_t c = vals[__ffsll((long long)m) - 1];
+  for (uint32_t m = len ? p.inj : 0u; __any(m != 0); m &= m - 1) {
+    const uint32_t c = r.get(R_VAL + (m ? (uint32_t)__ffs((int)m) - 1 : 0u));
 #pragma unroll
-    for (int u = 0; u < BFS_UNROLL; ++u) ok[u] = ok[u] && mv[u] != c;
+    for (int u = 0; u < BFS_UNROLL; ++u) ok[u] = ok[u] && !(m && mv[u] == c);
   }
-  // a lane without a row (len 0) may name a plan of fewer positions
-  const uint32_t bo = P.back_off[nk], nb = len ? P.back_off[nk + 1] - bo : 0u;
-  for (uint32_t b = 0; b < nb; ++b) {
-    // the source's own edge holds; the parent's is tested in its place
-    const uint32_t bv = vals[src == 1 + b ? P.par[nk] : P.backs[bo + b]];
-    const uint32_t hb = a.j.hub_of[bv];
-    if (hb != ~0u) {
-      const uint32_t* bm = a.j.hub_bits + (size_t)hb * a.j.W;
+  const uint32_t nb = len ? p.nb : 0u;
+  for (uint32_t b = 0; __any(b < nb); ++b) {
+    const uint32_t hub = __shfl(r.hub, r.lane0 + b, WAVE);
+    const uint32_t p0 = __shfl(r.p0, r.lane0 + b, WAVE);
+    uint32_t n = __shfl(r.n, r.lane0 + b, WAVE);
+    if (b >= nb) continue;
+    if (hub != ~0u) {
+      const uint32_t* bm = a.j.hub_bits + (size_t)hub * a.j.W;
       uint32_t wd[BFS_UNROLL];
 #pragma unroll
       for (int u = 0; u < BFS_UNROLL; ++u) wd[u] = ok[u] ? bm[mv[u] >> 5] >> (mv[u] & 31) : 0u;
@@ -267,8 +346,6 @@ __device__ __forceinline__ void test_candidates(const BfsArgs& a, const JoinPlan
       for (int u = 0; u < BFS_UNROLL; ++u) ok[u] = ok[u] && (wd[u] & 1u);
     } else {
       // a short row: its piece towards the candidates' label is shorter still
-      uint32_t p0, n;
-      piece(a.j.pieces, bv, d.w_lo, p0, n);
       const uint32_t* e[BFS_UNROLL];
 #pragma unroll
       for (int u = 0; u < BFS_UNROLL; ++u) {
@@ -288,20 +365,19 @@ __device__ __forceinline__ void test_candidates(const BfsArgs& a, const JoinPlan
 
 // Staged survivors from .. n - 1 become rows, 64 at a time.  The first one
 // not written (n when all are).
-__device__ __forceinline__ uint32_t drain(const BfsArgs& a, PlanAcc* acc, Slots& slots, const WaveStage& G,
-                                          uint32_t from, uint32_t n) {
-  const uint32_t lane = lane_id(), nk = a.level + 1;
+__device__ __forceinline__ uint32_t drain(const BfsArgs& a, const PlanLevel* plans, PlanAcc* acc, Slots& slots,
+                                          const WaveStage& G, const RowRegs& regs, uint32_t from, uint32_t n) {
+  const uint32_t lane = lane_id();
   for (uint32_t s0 = from; s0 < n; s0 += WAVE) {
     const bool has = s0 + lane < n;
     const uint32_t mv = has ? G.mv[s0 + lane] : 0u;
-    const uint32_t* row = G.row[has ? G.grp[s0 + lane] : 0u];
-    uint32_t plan = 0;
-    unsigned long long h = 0;
-    if (has) {
-      plan = row[R_PLAN];
-      h = (((unsigned long long)row[1] << 32) | row[0]) * tuple_term(a.j.plans[plan].order[nk], a.j.ids[mv]);
-    }
-    if (!finish_rows(a, acc, slots, has, row + R_VAL, a.level, plan, mv, h)) return s0;
+    RowRegs r = regs;
+    r.lane0 = has ? G.lane0[s0 + lane] : 0u;
+    const uint32_t row_plan = r.get(R_PLAN), plan = has ? row_plan : 0u;
+    unsigned long long h = ((unsigned long long)r.get(1) << 32) | r.get(0);
+    if (has) h *= tuple_term(plans[plan].qid, a.j.ids[mv]);
+    if (!finish_rows(a, plans, acc, slots, has, [&](uint32_t c) { return r.get(R_VAL + c); }, a.level, plan, mv, h))
+      return s0;
   }
   return n;
 }
@@ -315,7 +391,7 @@ __device__ __forceinline__ void add_last(PlanAcc& x, unsigned long long cnt, uns
 
 // Stages the survivors of a step; their number.
 __device__ __forceinline__ uint32_t stage_step(WaveStage& G, const uint32_t (&mv)[BFS_UNROLL],
-                                               const bool (&ok)[BFS_UNROLL], bool keep, uint32_t grp) {
+                                               const bool (&ok)[BFS_UNROLL], bool keep, uint32_t lane0) {
   const uint32_t lane = lane_id();
   const unsigned long long below = lane ? (~0ULL >> (WAVE - lane)) : 0ULL;
   uint32_t n = 0;
@@ -326,31 +402,33 @@ __device__ __forceinline__ uint32_t stage_step(WaveStage& G, const uint32_t (&mv
     if (put) {
       const uint32_t at = n + (uint32_t)__popcll(bal & below);
       G.mv[at] = mv[u];
-      G.grp[at] = grp;
+      G.lane0[at] = lane0;
     }
     n += (uint32_t)__popcll(bal);
   }
   return n;
 }
 
-// Five waves per SIMD (96 VGPRs, 6 spilled): R-MAT 22 cliques 660 ms, cycles
-// 1297 ms per batch, against 753 and 1375 at four (no spill) and 643 and 1338
-// at six (32 spilled).  Bound by the back-edge probes: an n-bit hub bitmap is
-// 32 KB on 2^18 vertices, so nearly every probe is an L2 miss of its own (79
-// GB fetched in 16 ms, the copy rate of the card).
+// Eight waves per SIMD: 32 cycles and cliques on an R-MAT 18 graph 20.5-24.2
+// ms, 21.5-25.4 at six, 23.2-27.4 at five and four.  Bound by what a CU can
+// gather: a list entry and 1 to 2 back-edge bits a candidate, 2e9 candidates
+// and 4e9 loads in 20 ms; with the vertices numbered by label a hub bitmap's
+// bits of one label are a few lines, and 3 GB of 32 ms' worth come from HBM.
 // Level a.level -> a.level + 1.  A wave's place in the level's rows is a
 // cursor per kind of row: the row (or quad of rows), the step of its
 // candidates, and the step's survivors already written.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) bfs_expand_kernel(BfsArgs a) {
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) bfs_expand_kernel(BfsArgs a) {
   extern __shared__ unsigned char lds_raw[];
   PlanAcc* acc = reinterpret_cast<PlanAcc*>(lds_raw);
+  PlanLevel* plans = reinterpret_cast<PlanLevel*>(acc + a.nplans);
   __shared__ WaveStage stage[4];
   const uint32_t lane = lane_id(), wv = threadIdx.x / WAVE;
   WaveStage& G = stage[wv];
   for (uint32_t i = threadIdx.x; i < a.nplans; i += blockDim.x) acc[i] = {0, 0, 0, 0};
+  load_plans(a, plans);
   __syncthreads();
   Slots slots = {0, 0};
-  const uint32_t nk = a.level + 1;
+  const uint32_t words = R_VAL + a.level + 1;  // of a row
   const uint32_t wave = blockIdx.x * (256 / WAVE) + wv, nwaves = gridDim.x * (256 / WAVE);
   BfsCursor* cur = a.cursors + (uint64_t)wave * 2;
   bool full = false;  // the next level's buffer is full (uniform per wave)
@@ -364,23 +442,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
   uint32_t idx = blockIdx.x / share < rows_at_once ? blockIdx.x / share : ~0u, pos = first_pos, skip = 0;
   if (a.resume) idx = uniform(cur[0].idx), pos = uniform(cur[0].pos), skip = uniform(cur[0].skip);
   while (idx < nlong) {
-    const uint32_t* row = a.long_in + (uint64_t)idx * a.stride_in;
-    const uint32_t plan = uniform(row[R_PLAN]), st = uniform(row[R_START]), src = uniform(row[R_SRC]);
-    uint32_t len = uniform(row[R_LEN]);
+    RowRegs r = {};
+    r.word = lane < words ? a.long_in[(uint64_t)idx * a.stride_in + lane] : 0u;
+    const uint32_t plan = uniform(r.get(R_PLAN)), st = uniform(r.get(R_START)), src = uniform(r.get(R_SRC));
+    uint32_t len = uniform(r.get(R_LEN));
     if (len) {  // 0: reserved, not written
       if (a.j.budget && uniform((uint32_t)a.j.out[a.j.plans[plan].out].aborted)) len = 0;
-      const JoinPlan& P = a.j.plans[plan];
-      const CetDesc& d = a.j.cets[P.cet[nk]];
-      const bool final = nk + 1 == P.q;
-      const uint32_t qid = P.order[nk];
-      if (lane == 0) G.row[0] = row;
-      wave_sync();
+      const PlanLevel& p = plans[plan];
+      const bool final = p.final;
+      const uint32_t qid = p.qid;
+      load_backs(a, p, r, src, len != 0);
       unsigned long long hsum = 0;
       uint32_t cnt = 0;
       for (; pos * (WAVE * BFS_UNROLL) < len; pos += share * (256 / WAVE)) {
         uint32_t mv[BFS_UNROLL];
         bool ok[BFS_UNROLL];
-        test_candidates(a, P, d, row + R_VAL, nk, st, len, src, pos * (WAVE * BFS_UNROLL) + lane, WAVE, mv, ok);
+        test_candidates(a, p, r, st, len, src, pos * (WAVE * BFS_UNROLL) + lane, WAVE, mv, ok);
         if (final) {
 #pragma unroll
           for (int u = 0; u < BFS_UNROLL; ++u)
@@ -391,7 +468,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
         } else {
           const uint32_t n = stage_step(G, mv, ok, true, 0);
           wave_sync();
-          const uint32_t done = drain(a, acc, slots, G, skip, n);
+          const uint32_t done = drain(a, plans, acc, slots, G, r, skip, n);
           wave_sync();
           if (done < n) {
             skip = done;
@@ -403,7 +480,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
       }
       if (final) {
         const unsigned long long c = wave_sum(cnt), h = wave_sum64(hsum);
-        if (lane == 0) add_last(acc[plan], c, h * (((unsigned long long)row[1] << 32) | row[0]));
+        const unsigned long long of_row = ((unsigned long long)r.get(1) << 32) | r.get(0);
+        if (lane == 0) add_last(acc[plan], c, h * of_row);
       }
       if (full) break;
     }
@@ -413,41 +491,45 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
   }
   if (lane == 0) cur[0] = {idx, pos, skip};
 
-  // short rows: 16 lanes each, four per wave
+  // short rows: 16 lanes each, four per wave; the next quad's rows load while
+  // this one's candidates are tested
   const uint32_t nshort = min(a.cin[0], a.cap_in);
   const uint32_t gi = lane / GROUP, gl = lane % GROUP;
   constexpr uint32_t PER = WAVE / GROUP;
+  static_assert(R_VAL + BFS_MAXQ <= GROUP, "a row's words fit its lanes");
   const uint32_t nquad = (nshort + PER - 1) / PER;
   idx = wave, pos = 0, skip = 0;
   if (a.resume) idx = uniform(cur[1].idx), pos = uniform(cur[1].pos), skip = uniform(cur[1].skip);
+  auto word_of = [&](uint32_t i) {
+    const uint64_t row = (uint64_t)i * PER + gi;
+    return i < nquad && row < nshort && gl < words ? a.rows_in[row * a.stride_in + gl] : 0u;
+  };
+  uint32_t next = full ? 0u : word_of(idx);
   while (!full && idx < nquad) {
-    const uint32_t r = idx * PER + gi;
-    const uint32_t* row = a.rows_in + (uint64_t)min(r, nshort - 1) * a.stride_in;
-    uint32_t len = r < nshort ? row[R_LEN] : 0u;
+    RowRegs r = {};
+    r.lane0 = gi * GROUP;
+    r.word = next;
+    next = word_of(idx < ~0u - nwaves ? idx + nwaves : ~0u);
+    uint32_t len = r.get(R_LEN);
     if (__any(len != 0)) {
-      uint32_t plan = 0, st = 0, src = 0;
-      if (len) {
-        plan = row[R_PLAN];
-        st = row[R_START];
-        src = row[R_SRC];
-        if (a.j.budget && a.j.out[a.j.plans[plan].out].aborted) len = 0;
-      }
-      const JoinPlan& P = a.j.plans[plan];
-      const CetDesc& d = a.j.cets[P.cet[nk]];
-      const bool final = nk + 1 == P.q;
-      const uint32_t qid = P.order[nk];
-      if (gl == 0) G.row[gi] = row;
-      wave_sync();
+      // a reserved slot that holds no row has only its length
+      const uint32_t row_plan = r.get(R_PLAN), st = r.get(R_START), row_src = r.get(R_SRC);
+      const uint32_t plan = len ? row_plan : 0u, src = len ? row_src : 0u;
+      if (len && a.j.budget && a.j.out[a.j.plans[plan].out].aborted) len = 0;
+      const PlanLevel& p = plans[plan];
+      const bool final = p.final;
+      const uint32_t qid = p.qid;
+      load_backs(a, p, r, src, len != 0);
       unsigned long long hsum = 0;
       uint32_t cnt = 0;
       for (; __any(pos < len); pos += GROUP * BFS_UNROLL) {
         uint32_t mv[BFS_UNROLL];
         bool ok[BFS_UNROLL];
-        test_candidates(a, P, d, row + R_VAL, nk, st, len, src, pos + gl, GROUP, mv, ok);
-        const uint32_t n = stage_step(G, mv, ok, !final, gi);
+        test_candidates(a, p, r, st, len, src, pos + gl, GROUP, mv, ok);
+        const uint32_t n = stage_step(G, mv, ok, !final, r.lane0);
         if (n) {
           wave_sync();
-          const uint32_t done = drain(a, acc, slots, G, skip, n);
+          const uint32_t done = drain(a, plans, acc, slots, G, r, skip, n);
           wave_sync();
           if (done < n) {  // this step again later: its last-level rows are not counted yet
             skip = done;
@@ -472,8 +554,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
         c += dpp_or_0<0x112, 0xf>(c), h += dpp_or_0<0x112, 0xf>(h);
         c += dpp_or_0<0x114, 0xf>(c), h += dpp_or_0<0x114, 0xf>(h);
         c += dpp_or_0<0x118, 0xf>(c), h += dpp_or_0<0x118, 0xf>(h);
-        if (gl == GROUP - 1 && c)
-          add_last(acc[plan], c, h * (((unsigned long long)row[1] << 32) | row[0]));
+        const unsigned long long of_row = ((unsigned long long)r.get(1) << 32) | r.get(0);
+        if (gl == GROUP - 1 && c) add_last(acc[plan], c, h * of_row);
       }
       wave_sync();
       if (full) break;
@@ -496,16 +578,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) b
 uint32_t bfs_row_words(uint32_t level) { return (R_VAL + level + 1 + 1) & ~1u; }
 
 void launch_bfs_first(const BfsArgs& a, uint32_t nwg, hipStream_t s) {
-  hipLaunchKernelGGL(bfs_first_kernel, dim3(nwg), dim3(256), sizeof(PlanAcc) * a.nplans, s, a);
+  hipLaunchKernelGGL(bfs_first_kernel, dim3(nwg), dim3(256), (sizeof(PlanAcc) + sizeof(PlanLevel)) * a.nplans, s, a);
 }
 
 void launch_bfs_expand(const BfsArgs& a, uint32_t nwg, hipStream_t s) {
-  hipLaunchKernelGGL(bfs_expand_kernel, dim3(nwg), dim3(256), sizeof(PlanAcc) * a.nplans, s, a);
+  hipLaunchKernelGGL(bfs_expand_kernel, dim3(nwg), dim3(256), (sizeof(PlanAcc) + sizeof(PlanLevel)) * a.nplans, s, a);
 }
 
-uint32_t bfs_resident_per_cu() {
+uint32_t bfs_resident_per_cu(uint32_t nplans) {
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bfs_expand_kernel, 256, sizeof(PlanAcc) * BFS_PLANS) !=
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, bfs_expand_kernel, 256,
+                                                   (sizeof(PlanAcc) + sizeof(PlanLevel)) * nplans) !=
           hipSuccess ||
       per_cu < 1) {
     (void)hipGetLastError();

@@ -328,7 +328,7 @@ struct BfsArgs {
 uint32_t bfs_row_words(uint32_t level);
 void launch_bfs_first(const BfsArgs& a, uint32_t nwg, hipStream_t s);
 void launch_bfs_expand(const BfsArgs& a, uint32_t nwg, hipStream_t s);
-uint32_t bfs_resident_per_cu();
+uint32_t bfs_resident_per_cu(uint32_t nplans);
 // Join workgroups (of the timed variant of the kind's kernel) that are
 // resident on one CU at once for a batch whose widest query has qmax
 // vertices (LDS and registers); a persistent grid gains nothing from more.

@@ -38,33 +38,39 @@ __device__ __forceinline__ bool row_less(const uint32_t* __restrict__ a, const u
 }
 
 // 64 rows per workgroup; wave w counts the rows below them among the rows
-// 64w .. 64w + 63 of every 256.  Rows are compared by their top 64 bits, then
-// column by column.
+// 64w .. 64w + 63 of every 256.  Rows are compared by their top 128 bits from
+// LDS, then (more bits than that, an equal row other than itself) column by
+// column.  With 64 bits there a row of more met itself once, in another
+// iteration than any other lane: 1129 rows of 6 14-bit columns took 105 us, 17
+// so.
 __global__ void __launch_bounds__(256) rank_tuples_kernel(const uint32_t* __restrict__ tuples, uint32_t q,
                                                           uint32_t bits, const unsigned long long* __restrict__ count,
                                                           uint32_t cap, uint32_t* __restrict__ out) {
   const unsigned long long total = *count;
   if (total > cap || (uint64_t)blockIdx.x * WAVE >= total) return;
   const uint32_t n = (uint32_t)total;
-  __shared__ unsigned long long key[256];
+  __shared__ unsigned long long key[256], rest[256];
   __shared__ uint32_t part[4][WAVE];
   const uint32_t lane = lane_id(), w = threadIdx.x / WAVE;
-  const uint32_t width = q * bits, top = min(width, 64u);
+  const uint32_t width = q * bits, top = min(width, 64u), next = min(width - top, 64u);
   const uint32_t i = blockIdx.x * WAVE + lane;
   const bool mine = i < n;
   const uint32_t* ri = tuples + (size_t)min(i, n - 1) * q;
   const unsigned long long ki = row_bits(ri, q, bits, width - top, top);
+  const unsigned long long li = next ? row_bits(ri, q, bits, width - top - next, next) : 0ull;
   uint32_t below = 0;
   for (uint32_t j0 = 0; j0 < n; j0 += 256) {
     const uint32_t j = j0 + threadIdx.x;
     __syncthreads();
     key[threadIdx.x] = j < n ? row_bits(tuples + (size_t)j * q, q, bits, width - top, top) : ~0ull;
+    rest[threadIdx.x] = j < n && next ? row_bits(tuples + (size_t)j * q, q, bits, width - top - next, next) : 0ull;
     __syncthreads();
     const uint32_t m = min(WAVE * (w + 1), n > j0 ? n - j0 : 0u);
     for (uint32_t x = WAVE * w; x < m; ++x) {
-      const unsigned long long kj = key[x];
-      below += kj < ki;
-      if (kj == ki && width > 64 && row_less(tuples + (size_t)(j0 + x) * q, ri, q)) ++below;
+      const unsigned long long kj = key[x], lj = rest[x];
+      below += kj < ki || (kj == ki && lj < li);
+      if (width > 128 && kj == ki && lj == li && j0 + x != i && row_less(tuples + (size_t)(j0 + x) * q, ri, q))
+        ++below;
     }
   }
   part[w][lane] = below;
