@@ -264,6 +264,7 @@ void gpsm_shutdown(gpsm_ctx* c) {
   for (auto& b : c->bufs) b.release();
   for (auto& b : c->h_stage) b.release();
   c->arena.release();
+  c->stager.release();
   c->pool.release();
   hipEventDestroy(c->ev0);
   hipEventDestroy(c->ev1);
@@ -366,7 +367,7 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   uint32_t* dlab = tmp + head;
   uint32_t* ends = dlab + lw;
   launch_fill_u32(tmp, 0u, kRead, s);
-  if (hipMemcpyAsync(dlab, labels, sizeof(uint32_t) * n, hipMemcpyHostToDevice, s) != hipSuccess)
+  if (c->stager.to_device(dlab, labels, sizeof(uint32_t) * n, s) != hipSuccess)
     return fail(GPSM_EDEVICE);
   const uint32_t min_degree = std::max<uint32_t>(c->hub_min_degree, 1);
   if (check) launch_check_rows(d.row0, d.col0, n, tmp, s);
@@ -486,9 +487,8 @@ int gpsm_graph_upload(gpsm_ctx* c, uint32_t n, const uint32_t* row_offset, const
     delete g;
     return GPSM_ENOMEM;
   }
-  if (hipMemcpyAsync(d.row0, row_offset, sizeof(uint32_t) * (n + 1), hipMemcpyHostToDevice, c->stream) !=
-          hipSuccess ||
-      (A && hipMemcpyAsync(d.col0, col, sizeof(uint32_t) * A, hipMemcpyHostToDevice, c->stream) != hipSuccess)) {
+  if (c->stager.to_device(d.row0, row_offset, sizeof(uint32_t) * ((size_t)n + 1), c->stream) != hipSuccess ||
+      c->stager.to_device(d.col0, col, sizeof(uint32_t) * A, c->stream) != hipSuccess) {
     (void)hipGetLastError();
     (void)hipStreamSynchronize(c->stream);
     free_graph_arrays(c, d);
@@ -510,7 +510,7 @@ int gpsm_graph_upload_edges(gpsm_ctx* c, uint32_t n, uint64_t m, const uint32_t*
   DevGraph& d = g->dg;
   d.n = n;
   uint64_t adj = 0;
-  int rc = build_csr_from_edges(n, m, src, dst, c->pool, c->stream, &d.row0, &d.col0, &adj);
+  int rc = build_csr_from_edges(n, m, src, dst, c->pool, c->stager, c->stream, &d.row0, &d.col0, &adj);
   if (rc) {
     free_graph_arrays(c, d);
     delete g;
@@ -533,11 +533,9 @@ int gpsm_graph_csr(const gpsm_graph* g, uint32_t* row_offset, uint32_t* col) {
   if (!g || !row_offset || (g->dg.adj && !col)) return GPSM_EINVAL;
   hipSetDevice(g->ctx->device);
   hipStream_t s = g->ctx->stream;
-  if (hipMemcpyAsync(row_offset, g->dg.row0, sizeof(uint32_t) * ((size_t)g->dg.n + 1), hipMemcpyDeviceToHost, s) !=
-          hipSuccess ||
-      (g->dg.adj &&
-       hipMemcpyAsync(col, g->dg.col0, sizeof(uint32_t) * g->dg.adj, hipMemcpyDeviceToHost, s) != hipSuccess) ||
-      hipStreamSynchronize(s) != hipSuccess) {
+  Stager& st = g->ctx->stager;
+  if (st.to_host(row_offset, g->dg.row0, sizeof(uint32_t) * ((size_t)g->dg.n + 1), s) != hipSuccess ||
+      st.to_host(col, g->dg.col0, sizeof(uint32_t) * g->dg.adj, s) != hipSuccess) {
     (void)hipGetLastError();
     return GPSM_EDEVICE;
   }
@@ -732,8 +730,7 @@ int sort_emitted(gpsm_ctx* c, const uint32_t* emit, uint64_t n, uint32_t q, uint
     uint32_t* scratch = dptr<uint32_t>(c, B_EMIT_SORT);
     launch_sort_tuples(emit, n, q, bits, scratch, scratch + words, s);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(host, scratch + words, bytes, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
+    HIPCHK(c->stager.to_host(host, scratch + words, bytes, s));
     return GPSM_OK;
   }
   std::vector<uint32_t> tup(n * q);

@@ -9,6 +9,7 @@
 #include "kernels/launch.h"
 #include "plan.h"
 #include "pool.h"
+#include "stager.h"
 
 namespace gpsm {
 
@@ -182,6 +183,7 @@ struct gpsm_ctx {
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   char name[256] = {0};
   uint32_t filter_resident[3] = {0, 0, 0};  // resident superstep workgroups of 64, 128, 256 threads (0: not asked yet)
+  gpsm::Stager stager;   // large copies from and to ordinary host memory
   gpsm::BlockPool pool;  // memory of this context's graphs
   gpsm::DevBuf bufs[gpsm::B_COUNT_];
   gpsm_ctx() {

@@ -12,6 +12,7 @@
 #include "gpsm.h"
 #include "launch.h"
 #include "pool.h"
+#include "stager.h"
 #include "wave.h"
 
 namespace gpsm {
@@ -81,7 +82,7 @@ uint32_t grid_for(uint64_t items) {
 }  // namespace
 
 int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint32_t* dst, BlockPool& pool,
-                         hipStream_t s, uint32_t** row, uint32_t** col, uint64_t* adj_out) {
+                         Stager& stager, hipStream_t s, uint32_t** row, uint32_t** col, uint64_t* adj_out) {
   *row = *col = nullptr;
   *adj_out = 0;
   const uint64_t M2 = 2 * m;
@@ -126,8 +127,8 @@ int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint
   // the sorted, deduplicated keys end up in `keys` (the passes ping-pong)
   unsigned long long* uniq = keys;
   if (!rc && M2) {
-    if (hipMemcpyAsync(d_src, src, sizeof(uint32_t) * m, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(d_dst, dst, sizeof(uint32_t) * m, hipMemcpyHostToDevice, s) != hipSuccess) {
+    if (stager.to_device(d_src, src, sizeof(uint32_t) * m, s) != hipSuccess ||
+        stager.to_device(d_dst, dst, sizeof(uint32_t) * m, s) != hipSuccess) {
       rc = GPSM_EDEVICE;
     } else {
       hipLaunchKernelGGL(edge_keys_kernel, dim3(grid_for(m)), dim3(256), 0, s, d_src, d_dst, m, n, keys, d_bad);

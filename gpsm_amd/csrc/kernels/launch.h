@@ -118,8 +118,9 @@ void launch_hubs(const DevGraph& g, uint32_t* scratch, hipStream_t s);
 // the device.  *row (n+1) and *col (*adj) are taken from pool, as is what the
 // build itself needs.  GPSM_EINVAL if an endpoint is >= n.
 class BlockPool;
+class Stager;
 int build_csr_from_edges(uint32_t n, uint64_t m, const uint32_t* src, const uint32_t* dst, BlockPool& pool,
-                         hipStream_t s, uint32_t** row, uint32_t** col, uint64_t* adj);
+                         Stager& stager, hipStream_t s, uint32_t** row, uint32_t** col, uint64_t* adj);
 
 void launch_neighbour_keys(const DevGraph& g, hipStream_t s);
 

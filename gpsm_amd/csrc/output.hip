@@ -1,7 +1,8 @@
 // gpsm_format_tuples / gpsm_write_tuples: the embedding lines of IO::output
 // (io/IO.cpp:207-213) formatted on the device (kernels/text.hip), chunk by
 // chunk so that device and host staging stay bounded whatever the result
-// size.
+// size: rows go to the device and text comes back through the context's
+// staging, straight into the caller's buffer.
 #include <hip/hip_runtime.h>
 #include <unistd.h>
 
@@ -17,10 +18,11 @@ using namespace gpsm;
 
 namespace {
 
-constexpr uint64_t kChunkOutBytes = 256ull << 20;  // device/host staging of one chunk's text
+constexpr uint64_t kChunkOutBytes = 256ull << 20;  // device staging of one chunk's text
 
-// Formats rows [0, n_rows) chunk by chunk; sink(text, bytes) receives every
-// chunk's text in order and returns nonzero to stop.
+// Formats rows [0, n_rows) chunk by chunk; sink(text, bytes, at) receives every
+// chunk's text (device memory) in order, at bytes of text before it, and returns
+// nonzero to stop.
 template <typename Sink>
 int format_chunks(gpsm_ctx* c, const uint32_t* tuples, uint64_t n_rows, uint32_t q, const uint8_t* keep,
                   uint64_t* bytes, Sink sink) {
@@ -36,8 +38,7 @@ int format_chunks(gpsm_ctx* c, const uint32_t* tuples, uint64_t n_rows, uint32_t
   const uint64_t nwg_cap = (rows_cap + R - 1) / R;
   const uint64_t sw = scan_scratch_words(nwg_cap) + 2;
   const uint64_t out_cap = rows_cap * maxlen;
-  // device buffers are the context's (reused across calls); the host
-  // staging is ordinary memory
+  // device buffers are the context's (reused across calls)
   if (c->bufs[B_TEXT_IN].ensure(sizeof(uint32_t) * rows_cap * q) ||
       c->bufs[B_TEXT_WG].ensure(sizeof(uint32_t) * (2 * nwg_cap + sw)) ||
       (keep && c->bufs[B_TEXT_KEEP].ensure(rows_cap)) || c->bufs[B_TEXT_OUT].ensure(out_cap))
@@ -48,7 +49,6 @@ int format_chunks(gpsm_ctx* c, const uint32_t* tuples, uint64_t n_rows, uint32_t
   uint32_t* doff = dlen + nwg_cap;
   uint8_t* dk = keep ? reinterpret_cast<uint8_t*>(c->bufs[B_TEXT_KEEP].ptr) : nullptr;
   char* dout = reinterpret_cast<char*>(c->bufs[B_TEXT_OUT].ptr);
-  std::unique_ptr<char[]> hout(new char[out_cap]);
   unsigned long long* dtot = reinterpret_cast<unsigned long long*>(scr);
   uint64_t written = 0;
   int rc = GPSM_OK;
@@ -56,8 +56,7 @@ int format_chunks(gpsm_ctx* c, const uint32_t* tuples, uint64_t n_rows, uint32_t
     const uint64_t rows = std::min(ch, n_rows - base);
     const uint64_t nwg = (rows + R - 1) / R;
     unsigned long long tot = 0;
-    if (hipMemcpyAsync(dt, tuples + base * q, sizeof(uint32_t) * rows * q, hipMemcpyHostToDevice, s) !=
-            hipSuccess ||
+    if (c->stager.to_device(dt, tuples + base * q, sizeof(uint32_t) * rows * q, s) != hipSuccess ||
         (keep && hipMemcpyAsync(dk, keep + base, rows, hipMemcpyHostToDevice, s) != hipSuccess)) {
       rc = GPSM_EDEVICE;
       break;
@@ -70,11 +69,7 @@ int format_chunks(gpsm_ctx* c, const uint32_t* tuples, uint64_t n_rows, uint32_t
       rc = GPSM_EDEVICE;
       break;
     }
-    if (tot && hipMemcpy(hout.get(), dout, tot, hipMemcpyDeviceToHost) != hipSuccess) {
-      rc = GPSM_EDEVICE;
-      break;
-    }
-    rc = sink(hout.get(), tot, written);
+    rc = sink(dout, tot, written);
     written += tot;
   }
   if (bytes) *bytes = written;
@@ -90,13 +85,9 @@ int gpsm_format_tuples(gpsm_ctx* c, const uint32_t* tuples, uint64_t n_rows, uin
   if (!c || !q || q > GPSM_MAX_QV || (n_rows && !tuples) || (cap && !out)) return GPSM_EINVAL;
   bool over = false;
   const int rc = format_chunks(c, tuples, n_rows, q, keep, bytes, [&](const char* text, uint64_t n, uint64_t at) {
-    if (at + n > cap) {
-      over = true;
-      if (at < cap) std::memcpy(out + at, text, cap - at);
-    } else {
-      std::memcpy(out + at, text, n);
-    }
-    return GPSM_OK;
+    over |= at + n > cap;
+    const uint64_t fit = at < cap ? std::min(n, cap - at) : 0;
+    return !fit || c->stager.to_host(out + at, text, fit, c->stream) == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
   });
   if (rc != GPSM_OK) return rc;
   return over ? GPSM_EOVERFLOW : GPSM_OK;
@@ -105,17 +96,22 @@ int gpsm_format_tuples(gpsm_ctx* c, const uint32_t* tuples, uint64_t n_rows, uin
 int gpsm_write_tuples(gpsm_ctx* c, int fd, const uint32_t* tuples, uint64_t n_rows, uint32_t q, const uint8_t* keep,
                       uint64_t* bytes) {
   if (!c || fd < 0 || !q || q > GPSM_MAX_QV || (n_rows && !tuples)) return GPSM_EINVAL;
-  return format_chunks(c, tuples, n_rows, q, keep, bytes, [&](const char* text, uint64_t n, uint64_t) {
+  std::unique_ptr<char[]> host;  // a chunk's text; the first chunk has the most rows, not always the most text
+  uint64_t room = 0;
+  return format_chunks(c, tuples, n_rows, q, keep, bytes, [&](const char* dev, uint64_t n, uint64_t) {
+    if (n > room) host.reset(new char[room = n]);
+    if (c->stager.to_host(host.get(), dev, n, c->stream) != hipSuccess) return (int)GPSM_EDEVICE;
+    const char* text = host.get();
     while (n) {
       const ssize_t w = ::write(fd, text, n);
       if (w < 0) {
         if (errno == EINTR) continue;
-        return GPSM_EINVAL;
+        return (int)GPSM_EINVAL;
       }
       text += w;
       n -= (uint64_t)w;
     }
-    return GPSM_OK;
+    return (int)GPSM_OK;
   });
 }
 

@@ -38,8 +38,7 @@ int filter_hook(void* user, gpsm_ctx* c, const uint32_t* bitmaps, const uint32_t
     bitmaps = out;
   }
   if (fo->bitmaps &&
-      hipMemcpyAsync(fo->bitmaps, bitmaps, sizeof(uint32_t) * (size_t)nslots * W, hipMemcpyDeviceToHost,
-                     c->stream) != hipSuccess)
+      c->stager.to_host(fo->bitmaps, bitmaps, sizeof(uint32_t) * (size_t)nslots * W, c->stream) != hipSuccess)
     fo->rc = GPSM_EDEVICE;
   if (hipStreamSynchronize(c->stream) != hipSuccess) fo->rc = GPSM_EDEVICE;
   if (fo->counts) std::memcpy(fo->counts, counts, sizeof(uint32_t) * nslots);
