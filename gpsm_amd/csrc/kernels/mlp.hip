@@ -285,7 +285,7 @@ __global__ void refresh_kernel(const float* __restrict__ m, __bf16* __restrict__
   }
 }
 
-__global__ void adam_kernel(float* __restrict__ p, float* __restrict__ g, float* __restrict__ m,
+__global__ void adam_kernel(float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
                             float* __restrict__ v, float lr, float c1, float c2) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= NP) return;
@@ -296,7 +296,6 @@ __global__ void adam_kernel(float* __restrict__ p, float* __restrict__ g, float*
   m[i] = mi;
   v[i] = vi;
   p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  g[i] = 0.0f;
 }
 
 }  // namespace
@@ -304,17 +303,16 @@ __global__ void adam_kernel(float* __restrict__ p, float* __restrict__ g, float*
 struct gpsm_mlp {
   gpsm_ctx* ctx = nullptr;
   float* p = nullptr;  // FP32 masters [NP]
-  float* g = nullptr;  // gradients
+  float* g = nullptr;  // gradients [NP], then the loss
   float* m = nullptr;
   float* v = nullptr;
   __bf16* w1 = nullptr;
   __bf16* w2 = nullptr;
   __bf16* w2t = nullptr;
-  float* loss = nullptr;
   float* norm = nullptr;  // mu[F], inv_sd[F]
-  DevBuf x, t, y;
+  DevBuf x, y;  // x: features, then (gradients) targets
   DevBuf act;  // the weight-gradient GEMMs' operands (mlp_grad_kernel)
-  HostBuf hx, hy;  // pinned staging of forward's features and outputs
+  HostBuf hx, hy;  // pinned staging of inputs and outputs
   int step = 0;
 };
 
@@ -328,16 +326,23 @@ int refresh(gpsm_mlp* mm) {
   return hipGetLastError() == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
 }
 
+// Features and targets to the device: a mini-batch as one queued copy from
+// pinned memory, large ones through the context's staging.  With two pageable
+// copies in, two out and four hipMemsetAsync the gradients of 256 samples took
+// 129 us, 33 of them the kernels.
 int stage(gpsm_mlp* mm, const float* x, const float* t, uint32_t B) {
   hipStream_t s = mm->ctx->stream;
-  if (mm->x.ensure(sizeof(float) * (size_t)B * F) || mm->y.ensure(sizeof(float) * B) ||
-      (t && mm->t.ensure(sizeof(float) * B)))
-    return GPSM_ENOMEM;
-  if (hipMemcpyAsync(mm->x.ptr, x, sizeof(float) * (size_t)B * F, hipMemcpyHostToDevice, s) != hipSuccess)
-    return GPSM_EDEVICE;
-  if (t && hipMemcpyAsync(mm->t.ptr, t, sizeof(float) * B, hipMemcpyHostToDevice, s) != hipSuccess)
-    return GPSM_EDEVICE;
-  return GPSM_OK;
+  const size_t xb = sizeof(float) * (size_t)B * F, tb = sizeof(float) * B;
+  if (mm->x.ensure(xb + tb)) return GPSM_ENOMEM;
+  char* d = static_cast<char*>(mm->x.ptr);
+  if (xb >= Stager::kMin)
+    return mm->ctx->stager.to_device(d, x, xb, s) == hipSuccess && mm->ctx->stager.to_device(d + xb, t, tb, s) == hipSuccess
+               ? GPSM_OK
+               : GPSM_EDEVICE;
+  if (mm->hx.ensure(xb + tb)) return GPSM_ENOMEM;
+  std::memcpy(mm->hx.ptr, x, xb);
+  std::memcpy(static_cast<char*>(mm->hx.ptr) + xb, t, tb);
+  return hipMemcpyAsync(d, mm->hx.ptr, xb + tb, hipMemcpyHostToDevice, s) == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
 }
 
 int run_grad(gpsm_mlp* mm, uint32_t B) {
@@ -345,10 +350,10 @@ int run_grad(gpsm_mlp* mm, uint32_t B) {
   const uint32_t Bp = (B + 31) / 32 * 32;
   if (mm->act.ensure(sizeof(__bf16) * (size_t)(3 * H + F) * Bp)) return GPSM_ENOMEM;
   __bf16* act = reinterpret_cast<__bf16*>(mm->act.ptr);
-  hipMemsetAsync(mm->loss, 0, sizeof(float), s);
-  hipLaunchKernelGGL(mlp_grad_kernel, dim3(Bp / 32), dim3(64), 0, s, weights_of(mm),
-                     reinterpret_cast<const float*>(mm->x.ptr), reinterpret_cast<const float*>(mm->t.ptr), B, Bp,
-                     mm->g, mm->loss, act);
+  launch_fill_u32(reinterpret_cast<uint32_t*>(mm->g), 0u, NP + 1, s);
+  const float* x = reinterpret_cast<const float*>(mm->x.ptr);
+  hipLaunchKernelGGL(mlp_grad_kernel, dim3(Bp / 32), dim3(64), 0, s, weights_of(mm), x, x + (size_t)B * F, B, Bp,
+                     mm->g, mm->g + NP, act);
   // split K: at most 64 workgroups of at least 256 samples (a multiple of 16)
   const uint32_t chunks = std::min<uint32_t>(64, std::max<uint32_t>(1, Bp / 256));
   const uint32_t KC = ((Bp + chunks - 1) / chunks + 15) / 16 * 16;
@@ -368,10 +373,10 @@ int gpsm_mlp_create(gpsm_ctx* c, uint64_t seed, gpsm_mlp** out) {
   hipSetDevice(c->device);
   gpsm_mlp* mm = new gpsm_mlp();
   mm->ctx = c;
-  if (hipMalloc(&mm->p, sizeof(float) * NP) || hipMalloc(&mm->g, sizeof(float) * NP) ||
+  if (hipMalloc(&mm->p, sizeof(float) * NP) || hipMalloc(&mm->g, sizeof(float) * (NP + 1)) ||
       hipMalloc(&mm->m, sizeof(float) * NP) || hipMalloc(&mm->v, sizeof(float) * NP) ||
       hipMalloc(&mm->w1, sizeof(__bf16) * H * F) || hipMalloc(&mm->w2, sizeof(__bf16) * H * H) ||
-      hipMalloc(&mm->w2t, sizeof(__bf16) * H * H) || hipMalloc(&mm->loss, sizeof(float)) ||
+      hipMalloc(&mm->w2t, sizeof(__bf16) * H * H) ||
       hipMalloc(&mm->norm, sizeof(float) * 2 * F)) {
     gpsm_mlp_free(mm);
     return GPSM_ENOMEM;
@@ -406,12 +411,10 @@ void gpsm_mlp_free(gpsm_mlp* mm) {
   hipFree(mm->w1);
   hipFree(mm->w2);
   hipFree(mm->w2t);
-  hipFree(mm->loss);
   hipFree(mm->norm);
   mm->x.release();
   mm->hx.release();
   mm->hy.release();
-  mm->t.release();
   mm->y.release();
   mm->act.release();
   delete mm;
@@ -421,7 +424,7 @@ int gpsm_mlp_set_params(gpsm_mlp* mm, const float* in) {
   if (!mm || !in) return GPSM_EINVAL;
   hipStream_t s = mm->ctx->stream;
   if (hipMemcpyAsync(mm->p, in, sizeof(float) * NP, hipMemcpyHostToDevice, s) ||
-      hipMemsetAsync(mm->g, 0, sizeof(float) * NP, s) || hipMemsetAsync(mm->m, 0, sizeof(float) * NP, s) ||
+      hipMemsetAsync(mm->m, 0, sizeof(float) * NP, s) ||
       hipMemsetAsync(mm->v, 0, sizeof(float) * NP, s))
     return GPSM_EDEVICE;
   mm->step = 0;
@@ -464,15 +467,14 @@ int gpsm_mlp_grad(gpsm_mlp* mm, const float* x, const float* t, uint32_t B, floa
   int rc = stage(mm, x, t, B);
   if (rc) return rc;
   hipStream_t s = mm->ctx->stream;
-  hipMemsetAsync(mm->g, 0, sizeof(float) * NP, s);
   if ((rc = run_grad(mm, B))) return rc;
-  float l = 0;
-  if (hipMemcpyAsync(grad, mm->g, sizeof(float) * NP, hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipMemcpyAsync(&l, mm->loss, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
+  if (mm->hy.ensure(sizeof(float) * (NP + 1))) return GPSM_ENOMEM;
+  const float* out = static_cast<const float*>(mm->hy.ptr);
+  if (hipMemcpyAsync(mm->hy.ptr, mm->g, sizeof(float) * (NP + 1), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return GPSM_EDEVICE;
-  hipMemsetAsync(mm->g, 0, sizeof(float) * NP, s);
-  if (loss) *loss = l;
+  std::memcpy(grad, out, sizeof(float) * NP);
+  if (loss) *loss = out[NP];
   return GPSM_OK;
 }
 
@@ -487,7 +489,7 @@ int gpsm_mlp_train_step(gpsm_mlp* mm, const float* x, const float* t, uint32_t B
   hipLaunchKernelGGL(adam_kernel, dim3((NP + 255) / 256), dim3(256), 0, s, mm->p, mm->g, mm->m, mm->v, lr, c1, c2);
   if ((rc = refresh(mm))) return rc;
   float l = 0;
-  if (hipMemcpyAsync(&l, mm->loss, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
+  if (hipMemcpyAsync(&l, mm->g + NP, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return GPSM_EDEVICE;
   if (loss) *loss = l;

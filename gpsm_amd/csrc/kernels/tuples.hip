@@ -38,19 +38,22 @@ __device__ __forceinline__ bool row_less(const uint32_t* __restrict__ a, const u
 }
 
 // 64 rows per workgroup; wave w counts the rows below them among the rows
-// 64w .. 64w + 63 of every 256.  Rows are compared by their top 128 bits from
-// LDS, then (more bits than that, an equal row other than itself) column by
-// column.  With 64 bits there a row of more met itself once, in another
-// iteration than any other lane: 1129 rows of 6 14-bit columns took 105 us, 17
-// so.
-__global__ void __launch_bounds__(256) rank_tuples_kernel(const uint32_t* __restrict__ tuples, uint32_t q,
-                                                          uint32_t bits, const unsigned long long* __restrict__ count,
-                                                          uint32_t cap, uint32_t* __restrict__ out) {
+// 64w .. 64w + 63 of every RANK_ROWS.  Rows are compared by their top 128 bits
+// from LDS, then (more bits than that, an equal row other than itself) column
+// by column.  With 64 bits there and 256 rows at a time 1129 rows of 6 14-bit
+// columns took 105 us (a row met itself once, in another iteration than any
+// other lane), 64 us with 128 bits, 20 us so.
+constexpr uint32_t RANK_ROWS = 1024;
+
+__global__ void __launch_bounds__(RANK_ROWS) rank_tuples_kernel(const uint32_t* __restrict__ tuples, uint32_t q,
+                                                                uint32_t bits,
+                                                                const unsigned long long* __restrict__ count,
+                                                                uint32_t cap, uint32_t* __restrict__ out) {
   const unsigned long long total = *count;
   if (total > cap || (uint64_t)blockIdx.x * WAVE >= total) return;
   const uint32_t n = (uint32_t)total;
-  __shared__ unsigned long long key[256], rest[256];
-  __shared__ uint32_t part[4][WAVE];
+  __shared__ unsigned long long key[RANK_ROWS], rest[RANK_ROWS];
+  __shared__ uint32_t part[RANK_ROWS / WAVE][WAVE];
   const uint32_t lane = lane_id(), w = threadIdx.x / WAVE;
   const uint32_t width = q * bits, top = min(width, 64u), next = min(width - top, 64u);
   const uint32_t i = blockIdx.x * WAVE + lane;
@@ -59,25 +62,29 @@ __global__ void __launch_bounds__(256) rank_tuples_kernel(const uint32_t* __rest
   const unsigned long long ki = row_bits(ri, q, bits, width - top, top);
   const unsigned long long li = next ? row_bits(ri, q, bits, width - top - next, next) : 0ull;
   uint32_t below = 0;
-  for (uint32_t j0 = 0; j0 < n; j0 += 256) {
+  for (uint32_t j0 = 0; j0 < n; j0 += RANK_ROWS) {
     const uint32_t j = j0 + threadIdx.x;
     __syncthreads();
-    key[threadIdx.x] = j < n ? row_bits(tuples + (size_t)j * q, q, bits, width - top, top) : ~0ull;
-    rest[threadIdx.x] = j < n && next ? row_bits(tuples + (size_t)j * q, q, bits, width - top - next, next) : 0ull;
+    if (j < n) {
+      key[threadIdx.x] = row_bits(tuples + (size_t)j * q, q, bits, width - top, top);
+      rest[threadIdx.x] = next ? row_bits(tuples + (size_t)j * q, q, bits, width - top - next, next) : 0ull;
+    }
     __syncthreads();
-    const uint32_t m = min(WAVE * (w + 1), n > j0 ? n - j0 : 0u);
+    const uint32_t m = min(WAVE * (w + 1), n - j0);
     for (uint32_t x = WAVE * w; x < m; ++x) {
       const unsigned long long kj = key[x], lj = rest[x];
       below += kj < ki || (kj == ki && lj < li);
-      if (width > 128 && kj == ki && lj == li && j0 + x != i && row_less(tuples + (size_t)(j0 + x) * q, ri, q))
-        ++below;
     }
+    if (width > 128)
+      for (uint32_t x = WAVE * w; x < m; ++x)
+        if (key[x] == ki && rest[x] == li && j0 + x != i && row_less(tuples + (size_t)(j0 + x) * q, ri, q)) ++below;
   }
   part[w][lane] = below;
   __syncthreads();
-  const uint32_t at = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+  uint32_t at = 0;
+  for (uint32_t x = 0; x < RANK_ROWS / WAVE; ++x) at += part[x][lane];
   if (mine)
-    for (uint32_t c = w; c < q; c += 4) out[(size_t)at * q + c] = ri[c];
+    for (uint32_t c = w; c < q; c += RANK_ROWS / WAVE) out[(size_t)at * q + c] = ri[c];
 }
 
 __global__ void tuple_keys_kernel(const uint32_t* __restrict__ tuples, uint64_t n, uint32_t q, uint32_t bits,
@@ -109,8 +116,8 @@ uint32_t grid_for(uint64_t items) {
 
 void launch_rank_tuples(const uint32_t* tuples, uint32_t q, uint32_t bits, const unsigned long long* count,
                         uint32_t cap, uint32_t* out, hipStream_t s) {
-  hipLaunchKernelGGL(rank_tuples_kernel, dim3((cap + WAVE - 1) / WAVE), dim3(256), 0, s, tuples, q, bits, count, cap,
-                     out);
+  hipLaunchKernelGGL(rank_tuples_kernel, dim3((cap + WAVE - 1) / WAVE), dim3(RANK_ROWS), 0, s, tuples, q, bits, count,
+                     cap, out);
 }
 
 uint64_t tuple_sort_words(uint64_t n) {
