@@ -15,6 +15,8 @@
 // staged in LDS and written back coalesced.  The same pass writes the rank
 // index (set bits before each 256-bit block, row-relative) the join uses to
 // find a vertex's candidate-edge list.
+#include <algorithm>
+
 #include "launch.h"
 #include "wave.h"
 
@@ -221,90 +223,134 @@ __global__ void __launch_bounds__(256) compact_rows_kernel(const uint32_t* __res
   }
 }
 
-// Reduce-then-scan for generic u32 arrays (wrapping u32 values, u64 total).
-constexpr uint32_t SCAN_ITEMS = 16;
-constexpr uint32_t SCAN_TILE = 256 * SCAN_ITEMS;
+// Exclusive scan of generic u32 arrays (wrapping u32 values, u64 total) in one
+// pass: a workgroup takes the next tile (a counter, so that every tile before
+// its own is taken by a workgroup that runs), publishes the tile's sum, adds up
+// the tiles before it - 64 at a time, back to the first that has published its
+// inclusive sum - and publishes its own.  It waits only for tiles taken before
+// its own, whose sums are published before anything is waited for.
+// A state is one word (2 bits what it holds, 62 bits of sum: at most 2^30
+// values of 32 bits a launch), read and written whole at agent scope.
+// The sums first and the tiles in a second pass read everything twice: 95 +
+// 14 + 119 us for 1e8 values, 245 us with the call; in one pass 217 us.  The
+// known sum moves on by the 64 tiles of one look per exchange of states across
+// the XCDs, about 1.4 us, so tiles are large: 271 us with 8192 values, 228 with
+// 16384, 217 with 32768, 255 with 49152 (too few waves).  Looking at 128 or 256
+// tiles at a time is slower (233, 241 us at 16384): more reads of the states
+// that others write.
+constexpr uint32_t SCAN_NT = 1024, SCAN_QUADS = 8;
+constexpr uint32_t SCAN_TILE = SCAN_NT * SCAN_QUADS * 4;
+constexpr uint64_t SCAN_MOST = 1ull << 30;  // values a launch
+constexpr unsigned long long ST_SUM = 1ull << 62, ST_INCL = 2ull << 62, ST_VALUE = ST_SUM - 1;
 
-__global__ void __launch_bounds__(256) scan_reduce_kernel(const uint32_t* __restrict__ in, uint64_t n,
-                                                          unsigned long long* __restrict__ sums) {
-  __shared__ unsigned long long part[4];
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-  uint32_t v[SCAN_ITEMS];
-  if (base + SCAN_TILE <= n) {  // a whole tile: every load unconditional, all in flight together
-#pragma unroll
-    for (uint32_t j = 0; j < SCAN_ITEMS; ++j) v[j] = in[base + (uint64_t)j * 256 + threadIdx.x];
-  } else {
-#pragma unroll
-    for (uint32_t j = 0; j < SCAN_ITEMS; ++j) {
-      const uint64_t i = base + (uint64_t)j * 256 + threadIdx.x;
-      v[j] = i < n ? in[i] : 0u;
-    }
-  }
-  unsigned long long s = 0;
-#pragma unroll
-  for (uint32_t j = 0; j < SCAN_ITEMS; ++j) s += v[j];
-  s = wave_sum64(s);
-  if (lane_id() == 0) part[threadIdx.x / WAVE] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) sums[blockIdx.x] = part[0] + part[1] + part[2] + part[3];
+// Before the states in scratch: the tile counter, the sum of earlier launches.
+struct ScanHead {
+  unsigned int next, pad;
+  unsigned long long carry;
+};
+
+__device__ __forceinline__ uint4 load_quad(const uint32_t* in, uint64_t i, uint64_t n, bool wide) {
+  if (wide && i + 4 <= n) return *reinterpret_cast<const uint4*>(in + i);
+  uint4 v;
+  v.x = i < n ? in[i] : 0u;
+  v.y = i + 1 < n ? in[i + 1] : 0u;
+  v.z = i + 2 < n ? in[i + 2] : 0u;
+  v.w = i + 3 < n ? in[i + 3] : 0u;
+  return v;
 }
 
-// The tile sums' exclusive scan, in place, and their total: one workgroup
-// of 1024 threads, 4096 sums per step.  (A single thread's serial loop over
-// them took 3.8 ms for 32,768 sums; 256 threads with 16 sums each, 45 us.)
-__global__ void __launch_bounds__(1024) scan_sums_kernel(unsigned long long* __restrict__ sums, uint32_t nb,
-                                                         unsigned long long* __restrict__ total) {
-  const unsigned long long t = block_scan_in_place<unsigned long long, 1024, 4>(sums, nb);
-  if (threadIdx.x == 0 && total) *total = t;
-}
-
-// A tile in striped order: thread t holds values j * 256 + t (every load
-// and store instruction moves 256 contiguous bytes per wave).  Each wave
-// scans its 64 values of every row j with shuffles, one wave scans the 64
-// (row, wave) totals in element order, and each value gets the tile's base,
-// its (row, wave) offset and its place in its wave's scan: two barriers per
-// tile.
-__global__ void __launch_bounds__(256) scan_tile_kernel(const uint32_t* in, uint32_t* out, uint64_t n,
-                                                        const unsigned long long* __restrict__ sums) {
-  __shared__ uint32_t wt[SCAN_ITEMS * 4];  // (row j, wave w) totals at j * 4 + w, then their offsets
+// wide: in and out are 16-byte aligned.  first: no earlier launch's sum.
+__global__ void __launch_bounds__(SCAN_NT) scan_kernel(const uint32_t* in, uint32_t* out, uint64_t n, bool wide,
+                                                       bool first, ScanHead* head,
+                                                       unsigned long long* __restrict__ state,
+                                                       unsigned long long* __restrict__ total) {
+  constexpr uint32_t NW = SCAN_NT / WAVE;
+  __shared__ uint32_t wt[SCAN_QUADS * NW];  // (quad k, wave w) totals at k * NW + w, then their offsets
+  __shared__ unsigned long long part[NW], before;
+  __shared__ uint32_t taken;
   const uint32_t lane = lane_id(), w = threadIdx.x / WAVE;
-  const uint64_t base = (uint64_t)blockIdx.x * SCAN_TILE;
-  const bool whole = base + SCAN_TILE <= n;
-  uint32_t v[SCAN_ITEMS];
-  if (whole) {
-#pragma unroll
-    for (uint32_t j = 0; j < SCAN_ITEMS; ++j) v[j] = in[base + (uint64_t)j * 256 + threadIdx.x];
-  } else {
-#pragma unroll
-    for (uint32_t j = 0; j < SCAN_ITEMS; ++j) {
-      const uint64_t i = base + (uint64_t)j * 256 + threadIdx.x;
-      v[j] = i < n ? in[i] : 0u;
-    }
-  }
-#pragma unroll
-  for (uint32_t j = 0; j < SCAN_ITEMS; ++j) {
-    const uint32_t incl = wave_incl_scan(v[j]);
-    if (lane == WAVE - 1) wt[j * 4 + w] = incl;
-    v[j] = incl - v[j];  // exclusive within the wave's 64 values of row j
-  }
+  if (threadIdx.x == 0) taken = gridDim.x > 1 ? atomicAdd(&head->next, 1u) : 0u;
   __syncthreads();
-  static_assert(SCAN_ITEMS * 4 == WAVE, "one wave scans the (row, wave) totals");
+  const uint32_t tile = taken;
+  const uint64_t base = (uint64_t)tile * SCAN_TILE;
+  uint4 v[SCAN_QUADS];
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_QUADS; ++k)
+    v[k] = load_quad(in, base + ((uint64_t)k * SCAN_NT + threadIdx.x) * 4, n, wide);
+  unsigned long long mine = 0;
+  uint32_t ex[SCAN_QUADS];
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_QUADS; ++k) {
+    mine += (unsigned long long)v[k].x + v[k].y + ((unsigned long long)v[k].z + v[k].w);
+    const uint32_t s = v[k].x + v[k].y + v[k].z + v[k].w, incl = wave_incl_scan(s);
+    if (lane == WAVE - 1) wt[k * NW + w] = incl;
+    ex[k] = incl - s;
+  }
+  mine = wave_sum64(mine);
+  if (lane == 0) part[w] = mine;
+  __syncthreads();
   if (w == 0) {
-    const uint32_t x = wt[lane];
-    wt[lane] = wave_incl_scan(x) - x;
-  }
-  __syncthreads();
-  const uint32_t off = (uint32_t)sums[blockIdx.x];
-  if (whole) {
+    static_assert(SCAN_QUADS * NW % WAVE == 0, "one wave scans the (quad, wave) totals");
+    uint32_t run = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < SCAN_ITEMS; ++j) out[base + (uint64_t)j * 256 + threadIdx.x] = off + wt[j * 4 + w] + v[j];
-  } else {
-#pragma unroll
-    for (uint32_t j = 0; j < SCAN_ITEMS; ++j) {
-      const uint64_t i = base + (uint64_t)j * 256 + threadIdx.x;
-      if (i < n) out[i] = off + wt[j * 4 + w] + v[j];
+    for (uint32_t c = 0; c < SCAN_QUADS * NW; c += WAVE) {
+      const uint32_t x = wt[c + lane], incl = wave_incl_scan(x);
+      wt[c + lane] = run + incl - x;
+      run += __shfl(incl, WAVE - 1, WAVE);
+    }
+    unsigned long long sum = 0;
+    for (uint32_t i = 0; i < NW; ++i) sum += part[i];
+    unsigned long long excl = 0;
+    if (gridDim.x > 1) {
+      if (lane == 0)
+        __hip_atomic_store(&state[tile], (tile ? ST_SUM : ST_INCL) | sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (uint32_t hi = tile; hi > 0;) {  // tiles below hi are still to be added
+        const unsigned long long st =
+            lane < hi ? __hip_atomic_load(&state[hi - 1 - lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : ST_INCL;
+        const unsigned long long incl_at = __ballot((st & ST_INCL) != 0), none = __ballot(st == 0);
+        // lanes up to the first inclusive sum count
+        const unsigned long long use = incl_at ? (incl_at & (0ull - incl_at)) * 2 - 1 : ~0ull;
+        if (none & use) {
+          __builtin_amdgcn_s_sleep(1);
+          continue;
+        }
+        excl += wave_sum64((use >> lane) & 1 ? st & ST_VALUE : 0ull);
+        hi = incl_at ? 0u : hi - WAVE;
+      }
+      if (tile && lane == 0)
+        __hip_atomic_store(&state[tile], ST_INCL | (excl + sum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const unsigned long long carry = first ? 0ull : head->carry;
+    if (lane == 0) {
+      before = carry + excl;
+      if (tile == gridDim.x - 1 && total) *total = carry + excl + sum;
     }
   }
+  __syncthreads();
+  const uint32_t off = (uint32_t)before;
+#pragma unroll
+  for (uint32_t k = 0; k < SCAN_QUADS; ++k) {
+    const uint64_t i = base + ((uint64_t)k * SCAN_NT + threadIdx.x) * 4;
+    uint4 o;
+    o.x = off + wt[k * NW + w] + ex[k];
+    o.y = o.x + v[k].x;
+    o.z = o.y + v[k].y;
+    o.w = o.z + v[k].z;
+    if (wide && i + 4 <= n) {
+      *reinterpret_cast<uint4*>(out + i) = o;
+    } else {
+      if (i < n) out[i] = o.x;
+      if (i + 1 < n) out[i + 1] = o.y;
+      if (i + 2 < n) out[i + 2] = o.z;
+      if (i + 3 < n) out[i + 3] = o.w;
+    }
+  }
+}
+
+// The sum so far is carried to the next launch, whose tiles start over.
+__global__ void scan_next_kernel(ScanHead* head, const unsigned long long* __restrict__ sum) {
+  head->carry = *sum;
+  head->next = 0;
 }
 
 __global__ void fill_u32_kernel(uint32_t* __restrict__ p, uint32_t v, uint64_t n) {
@@ -340,16 +386,32 @@ void launch_compact_rows(const DevGraph& g, const uint32_t* bitmaps, uint32_t nr
                      clist, bprefix);
 }
 
-uint64_t scan_scratch_words(uint64_t n) { return 2 * ((n + SCAN_TILE - 1) / SCAN_TILE) + 2; }
+namespace {
+uint64_t scan_tiles(uint64_t n) { return (std::min(n, SCAN_MOST) + SCAN_TILE - 1) / SCAN_TILE; }
+constexpr uint64_t kScanHead = (sizeof(ScanHead) + sizeof(unsigned long long)) / sizeof(uint32_t);  // and a total
+}  // namespace
+
+uint64_t scan_scratch_words(uint64_t n) { return kScanHead + 2 * scan_tiles(n); }
 
 void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, unsigned long long* total,
                            uint32_t* scratch, uint64_t scratch_words, hipStream_t s) {
-  const uint64_t nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-  if (nb == 0 || scratch_words < 2 * nb) return;
-  unsigned long long* sums = reinterpret_cast<unsigned long long*>(scratch);
-  hipLaunchKernelGGL(scan_reduce_kernel, dim3((uint32_t)nb), dim3(256), 0, s, in, n, sums);
-  hipLaunchKernelGGL(scan_sums_kernel, dim3(1), dim3(1024), 0, s, sums, (uint32_t)nb, total);
-  hipLaunchKernelGGL(scan_tile_kernel, dim3((uint32_t)nb), dim3(256), 0, s, in, out, n, sums);
+  if (!n || scratch_words < scan_scratch_words(n)) return;
+  ScanHead* head = reinterpret_cast<ScanHead*>(scratch);
+  unsigned long long* sum = reinterpret_cast<unsigned long long*>(head + 1);
+  unsigned long long* state = sum + 1;
+  const bool wide = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+  for (uint64_t at = 0; at < n; at += SCAN_MOST) {
+    const uint64_t m = std::min(SCAN_MOST, n - at), tiles = scan_tiles(m);
+    const bool last = at + m == n;
+    if (at) {
+      hipLaunchKernelGGL(scan_next_kernel, dim3(1), dim3(1), 0, s, head, sum);
+      launch_fill_u32(reinterpret_cast<uint32_t*>(state), 0u, 2 * tiles, s);
+    } else if (tiles > 1) {
+      launch_fill_u32(scratch, 0u, kScanHead + 2 * tiles, s);
+    }
+    hipLaunchKernelGGL(scan_kernel, dim3((uint32_t)tiles), dim3(SCAN_NT), 0, s, in + at, out + at, m, wide, at == 0,
+                       head, state, last ? total : sum);
+  }
 }
 
 uint64_t compact_scratch_words(uint64_t nbits) {

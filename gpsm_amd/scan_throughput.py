@@ -61,7 +61,9 @@ def summarise(trace_csv, rec, out_md, command, append):
         m = re.search(r"(\w+_kernel)", r["Kernel_Name"])
         if m:
             dur[m.group(1)].append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-3)
-    byt = kernel_bytes(rec["mode"], rec["n"], rec.get("ids", 0))
+    # the one-pass scan, or a trace of the three kernels before it
+    byt = {"scan_kernel": 8 * rec["n"]} if "scan_kernel" in dur else kernel_bytes(rec["mode"], rec["n"],
+                                                                                  rec.get("ids", 0))
     lines = [] if append else [
         "# Scan and compaction kernels: HBM throughput", "",
         "Each configuration is one rocprofv3 --kernel-trace run (commands below); per kernel the average of its "

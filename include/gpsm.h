@@ -257,8 +257,9 @@ int gpsm_scan_u32(gpsm_ctx* ctx, const uint32_t* in, uint32_t* out, uint64_t n, 
  * (GPSM_ESCRATCH beyond it).  Runs on the context's stream and waits for it.
  * Calls that overlap on one device share that array and race. */
 #define GPSM_SCAN_NOALLOC_SCRATCH_BYTES (256u * 1024u)
-/* 2 words hold the total, 2 words per block of 4096 values hold its sum:
- * (65536 - 2) / 2 = 32767 blocks */
+/* 2 words hold the total; 2 words per block of 4096 values would fit the
+ * rest, (65536 - 2) / 2 = 32767 blocks (a block's sum takes 2 words, and
+ * blocks are 32768 values) */
 #define GPSM_SCAN_NOALLOC_MAX (32767ull * 4096ull)
 int gpsm_scan_u32_noalloc(gpsm_ctx* ctx, const uint32_t* d_in, uint32_t* d_out, uint64_t n, uint64_t* total);
 
