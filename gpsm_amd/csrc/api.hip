@@ -598,7 +598,7 @@ constexpr double kLevelBytes = 16.0 * (1ull << 30);
 // First-table rows of the plans joined breadth-first at a time (1 GB of rows).
 constexpr uint64_t kBfsRows = 1ull << 25;
 
-// Words of B_CTR: 0 .. 2 the launches' task counters, 16 .. 17 the tuples
+// Words of the join's counters (after B_JOUT's results): 0 .. 2 the launches' task counters, 16 .. 17 the tuples
 // emitted, and of the breadth-first join, per level, two row counts and the
 // waves that stopped at a full buffer.
 constexpr uint32_t kCtrRows = 64, kCtrPending = kCtrRows + 2 * (BFS_MAXQ + 2), kCtrWords = 128;
@@ -606,7 +606,7 @@ static_assert(kCtrPending + BFS_MAXQ <= kCtrWords, "levels 0 .. BFS_MAXQ - 1");
 
 template <typename T>
 T* dptr(gpsm_ctx* c, int b) {
-  return reinterpret_cast<T*>(c->bufs[b].ptr);
+  return reinterpret_cast<T*>(c->part[b] ? c->part[b] : c->bufs[b].ptr);
 }
 
 template <typename T>
@@ -621,6 +621,55 @@ int upload(gpsm_ctx* c, int b, const std::vector<T>& v) {
   if (hipMemcpyAsync(c->bufs[b].ptr, h, sizeof(T) * v.size(), hipMemcpyHostToDevice, c->stream) != hipSuccess)
     return GPSM_EDEVICE;
   return GPSM_OK;
+}
+
+// A phase's arrays to the device in one copy (a copy of its own for each took
+// a third of the smallest call): dptr(id) is where they are.  An array's place
+// depends on the sizes before it rounded up, so that batches alike in size
+// reuse a captured graph.
+struct Part {
+  int id;
+  const void* p;
+  size_t bytes;
+};
+
+template <typename T>
+Part part(int id, const std::vector<T>& v) {
+  return {id, v.data(), sizeof(T) * v.size()};
+}
+
+int upload_parts(gpsm_ctx* c, int buf, std::initializer_list<Part> parts) {
+  auto room = [](size_t bytes) {
+    size_t r = 256;
+    while (r < bytes && r < 65536) r *= 2;
+    return (std::max(r, bytes) + r - 1) / r * r;
+  };
+  size_t at = 0, end = 0;
+  for (const Part& x : parts) {
+    end = at + x.bytes;
+    at += room(x.bytes);
+  }
+  if (int rc = c->bufs[buf].ensure(at)) return rc;
+  char* h = static_cast<char*>(c->arena.take(at));
+  if (!h) return GPSM_ENOMEM;
+  char* d = static_cast<char*>(c->bufs[buf].ptr);
+  at = 0;
+  for (const Part& x : parts) {
+    if (x.bytes) std::memcpy(h + at, x.p, x.bytes);
+    c->part[x.id] = d + at;
+    at += room(x.bytes);
+  }
+  return hipMemcpyAsync(d, h, std::max<size_t>(end, 1), hipMemcpyHostToDevice, c->stream) == hipSuccess
+             ? GPSM_OK
+             : GPSM_EDEVICE;
+}
+
+// Chunks of 64 candidates in the tables before each of v, and in all.
+template <typename Desc>
+std::vector<uint32_t> chunks_before(const std::vector<Desc>& v) {
+  std::vector<uint32_t> base(1, 0);
+  for (const auto& d : v) base.push_back(base.back() + (d.ncand + 63) / 64);
+  return base;
 }
 
 struct QState {
@@ -881,10 +930,8 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   fill_off[maxsteps] = (uint32_t)fills.size();
   const size_t ncounters = (size_t)maxsteps + nexplore;  // listed items per superstep, candidates per explore op
   if ((rc = c->bufs[B_BITMAPS].ensure(sizeof(uint32_t) * (size_t)std::max<uint32_t>(erows, 1) * W)) ||
-      (rc = upload(c, B_FILLS, fills)))
-    return rc;
-  if ((rc = upload(c, B_INIT, init)) || (rc = upload(c, B_FOPS, fops)) || (rc = upload(c, B_NBR_SLOT, nbr_slot)) ||
-      (rc = upload(c, B_NBR_LO, nbr_lo)) || (rc = upload(c, B_NBR_HI, nbr_hi)))
+      (rc = upload_parts(c, B_UP_A, {part(B_INIT, init), part(B_FOPS, fops), part(B_FILLS, fills),
+                                     part(B_NBR_SLOT, nbr_slot), part(B_NBR_LO, nbr_lo), part(B_NBR_HI, nbr_hi)})))
     return rc;
   if ((rc = c->bufs[B_COUNTS].ensure(sizeof(uint32_t) * std::max<uint32_t>(nslots, 1)))) return rc;
   if ((rc = c->bufs[B_SEGC].ensure(sizeof(uint32_t) * std::max<uint64_t>((uint64_t)nslots * segs_of(W), 1))))
@@ -893,9 +940,9 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   for (uint32_t sidx = 0; sidx < maxsteps; ++sidx)
     max_items = std::max(max_items, (uint64_t)(step_off[sidx + 1] - step_off[sidx]) * step_ranges[sidx]);
   if ((rc = c->bufs[B_FITEMS].ensure(sizeof(uint2) * max_items)) ||
-      (rc = c->bufs[B_FNITEMS].ensure(sizeof(uint32_t) * std::max<size_t>(ncounters, 1))) ||
-      (rc = c->bufs[B_RFLAGS].ensure(sizeof(uint32_t) * 4 * (uint64_t)std::max<uint32_t>(nq, 1))))
+      (rc = c->bufs[B_FNITEMS].ensure(sizeof(uint32_t) * (ncounters + 4 * (uint64_t)std::max<uint32_t>(nq, 1)))))
     return rc;
+  uint32_t* rflags = dptr<uint32_t>(c, B_FNITEMS) + ncounters;
   // work counters (profile mode 2): one slot per filter superstep, then the
   // candidate-edge count of phase B, the count of phase C and the write
   const size_t fstat_step = (size_t)STAT_COPIES * STAT_STRIDE;
@@ -909,9 +956,9 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if (o.use_graph) {
     sig_a.add(uint64_t{0});
     sig_a.add_graph(dg);
-    for (int i : {B_FILLS, B_BITMAPS, B_FNITEMS, B_RFLAGS, B_INIT, B_FOPS, B_NBR_SLOT, B_NBR_LO, B_NBR_HI, B_FITEMS, B_SEGC,
+    for (int i : {B_FILLS, B_BITMAPS, B_FNITEMS, B_INIT, B_FOPS, B_NBR_SLOT, B_NBR_LO, B_NBR_HI, B_FITEMS, B_SEGC,
                   B_COUNTS})
-      sig_a.add(c->bufs[i].ptr);
+      sig_a.add(dptr<uint32_t>(c, i));
     sig_a.add(nslots), sig_a.add(maxsteps), sig_a.add(nq), sig_a.add(init.size()), sig_a.add(fblock);
     for (uint32_t v : step_off) sig_a.add(v);
     for (uint32_t v : fill_off) sig_a.add(v);
@@ -924,8 +971,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     bool captured = false;
     if (o.use_graph && hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) captured = true;
     launch_fill_u32(bitmaps, 0u, (uint64_t)erows * W, s);
-    if (ncounters) launch_fill_u32(dptr<uint32_t>(c, B_FNITEMS), 0u, ncounters, s);
-    launch_fill_u32(dptr<uint32_t>(c, B_RFLAGS), 0u, 4ull * std::max<uint32_t>(nq, 1), s);
+    launch_fill_u32(dptr<uint32_t>(c, B_FNITEMS), 0u, ncounters + 4ull * std::max<uint32_t>(nq, 1), s);
     if (counters) launch_fill_u32(reinterpret_cast<uint32_t*>(fstats), 0u, 2ull * fstat_step * nstat_slots, s);
     {
       hipEvent_t a = pbegin(K_INIT);
@@ -940,7 +986,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
                          dptr<uint32_t>(c, B_NBR_LO), dptr<uint32_t>(c, B_NBR_HI),
                          dptr<FillOp>(c, B_FILLS) + fill_off[sidx], fill_off[sidx + 1] - fill_off[sidx], bitmaps,
                          step_ranges[sidx], fblock, fresident, dptr<uint2>(c, B_FITEMS), dptr<uint32_t>(c, B_FNITEMS) + sidx,
-                         dptr<uint32_t>(c, B_RFLAGS), dptr<uint32_t>(c, B_FNITEMS) + maxsteps,
+                         rflags, dptr<uint32_t>(c, B_FNITEMS) + maxsteps,
                          counters ? fstats + fstat_step * sidx : nullptr, s);
       pend(K_FILTER, a, 4.0 * W * nops_s, counters ? (int)sidx : -1);
     }
@@ -973,15 +1019,8 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // ---------------- phase B: compaction + forward |CET| ----------------
   std::vector<uint64_t> coff(std::max<uint32_t>(nslots, 1) + 1, 0);
   for (uint32_t r = 0; r < nslots; ++r) coff[r + 1] = coff[r] + counts[r];
-  if ((rc = upload(c, B_COFF, coff))) return rc;
   if ((rc = c->bufs[B_CLIST].ensure(sizeof(uint32_t) * std::max<uint64_t>(coff[nslots], 1)))) return rc;
   if ((rc = c->bufs[B_BPREFIX].ensure(sizeof(uint32_t) * (size_t)std::max<uint32_t>(nslots, 1) * NB))) return rc;
-  {
-    hipEvent_t a = pbegin(K_COMPACT);
-    launch_compact_rows(dg, bitmaps, nslots, dptr<uint32_t>(c, B_SEGC), dptr<uint64_t>(c, B_COFF),
-                        dptr<uint32_t>(c, B_CLIST), dptr<uint32_t>(c, B_BPREFIX), s);
-    pend(K_COMPACT, a, (double)nslots * 4.0 * (W + NB) + 4.0 * coff[nslots], -1);
-  }
   std::vector<CetDesc> fdesc;
   std::vector<uint32_t> fdesc_of_q(nq, 0);
   for (uint32_t b = 0; b < nq; ++b) {
@@ -1010,14 +1049,20 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     rev_bound += counts[d.w_slot] + 1;
   }
   const uint32_t cgrid = std::max<uint32_t>(c->ncu * 8, 64);
-  if ((rc = upload(c, B_FDESC, fdesc))) return rc;
-  if ((rc = c->bufs[B_CHUNKS].ensure(sizeof(uint32_t) * (fdesc.size() + 2)))) return rc;
+  if ((rc = upload_parts(c, B_UP_B, {part(B_COFF, coff), part(B_FDESC, fdesc), part(B_FCHUNK, chunks_before(fdesc))})))
+    return rc;
+  {
+    hipEvent_t a = pbegin(K_COMPACT);
+    launch_compact_rows(dg, bitmaps, nslots, dptr<uint32_t>(c, B_SEGC), dptr<uint64_t>(c, B_COFF),
+                        dptr<uint32_t>(c, B_CLIST), dptr<uint32_t>(c, B_BPREFIX), s);
+    pend(K_COMPACT, a, (double)nslots * 4.0 * (W + NB) + 4.0 * coff[nslots], -1);
+  }
   if ((rc = c->bufs[B_OFFSETS].ensure(sizeof(uint32_t) * std::max<uint64_t>(fwd_words + rev_bound, 1)))) return rc;
   const uint64_t off_capacity = c->bufs[B_OFFSETS].bytes / sizeof(uint32_t);
   {
     hipEvent_t a = pbegin(K_CET_COUNT);
     launch_cet_count(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_FDESC), (uint32_t)fdesc.size(),
-                     dptr<uint32_t>(c, B_OFFSETS), 1, dptr<uint32_t>(c, B_CHUNKS), cgrid, s,
+                     dptr<uint32_t>(c, B_OFFSETS), 1, dptr<uint32_t>(c, B_FCHUNK), cgrid, s,
                      counters ? fstats + fstat_step * slot_cet_b : nullptr);
     pend(K_CET_COUNT, a, 0.0, counters ? slot_cet_b : -1);
   }
@@ -1284,8 +1329,6 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // ---------------- phase C: candidate-edge tables ----------------
   wall(K_WALL_PLAN);
   term_start.push_back(term_words);
-  if ((rc = upload(c, B_JDESC, jdesc)) || (rc = upload(c, B_PLANS, plans)) || (rc = upload(c, B_TERM_DESC, term_desc)) || (rc = upload(c, B_TERM_START, term_start)))
-    return rc;
   if ((rc = c->bufs[B_TERMS].ensure(sizeof(uint64_t) * std::max<uint64_t>(term_words, 1)))) return rc;
   std::vector<CetDesc> cdesc;
   for (uint32_t i : recount) cdesc.push_back(jdesc[i]);
@@ -1296,34 +1339,30 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   for (uint32_t i : wtab) no_list[i] = 1, wdesc.push_back(jdesc[i]);
   for (size_t i = 0; i < jdesc.size(); ++i)
     if (!no_list[i]) ldesc.push_back(jdesc[i]);
-  auto chunks_before = [](const auto& v) {
-    std::vector<uint32_t> base(1, 0);
-    for (const auto& d : v) base.push_back(base.back() + (d.ncand + 63) / 64);
-    return base;
-  };
-  if ((rc = upload(c, B_LDESC, ldesc)) || (rc = upload(c, B_WDESC, wdesc)) || (rc = upload(c, B_ADESC, adesc)) ||
-      (!wdesc.empty() && (rc = upload(c, B_WCHUNK, chunks_before(wdesc)))) ||
-      (!adesc.empty() && (rc = upload(c, B_ACHUNK, chunks_before(adesc)))) ||
+  if ((rc = upload_parts(c, B_UP_C, {part(B_JDESC, jdesc), part(B_PLANS, plans), part(B_TERM_DESC, term_desc),
+                                     part(B_TERM_START, term_start), part(B_LDESC, ldesc),
+                                     part(B_LCHUNK, chunks_before(ldesc)), part(B_CDESC, cdesc),
+                                     part(B_CCHUNK, chunks_before(cdesc)), part(B_WDESC, wdesc),
+                                     part(B_WCHUNK, chunks_before(wdesc)), part(B_ADESC, adesc),
+                                     part(B_ACHUNK, chunks_before(adesc))})) ||
       (rc = c->bufs[B_AGGS].ensure(sizeof(CetAgg) * std::max<uint64_t>(agg_words, 1))))
     return rc;
   if (off_words > off_capacity) return GPSM_EINVAL;  // cannot happen: rev_bound covers every reversed table
-  if ((rc = upload(c, B_CDESC, cdesc)) ||
-      (rc = c->bufs[B_LISTS].ensure(sizeof(uint32_t) * std::max<uint64_t>(list_words, 1))) ||
-      (rc = c->bufs[B_CHUNKS].ensure(sizeof(uint32_t) * (jdesc.size() + 2))))
-    return rc;
+  if ((rc = c->bufs[B_LISTS].ensure(sizeof(uint32_t) * std::max<uint64_t>(list_words, 1)))) return rc;
   const uint32_t nplans = (uint32_t)plans.size();
-  if ((rc = c->bufs[B_JOUT].ensure(sizeof(JoinOut) * std::max<uint32_t>(nplans, 1))) ||
+  const uint64_t jout_words = sizeof(JoinOut) / 4 * (uint64_t)std::max<uint32_t>(nplans, 1);
+  if ((rc = c->bufs[B_JOUT].ensure(sizeof(uint32_t) * (jout_words + kCtrWords))) ||
       (rc = c->h_stage[2].ensure(sizeof(JoinOut) * std::max<uint32_t>(nplans, 1))))
     return rc;
-  if ((rc = c->bufs[B_CTR].ensure(4 * kCtrWords))) return rc;
+  uint32_t* ctr = dptr<uint32_t>(c, B_JOUT) + jout_words;
   if (emit_cap && (rc = c->bufs[B_EMIT].ensure(sizeof(uint32_t) * emit_cap * qmax))) return rc;
   PhaseSig sig_c;
   if (o.use_graph) {
     sig_c.add(uint64_t{1});
     sig_c.add_graph(dg);
-    for (int i : {B_BITMAPS, B_CLIST, B_CDESC, B_OFFSETS, B_CHUNKS, B_JDESC, B_LISTS, B_TERM_DESC, B_TERM_START,
-                  B_TERMS, B_JOUT, B_CTR, B_LDESC, B_WDESC, B_WCHUNK, B_ADESC, B_ACHUNK, B_AGGS, B_BPREFIX})
-      sig_c.add(c->bufs[i].ptr);
+    for (int i : {B_BITMAPS, B_CLIST, B_CDESC, B_OFFSETS, B_CCHUNK, B_JDESC, B_LISTS, B_TERM_DESC, B_TERM_START,
+                  B_TERMS, B_JOUT, B_LDESC, B_LCHUNK, B_WDESC, B_WCHUNK, B_ADESC, B_ACHUNK, B_AGGS, B_BPREFIX})
+      sig_c.add(dptr<uint32_t>(c, i));
     for (uint64_t v : {(uint64_t)cdesc.size(), (uint64_t)cgrid, (uint64_t)jdesc.size(), (uint64_t)term_desc.size(),
                        (uint64_t)term_words, (uint64_t)nplans, (uint64_t)ldesc.size(), (uint64_t)wdesc.size(),
                        (uint64_t)adesc.size()})
@@ -1337,13 +1376,13 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     hipEvent_t pa = pbegin(K_CET_COUNT);
     if (!cdesc.empty())
       launch_cet_count(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_CDESC), (uint32_t)cdesc.size(),
-                       dptr<uint32_t>(c, B_OFFSETS), 1, dptr<uint32_t>(c, B_CHUNKS), cgrid, s,
+                       dptr<uint32_t>(c, B_OFFSETS), 1, dptr<uint32_t>(c, B_CCHUNK), cgrid, s,
                        counters ? fstats + fstat_step * slot_cet_c : nullptr);
     pend(K_CET_COUNT, pa, 0.0, counters ? slot_cet_c : -1);
     launch_cet_offsets(dptr<CetDesc>(c, B_LDESC), (uint32_t)ldesc.size(), dptr<uint32_t>(c, B_OFFSETS), s);
     pa = pbegin(K_CET_WRITE);
     launch_cet_write(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_LDESC), (uint32_t)ldesc.size(),
-                     dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_LISTS), dptr<uint32_t>(c, B_CHUNKS), cgrid, s,
+                     dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_LISTS), dptr<uint32_t>(c, B_LCHUNK), cgrid, s,
                      counters ? fstats + fstat_step * slot_cet_w : nullptr);
     launch_cet_sums(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_WDESC), (uint32_t)wdesc.size(),
                     dptr<uint32_t>(c, B_WCHUNK), dptr<CetAgg>(c, B_AGGS), cgrid, s,
@@ -1355,8 +1394,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
                      dptr<uint64_t>(c, B_TERM_START), (uint32_t)term_desc.size(), term_words,
                      dptr<unsigned long long>(c, B_TERMS), s);
     pend(K_CET_WRITE, pa, 0.0, counters ? slot_cet_w : -1);
-    launch_fill_u32(dptr<uint32_t>(c, B_JOUT), 0u, sizeof(JoinOut) / 4 * (uint64_t)std::max<uint32_t>(nplans, 1), s);
-    launch_fill_u32(dptr<uint32_t>(c, B_CTR), 0u, kCtrWords, s);
+    launch_fill_u32(dptr<uint32_t>(c, B_JOUT), 0u, jout_words + kCtrWords, s);
     if (captured && (rc = launch_captured(c, 1, s, sig_c.w))) return rc;
   }
   // ---------------- phase D: join ----------------
@@ -1384,7 +1422,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     ja.out = dptr<JoinOut>(c, B_JOUT);
     if (emit_cap) {
       ja.emit = dptr<uint32_t>(c, B_EMIT);
-      ja.emit_ctr = reinterpret_cast<unsigned long long*>(dptr<uint32_t>(c, B_CTR) + 16);
+      ja.emit_ctr = reinterpret_cast<unsigned long long*>(ctr + 16);
       ja.emit_cap = emit_cap;
     }
     ja.budget = o.work_budget;
@@ -1429,7 +1467,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
         JoinArgs jl = ja;
         jl.tasks = dptr<JoinTask>(c, B_TASKS) + task0[i];
         jl.ntasks = (uint32_t)ltasks[i].size();
-        jl.task_counter = dptr<unsigned int>(c, B_CTR) + i;
+        jl.task_counter = ctr + i;
         jl.levels = dptr<uint32_t>(c, B_LEVELS) + lw * level0;
         level0 += lwg[i];
         if (i == 2 && fork) {
@@ -1450,7 +1488,6 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     // levels the host reads which of them stopped at a full buffer; the
     // deepest one goes on first, into buffers emptied by then.
     auto breadth_first = [&]() -> int {
-      uint32_t* ctr = dptr<uint32_t>(c, B_CTR);
       for (size_t q0 = 0, q1; q0 < bfs_q.size(); q0 = q1) {
         uint64_t first_rows = 0;
         for (q1 = q0; q1 < bfs_q.size() && q1 < q0 + BFS_PLANS; ++q1) {
@@ -1565,7 +1602,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     }
     unsigned long long emitted = 0;
     if (emit_cap)
-      HIPCHK(hipMemcpyAsync(&emitted, dptr<uint32_t>(c, B_CTR) + 16, sizeof(emitted), hipMemcpyDeviceToHost, s));
+      HIPCHK(hipMemcpyAsync(&emitted, ctr + 16, sizeof(emitted), hipMemcpyDeviceToHost, s));
     HIPCHK(hipMemcpyAsync(c->h_stage[2].ptr, dptr<JoinOut>(c, B_JOUT), sizeof(JoinOut) * nplans,
                           hipMemcpyDeviceToHost, s));
     hipEventRecord(c->ev1, s);

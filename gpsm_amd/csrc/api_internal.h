@@ -66,8 +66,7 @@ enum BufId {
   B_LISTS,
   B_PLANS,
   B_TASKS,
-  B_JOUT,
-  B_CTR,
+  B_JOUT,        // the plans' results, then the join's counters
   B_LEVELS,
   B_EMIT,
   B_EMIT_SORT,   // sorting the emitted tuples: scratch, then the sorted rows
@@ -82,10 +81,14 @@ enum BufId {
   B_TEXT_WG,     // ... scan scratch, per-workgroup lengths and offsets
   B_TEXT_OUT,    // ... the chunk's text
   B_FITEMS,      // filter superstep: (op, vertex range) pairs with candidates
-  B_FNITEMS,     // ... their number, one counter per superstep, then the explore ops' candidate counts
+  B_FNITEMS,     // ... their number, one counter per superstep, then the explore ops' candidate counts, then the
+                 // refine rounds that removed a candidate, 4 per query
   B_FILLS,       // explore ops' neighbours (FillOp)
+  B_FCHUNK,      // chunks of 64 candidates before each forward table
   B_CDESC,       // candidate-edge tables of reversed plan edges (counted again)
+  B_CCHUNK,      // ... chunks before each
   B_LDESC,       // candidate-edge tables whose lists are written
+  B_LCHUNK,      // ... chunks before each
   B_WDESC,       // last levels' tables counted from records
   B_WCHUNK,      // ... chunks of 64 candidates before each
   B_ADESC,       // tables of the level before (AggDesc)
@@ -95,7 +98,9 @@ enum BufId {
   B_BFIRST,      // ... first-table rows before each
   B_BROWS,       // ... rows of their levels
   B_BCURS,       // ... where each wave of a level stands
-  B_RFLAGS,      // refine rounds that removed a candidate, 4 per query
+  B_UP_A,        // uploads of the filter, of the candidate-edge counts, of tables and plans: one copy each
+  B_UP_B,
+  B_UP_C,
   B_COUNT_
 };
 
@@ -186,6 +191,7 @@ struct gpsm_ctx {
   gpsm::Stager stager;   // large copies from and to ordinary host memory
   gpsm::BlockPool pool;  // memory of this context's graphs
   gpsm::DevBuf bufs[gpsm::B_COUNT_];
+  void* part[gpsm::B_COUNT_] = {};  // where a batch's packed uploads are (parts of B_UP_*)
   gpsm_ctx() {
     for (auto& b : bufs) b.pool = &pool;
   }

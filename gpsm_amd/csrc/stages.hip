@@ -75,12 +75,16 @@ int cet_hook(void* user, gpsm_ctx* c, const CetDesc* fdesc, uint32_t nf) {
     co->rc = GPSM_EOVERFLOW;
     return STOP;
   }
-  for (auto& x : d) x.total = 0;
+  std::vector<uint32_t> chunks(1, 0);
+  for (auto& x : d) {
+    x.total = 0;
+    chunks.push_back(chunks.back() + (x.ncand + 63) / 64);
+  }
   hipStream_t s = c->stream;
   if (c->bufs[B_JDESC].ensure(sizeof(CetDesc) * std::max<uint32_t>(nf, 1)) ||
       c->bufs[B_OFFSETS].ensure(sizeof(uint32_t) * std::max<uint64_t>(offw, 1)) ||
       c->bufs[B_LISTS].ensure(sizeof(uint32_t) * std::max<uint64_t>(listw, 1)) ||
-      c->bufs[B_CHUNKS].ensure(sizeof(uint32_t) * (nf + 2))) {
+      c->bufs[B_CHUNKS].ensure(sizeof(uint32_t) * chunks.size())) {
     co->rc = GPSM_ENOMEM;
     return STOP;
   }
@@ -91,11 +95,12 @@ int cet_hook(void* user, gpsm_ctx* c, const CetDesc* fdesc, uint32_t nf) {
   const uint32_t* bitmaps = reinterpret_cast<const uint32_t*>(c->bufs[B_BITMAPS].ptr);
   const DevGraph& dg = co->g->dg;
   const uint32_t grid = std::max<uint32_t>(c->ncu * 8, 64);
+  uint32_t* dchunks = reinterpret_cast<uint32_t*>(c->bufs[B_CHUNKS].ptr);
   hipMemcpyAsync(dd, d.data(), sizeof(CetDesc) * nf, hipMemcpyHostToDevice, s);
-  launch_cet_count(dg, bitmaps, clist, dd, nf, offs, 1, reinterpret_cast<uint32_t*>(c->bufs[B_CHUNKS].ptr), grid, s);
+  hipMemcpyAsync(dchunks, chunks.data(), sizeof(uint32_t) * chunks.size(), hipMemcpyHostToDevice, s);
+  launch_cet_count(dg, bitmaps, clist, dd, nf, offs, 1, dchunks, grid, s);
   launch_cet_offsets(dd, nf, offs, s);
-  launch_cet_write(dg, bitmaps, clist, dd, nf, offs, lists, reinterpret_cast<uint32_t*>(c->bufs[B_CHUNKS].ptr), grid,
-                   s);
+  launch_cet_write(dg, bitmaps, clist, dd, nf, offs, lists, dchunks, grid, s);
   uint64_t cmax = 0;
   for (auto& x : d) cmax = std::max<uint64_t>(cmax, x.clist_off + x.ncand);
   if (dg.row != dg.row0) {
