@@ -21,6 +21,7 @@ N_PARAMS = HIDDEN * FEAT + HIDDEN + HIDDEN * HIDDEN + HIDDEN + HIDDEN + 1
 ORDER_HEURISTIC, ORDER_LEARNED, ORDER_EXPLICIT = 0, 1, 2
 Q_WALK_TREE, Q_WALK_INDUCED, Q_WALK_HALF, Q_CYCLE, Q_CLIQUE = 0, 1, 2, 3, 4
 
+EOVERFLOW = -5
 ERRORS = {
     0: "ok", -1: "invalid argument", -2: "out of memory", -3: "HIP runtime error", -4: "query too large",
     -5: "tuple capacity exceeded", -6: "no HIP device", -7: "query disconnected or without edges",

@@ -350,14 +350,18 @@ class ResidentGraph:
         ef = np.zeros(E, dtype=np.uint32)
         et = np.zeros(E, dtype=np.uint32)
         size = np.zeros(E, dtype=np.uint32)
-        check(_lib.lib().gpsm_candidate_edges(self.ctx.h, self.h, C.byref(qs), ptr(ef), ptr(et), ptr(size), None, 0,
-                                              None), "gpsm_candidate_edges")
-        m = [int(cand[ef[e]]) for e in range(E)]
-        cap_words = sum(2 * m[e] + 1 + int(size[e]) for e in range(E))
-        buf = np.zeros(max(cap_words, 1), dtype=np.uint32)
+        # the tables' size is known after a pass: most fit the first buffer
+        cap_words = 1 << 20
         toff = np.zeros(max(E, 1), dtype=np.uint64)
-        check(_lib.lib().gpsm_candidate_edges(self.ctx.h, self.h, C.byref(qs), ptr(ef), ptr(et), ptr(size),
-                                              ptr(buf), cap_words, ptr(toff)), "gpsm_candidate_edges")
+        for _ in range(2):
+            buf = np.zeros(max(cap_words, 1), dtype=np.uint32)
+            rc = _lib.lib().gpsm_candidate_edges(self.ctx.h, self.h, C.byref(qs), ptr(ef), ptr(et), ptr(size),
+                                                 ptr(buf), cap_words, ptr(toff))
+            m = [int(cand[ef[e]]) for e in range(E)]
+            cap_words = sum(2 * m[e] + 1 + int(size[e]) for e in range(E))
+            if rc != _lib.EOVERFLOW:
+                break
+        check(rc, "gpsm_candidate_edges")
         out = []
         for e in range(E):
             t = buf[int(toff[e]):]
