@@ -357,7 +357,6 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   st.n = n;
   st.adj = d.adj;
   d.W = words_of(n);
-  d.NB = nblocks_of(n);
   // scratch: what the host reads (row check, number of ranges, label and hub
   // counts), the labels, the ranges' ends
   // (the counts' words later take the labels' values, starts and ranges)
@@ -738,7 +737,7 @@ struct PhaseSig {
   void add(uint64_t v) { w.push_back(v); }
   void add(const void* p) { w.push_back((uint64_t)(uintptr_t)p); }
   void add_graph(const DevGraph& g) {
-    add(g.n), add(g.adj), add(g.W), add(g.NB), add(g.ids), add(g.row), add(g.lrow), add(g.ngroup), add(g.gshift), add(g.col), add(g.key), add(g.ckey), add(g.fchunk),
+    add(g.n), add(g.adj), add(g.W), add(g.ids), add(g.row), add(g.lrow), add(g.ngroup), add(g.gshift), add(g.col), add(g.key), add(g.ckey), add(g.fchunk),
         add(g.nfchunk), add(g.wrange), add(g.hparts), add(g.nhparts), add(g.hub_of), add(g.hub_bits), add(g.nhub), add(g.hub_degree);
   }
 };
@@ -836,7 +835,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     maxsteps = std::max<uint32_t>(maxsteps, (uint32_t)S.fs.steps.size());
     qmax = std::max(qmax, S.hq.n);
   }
-  const uint32_t W = dg.W, NB = dg.NB;
+  const uint32_t W = dg.W;
   int rc;
   // per-launch timing (not inside captured graphs)
   const bool prof = c->prof.mode > 0 && !o.use_graph;
@@ -1020,7 +1019,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   std::vector<uint64_t> coff(std::max<uint32_t>(nslots, 1) + 1, 0);
   for (uint32_t r = 0; r < nslots; ++r) coff[r + 1] = coff[r] + counts[r];
   if ((rc = c->bufs[B_CLIST].ensure(sizeof(uint32_t) * std::max<uint64_t>(coff[nslots], 1)))) return rc;
-  if ((rc = c->bufs[B_BPREFIX].ensure(sizeof(uint32_t) * (size_t)std::max<uint32_t>(nslots, 1) * NB))) return rc;
+  if ((rc = c->bufs[B_BPREFIX].ensure(sizeof(uint32_t) * (size_t)std::max<uint32_t>(nslots, 1) * W))) return rc;
   std::vector<CetDesc> fdesc;
   std::vector<uint32_t> fdesc_of_q(nq, 0);
   for (uint32_t b = 0; b < nq; ++b) {
@@ -1055,7 +1054,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     hipEvent_t a = pbegin(K_COMPACT);
     launch_compact_rows(dg, bitmaps, nslots, dptr<uint32_t>(c, B_SEGC), dptr<uint64_t>(c, B_COFF),
                         dptr<uint32_t>(c, B_CLIST), dptr<uint32_t>(c, B_BPREFIX), s);
-    pend(K_COMPACT, a, (double)nslots * 4.0 * (W + NB) + 4.0 * coff[nslots], -1);
+    pend(K_COMPACT, a, (double)nslots * 8.0 * W + 4.0 * coff[nslots], -1);
   }
   if ((rc = c->bufs[B_OFFSETS].ensure(sizeof(uint32_t) * std::max<uint64_t>(fwd_words + rev_bound, 1)))) return rc;
   const uint64_t off_capacity = c->bufs[B_OFFSETS].bytes / sizeof(uint32_t);
@@ -1417,7 +1416,6 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     ja.cets = dptr<CetDesc>(c, B_JDESC);
     ja.plans = dptr<JoinPlan>(c, B_PLANS);
     ja.W = W;
-    ja.NB = NB;
     ja.qmax = qmax;
     ja.out = dptr<JoinOut>(c, B_JOUT);
     if (emit_cap) {

@@ -8,7 +8,7 @@
 // Per batch of queries (one arena, bump-allocated):
 //   bitmaps[slot][W]   candidate set C(u) of every query vertex ("slot" =
 //                      batch-wide vertex index), W = ceil(n/32) words
-//   bprefix[slot][NB]  set bits before each 256-bit block (rank index)
+//   bprefix[slot][W]   set bits before each word (rank index)
 //   clist[coff[slot]]  ascending ids of C(u)
 //   per directed query edge x->w used by a join: off[|C(x)|+1] and
 //                      list[|CET|], the candidate-edge table
@@ -21,10 +21,8 @@ constexpr uint32_t KEY_DEG_BITS = 20;
 constexpr uint32_t KEY_DEG_MASK = (1u << KEY_DEG_BITS) - 1;
 constexpr uint32_t MAX_LABELS = (1u << (32 - KEY_DEG_BITS)) - 1;
 constexpr uint32_t MAXQ = 64;
-constexpr uint32_t BLOCK_BITS = 256;  // rank-index block
 
 inline uint32_t words_of(uint32_t n) { return (n + 31) / 32; }
-inline uint32_t nblocks_of(uint32_t n) { return (words_of(n) + 7) / 8 + 1; }
 
 // A data graph's rows in pieces by the neighbours' label (DevGraph::lrow).
 struct Pieces {

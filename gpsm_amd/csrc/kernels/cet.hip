@@ -377,7 +377,7 @@ struct AggLds {
 
 __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict__ ids,
                                                       const uint32_t* __restrict__ bitmaps,
-                                                      const uint32_t* __restrict__ bprefix, uint32_t W, uint32_t NB,
+                                                      const uint32_t* __restrict__ bprefix, uint32_t W,
                                                       const AggDesc* __restrict__ descs, uint32_t ndesc,
                                                       const uint32_t* __restrict__ chunk_base,
                                                       const uint32_t* __restrict__ offsets,
@@ -403,7 +403,7 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
     L.s[lane] = L.a[lane] = L.b[lane] = 0;
     wave_sync();
     const uint32_t* bm_y = bitmaps + (size_t)d.y_slot * W;
-    const uint32_t* bp_y = bprefix + (size_t)d.y_slot * NB;
+    const uint32_t* bp_y = bprefix + (size_t)d.y_slot * W;
     const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
     const uint32_t* lst = lists + d.list_base;
     for (uint32_t f = 0; f < D; f += WAVE * AGG_UNROLL) {
@@ -522,7 +522,7 @@ void launch_cet_aggs(const DevGraph& g, const uint32_t* bitmaps, const uint32_t*
                      uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
                      CetAgg* aggs, uint32_t grid, hipStream_t s) {
   if (!ndesc) return;
-  hipLaunchKernelGGL(cet_agg_kernel, dim3(grid), dim3(256), 0, s, g.ids, bitmaps, bprefix, g.W, g.NB, descs, ndesc,
+  hipLaunchKernelGGL(cet_agg_kernel, dim3(grid), dim3(256), 0, s, g.ids, bitmaps, bprefix, g.W, descs, ndesc,
                      chunk_base, offsets, lists, aggs);
 }
 

@@ -11,7 +11,7 @@
 //    (k+1 bound vertices) with one bounded column-major buffer per level, so
 //    memory is O(cap * q^2) per workgroup whatever the result size;
 //  * a row's candidate list is found in O(1) through the rank index of C(x)
-//    (set bits before each 256-bit block + popcounts);
+//    (set bits before each word + a popcount);
 //  * a window of 256 rows is expanded flattened: 256 threads take 256
 //    consecutive (row, candidate) pairs, so rows of any fan-out share lanes;
 //  * join-mode edges become edge-membership checks (binary search in the
@@ -151,7 +151,7 @@ __device__ __forceinline__ void flush_agg_work(const JoinArgs& a, const JoinPlan
 }
 
 __device__ __forceinline__ CetAgg agg_of(const JoinArgs& a, const CetDesc& d, uint32_t x) {
-  return a.aggs[d.agg_base + rank_of(a.bitmaps + (size_t)d.x_slot * a.W, a.bprefix + (size_t)d.x_slot * a.NB, x)];
+  return a.aggs[d.agg_base + rank_of(a.bitmaps + (size_t)d.x_slot * a.W, a.bprefix + (size_t)d.x_slot * a.W, x)];
 }
 
 // Whether u is in the candidate-edge list of mu in table d: u in C(w) and
@@ -179,7 +179,7 @@ __device__ __forceinline__ void count_last_level(const JoinArgs& a, const JoinPl
   const uint32_t qid = P.order[w];
   const uint32_t mu = val[P.par[w] * WROWS + tid];
   const CetAgg r = agg_of(a, d, mu);
-  if (BYTES) bytes += 4 + 4 * (((mu >> 5) & 7) + 1) + sizeof(CetAgg);
+  if (BYTES) bytes += 4 + 4 + sizeof(CetAgg);
   unsigned long long len = r.len, s = r.s;
   for (uint64_t m = P.inj[w]; m; m &= m - 1) {
     const uint32_t u = val[(uint32_t)(__ffsll((long long)m) - 1) * WROWS + tid];
@@ -222,7 +222,7 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
   if (tid < nw) {
     mu = val[py * WROWS + tid];
     const CetAgg r = agg_of(a, dy, mu);
-    if (BYTES) bytes += 4 + 4 * (((mu >> 5) & 7) + 1) + sizeof(CetAgg);
+    if (BYTES) bytes += 4 + 4 + sizeof(CetAgg);
     st_y = r.off;
     len_y = r.len;
     unsigned long long n = r.len, ty = r.s, ra = r.a, rb = r.b;
@@ -234,7 +234,7 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
       ty -= t;
       if (chain) {
         const CetAgg x = agg_of(a, dw, u);
-        if (BYTES) bytes += 4 + 4 * (((u >> 5) & 7) + 1) + sizeof(CetAgg);
+        if (BYTES) bytes += 4 + 4 + sizeof(CetAgg);
         ra -= x.len;
         rb -= t * x.s;
       } else if (sibling && bit_of(bm_w, u)) {
@@ -254,7 +254,7 @@ __device__ __forceinline__ void count_last_two(const JoinArgs& a, const JoinPlan
     } else {
       const uint32_t mw = val[pw * WROWS + tid];
       const CetAgg x = agg_of(a, dw, mw);
-      if (BYTES) bytes += 4 + 4 * (((mw >> 5) & 7) + 1) + sizeof(CetAgg);
+      if (BYTES) bytes += 4 + 4 + sizeof(CetAgg);
       aw.work_w += n * x.len;
       unsigned long long lw = x.len, sw = x.s;
       for (uint64_t m = iw & ~(1ull << y); m; m &= m - 1) {
@@ -444,7 +444,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
         const uint32_t p = P.par[nk];
         const CetDesc dn = a.cets[P.cet[nk]];
         const uint32_t* bm_x = a.bitmaps + (size_t)dn.x_slot * a.W;
-        const uint32_t* bp_x = a.bprefix + (size_t)dn.x_slot * a.NB;
+        const uint32_t* bp_x = a.bprefix + (size_t)dn.x_slot * a.W;
         const uint32_t* offn = a.offsets + dn.off_base;
         const uint32_t bo = P.back_off[nk], be = CYCLIC ? P.back_off[nk + 1] : bo;  // a tree plan has none
         const uint64_t inj = P.inj[nk];
@@ -489,7 +489,7 @@ __device__ __forceinline__ void join_body(const JoinArgs& a) {
         }
         if (tid < nw) {
           // row values, rank index (prefix + words) and the offset pair
-          if (BYTES) my_bytes += (k == 1 ? 8 : 4 * (k + 1)) + 4 + 4 * (((val[p * WROWS + tid] >> 5) & 7) + 1) + 8;
+          if (BYTES) my_bytes += (k == 1 ? 8 : 4 * (k + 1)) + 4 + 4 + 8;
           const uint32_t j = rank_of(bm_x, bp_x, val[p * WROWS + tid]);
           st = offn[j];
           ub = offn[j + 1] - st;

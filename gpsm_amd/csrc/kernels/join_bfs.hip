@@ -145,7 +145,7 @@ __device__ __forceinline__ bool finish_rows(const BfsArgs& a, const PlanLevel* p
   const uint32_t bound = val(min(pp, k));
   if (has) {
     const uint32_t x = pp == k + 1 ? mv : bound;
-    const uint32_t j = rank_of(a.j.bitmaps + (size_t)p.x_slot * a.j.W, a.j.bprefix + (size_t)p.x_slot * a.j.NB, x);
+    const uint32_t j = rank_of(a.j.bitmaps + (size_t)p.x_slot * a.j.W, a.j.bprefix + (size_t)p.x_slot * a.j.W, x);
     const uint32_t* off = a.j.offsets + p.off;
     st = off[j];
     full = off[j + 1] - st;

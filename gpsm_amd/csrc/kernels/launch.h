@@ -13,7 +13,6 @@ struct DevGraph {
   uint32_t n = 0;
   uint64_t adj = 0;
   uint32_t W = 0;   // bitmap words per query vertex
-  uint32_t NB = 0;  // rank-index entries per query vertex
   // The vertices are numbered by (label, id) on the device, so that a
   // candidate set, all of one label, is one dense piece of every bitmap and of
   // every hub's: ids[i] is the id of vertex i, pos its inverse.  row / col and
@@ -272,7 +271,7 @@ struct JoinArgs {
   const JoinPlan* plans;
   const JoinTask* tasks;
   uint32_t ntasks;
-  uint32_t W, NB;
+  uint32_t W;
   uint32_t cap;       // rows per level buffer
   uint32_t qmax;      // widest query of the batch
   uint32_t* levels;   // per workgroup: (qmax-2) buffers of cap rows, column-major

@@ -13,8 +13,7 @@
 // and compacts the four one after the other (each
 // thread owns eight consecutive words, one block scan places them), ids
 // staged in LDS and written back coalesced.  The same pass writes the rank
-// index (set bits before each 256-bit block, row-relative) the join uses to
-// find a vertex's candidate-edge list.
+// index (set bits before each word, row-relative) the join uses to find a vertex's candidate-edge list.
 #include <algorithm>
 
 #include "launch.h"
@@ -114,8 +113,8 @@ __global__ void __launch_bounds__(256) seg_offsets_kernel(uint32_t* __restrict__
 // after the other: thread t holds the words j * 256 + t of a segment (eight
 // loads in flight, and the next segment's eight issued before the current
 // one is scanned); a wave scan per row j of its words' popcounts and one
-// scan of the (row, wave) totals give every word its output position, the
-// first word of each 256-bit block writes its rank-index entry, and the ids
+// scan of the (row, wave) totals give every word its output position,
+// which is its rank-index entry, and the ids
 // go through LDS (in rounds of STAGE_IDS output positions when the segment
 // holds more) and are written back coalesced.  The row's set bits before
 // the group come from the segment popcounts; within the group the
@@ -147,7 +146,7 @@ __device__ __forceinline__ void load_words(const uint32_t* __restrict__ bm, uint
 }
 
 __global__ void __launch_bounds__(256) compact_rows_kernel(const uint32_t* __restrict__ bitmaps, uint32_t W,
-                                                           uint32_t NB, uint32_t nseg,
+                                                           uint32_t nseg,
                                                            const uint32_t* __restrict__ segc,
                                                            const uint64_t* __restrict__ coff,
                                                            uint32_t* __restrict__ clist,
@@ -160,7 +159,7 @@ __global__ void __launch_bounds__(256) compact_rows_kernel(const uint32_t* __res
   const uint32_t r = blockIdx.x / ngrp, sg0 = (blockIdx.x % ngrp) * COMPACT_GROUP;
   const uint32_t sg1 = min(nseg, sg0 + COMPACT_GROUP);
   const uint32_t* bm = bitmaps + (size_t)r * W;
-  uint32_t* bp = bprefix + (size_t)r * NB;
+  uint32_t* bp = bprefix + (size_t)r * W;
   uint32_t* out = clist + coff[r];
   if (threadIdx.x == 0) rel = segc[(size_t)r * nseg + sg0];  // set bits of the row's segments before the group
   uint32_t w[CW];
@@ -192,7 +191,7 @@ __global__ void __launch_bounds__(256) compact_rows_kernel(const uint32_t* __res
     for (uint32_t j = 0; j < CW; ++j) {
       pos[j] += wt[j * 4 + wv];
       const uint32_t wi = s0 + j * 256 + threadIdx.x;
-      if ((threadIdx.x & 7) == 0 && wi < W) bp[wi >> 3] = carry + pos[j];  // first word of its 256-bit block
+      if (bprefix && wi < W) bp[wi] = carry + pos[j];
     }
     // ids through LDS, in rounds of STAGE_IDS output positions when the
     // segment holds more, written back coalesced
@@ -216,7 +215,6 @@ __global__ void __launch_bounds__(256) compact_rows_kernel(const uint32_t* __res
     // every thread has read wt (and stage): the last round ends with a
     // barrier, and a segment without set bits has none
     if (total == 0) __syncthreads();
-    if (sg == nseg - 1 && threadIdx.x == 0) bp[NB - 1] = carry + total;
     if (threadIdx.x == 0) rel = carry + total;  // read after the next segment's first barrier
 #pragma unroll
     for (uint32_t j = 0; j < CW; ++j) w[j] = nx[j];
@@ -382,7 +380,7 @@ void launch_compact_rows(const DevGraph& g, const uint32_t* bitmaps, uint32_t nr
   if (!nrows) return;
   const uint32_t nseg = segs_of(g.W);
   const uint32_t ngrp = (nseg + COMPACT_GROUP - 1) / COMPACT_GROUP;
-  hipLaunchKernelGGL(compact_rows_kernel, dim3(nrows * ngrp), dim3(256), 0, s, bitmaps, g.W, g.NB, nseg, segc, coff,
+  hipLaunchKernelGGL(compact_rows_kernel, dim3(nrows * ngrp), dim3(256), 0, s, bitmaps, g.W, nseg, segc, coff,
                      clist, bprefix);
 }
 
@@ -416,26 +414,23 @@ void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint64_t n, unsign
 
 uint64_t compact_scratch_words(uint64_t nbits) {
   const uint64_t W = (nbits + 31) / 32;
-  return 2 + ((W + 7) / 8 + 1) + segs_of((uint32_t)W) + 1;
+  return 2 + segs_of((uint32_t)W) + 1;
 }
 
 void launch_compact_bitmap(const uint32_t* bits, uint64_t nbits, uint32_t* ids, unsigned long long* count,
                            uint32_t* scratch, hipStream_t s) {
   // one row of ceil(nbits/32) words through the row compaction; scratch
-  // holds the row offset (2 words), the rank index, the segment counts and
-  // the row count
+  // holds the row offset (2 words), the segment counts and the row count
   DevGraph g;
   g.W = (uint32_t)((nbits + 31) / 32);
-  g.NB = (g.W + 7) / 8 + 1;
   uint64_t* coff = reinterpret_cast<uint64_t*>(scratch);
-  uint32_t* bp = scratch + 2;
-  uint32_t* segc = bp + g.NB;
+  uint32_t* segc = scratch + 2;
   uint32_t* rowc = segc + segs_of(g.W);
   hipMemsetAsync(coff, 0, sizeof(uint64_t), s);
   launch_row_popcount(g, bits, 1, segc, rowc, s);
-  launch_compact_rows(g, bits, 1, segc, coff, ids, bp, s);
+  launch_compact_rows(g, bits, 1, segc, coff, ids, nullptr, s);
   hipMemsetAsync(count, 0, sizeof(unsigned long long), s);
-  hipMemcpyAsync(count, bp + g.NB - 1, sizeof(uint32_t), hipMemcpyDeviceToDevice, s);
+  hipMemcpyAsync(count, rowc, sizeof(uint32_t), hipMemcpyDeviceToDevice, s);
 }
 
 }  // namespace gpsm

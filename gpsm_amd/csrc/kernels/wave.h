@@ -70,14 +70,11 @@ __device__ __forceinline__ unsigned long long wave_sum64(unsigned long long x) {
 __device__ __forceinline__ uint32_t bit_of(const uint32_t* bm, uint32_t v) { return (bm[v >> 5] >> (v & 31)) & 1u; }
 
 // Position of x among the set bits of a bitmap (x's own bit not counted): the
-// rank index's count before its 256-bit block plus the block's words up to it.
+// rank index's count before its word plus the word's bits below it.  With an
+// entry per 256 bits up to seven words more were read, one after the other.
 __device__ __forceinline__ uint32_t rank_of(const uint32_t* __restrict__ bm, const uint32_t* __restrict__ bp,
                                             uint32_t x) {
-  const uint32_t blk = x >> 8;
-  uint32_t r = bp[blk];
-  const uint32_t w0 = blk * 8, wx = x >> 5;
-  for (uint32_t w = w0; w < wx; ++w) r += __popc(bm[w]);
-  return r + __popc(bm[wx] & ((1u << (x & 31)) - 1u));
+  return bp[x >> 5] + __popc(bm[x >> 5] & ((1u << (x & 31)) - 1u));
 }
 
 // Sets bit v, reading first so that already-set bits cost no atomic.
