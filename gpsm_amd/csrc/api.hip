@@ -263,6 +263,7 @@ void gpsm_shutdown(gpsm_ctx* c) {
     if (e) hipGraphExecDestroy(e);
   for (auto& b : c->bufs) b.release();
   for (auto& b : c->h_stage) b.release();
+  for (auto& b : c->h_net) b.release();
   c->arena.release();
   c->stager.release();
   c->pool.release();

@@ -201,6 +201,8 @@ struct gpsm_ctx {
   // pinned readbacks of a batch: counts, |CET| descriptors, join results, join
   // flag, few sorted tuples
   gpsm::HostBuf h_stage[5];
+  // ... inputs and outputs of a network call (each waits for its own)
+  gpsm::HostBuf h_net[2];
   gpsm::PinnedArena arena;   // pinned sources of a batch's uploads
   // Instantiated hipGraphs of a batch's two captured phases (filter;
   // candidate-edge tables), kept across batches: a batch whose launches

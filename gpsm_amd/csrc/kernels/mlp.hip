@@ -312,7 +312,6 @@ struct gpsm_mlp {
   float* norm = nullptr;  // mu[F], inv_sd[F]
   DevBuf x, y;  // x: features, then (gradients) targets
   DevBuf act;  // the weight-gradient GEMMs' operands (mlp_grad_kernel)
-  HostBuf hx, hy;  // pinned staging of inputs and outputs
   int step = 0;
 };
 
@@ -339,10 +338,10 @@ int stage(gpsm_mlp* mm, const float* x, const float* t, uint32_t B) {
     return mm->ctx->stager.to_device(d, x, xb, s) == hipSuccess && mm->ctx->stager.to_device(d + xb, t, tb, s) == hipSuccess
                ? GPSM_OK
                : GPSM_EDEVICE;
-  if (mm->hx.ensure(xb + tb)) return GPSM_ENOMEM;
-  std::memcpy(mm->hx.ptr, x, xb);
-  std::memcpy(static_cast<char*>(mm->hx.ptr) + xb, t, tb);
-  return hipMemcpyAsync(d, mm->hx.ptr, xb + tb, hipMemcpyHostToDevice, s) == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
+  if (mm->ctx->h_net[0].ensure(xb + tb)) return GPSM_ENOMEM;
+  std::memcpy(mm->ctx->h_net[0].ptr, x, xb);
+  std::memcpy(static_cast<char*>(mm->ctx->h_net[0].ptr) + xb, t, tb);
+  return hipMemcpyAsync(d, mm->ctx->h_net[0].ptr, xb + tb, hipMemcpyHostToDevice, s) == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
 }
 
 int run_grad(gpsm_mlp* mm, uint32_t B) {
@@ -413,8 +412,6 @@ void gpsm_mlp_free(gpsm_mlp* mm) {
   hipFree(mm->w2t);
   hipFree(mm->norm);
   mm->x.release();
-  mm->hx.release();
-  mm->hy.release();
   mm->y.release();
   mm->act.release();
   delete mm;
@@ -448,17 +445,17 @@ int gpsm_mlp_forward(gpsm_mlp* mm, const float* x, uint32_t B, float* y) {
   if (!mm || (B && (!x || !y))) return GPSM_EINVAL;
   if (!B) return GPSM_OK;
   const size_t xb = sizeof(float) * (size_t)B * F, yb = sizeof(float) * B;
-  if (mm->x.ensure(xb) || mm->y.ensure(yb) || mm->hx.ensure(xb) || mm->hy.ensure(yb)) return GPSM_ENOMEM;
+  if (mm->x.ensure(xb) || mm->y.ensure(yb) || mm->ctx->h_net[0].ensure(xb) || mm->ctx->h_net[1].ensure(yb)) return GPSM_ENOMEM;
   hipStream_t s = mm->ctx->stream;
-  std::memcpy(mm->hx.ptr, x, xb);
-  if (hipMemcpyAsync(mm->x.ptr, mm->hx.ptr, xb, hipMemcpyHostToDevice, s) != hipSuccess) return GPSM_EDEVICE;
+  std::memcpy(mm->ctx->h_net[0].ptr, x, xb);
+  if (hipMemcpyAsync(mm->x.ptr, mm->ctx->h_net[0].ptr, xb, hipMemcpyHostToDevice, s) != hipSuccess) return GPSM_EDEVICE;
   hipLaunchKernelGGL(mlp_forward_kernel, dim3((B + 31) / 32), dim3(64), 0, s, weights_of(mm),
                      reinterpret_cast<const float*>(mm->x.ptr), B, reinterpret_cast<float*>(mm->y.ptr));
   if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(mm->hy.ptr, mm->y.ptr, yb, hipMemcpyDeviceToHost, s) != hipSuccess ||
+      hipMemcpyAsync(mm->ctx->h_net[1].ptr, mm->y.ptr, yb, hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return GPSM_EDEVICE;
-  std::memcpy(y, mm->hy.ptr, yb);
+  std::memcpy(y, mm->ctx->h_net[1].ptr, yb);
   return GPSM_OK;
 }
 
@@ -468,9 +465,9 @@ int gpsm_mlp_grad(gpsm_mlp* mm, const float* x, const float* t, uint32_t B, floa
   if (rc) return rc;
   hipStream_t s = mm->ctx->stream;
   if ((rc = run_grad(mm, B))) return rc;
-  if (mm->hy.ensure(sizeof(float) * (NP + 1))) return GPSM_ENOMEM;
-  const float* out = static_cast<const float*>(mm->hy.ptr);
-  if (hipMemcpyAsync(mm->hy.ptr, mm->g, sizeof(float) * (NP + 1), hipMemcpyDeviceToHost, s) != hipSuccess ||
+  if (mm->ctx->h_net[1].ensure(sizeof(float) * (NP + 1))) return GPSM_ENOMEM;
+  const float* out = static_cast<const float*>(mm->ctx->h_net[1].ptr);
+  if (hipMemcpyAsync(mm->ctx->h_net[1].ptr, mm->g, sizeof(float) * (NP + 1), hipMemcpyDeviceToHost, s) != hipSuccess ||
       hipStreamSynchronize(s) != hipSuccess)
     return GPSM_EDEVICE;
   std::memcpy(grad, out, sizeof(float) * NP);
