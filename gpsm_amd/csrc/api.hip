@@ -370,7 +370,7 @@ int finish_graph(gpsm_ctx* c, gpsm_graph* g, const uint32_t* labels, bool check)
   if (c->stager.to_device(dlab, labels, sizeof(uint32_t) * n, s) != hipSuccess)
     return fail(GPSM_EDEVICE);
   const uint32_t min_degree = std::max<uint32_t>(c->hub_min_degree, 1);
-  if (check) launch_check_rows(d.row0, d.col0, n, tmp, s);
+  if (check) launch_check_rows(d.row0, d.col0, n, d.adj, tmp, s);
   launch_vertex_stats(d.row0, dlab, n, min_degree, tmp + 4, tmp + 4 + LABEL_HIST + 1, s);
   uint32_t h[kRead];
   if (hipMemcpyAsync(h, tmp, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||

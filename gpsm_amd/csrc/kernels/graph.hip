@@ -16,24 +16,35 @@ namespace gpsm {
 
 namespace {
 
-// One wave per 64 pieces, flattened over their entries; a hub's entry sets its
-// neighbour's bit.
-__global__ void __launch_bounds__(256) hub_bits_kernel(const uint32_t* __restrict__ lrow, uint64_t npieces, uint32_t n,
+// Calls f(segment, entry) for every entry of segments off[0] .. off[nseg] (off[0]
+// = 0), one wave per ENTRY_BLOCK consecutive entries: its first and last
+// segment by a search in all offsets, an entry's by one between them.  (With a
+// wave per 64 segments the first rows of a graph whose ids descend by degree,
+// a million entries, were one wave's: 8.6 ms of a 1M-vertex graph's upload.)
+constexpr uint32_t ENTRY_BLOCK = 1024;
+
+template <typename F>
+__device__ __forceinline__ void for_entries(const uint32_t* __restrict__ off, uint32_t nseg, F f) {
+  const uint32_t lane = lane_id(), total = off[nseg];
+  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
+  const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / WAVE;
+  for (uint64_t e0 = wave * ENTRY_BLOCK; e0 < total; e0 += nwaves * ENTRY_BLOCK) {
+    const uint32_t e1 = (uint32_t)min((uint64_t)total, e0 + ENTRY_BLOCK);
+    const uint32_t lo = seg_search(off, nseg, (uint32_t)e0);
+    const uint32_t ns = seg_search(off + lo, nseg - lo, e1 - 1) + 1;
+    for (uint32_t e = (uint32_t)e0 + lane; e < e1; e += WAVE) f(lo + seg_search(off + lo, ns, e), e);
+  }
+}
+
+// A hub's entry sets its neighbour's bit.
+__global__ void __launch_bounds__(256) hub_bits_kernel(const uint32_t* __restrict__ lrow, uint32_t npieces, uint32_t n,
                                                        const uint32_t* __restrict__ col,
                                                        const uint32_t* __restrict__ hub_of, uint32_t W,
                                                        uint32_t* __restrict__ bits) {
-  const uint32_t lane = lane_id();
-  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-  const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
-  for (uint64_t p0 = wave * WAVE; p0 < npieces; p0 += nwaves * WAVE) {
-    const uint32_t np = (uint32_t)min((uint64_t)WAVE, npieces - p0);
-    const uint32_t e1 = lrow[p0 + np];
-    for (uint32_t e = lrow[p0] + lane; e < e1; e += WAVE) {
-      const uint32_t h = hub_of[(uint32_t)((p0 + seg_search(lrow + p0, np, e)) % n)];
-      const uint32_t w = col[e];
-      if (h != ~0u) atomicOr(bits + (size_t)h * W + (w >> 5), 1u << (w & 31));
-    }
-  }
+  for_entries(lrow, npieces, [&](uint32_t p, uint32_t e) {
+    const uint32_t h = hub_of[p % n], w = col[e];
+    if (h != ~0u) atomicOr(bits + (size_t)h * W + (w >> 5), 1u << (w & 31));
+  });
 }
 
 // Label statistics and hub counts of a graph, and its rows' order, in one
@@ -70,20 +81,11 @@ __global__ void __launch_bounds__(256) vertex_stats_kernel(const uint32_t* __res
 // *bad |= 1 if a row is not strictly ascending, names a vertex >= n or its own.
 __global__ void check_rows_kernel(const uint32_t* __restrict__ row, const uint32_t* __restrict__ col, uint32_t n,
                                   uint32_t* __restrict__ bad) {
-  // one wave per 64 rows, flattened over their entries by a search in the offsets
-  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-  const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / WAVE;
-  const uint32_t lane = lane_id();
   bool wrong = false;
-  for (uint64_t v0 = wave * WAVE; v0 < n; v0 += nwaves * WAVE) {
-    const uint32_t nv = (uint32_t)min((uint64_t)WAVE, n - v0);
-    const uint32_t e1 = row[v0 + nv];
-    for (uint32_t e = row[v0] + lane; e < e1; e += WAVE) {
-      const uint32_t i = seg_search(row + v0, nv, e);  // the last row starting at or before e: it holds e
-      const uint32_t c = col[e];
-      wrong |= c >= n || c == v0 + i || (e > row[v0 + i] && col[e - 1] >= c);
-    }
-  }
+  for_entries(row, n, [&](uint32_t v, uint32_t e) {
+    const uint32_t c = col[e];
+    wrong |= c >= n || c == v || (e > row[v] && col[e - 1] >= c);
+  });
   if (wrong) atomicOr(bad, 1u);
 }
 
@@ -116,27 +118,19 @@ __global__ void numbering_kernel(const unsigned long long* __restrict__ place, c
 
 // The entries of vertex 0, 1, ... as (label group, vertex, label, neighbour)
 // keys: the vertex and the neighbour in pb bits, the label in lb (0: left
-// out).  One wave per 64 vertices, flattened over their entries.
+// out).
 __global__ void row_entries_kernel(const uint32_t* __restrict__ row0, const uint32_t* __restrict__ col0,
                                    const uint32_t* __restrict__ ids, const uint32_t* __restrict__ pos,
                                    const uint32_t* __restrict__ key, const uint32_t* __restrict__ row, uint32_t n,
                                    uint32_t pb, uint32_t lb, uint32_t gshift,
                                    unsigned long long* __restrict__ entry) {
-  const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
-  const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / WAVE;
-  const uint32_t lane = lane_id();
-  for (uint64_t v0 = wave * WAVE; v0 < n; v0 += nwaves * WAVE) {
-    const uint32_t nv = (uint32_t)min((uint64_t)WAVE, n - v0);
-    const uint32_t e1 = row[v0 + nv];
-    for (uint32_t e = row[v0] + lane; e < e1; e += WAVE) {
-      const uint32_t i = seg_search(row + v0, nv, e);
-      const uint32_t x = pos[col0[row0[ids[v0 + i]] + (e - row[v0 + i])]];
-      const uint32_t l = (key[x] >> KEY_DEG_BITS) - 1;
-      unsigned long long k = ((unsigned long long)(l >> gshift) << pb) | (v0 + i);
-      if (lb) k = (k << lb) | l;
-      entry[e] = (k << pb) | x;
-    }
-  }
+  for_entries(row, n, [&](uint32_t v, uint32_t e) {
+    const uint32_t x = pos[col0[row0[ids[v]] + (e - row[v])]];
+    const uint32_t l = (key[x] >> KEY_DEG_BITS) - 1;
+    unsigned long long k = ((unsigned long long)(l >> gshift) << pb) | v;
+    if (lb) k = (k << lb) | l;
+    entry[e] = (k << pb) | x;
+  });
 }
 
 // lrow[p] for the pieces p = 256 b .. 256 b + 255 of a workgroup, and the end:
@@ -291,6 +285,9 @@ uint32_t grid_for(uint64_t items) {
   return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((items + 255) / 256, 16384));
 }
 
+// Workgroups of 256 threads, a wave per ENTRY_BLOCK entries.
+uint32_t entry_grid(uint64_t adj) { return grid_for((adj + ENTRY_BLOCK - 1) / ENTRY_BLOCK * WAVE); }
+
 // Bits of x.
 uint32_t bits_of(uint32_t x) { return x ? 32 - (uint32_t)__builtin_clz(x) : 0; }
 
@@ -304,8 +301,9 @@ void launch_vertex_stats(const uint32_t* row, const uint32_t* label, uint32_t n,
                      min_degree, hist, hubs);
 }
 
-void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uint32_t* bad, hipStream_t s) {
-  hipLaunchKernelGGL(check_rows_kernel, dim3(grid_for(n)), dim3(256), 0, s, row, col, n, bad);
+void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uint64_t adj, uint32_t* bad,
+                       hipStream_t s) {
+  hipLaunchKernelGGL(check_rows_kernel, dim3(entry_grid(adj)), dim3(256), 0, s, row, col, n, bad);
 }
 
 uint64_t relabel_words(uint32_t n, uint64_t adj) {
@@ -346,7 +344,7 @@ void launch_relabel(const DevGraph& g, const uint32_t* label, const uint32_t* va
   const bool exact = g.gshift == 0;
   uint32_t lb = exact ? 0 : bits_of(nl - 1);
   if (gb + 2 * pb + lb > 64) lb = 0;
-  hipLaunchKernelGGL(row_entries_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.row0, g.col0, g.ids, g.pos, g.key,
+  hipLaunchKernelGGL(row_entries_kernel, dim3(entry_grid(g.adj)), dim3(256), 0, s, g.row0, g.col0, g.ids, g.pos, g.key,
                      g.row, g.n, pb, lb, g.gshift, a);
   for (uint32_t shift = exact ? 2 * pb : lb ? pb : 0; shift < gb + 2 * pb + lb; shift += 8) {
     launch_radix_pass(a, b, nullptr, nullptr, g.adj, shift, hist, hstart, scan, sw, s);
@@ -364,7 +362,8 @@ void choose_pieces(DevGraph& g, uint32_t nl) {
   g.gshift = 0;
   for (;; ++g.gshift) {
     g.ngroup = ((nl - 1) >> g.gshift) + 1;
-    if (g.ngroup == 1 || (g.ngroup <= PIECE_GROUPS && (uint64_t)g.ngroup * g.n <= 4 * g.adj + g.n &&
+    const uint64_t words = (uint64_t)g.ngroup * g.n;
+    if (g.ngroup == 1 || (g.ngroup <= PIECE_GROUPS && words <= 4 * g.adj + g.n && words < 1ull << 32 &&
                           bits_of(g.ngroup - 1) + 2 * bits_of(g.n - 1) <= 64))
       return;
   }
@@ -416,8 +415,8 @@ void launch_hubs(const DevGraph& g, uint32_t* scratch, hipStream_t s) {
   hipLaunchKernelGGL(hub_list_kernel, dim3(grid_for(g.n)), dim3(256), 0, s, g.row, g.n, g.hub_degree, before,
                      g.hub_of);
   const uint64_t np = (uint64_t)g.n * g.ngroup;
-  hipLaunchKernelGGL(hub_bits_kernel, dim3(grid_for(np)), dim3(256), 0, s, g.lrow, np, g.n, g.col, g.hub_of, g.W,
-                     g.hub_bits);
+  hipLaunchKernelGGL(hub_bits_kernel, dim3(entry_grid(g.adj)), dim3(256), 0, s, g.lrow, (uint32_t)np, g.n,
+                     g.col, g.hub_of, g.W, g.hub_bits);
 }
 
 void launch_neighbour_keys(const DevGraph& g, hipStream_t s) {

@@ -78,7 +78,8 @@ void launch_vertex_stats(const uint32_t* row, const uint32_t* label, uint32_t n,
 // Sets *bad (zeroed by the caller) if a row of the CSR (offsets monotone, the
 // last one the length of col) is not strictly ascending, holds its own vertex
 // or one >= n.
-void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uint32_t* bad, hipStream_t s);
+void launch_check_rows(const uint32_t* row, const uint32_t* col, uint32_t n, uint64_t adj, uint32_t* bad,
+                       hipStream_t s);
 // From row0 / col0, the vertices' labels (by id) and the nl distinct label
 // values, ascending: ids, pos, row, col and lrow (unless they are row0 / col0:
 // the vertices then keep their ids) and key.  scratch: relabel_words(n, adj)

@@ -89,3 +89,26 @@ def test_no_edges(ctx):
     q = G.Query(np.array([1, 2], dtype=np.uint32), np.array([0], dtype=np.uint32), np.array([1], dtype=np.uint32))
     assert ctx.upload(g).match(q).count == 0
     assert ctx.upload_edges(300, [], [], np.arange(300) % 5 + 1).match(q).count == 0
+
+
+# 1024 entries a wave: a path's 2 (m - 1) just below, at and above, behind and
+# before vertices without entries, and a star whose hub's fill several waves
+@pytest.mark.parametrize("m", [512, 513, 514, 1025, 1537])
+@pytest.mark.parametrize("gap", [0, 70])
+def test_entry_blocks(ctx, m, gap):
+    n = m + 2 * gap
+    lab = np.arange(n) % 3 + 1
+    v = np.arange(gap, gap + m)
+    for src, dst in ((v[:-1], v[1:]), (np.full(m - 1, gap), v[1:])):
+        g = G.from_edges(n, src, dst, lab)
+        rg, re = ctx.upload(g), ctx.upload_edges(n, src, dst, lab)
+        assert np.array_equal(re.g.row_offset, g.row_offset) and np.array_equal(re.g.col, g.col)
+        for l in ([1, 2], [2, 1, 3], [3, 1, 3]):
+            q = G.Query(np.array(l, dtype=np.uint32), np.arange(len(l) - 1, dtype=np.uint32),
+                        np.arange(1, len(l), dtype=np.uint32))
+            check(rg, g, q, l)
+            check(re, g, q, l)
+    bad = g.col.copy()
+    bad[-1] = n
+    with pytest.raises(_lib.GpsmError):
+        ctx.upload(G.DataGraph(g.row_offset, bad, g.labels))
