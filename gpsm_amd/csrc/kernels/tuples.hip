@@ -42,7 +42,7 @@ __device__ __forceinline__ bool row_less(const uint32_t* __restrict__ a, const u
 // from LDS, then (more bits than that, an equal row other than itself) column
 // by column.  With 64 bits there and 256 rows at a time 1129 rows of 6 14-bit
 // columns took 105 us (a row met itself once, in another iteration than any
-// other lane), 64 us with 128 bits, 20 us so.
+// other lane), 64 us with 128 bits, 21 us so.
 constexpr uint32_t RANK_ROWS = 1024;
 
 __global__ void __launch_bounds__(RANK_ROWS) rank_tuples_kernel(const uint32_t* __restrict__ tuples, uint32_t q,

@@ -116,7 +116,7 @@ int gpsm_verify_directed(gpsm_ctx* c, const gpsm_graph* g, uint32_t q, uint32_t 
   hipSetDevice(c->device);
   hipStream_t s = c->stream;
   // tuples go through the device in chunks of at most 256 MB, in the context's
-  // buffers (six allocations and frees took 0.5 ms of a call)
+  // buffers
   const uint64_t chunk = std::min<uint64_t>(n_tuples, (256ull << 20) / (sizeof(uint32_t) * q));
   if (c->bufs[B_TEXT_IN].ensure(sizeof(uint32_t) * chunk * q) || c->bufs[B_TEXT_KEEP].ensure(chunk) ||
       c->bufs[B_TEXT_WG].ensure(sizeof(uint32_t) * (2 + 3 * (uint64_t)m)))
