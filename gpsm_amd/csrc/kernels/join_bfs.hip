@@ -515,7 +515,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) b
       // a reserved slot that holds no row has only its length
       const uint32_t row_plan = r.get(R_PLAN), st = r.get(R_START), row_src = r.get(R_SRC);
       const uint32_t plan = len ? row_plan : 0u, src = len ? row_src : 0u;
-      if (len && a.j.budget && a.j.out[a.j.plans[plan].out].aborted) len = 0;
+      // rows of a plan over its budget end here, but not while part of a step is
+      // written: skip counts that step's survivors over all four rows
+      if (len && !skip && a.j.budget && a.j.out[a.j.plans[plan].out].aborted) len = 0;
       const PlanLevel& p = plans[plan];
       const bool final = p.final;
       const uint32_t qid = p.qid;
