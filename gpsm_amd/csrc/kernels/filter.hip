@@ -18,6 +18,7 @@
 #include <type_traits>
 
 #include "launch.h"
+#include "steps.h"
 #include "wave.h"
 
 namespace gpsm {
@@ -448,12 +449,13 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
     uint32_t C = 0;
     if (pull) {
       // the range's vertices with v's label and degree, ascending
-      for (uint32_t v0 = v_lo; v0 < v_hi; v0 += WAVE) {
-        const uint32_t v = v0 + lane, k = v < v_hi ? key[v] : 0u;
+      for_steps(v_lo, v_hi, [&](uint64_t v0) {
+        const uint64_t v = v0 + lane;
+        const uint32_t k = v < v_hi ? key[v] : 0u;
         const unsigned long long m = __ballot(k >= lo && k <= hi && v < v_hi);
-        if ((m >> lane) & 1ULL) L.cand[C + (uint32_t)__popcll(lane ? m & (~0ULL >> (WAVE - lane)) : 0ULL)] = v;
+        if ((m >> lane) & 1ULL) L.cand[C + (uint32_t)__popcll(lane ? m & (~0ULL >> (WAVE - lane)) : 0ULL)] = (uint32_t)v;
         C += (uint32_t)__popcll(m);
-      }
+      });
       L.word[lane] = 0;
     } else {
       uint32_t w = 0;

@@ -10,6 +10,7 @@
 #include <algorithm>
 
 #include "launch.h"
+#include "steps.h"
 #include "wave.h"
 
 namespace gpsm {
@@ -32,7 +33,10 @@ __device__ __forceinline__ void for_entries(const uint32_t* __restrict__ off, ui
     const uint32_t e1 = (uint32_t)min((uint64_t)total, e0 + ENTRY_BLOCK);
     const uint32_t lo = seg_search(off, nseg, (uint32_t)e0);
     const uint32_t ns = seg_search(off + lo, nseg - lo, e1 - 1) + 1;
-    for (uint32_t e = (uint32_t)e0 + lane; e < e1; e += WAVE) f(lo + seg_search(off + lo, ns, e), e);
+    for_steps(e0, e1, [&](uint64_t x) {
+      const uint64_t e = x + lane;
+      if (e < e1) f(lo + seg_search(off + lo, ns, (uint32_t)e), (uint32_t)e);
+    });
   }
 }
 
