@@ -55,6 +55,12 @@ void set_error(const char* what, hipError_t e) {
   g_last_error = std::string(what) + ": " + hipGetErrorString(e);
 }
 
+// Guards a device's copy of scratch, which its contexts share.
+std::mutex& noalloc_mutex(int device) {
+  static std::mutex m[64];
+  return m[device % 64];
+}
+
 }  // namespace
 
 namespace gpsm {
@@ -285,16 +291,19 @@ int gpsm_scan_u32_noalloc(gpsm_ctx* c, const uint32_t* d_in, uint32_t* d_out, ui
   if (n > GPSM_SCAN_NOALLOC_MAX) return GPSM_ESCRATCH;
   if (hipSetDevice(c->device) != hipSuccess) return GPSM_EDEVICE;
   hipStream_t s = c->stream;
+  // the array is the device's, not the context's: one call at a time, until
+  // its stream is idle (a second call would clear the tile states that the
+  // first one's workgroups wait for)
+  std::lock_guard<std::mutex> turn(noalloc_mutex(c->device));
   // words 0-1: the total; from word 2: two words per block sum
   uint32_t* scr = c->noalloc_scratch;
   unsigned long long* dtot = reinterpret_cast<unsigned long long*>(scr);
   const uint64_t words = GPSM_SCAN_NOALLOC_SCRATCH_BYTES / sizeof(uint32_t);
   launch_exclusive_scan(d_in, d_out, n, dtot, scr + 2, words - 2, s);
   unsigned long long t = 0;
-  if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(&t, dtot, sizeof(t), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
-    return GPSM_EDEVICE;
+  const bool queued = hipGetLastError() == hipSuccess &&
+                      hipMemcpyAsync(&t, dtot, sizeof(t), hipMemcpyDeviceToHost, s) == hipSuccess;
+  if (hipStreamSynchronize(s) != hipSuccess || !queued) return GPSM_EDEVICE;
   if (total) *total = t;
   return GPSM_OK;
 }

@@ -255,7 +255,8 @@ int gpsm_scan_u32(gpsm_ctx* ctx, const uint32_t* in, uint32_t* out, uint64_t n, 
  * of GPSM_SCAN_NOALLOC_SCRATCH_BYTES owned by the library (one per device,
  * held until the process ends), which bounds n at GPSM_SCAN_NOALLOC_MAX
  * (GPSM_ESCRATCH beyond it).  Runs on the context's stream and waits for it.
- * Calls that overlap on one device share that array and race. */
+ * The array is one per device: calls of several contexts or threads on one
+ * device take turns. */
 #define GPSM_SCAN_NOALLOC_SCRATCH_BYTES (256u * 1024u)
 /* 2 words hold the total; 2 words per block of 4096 values would fit the
  * rest, (65536 - 2) / 2 = 32767 blocks (a block's sum takes 2 words, and
