@@ -71,15 +71,7 @@ int DevBuf::ensure(size_t nbytes) {
   ptr = nullptr;
   bytes = 0;
   size_t want = std::max<size_t>(nbytes + nbytes / 4, 4096);
-  if (hipMalloc(&ptr, want) != hipSuccess) {
-    (void)hipGetLastError();
-    if (pool) pool->release();
-    if (!pool || hipMalloc(&ptr, want) != hipSuccess) {
-      ptr = nullptr;
-      (void)hipGetLastError();
-      return GPSM_ENOMEM;
-    }
-  }
+  if (!device_malloc(&ptr, want)) return GPSM_ENOMEM;
   bytes = want;
   return GPSM_OK;
 }

@@ -17,7 +17,6 @@ namespace gpsm {
 struct DevBuf {
   void* ptr = nullptr;
   size_t bytes = 0;
-  BlockPool* pool = nullptr;  // asked to return its idle blocks when an allocation fails
   int ensure(size_t nbytes);
   void release();
 };
@@ -192,9 +191,6 @@ struct gpsm_ctx {
   gpsm::BlockPool pool;  // memory of this context's graphs
   gpsm::DevBuf bufs[gpsm::B_COUNT_];
   void* part[gpsm::B_COUNT_] = {};  // where a batch's packed uploads are (parts of B_UP_*)
-  gpsm_ctx() {
-    for (auto& b : bufs) b.pool = &pool;
-  }
   gpsm::Tuning tune;
   gpsm_mlp* planner = nullptr;
   std::vector<uint32_t> h_counts;

@@ -372,11 +372,10 @@ int gpsm_mlp_create(gpsm_ctx* c, uint64_t seed, gpsm_mlp** out) {
   hipSetDevice(c->device);
   gpsm_mlp* mm = new gpsm_mlp();
   mm->ctx = c;
-  if (hipMalloc(&mm->p, sizeof(float) * NP) || hipMalloc(&mm->g, sizeof(float) * (NP + 1)) ||
-      hipMalloc(&mm->m, sizeof(float) * NP) || hipMalloc(&mm->v, sizeof(float) * NP) ||
-      hipMalloc(&mm->w1, sizeof(__bf16) * H * F) || hipMalloc(&mm->w2, sizeof(__bf16) * H * H) ||
-      hipMalloc(&mm->w2t, sizeof(__bf16) * H * H) ||
-      hipMalloc(&mm->norm, sizeof(float) * 2 * F)) {
+  if (!device_malloc(&mm->p, sizeof(float) * NP) || !device_malloc(&mm->g, sizeof(float) * (NP + 1)) ||
+      !device_malloc(&mm->m, sizeof(float) * NP) || !device_malloc(&mm->v, sizeof(float) * NP) ||
+      !device_malloc(&mm->w1, sizeof(__bf16) * H * F) || !device_malloc(&mm->w2, sizeof(__bf16) * H * H) ||
+      !device_malloc(&mm->w2t, sizeof(__bf16) * H * H) || !device_malloc(&mm->norm, sizeof(float) * 2 * F)) {
     gpsm_mlp_free(mm);
     return GPSM_ENOMEM;
   }

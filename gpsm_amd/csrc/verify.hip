@@ -61,11 +61,7 @@ __global__ void verify_kernel(const uint32_t* __restrict__ orow, const uint32_t*
 
 template <typename T>
 int to_device(const T* h, size_t n, T** d, hipStream_t s) {
-  if (hipMalloc(d, sizeof(T) * std::max<size_t>(n, 1)) != hipSuccess) {
-    (void)hipGetLastError();
-    *d = nullptr;
-    return GPSM_ENOMEM;
-  }
+  if (!device_malloc(d, sizeof(T) * std::max<size_t>(n, 1))) return GPSM_ENOMEM;
   if (n && hipMemcpyAsync(*d, h, sizeof(T) * n, hipMemcpyHostToDevice, s) != hipSuccess) return GPSM_EDEVICE;
   return GPSM_OK;
 }

@@ -128,6 +128,10 @@ int gpsm_graph_info(const gpsm_graph* g, uint32_t* n, uint64_t* adj);
 /* Copies a resident graph's CSR to host buffers row_offset[n+1], col[adj]
  * (e.g. to write a binary cache of a graph built on the device). */
 int gpsm_graph_csr(const gpsm_graph* g, uint32_t* row_offset, uint32_t* col);
+/* Frees a graph; any thread may, while no call uses it.  Up to 8 GiB of freed
+ * graphs' device memory waits in the context for its next graphs and goes back
+ * to the driver with the context, or when an allocation of any context of the
+ * process finds no memory. */
 int gpsm_graph_free(gpsm_graph* g);
 /* Bytes of device memory the resident graph occupies. */
 uint64_t gpsm_graph_device_bytes(const gpsm_graph* g);
