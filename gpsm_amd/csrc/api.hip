@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "api_internal.h"
+#include "bfs_sizes.h"
 #include "gpsm.h"
 #include "kernels/launch.h"
 #include "plan.h"
@@ -596,7 +597,8 @@ namespace {
 // workgroup, so the bound matters only for very wide queries.
 constexpr double kLevelBytes = 16.0 * (1ull << 30);
 
-// First-table rows of the plans joined breadth-first at a time (1 GB of rows).
+// First-table rows of the plans joined breadth-first at a time: their rows take
+// 64 bytes each, a short row's place and a long one's (2 GB).
 constexpr uint64_t kBfsRows = 1ull << 25;
 
 // Words of the join's counters (after B_JOUT's results): 0 .. 2 the launches' task counters, 16 .. 17 the tuples
@@ -1284,7 +1286,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   // the depth-first tasks share them well).
   // Depth-first, a cycle or clique of an R-MAT graph has a few thousand
   // first-table rows and most of its work under a few of them.
-  std::vector<uint32_t> bfs_q;
+  std::vector<uint32_t> bfs_q, bfs_left;  // queries; those of them left to the depth-first join
   uint64_t rows_total = 0;
   double est_total = 0;
   for (uint32_t b = 0; b < nq; ++b) {
@@ -1484,9 +1486,10 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     };
     // Breadth-first launches, BFS_PLANS plans at a time: a buffer per level,
     // for sixteen times the rows expected at the busiest level (the estimate
-    // is rough), 2^18 to 2^24 rows within kLevelBytes.  After a pass over the
-    // levels the host reads which of them stopped at a full buffer; the
-    // deepest one goes on first, into buffers emptied by then.
+    // is rough), 2^18 to 2^24 rows within kLevelBytes, fewer where the device
+    // has less room (bfs_sizes.h).  After a pass over the levels the host reads
+    // which of them stopped at a full buffer; the deepest one goes on first,
+    // into buffers emptied by then.
     auto breadth_first = [&]() -> int {
       for (size_t q0 = 0, q1; q0 < bfs_q.size(); q0 = q1) {
         uint64_t first_rows = 0;
@@ -1509,23 +1512,15 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
         const uint32_t nwg_b = std::max<uint32_t>(1, c->ncu * bfs_resident_per_cu((uint32_t)bp.size()));
         const uint64_t nwave = (uint64_t)nwg_b * 4;
         const uint32_t block = (uint32_t)std::min(64.0, std::max(4.0, rows / (4.0 * nwave)));
-        uint64_t words_per_row = 1;
-        for (uint32_t l = 2; l + 1 < widest; ++l) words_per_row += bfs_row_words(l);
         const uint64_t slack = nwave * block;  // slots of blocks not filled
-        const uint64_t most = std::max<uint64_t>((uint64_t)(kLevelBytes / (4.5 * words_per_row)), 1u << 18);
-        const uint64_t rcap =
-            slack + std::min<uint64_t>(most, (uint64_t)std::min(std::max(16.0 * rows, 262144.0), 16777216.0));
-        const uint64_t cap1 = first.back() + slack;  // every level-1 row
-        auto cap_of = [&](uint32_t l) { return l == 1 ? cap1 : rcap; };
-        auto long_of = [&](uint32_t l) { return l == 1 ? first.back() : rcap / 16; };
-        uint64_t at[BFS_MAXQ] = {0}, words = 0;  // each level's short rows, its long rows after them
-        for (uint32_t l = 1; l + 1 < widest; ++l) {
-          at[l] = words;
-          words += (cap_of(l) + long_of(l)) * bfs_row_words(l);
+        BfsSizes z;
+        if (!bfs_fit(widest, first.back(), slack, bfs_rows(widest, first.back(), slack, rows, kLevelBytes), z,
+                     [&](size_t bytes) { return c->bufs[B_BROWS].ensure(bytes) == GPSM_OK; })) {
+          bfs_left.insert(bfs_left.end(), bfs_q.begin() + q0, bfs_q.begin() + q1);
+          continue;
         }
         int rc;
-        if ((rc = c->bufs[B_BROWS].ensure(sizeof(uint32_t) * words)) || (rc = upload(c, B_BPLANS, bp)) ||
-            (rc = upload(c, B_BFIRST, first)) ||
+        if ((rc = upload(c, B_BPLANS, bp)) || (rc = upload(c, B_BFIRST, first)) ||
             (rc = c->bufs[B_BCURS].ensure(sizeof(BfsCursor) * 2 * nwave * BFS_MAXQ)))
           return rc;
         if (q0) launch_fill_u32(ctr + kCtrRows, 0u, kCtrWords - kCtrRows, s);
@@ -1539,10 +1534,10 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
         uint32_t* rows_base = dptr<uint32_t>(c, B_BROWS);
         auto out_level = [&](uint32_t l) {
           const bool kept = l + 1 < widest;
-          a.rows_out = kept ? rows_base + at[l] : nullptr;
-          a.long_out = kept ? a.rows_out + cap_of(l) * bfs_row_words(l) : nullptr;
-          a.cap = kept ? (uint32_t)cap_of(l) : 0;
-          a.long_cap = kept ? (uint32_t)long_of(l) : 0;
+          a.rows_out = kept ? rows_base + z.at[l] : nullptr;
+          a.long_out = kept ? a.rows_out + z.cap[l] * bfs_row_words(l) : nullptr;
+          a.cap = kept ? (uint32_t)z.cap[l] : 0;
+          a.long_cap = kept ? (uint32_t)z.long_cap[l] : 0;
           a.stride_out = bfs_row_words(l);
           a.cout = ctr + kCtrRows + 2 * l;
         };
@@ -1588,6 +1583,12 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     // timed together as one join
     hipEvent_t pa = pbegin(K_JOIN);
     if (!bfs_q.empty() && (rc = breadth_first())) return rc;
+    // those without room for their levels join the depth-first tasks
+    for (uint32_t b : bfs_left) {
+      rows_total += Q[b].cet_size[Q[b].plan.first_edge];
+      est_total += est[b];
+    }
+    for (uint32_t b : bfs_left) add_tasks(b);
     if ((rc = depth_first())) return rc;
     pend(K_JOIN, pa, 0.0, -1);
     HIPCHK(hipGetLastError());

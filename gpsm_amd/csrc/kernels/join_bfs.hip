@@ -39,6 +39,7 @@ namespace {
 // their number (0: no row), 5 their source (0: the parent's list, 1 + b: the
 // adjacency of the vertex at back position b), then the level + 1 vertices
 constexpr uint32_t R_PLAN = 2, R_START = 3, R_LEN = 4, R_SRC = 5, R_VAL = 6;
+static_assert(bfs_row_words(1) == ((R_VAL + 2 + 1) & ~1u), "a row's words");
 constexpr uint32_t GROUP = 16;         // lanes per short row (one DPP row)
 constexpr uint32_t LONG_LIST = 512;    // candidates above which workgroups take the row
 constexpr int BFS_UNROLL = 4;          // candidates in flight per lane
@@ -576,8 +577,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) b
 }
 
 }  // namespace
-
-uint32_t bfs_row_words(uint32_t level) { return (R_VAL + level + 1 + 1) & ~1u; }
 
 void launch_bfs_first(const BfsArgs& a, uint32_t nwg, hipStream_t s) {
   hipLaunchKernelGGL(bfs_first_kernel, dim3(nwg), dim3(256), (sizeof(PlanAcc) + sizeof(PlanLevel)) * a.nplans, s, a);

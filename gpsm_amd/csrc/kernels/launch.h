@@ -5,6 +5,7 @@
 #include <cstdint>
 #include <vector>
 
+#include "bfs_sizes.h"
 #include "gpsm_dev.h"
 
 namespace gpsm {
@@ -304,7 +305,7 @@ uint64_t join_level_words(uint32_t qmax, uint32_t cap);
 // takes level to level + 1: all its rows, or (resume) those that an earlier
 // launch left when the next level's buffer was full.  j: plans (nplans of them, JoinPlan::out their
 // results), cets, lists, budget and out as for launch_join.
-constexpr uint32_t BFS_PLANS = 256, BFS_MAXQ = 8;
+constexpr uint32_t BFS_PLANS = 256;
 struct BfsCursor {
   uint32_t idx, pos, skip;
 };
@@ -326,7 +327,6 @@ struct BfsArgs {
   uint32_t resume;
   uint32_t* pending;   // waves that stopped at a full buffer (zeroed by the caller)
 };
-uint32_t bfs_row_words(uint32_t level);
 void launch_bfs_first(const BfsArgs& a, uint32_t nwg, hipStream_t s);
 void launch_bfs_expand(const BfsArgs& a, uint32_t nwg, hipStream_t s);
 uint32_t bfs_resident_per_cu(uint32_t nplans);
