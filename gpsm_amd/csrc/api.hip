@@ -262,7 +262,8 @@ void gpsm_shutdown(gpsm_ctx* c) {
     if (e) hipGraphExecDestroy(e);
   for (auto& b : c->bufs) b.release();
   for (auto& b : c->h_stage) b.release();
-  for (auto& b : c->h_net) b.release();
+  c->net_stages->idle.each([](NetStage& x) { x.release(); });
+  c->net_stages->context_ended = true;
   c->arena.release();
   c->stager.release();
   c->pool.release();

@@ -2,10 +2,13 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
+#include <memory>
 #include <vector>
 
 #include "gpsm.h"
+#include "leases.h"
 #include "kernels/launch.h"
 #include "plan.h"
 #include "pool.h"
@@ -28,6 +31,26 @@ struct HostBuf {
   size_t bytes = 0;
   int ensure(size_t nbytes);
   void release();
+};
+
+// Pinned staging of a network call: what goes in, what comes out.  Lent by the
+// network's context for the call: hipHostMalloc takes longer than a mini-batch's
+// gradients, and a network may be the planner of another context, whose thread
+// then calls it while this context's thread calls another.
+struct NetStage {
+  static constexpr size_t kKeep = 4u << 20;  // bytes kept without any network
+  HostBuf in, out;
+  void release() {
+    in.release();
+    out.release();
+  }
+};
+
+// Shared by a context and its networks (one may be freed after the context).
+struct NetStages {
+  Leases<NetStage> idle;
+  std::atomic<int> networks{0};
+  std::atomic<bool> context_ended{false};
 };
 
 // Pinned staging for a batch's uploads: take() hands out fresh regions (in
@@ -197,8 +220,7 @@ struct gpsm_ctx {
   // pinned readbacks of a batch: counts, |CET| descriptors, join results, join
   // flag, few sorted tuples
   gpsm::HostBuf h_stage[5];
-  // ... inputs and outputs of a network call (each waits for its own)
-  gpsm::HostBuf h_net[2];
+  std::shared_ptr<gpsm::NetStages> net_stages = std::make_shared<gpsm::NetStages>();
   gpsm::PinnedArena arena;   // pinned sources of a batch's uploads
   // Instantiated hipGraphs of a batch's two captured phases (filter;
   // candidate-edge tables), kept across batches: a batch whose launches

@@ -312,6 +312,7 @@ struct gpsm_mlp {
   float* norm = nullptr;  // mu[F], inv_sd[F]
   DevBuf x, y;  // x: features, then (gradients) targets
   DevBuf act;  // the weight-gradient GEMMs' operands (mlp_grad_kernel)
+  std::shared_ptr<NetStages> stages;  // the context's
   int step = 0;
 };
 
@@ -325,11 +326,30 @@ int refresh(gpsm_mlp* mm) {
   return hipGetLastError() == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
 }
 
+// The call's staging, given back at its end once the stream is idle.
+class StageLease {
+ public:
+  explicit StageLease(gpsm_mlp* mm) : mm_(mm), x_(mm->stages->idle.take()) {}
+  ~StageLease() {
+    if (!idle_) (void)hipStreamSynchronize(mm_->ctx->stream);  // a failed call's copies may still be queued
+    mm_->stages->idle.give(std::move(x_));
+  }
+  StageLease(const StageLease&) = delete;
+  NetStage* operator->() { return x_.get(); }
+  // Waits for what the call queued.
+  bool wait() { return idle_ = hipStreamSynchronize(mm_->ctx->stream) == hipSuccess; }
+
+ private:
+  gpsm_mlp* mm_;
+  std::unique_ptr<NetStage> x_;
+  bool idle_ = false;
+};
+
 // Features and targets to the device: a mini-batch as one queued copy from
 // pinned memory, large ones through the context's staging.  With two pageable
 // copies in, two out and four hipMemsetAsync the gradients of 256 samples took
 // 129 us, 33 of them the kernels.
-int stage(gpsm_mlp* mm, const float* x, const float* t, uint32_t B) {
+int stage(gpsm_mlp* mm, StageLease& st, const float* x, const float* t, uint32_t B) {
   hipStream_t s = mm->ctx->stream;
   const size_t xb = sizeof(float) * (size_t)B * F, tb = sizeof(float) * B;
   if (mm->x.ensure(xb + tb)) return GPSM_ENOMEM;
@@ -338,10 +358,10 @@ int stage(gpsm_mlp* mm, const float* x, const float* t, uint32_t B) {
     return mm->ctx->stager.to_device(d, x, xb, s) == hipSuccess && mm->ctx->stager.to_device(d + xb, t, tb, s) == hipSuccess
                ? GPSM_OK
                : GPSM_EDEVICE;
-  if (mm->ctx->h_net[0].ensure(xb + tb)) return GPSM_ENOMEM;
-  std::memcpy(mm->ctx->h_net[0].ptr, x, xb);
-  std::memcpy(static_cast<char*>(mm->ctx->h_net[0].ptr) + xb, t, tb);
-  return hipMemcpyAsync(d, mm->ctx->h_net[0].ptr, xb + tb, hipMemcpyHostToDevice, s) == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
+  if (st->in.ensure(xb + tb)) return GPSM_ENOMEM;
+  std::memcpy(st->in.ptr, x, xb);
+  std::memcpy(static_cast<char*>(st->in.ptr) + xb, t, tb);
+  return hipMemcpyAsync(d, st->in.ptr, xb + tb, hipMemcpyHostToDevice, s) == hipSuccess ? GPSM_OK : GPSM_EDEVICE;
 }
 
 int run_grad(gpsm_mlp* mm, uint32_t B) {
@@ -372,6 +392,8 @@ int gpsm_mlp_create(gpsm_ctx* c, uint64_t seed, gpsm_mlp** out) {
   hipSetDevice(c->device);
   gpsm_mlp* mm = new gpsm_mlp();
   mm->ctx = c;
+  mm->stages = c->net_stages;
+  ++mm->stages->networks;
   if (!device_malloc(&mm->p, sizeof(float) * NP) || !device_malloc(&mm->g, sizeof(float) * (NP + 1)) ||
       !device_malloc(&mm->m, sizeof(float) * NP) || !device_malloc(&mm->v, sizeof(float) * NP) ||
       !device_malloc(&mm->w1, sizeof(__bf16) * H * F) || !device_malloc(&mm->w2, sizeof(__bf16) * H * H) ||
@@ -401,7 +423,7 @@ int gpsm_mlp_create(gpsm_ctx* c, uint64_t seed, gpsm_mlp** out) {
 
 void gpsm_mlp_free(gpsm_mlp* mm) {
   if (!mm) return;
-  if (mm->ctx && mm->ctx->planner == mm) mm->ctx->planner = nullptr;
+  if (!mm->stages->context_ended && mm->ctx->planner == mm) mm->ctx->planner = nullptr;
   hipFree(mm->p);
   hipFree(mm->g);
   hipFree(mm->m);
@@ -413,6 +435,11 @@ void gpsm_mlp_free(gpsm_mlp* mm) {
   mm->x.release();
   mm->y.release();
   mm->act.release();
+  // the last network takes large staging with it
+  if (--mm->stages->networks == 0)
+    mm->stages->idle.each([](NetStage& x) {
+      if (x.in.bytes + x.out.bytes > NetStage::kKeep) x.release();
+    });
   delete mm;
 }
 
@@ -444,30 +471,31 @@ int gpsm_mlp_forward(gpsm_mlp* mm, const float* x, uint32_t B, float* y) {
   if (!mm || (B && (!x || !y))) return GPSM_EINVAL;
   if (!B) return GPSM_OK;
   const size_t xb = sizeof(float) * (size_t)B * F, yb = sizeof(float) * B;
-  if (mm->x.ensure(xb) || mm->y.ensure(yb) || mm->ctx->h_net[0].ensure(xb) || mm->ctx->h_net[1].ensure(yb)) return GPSM_ENOMEM;
+  StageLease st(mm);
+  if (mm->x.ensure(xb) || mm->y.ensure(yb) || st->in.ensure(xb) || st->out.ensure(yb)) return GPSM_ENOMEM;
   hipStream_t s = mm->ctx->stream;
-  std::memcpy(mm->ctx->h_net[0].ptr, x, xb);
-  if (hipMemcpyAsync(mm->x.ptr, mm->ctx->h_net[0].ptr, xb, hipMemcpyHostToDevice, s) != hipSuccess) return GPSM_EDEVICE;
+  std::memcpy(st->in.ptr, x, xb);
+  if (hipMemcpyAsync(mm->x.ptr, st->in.ptr, xb, hipMemcpyHostToDevice, s) != hipSuccess) return GPSM_EDEVICE;
   hipLaunchKernelGGL(mlp_forward_kernel, dim3((B + 31) / 32), dim3(64), 0, s, weights_of(mm),
                      reinterpret_cast<const float*>(mm->x.ptr), B, reinterpret_cast<float*>(mm->y.ptr));
   if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(mm->ctx->h_net[1].ptr, mm->y.ptr, yb, hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
+      hipMemcpyAsync(st->out.ptr, mm->y.ptr, yb, hipMemcpyDeviceToHost, s) != hipSuccess || !st.wait())
     return GPSM_EDEVICE;
-  std::memcpy(y, mm->ctx->h_net[1].ptr, yb);
+  std::memcpy(y, st->out.ptr, yb);
   return GPSM_OK;
 }
 
 int gpsm_mlp_grad(gpsm_mlp* mm, const float* x, const float* t, uint32_t B, float* loss, float* grad) {
   if (!mm || !x || !t || !B || !grad) return GPSM_EINVAL;
-  int rc = stage(mm, x, t, B);
+  StageLease st(mm);
+  int rc = stage(mm, st, x, t, B);
   if (rc) return rc;
   hipStream_t s = mm->ctx->stream;
   if ((rc = run_grad(mm, B))) return rc;
-  if (mm->ctx->h_net[1].ensure(sizeof(float) * (NP + 1))) return GPSM_ENOMEM;
-  const float* out = static_cast<const float*>(mm->ctx->h_net[1].ptr);
-  if (hipMemcpyAsync(mm->ctx->h_net[1].ptr, mm->g, sizeof(float) * (NP + 1), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
+  if (st->out.ensure(sizeof(float) * (NP + 1))) return GPSM_ENOMEM;
+  const float* out = static_cast<const float*>(st->out.ptr);
+  if (hipMemcpyAsync(st->out.ptr, mm->g, sizeof(float) * (NP + 1), hipMemcpyDeviceToHost, s) != hipSuccess ||
+      !st.wait())
     return GPSM_EDEVICE;
   std::memcpy(grad, out, sizeof(float) * NP);
   if (loss) *loss = out[NP];
@@ -476,7 +504,8 @@ int gpsm_mlp_grad(gpsm_mlp* mm, const float* x, const float* t, uint32_t B, floa
 
 int gpsm_mlp_train_step(gpsm_mlp* mm, const float* x, const float* t, uint32_t B, float lr, float* loss) {
   if (!mm || !x || !t || !B) return GPSM_EINVAL;
-  int rc = stage(mm, x, t, B);
+  StageLease st(mm);
+  int rc = stage(mm, st, x, t, B);
   if (rc) return rc;
   if ((rc = run_grad(mm, B))) return rc;
   hipStream_t s = mm->ctx->stream;
@@ -485,8 +514,7 @@ int gpsm_mlp_train_step(gpsm_mlp* mm, const float* x, const float* t, uint32_t B
   hipLaunchKernelGGL(adam_kernel, dim3((NP + 255) / 256), dim3(256), 0, s, mm->p, mm->g, mm->m, mm->v, lr, c1, c2);
   if ((rc = refresh(mm))) return rc;
   float l = 0;
-  if (hipMemcpyAsync(&l, mm->g + NP, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
-      hipStreamSynchronize(s) != hipSuccess)
+  if (hipMemcpyAsync(&l, mm->g + NP, sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess || !st.wait())
     return GPSM_EDEVICE;
   if (loss) *loss = l;
   return GPSM_OK;
