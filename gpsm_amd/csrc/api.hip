@@ -1037,7 +1037,8 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       d.w_slot = S.vbase + S.hq.et[e];
       d.ncand = counts[d.x_slot];
       d.clist_off = coff[d.x_slot];
-      key_range(S.hq, st, S.hq.et[e], d.w_lo, d.w_hi);
+      uint32_t hi;
+      key_range(S.hq, st, S.hq.et[e], d.w_lo, hi);
       fdesc.push_back(d);
     }
   }
@@ -1066,7 +1067,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   {
     hipEvent_t a = pbegin(K_CET_COUNT);
     launch_cet_count(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_FDESC), (uint32_t)fdesc.size(),
-                     dptr<uint32_t>(c, B_OFFSETS), 1, dptr<uint32_t>(c, B_FCHUNK), cgrid, s,
+                     dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_FCHUNK), cgrid, s,
                      counters ? fstats + fstat_step * slot_cet_b : nullptr);
     pend(K_CET_COUNT, a, 0.0, counters ? slot_cet_b : -1);
   }
@@ -1200,7 +1201,8 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
       d.list_base = list_words;
       d.list_cap = (uint32_t)S.cet_size[edge];
       d.term_base = ~0ull;
-      key_range(S.hq, st, wq, d.w_lo, d.w_hi);
+      uint32_t hi;
+      key_range(S.hq, st, wq, d.w_lo, hi);
       if (list) list_words += S.cet_size[edge];
       jdesc.push_back(d);
       return (uint32_t)jdesc.size() - 1;
@@ -1380,7 +1382,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
     hipEvent_t pa = pbegin(K_CET_COUNT);
     if (!cdesc.empty())
       launch_cet_count(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_CDESC), (uint32_t)cdesc.size(),
-                       dptr<uint32_t>(c, B_OFFSETS), 1, dptr<uint32_t>(c, B_CCHUNK), cgrid, s,
+                       dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_CCHUNK), cgrid, s,
                        counters ? fstats + fstat_step * slot_cet_c : nullptr);
     pend(K_CET_COUNT, pa, 0.0, counters ? slot_cet_c : -1);
     launch_cet_offsets(dptr<CetDesc>(c, B_LDESC), (uint32_t)ldesc.size(), dptr<uint32_t>(c, B_OFFSETS), s);

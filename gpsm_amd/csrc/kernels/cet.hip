@@ -3,10 +3,9 @@
 // mu in C(x) ascending, the data neighbours of mu that are in C(w), in
 // adjacency (ascending) order.
 //
-// One wave per 64 candidates of C(x), taken with a stride: of the N waves
-// of a table, wave j takes candidates j, j + N, j + 2N, ..., so the hubs of
-// a power-law graph (its lowest ids, the first candidates) land on
-// different waves.  The wave walks the concatenated adjacency of its
+// One wave per 64 candidates of C(x): some of the first, which on a power-law
+// graph are the hubs, spread over the table's waves, and runs of consecutive
+// ones (cand_index).  The wave walks the concatenated adjacency of its
 // candidates towards w's label (DevGraph::lrow: C(w) holds no vertex of
 // another) 64 entries per step (balanced across hub and leaf candidates) and
 // tests C(w) membership in the bitmap.  Outputs are per candidate (its
@@ -82,7 +81,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) c
                                                         const uint32_t* __restrict__ bitmaps, uint32_t W,
                                                         const uint32_t* __restrict__ clist, CetDesc* descs,
                                                         const uint32_t* __restrict__ chunk_base, uint32_t ndesc,
-                                                        uint32_t* __restrict__ offsets, int per_cand,
+                                                        uint32_t* __restrict__ offsets,
                                                         unsigned long long* __restrict__ stats) {
   __shared__ CetLds lds[4];
   CetTally tl;
@@ -102,8 +101,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) c
     const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
     uint32_t tot = 0;
     for (uint32_t f = 0; f < D; f += WAVE * CET_UNROLL) {
-      // CET_UNROLL entries per lane: all adjacency and key loads, then the
-      // probes of the entries whose key is in range
+      // CET_UNROLL entries per lane: all adjacency loads, then their probes
       uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], es[CET_UNROLL];
 #pragma unroll
       for (int u = 0; u < CET_UNROLL; ++u) cis[u] = f + u * WAVE + lane;
@@ -134,11 +132,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) c
       for (int u = 0; u < CET_UNROLL; ++u)
         if (pw[u] & 1u) {
           ++tot;
-          if (per_cand) atomicAdd(&L.cnt[cis[u]], 1u);
+          atomicAdd(&L.cnt[cis[u]], 1u);
         }
     }
     wave_sync();
-    if (per_cand && mine) offsets[d.off_base + cand_index(j, nch, lane)] = L.cnt[lane];
+    if (mine) offsets[d.off_base + cand_index(j, nch, lane)] = L.cnt[lane];
     tot = wave_sum(tot);
     if (lane == 0 && tot) atomicAdd(reinterpret_cast<unsigned long long*>(&descs[di].total), (unsigned long long)tot);
     wave_sync();
@@ -208,9 +206,8 @@ __global__ void __launch_bounds__(256) cet_write_kernel(Pieces pieces, const uin
     const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
     uint32_t* out = lists + d.list_base;
     for (uint32_t f = 0; f < D; f += WAVE * CET_UNROLL) {
-      // CET_UNROLL sub-steps of 64 entries: all adjacency and key loads, the
-      // probes of in-range entries, then the writes sub-step by sub-step
-      // (lists stay in adjacency order)
+      // CET_UNROLL sub-steps of 64 entries: all adjacency loads, their probes,
+      // then the writes sub-step by sub-step (lists stay in adjacency order)
       uint32_t cis[CET_UNROLL], mvs[CET_UNROLL];
       bool hits[CET_UNROLL];
       uint32_t es[CET_UNROLL];
@@ -276,7 +273,7 @@ __device__ __forceinline__ void seg_add(unsigned long long* cell, uint32_t seg, 
 }
 
 // Records of the last join levels' tables: one wave per 64 candidates of
-// C(x) with a stride, flattened over their adjacency as in cet_count, but an
+// C(x) (cand_index), flattened over their adjacency as in cet_count, but an
 // entry in C(w) adds its hash term (computed here, about 30 VALU
 // instructions, only in lanes with a hit) to its candidate's sum and is not
 // written: the join reads 32 bytes per candidate instead of 12 per list
@@ -363,8 +360,8 @@ __global__ void __launch_bounds__(256) cet_sum_kernel(Pieces pieces, const uint3
   if (stats) flush_tally(tl, stats);
 }
 
-// Records of the level before the last: one wave per 64 candidates with a
-// stride, flattened over their lists.  A list entry costs its hash term and,
+// Records of the level before the last: one wave per 64 candidates
+// (cand_index), flattened over their lists.  A list entry costs its hash term and,
 // where w's parent is the entry itself (AGG_CHAIN), its rank in C(y) and its
 // 32-byte record of the last table.
 constexpr int AGG_UNROLL = 2;  // list entries in flight per lane
@@ -488,11 +485,11 @@ __global__ void __launch_bounds__(256) cet_terms_kernel(const uint32_t* __restri
 }  // namespace
 
 void launch_cet_count(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, CetDesc* descs,
-                      uint32_t ndesc, uint32_t* offsets, int per_cand, const uint32_t* chunk_base, uint32_t grid,
-                      hipStream_t s, unsigned long long* stats) {
+                      uint32_t ndesc, uint32_t* offsets, const uint32_t* chunk_base, uint32_t grid, hipStream_t s,
+                      unsigned long long* stats) {
   if (!ndesc) return;
   hipLaunchKernelGGL(cet_count_kernel, dim3(grid), dim3(256), 0, s, pieces_of(g), g.col, bitmaps, g.W, clist,
-                     descs, chunk_base, ndesc, offsets, per_cand, stats);
+                     descs, chunk_base, ndesc, offsets, stats);
 }
 
 void launch_cet_offsets(CetDesc* descs, uint32_t ndesc, uint32_t* offsets, hipStream_t s) {

@@ -224,15 +224,15 @@ void launch_text_write(const uint32_t* tuples, uint64_t rows, uint32_t q, const 
 
 // cet.hip ----------------------------------------------------------------------
 // Per CetDesc: |CET| into desc.total (atomic); per-candidate counts into
-// offsets (when per_cand != 0) at desc.off_base.
+// offsets at desc.off_base.
 // chunk_base[d]: chunks of 64 candidates in the tables before d (ndesc + 1
 // entries); grid: workgroups (persistent).
 // stats (optional, STAT_COPIES x STAT_STRIDE u64, zeroed by the caller):
 // entries 0..3 = candidates, adjacency entries examined, bitmap probes, list
 // entries written (cet_write only), summed over the copies.
 void launch_cet_count(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, CetDesc* descs,
-                      uint32_t ndesc, uint32_t* offsets, int per_cand, const uint32_t* chunk_base, uint32_t grid,
-                      hipStream_t s, unsigned long long* stats = nullptr);
+                      uint32_t ndesc, uint32_t* offsets, const uint32_t* chunk_base, uint32_t grid, hipStream_t s,
+                      unsigned long long* stats = nullptr);
 // Segmented exclusive scan of the per-candidate counts of every desc.
 void launch_cet_offsets(CetDesc* descs, uint32_t ndesc, uint32_t* offsets, hipStream_t s);
 // Records of the last join levels' tables (CetAgg::s and len of every

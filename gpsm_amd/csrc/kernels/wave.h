@@ -125,17 +125,17 @@ __device__ __forceinline__ uint64_t fmix64(uint64_t k) {
   return k;
 }
 
-// One factor of a tuple's hash (odd): the tuple hash is the product of the
-// factors of its (query vertex, image) pairs mod 2^64, so it does not depend
-// on the order in which the join binds the vertices.
 // Entries off .. off + len - 1 of vertex v: those towards the label of key_lo
-// (a key of it), and, where several labels make a group, the group's others.
+// (a key of it: its label bits are at least 1), and, where several labels make a group, the group's others.
 __device__ __forceinline__ void piece(const Pieces& p, uint32_t v, uint32_t key_lo, uint32_t& off, uint32_t& len) {
   const uint32_t* r = p.lrow + (size_t)(((key_lo >> KEY_DEG_BITS) - 1) >> p.gshift) * p.n + v;
   off = r[0];
   len = r[1] - off;
 }
 
+// One factor of a tuple's hash (odd): the tuple hash is the product of the
+// factors of its (query vertex, image) pairs mod 2^64, so it does not depend
+// on the order in which the join binds the vertices.
 __device__ __forceinline__ uint64_t tuple_term(uint32_t qid, uint32_t v) {
   return fmix64((((uint64_t)qid << 32) | v) ^ 0x9E3779B97F4A7C15ULL) | 1ULL;
 }

@@ -98,7 +98,7 @@ int cet_hook(void* user, gpsm_ctx* c, const CetDesc* fdesc, uint32_t nf) {
   uint32_t* dchunks = reinterpret_cast<uint32_t*>(c->bufs[B_CHUNKS].ptr);
   hipMemcpyAsync(dd, d.data(), sizeof(CetDesc) * nf, hipMemcpyHostToDevice, s);
   hipMemcpyAsync(dchunks, chunks.data(), sizeof(uint32_t) * chunks.size(), hipMemcpyHostToDevice, s);
-  launch_cet_count(dg, bitmaps, clist, dd, nf, offs, 1, dchunks, grid, s);
+  launch_cet_count(dg, bitmaps, clist, dd, nf, offs, dchunks, grid, s);
   launch_cet_offsets(dd, nf, offs, s);
   launch_cet_write(dg, bitmaps, clist, dd, nf, offs, lists, dchunks, grid, s);
   uint64_t cmax = 0;
