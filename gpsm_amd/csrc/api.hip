@@ -1395,7 +1395,7 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
                     counters ? fstats + fstat_step * slot_cet_w : nullptr);
     launch_cet_aggs(dg, bitmaps, dptr<uint32_t>(c, B_BPREFIX), dptr<AggDesc>(c, B_ADESC), (uint32_t)adesc.size(),
                     dptr<uint32_t>(c, B_ACHUNK), dptr<uint32_t>(c, B_OFFSETS), dptr<uint32_t>(c, B_LISTS),
-                    dptr<CetAgg>(c, B_AGGS), cgrid, s);
+                    dptr<CetAgg>(c, B_AGGS), cgrid, s, counters ? fstats + fstat_step * slot_cet_w : nullptr);
     launch_cet_terms(dg, dptr<uint32_t>(c, B_LISTS), dptr<CetDesc>(c, B_JDESC), dptr<uint32_t>(c, B_TERM_DESC),
                      dptr<uint64_t>(c, B_TERM_START), (uint32_t)term_desc.size(), term_words,
                      dptr<unsigned long long>(c, B_TERMS), s);
@@ -1628,21 +1628,26 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
         hipEventElapsedTime(&kms, pnd.a, pnd.b);
         double bytes = pnd.bytes;
         if (pnd.stats_slot >= 0) {
-          unsigned long long f[5] = {0, 0, 0, 0, 0};
+          unsigned long long f[STAT_STRIDE] = {0};
           for (uint32_t cp = 0; cp < STAT_COPIES; ++cp)
-            for (int i = 0; i < 5; ++i) f[i] += fs[fstat_step * pnd.stats_slot + cp * STAT_STRIDE + i];
+            for (uint32_t i = 0; i < STAT_STRIDE; ++i) f[i] += fs[fstat_step * pnd.stats_slot + cp * STAT_STRIDE + i];
           if (pnd.kind == K_FILTER) {
-            // candidates: two row offsets; entries: column index or neighbour
-            // key; neighbour keys read beside the column index (explore's
-            // second pass); bitmap probes and bit writes count one bit each
+            // candidates and neighbours: two piece bounds; entries: column index
+            // or neighbour key; vertices' keys and neighbour keys read beside the
+            // column index; bitmap probes and bit writes count one bit each
             bytes += 8.0 * f[0] + 4.0 * f[1] + 4.0 * f[2] + (f[3] + f[4]) / 8.0;
           } else {
-            // candidate-edge count / write: per candidate its id and two row
-            // offsets, plus its count written (count) or its list offset read
-            // (write); per adjacency entry the column index and the
-            // neighbour's key; one bit per probe of C(w); 4 per list entry
-            // written
-            bytes += 16.0 * f[0] + 8.0 * f[1] + f[2] / 8.0 + 4.0 * f[3];
+            // candidate-edge count / write: per candidate its id, two piece
+            // bounds and its count written (count) or its list offset read
+            // (write); per adjacency entry the column index; one bit per probe of
+            // a candidate set; 4 per list entry written.  Records of the last
+            // table: per candidate its id, two piece bounds and the record
+            // written; of the table before: two list offsets and the record
+            // written, per list entry the entry, per record read two rank loads
+            // and the record.
+            constexpr double rec = sizeof(CetAgg);
+            bytes += 16.0 * f[0] + 4.0 * f[1] + f[2] / 8.0 + 4.0 * f[3] + (12.0 + rec) * f[4] + (8.0 + rec) * f[5] +
+                     4.0 * f[6] + (8.0 + rec) * f[7];
           }
         }
         Prof::Acc& acc = c->prof.acc[pnd.kind];

@@ -27,21 +27,27 @@ struct CetLds {
   uint32_t cnt[WAVE];
 };
 
-// Optional work counters (profiling): per lane, candidates loaded, adjacency
-// entries examined, bitmap probes and list entries written; one atomic per
-// counter per workgroup into copy blockIdx % STAT_COPIES of stats.
+// Optional work counters (profiling), per lane: of cet_count and cet_write the
+// candidates loaded, of all but cet_agg the adjacency entries examined, bitmap
+// probes, list entries written; cet_sum's candidates; cet_agg's candidates,
+// list entries and records read.  One atomic per counter per workgroup into
+// copy blockIdx % STAT_COPIES of stats.
+constexpr int CET_STATS = 8;
+static_assert(CET_STATS <= STAT_STRIDE, "a copy's counters");
 struct CetTally {
-  uint32_t cand = 0, ent = 0, probe = 0, wrote = 0;
+  uint32_t cand = 0, ent = 0, probe = 0, wrote = 0, sums = 0, aggs = 0, items = 0, recs = 0;
 };
 
 __device__ __forceinline__ void flush_tally(const CetTally& t, unsigned long long* stats) {
-  __shared__ unsigned long long red[4][4];
-  const unsigned long long v[4] = {wave_sum64(t.cand), wave_sum64(t.ent), wave_sum64(t.probe), wave_sum64(t.wrote)};
+  __shared__ unsigned long long red[4][CET_STATS];
+  const unsigned long long v[CET_STATS] = {wave_sum64(t.cand), wave_sum64(t.ent),  wave_sum64(t.probe),
+                                           wave_sum64(t.wrote), wave_sum64(t.sums), wave_sum64(t.aggs),
+                                           wave_sum64(t.items), wave_sum64(t.recs)};
   const uint32_t w = threadIdx.x / WAVE;
   if (lane_id() == 0)
-    for (int i = 0; i < 4; ++i) red[w][i] = v[i];
+    for (int i = 0; i < CET_STATS; ++i) red[w][i] = v[i];
   __syncthreads();
-  if (threadIdx.x < 4) {
+  if (threadIdx.x < CET_STATS) {
     unsigned long long tot = 0;
     for (uint32_t x = 0; x < blockDim.x / WAVE; ++x) tot += red[x][threadIdx.x];
     if (tot) atomicAdd(stats + (blockIdx.x % STAT_COPIES) * STAT_STRIDE + threadIdx.x, tot);
@@ -306,7 +312,7 @@ __global__ void __launch_bounds__(256) cet_sum_kernel(Pieces pieces, const uint3
     uint32_t D;
     L.s[lane] = 0;
     load_chunk(pieces, clist, d, j, nch, L.c, mine, D);
-    tl.cand += mine;
+    tl.sums += mine;
     const uint32_t* bm_w = bitmaps + (size_t)d.w_slot * W;
     for (uint32_t f = 0; f < D; f += WAVE * CET_UNROLL) {
       uint32_t cis[CET_UNROLL], mvs[CET_UNROLL], pw[CET_UNROLL];
@@ -378,8 +384,10 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
                                                       const AggDesc* __restrict__ descs, uint32_t ndesc,
                                                       const uint32_t* __restrict__ chunk_base,
                                                       const uint32_t* __restrict__ offsets,
-                                                      const uint32_t* __restrict__ lists, CetAgg* aggs) {
+                                                      const uint32_t* __restrict__ lists, CetAgg* aggs,
+                                                      unsigned long long* __restrict__ stats) {
   __shared__ AggLds lds[4];
+  CetTally tl;
   AggLds& L = lds[threadIdx.x / WAVE];
   const uint32_t lane = lane_id();
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
@@ -395,6 +403,12 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
     const uint32_t len = mine ? offsets[d.off_base + ci + 1] - off : 0u;
     const uint32_t incl = wave_incl_scan(len);
     const uint32_t D = uniform(__shfl(incl, WAVE - 1, WAVE));
+    if (stats) {
+      tl.aggs += mine;
+      tl.items += len;
+      if (d.mode == AGG_CHAIN) tl.recs += len;
+      if (d.mode == AGG_SIBLING) tl.probe += len;
+    }
     L.pre[lane] = incl - len;
     L.off[lane] = off;
     L.s[lane] = L.a[lane] = L.b[lane] = 0;
@@ -459,6 +473,7 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
     }
     wave_sync();
   }
+  if (stats) flush_tally(tl, stats);
 }
 
 // One thread per term: the table by a binary search over the term ranges.
@@ -517,10 +532,10 @@ void launch_cet_sums(const DevGraph& g, const uint32_t* bitmaps, const uint32_t*
 
 void launch_cet_aggs(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* bprefix, const AggDesc* descs,
                      uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
-                     CetAgg* aggs, uint32_t grid, hipStream_t s) {
+                     CetAgg* aggs, uint32_t grid, hipStream_t s, unsigned long long* stats) {
   if (!ndesc) return;
   hipLaunchKernelGGL(cet_agg_kernel, dim3(grid), dim3(256), 0, s, g.ids, bitmaps, bprefix, g.W, descs, ndesc,
-                     chunk_base, offsets, lists, aggs);
+                     chunk_base, offsets, lists, aggs, stats);
 }
 
 void launch_cet_write(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, const CetDesc* descs,

@@ -222,8 +222,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(Pieces pieces, const u
   const uint32_t wave = uniform((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
   const uint32_t nwaves = (gridDim.x * blockDim.x) / WAVE;
   // per-lane tallies for the optional byte accounting, over all items
-  unsigned long long t_cand = 0;
-  uint32_t t_ent = 0, t_probe = 0;
+  uint32_t t_piece = 0, t_ent = 0, t_probe = 0;
 
   // the next item's list entry is loaded while the current one runs
   uint2 nxt = list && wave < items ? list[wave] : make_uint2(0u, 0u);
@@ -262,7 +261,6 @@ __global__ void __launch_bounds__(256) filter_step_kernel(Pieces pieces, const u
     const uint32_t incl = wave_incl_scan(pc);
     const uint32_t C = uniform(__shfl(incl, WAVE - 1, WAVE));
     if (C == 0) continue;
-    if (lane == 0) t_cand += C;
     {
       uint32_t pos = incl - pc, x = w;
       while (x) {
@@ -289,6 +287,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(Pieces pieces, const u
         uint32_t noff = 0, nlen = 0;
         if (i + 1 < nv) piece(pieces, id, nbr_lo[nb + i + 1], noff, nlen);
         const bool alive = mine && ff == nv;
+        if (stats) t_piece += alive;
         L.hit[lane] = 0;
         uint32_t cur = 0;  // entries of this candidate already examined
         bool h = !alive;
@@ -368,7 +367,7 @@ __global__ void __launch_bounds__(256) filter_step_kernel(Pieces pieces, const u
   if (stats) {
     // one atomic per counter per workgroup, spread over STAT_COPIES copies
     __shared__ unsigned long long red[4][5];
-    const unsigned long long v[5] = {t_cand, wave_sum64(t_ent), 0, wave_sum64(t_probe), 0};
+    const unsigned long long v[5] = {wave_sum64(t_piece), wave_sum64(t_ent), 0, wave_sum64(t_probe), 0};
     const uint32_t w = threadIdx.x / WAVE;
     if (lane == 0)
       for (int i = 0; i < 5; ++i) red[w][i] = v[i];
@@ -417,7 +416,7 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
   const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / WAVE;
   const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) / WAVE;
   const uint64_t pairs = (uint64_t)nfill * max_ranges, items = pairs + (uint64_t)nfill * nhp;
-  uint32_t t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
+  uint32_t t_piece = 0, t_ent = 0, t_key = 0, t_probe = 0, t_set = 0;
   for (uint64_t it = wave; it < items; it += nwaves) {
     const bool part = it >= pairs;
     const uint64_t x = part ? it - pairs : it;
@@ -452,6 +451,7 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
       for_steps(v_lo, v_hi, [&](uint64_t v0) {
         const uint64_t v = v0 + lane;
         const uint32_t k = v < v_hi ? key[v] : 0u;
+        if (stats) t_key += v < v_hi;
         const unsigned long long m = __ballot(k >= lo && k <= hi && v < v_hi);
         if ((m >> lane) & 1ULL) L.cand[C + (uint32_t)__popcll(lane ? m & (~0ULL >> (WAVE - lane)) : 0ULL)] = (uint32_t)v;
         C += (uint32_t)__popcll(m);
@@ -477,6 +477,7 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
       const bool mine = s0 + lane < C;
       const uint32_t id = mine ? L.cand[s0 + lane] : 0u;
       uint32_t off = 0, len = 0;
+      if (stats) t_piece += mine;
       if (mine) {
         piece(pieces, id, pull ? u_lo : lo, off, len);
         off += first;
@@ -569,10 +570,11 @@ __global__ void __launch_bounds__(256) fill_kernel(const uint32_t* __restrict__ 
     wave_sync();
   }
   if (stats) {
-    const unsigned long long v[4] = {wave_sum64(t_ent), wave_sum64(t_key), wave_sum64(t_probe), wave_sum64(t_set)};
+    const unsigned long long v[5] = {wave_sum64(t_piece), wave_sum64(t_ent), wave_sum64(t_key), wave_sum64(t_probe),
+                                     wave_sum64(t_set)};
     if (lane == 0)
-      for (int i = 0; i < 4; ++i)
-        if (v[i]) atomicAdd(stats + (blockIdx.x % STAT_COPIES) * STAT_STRIDE + 1 + i, v[i]);
+      for (int i = 0; i < 5; ++i)
+        if (v[i]) atomicAdd(stats + (blockIdx.x % STAT_COPIES) * STAT_STRIDE + i, v[i]);
   }
 }
 

@@ -131,8 +131,9 @@ void launch_init(const DevGraph& g, const InitOp* ops, uint32_t nops, uint32_t* 
 // One superstep: every op (one per query) explores or refines its C(u); the
 // explore ops' neighbours are filled by a second launch (fills, one per
 // neighbour).  stats (optional, STAT_COPIES x STAT_STRIDE u64, zeroed by the
-// caller): copy c, entries 0..4 = candidates, adjacency entries read, key
-// gathers, bitmap probes, bits set, added by the workgroups with blockIdx %
+// caller): copy c, entries 0..4 = pieces looked up (one per candidate and
+// neighbour), adjacency entries read, vertex and second entry keys read, bitmap
+// probes, bits set, added by the workgroups with blockIdx %
 // copies == c (the sum over copies is the launch's total).
 // Of more than FILTER_DIRECT (op, vertex range) pairs the superstep visits
 // only those whose range holds a candidate of C(u): a first kernel lists them
@@ -228,8 +229,9 @@ void launch_text_write(const uint32_t* tuples, uint64_t rows, uint32_t q, const 
 // chunk_base[d]: chunks of 64 candidates in the tables before d (ndesc + 1
 // entries); grid: workgroups (persistent).
 // stats (optional, STAT_COPIES x STAT_STRIDE u64, zeroed by the caller):
-// entries 0..3 = candidates, adjacency entries examined, bitmap probes, list
-// entries written (cet_write only), summed over the copies.
+// entries 0..3 = candidates (cet_count, cet_write), adjacency entries examined,
+// bitmap probes, list entries written, 4 = cet_sum's candidates, 5..7 = cet_agg's
+// candidates, list entries and records read, summed over the copies.
 void launch_cet_count(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* clist, CetDesc* descs,
                       uint32_t ndesc, uint32_t* offsets, const uint32_t* chunk_base, uint32_t grid, hipStream_t s,
                       unsigned long long* stats = nullptr);
@@ -244,7 +246,7 @@ void launch_cet_sums(const DevGraph& g, const uint32_t* bitmaps, const uint32_t*
 // the last tables' records.
 void launch_cet_aggs(const DevGraph& g, const uint32_t* bitmaps, const uint32_t* bprefix, const AggDesc* descs,
                      uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
-                     CetAgg* aggs, uint32_t grid, hipStream_t s);
+                     CetAgg* aggs, uint32_t grid, hipStream_t s, unsigned long long* stats = nullptr);
 // Hash terms of the last join levels' lists: for table term_desc[i] (terms
 // [term_start[i], term_start[i+1]) of terms), tuple_term(term_qid, id of list[e]).
 void launch_cet_terms(const DevGraph& g, const uint32_t* lists, const CetDesc* descs, const uint32_t* term_desc,
