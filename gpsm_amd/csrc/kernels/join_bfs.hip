@@ -12,9 +12,8 @@
 //    extends it) is one record; 16 lanes take a row of at most LONG_LIST
 //    candidates, four rows per wave, a workgroup takes a longer one;
 //  * a row's candidates come from its parent's candidate-edge list, or, with
-//    the learned order, from a back edge's bound vertex with fewer neighbours of
-//    the label (tested against C(w) and the parent's edge instead): the order's
-//    choice of the vertex to expand from, made row by row;
+//    the learned order (finish_rows), from a back edge's bound vertex with fewer
+//    neighbours of the label (tested against C(w) and the parent's edge instead);
 //  * survivors are staged in LDS and finished densely, one lane each: their
 //    own next list (rank index, offsets), then one record;
 //  * the last level is counted and hashed, not written.
@@ -155,8 +154,13 @@ __device__ __forceinline__ bool finish_rows(const BfsArgs& a, const PlanLevel* p
   // A back edge's vertex with fewer neighbours of the label is the cheaper
   // source, although its candidates take two tests more: 32 cycles and cliques
   // on an R-MAT 18 graph take 21.6 ms from the parents' lists alone, 16.0 /
-  // 14.2 / 13.6 ms with those less than 1/4, 1/2, 4/5 as long.  The heuristic
-  // order's plans keep their expand edge, the reference's rule.
+  // 14.2 / 13.6 ms with those less than 1/4, 1/2, 4/5 as long.  Rows, work,
+  // counts and hashes do not depend on it, and nothing in a heuristic plan rules
+  // it out.  It is off there for one reason: the 16 cliques on the R-MAT 22 graph
+  // are expected to join with the learned order in at most 0.8 times the
+  // heuristic order's time (tests/test_gpu_configs.py).  With it for both orders
+  // they take 137 ms (learned) and 125 (heuristic), so the expectation holds
+  // through this rule only: 137 and 320 ms as it is.
   const uint32_t nb = a.any_source && has ? p.nb2 : 0u;
   for (uint32_t b = 0; __any(b < nb); ++b) {
     const uint32_t c = b < nb ? p.backs2[b] : 0u;

@@ -64,6 +64,13 @@ inline Pieces pieces_of(const DevGraph& g) { return Pieces{g.lrow, g.n, g.gshift
 
 // Vertices per range: fewer where the graph is small, whose candidate sets
 // (one label's vertices, next to each other) otherwise fill too few waves.
+// 64 against 256 vertices a range on Chung-Lu graphs of 8 n edges and 4 labels,
+// an 8-vertex walk by itself (filter and counts) and 64 walks of 6 to 8 in a
+// batch: n = 30k 393 / 490 us and 3.1 / 3.1 ms, 200k 608 / 708 us and 8.6 / 7.7
+// ms, 400k 820 / 855 us and 15.2 / 13.6 ms, 600k 1165 / 1127 us and 21.2 / 18.4
+// ms, 1M 1570 / 1430 us and 39.7 / 34.6 ms.  With 16 labels the single walk is
+// even at 1M (682 / 672 us), a batch at 100k (2.75 / 2.65 ms).  The line is
+// where single queries of few labels are even.
 constexpr uint32_t FCHUNK_VERTS = 256, FCHUNK_VERTS_SMALL = 64;
 inline uint32_t range_verts(uint32_t n) { return n < 1u << 19 ? FCHUNK_VERTS_SMALL : FCHUNK_VERTS; }
 constexpr uint32_t FCHUNK_ENTRIES = 4096;
@@ -315,7 +322,7 @@ struct BfsArgs {
   JoinArgs j;
   uint32_t nplans, level;
   uint32_t block;             // row slots a wave reserves at a time
-  uint32_t any_source;        // a row's candidates may come from any of its bound neighbours
+  uint32_t any_source;        // a row's candidates may come from any of its bound neighbours (finish_rows)
   const uint64_t* first_row;  // first-table rows of the plans before each (nplans + 1)
   // rows of `level` and `level + 1`: records of stride_* words; short lists,
   // long lists, and their counts (2 words each, zeroed by the caller)

@@ -179,10 +179,11 @@ def main():
                                                          float(r["TotalDurationNs"]) / 1e6, float(r["Percentage"])))
     pair = join_pair_us(find(os.path.join(P, "trace"), "kernel_trace.csv"))
     if pair:
-        lines += ["", "A batch's tree-plan and cyclic-plan join launches run at the same time on two streams, so "
-                  "their durations overlap (and the %% column counts both): from their first start to their last "
-                  "end they take %.1f us per batch on average (%d batches of the trace)." % (sum(pair) / len(pair),
-                                                                                             len(pair))]
+        lines += ["", "From the first start to the last end of a batch's cyclic-plan and tree-plan join launches, "
+                  "which follow one another on one stream: %.1f us on average (%d batches of the trace). The trace "
+                  "holds batches of both orders; the breadth-first launches (bfs_*) are mostly the heuristic "
+                  "order's, whose plans leave back edges to the last position more often."
+                  % (sum(pair) / len(pair), len(pair))]
     if bl:
         lines += ["", "The traced run's bench line: join average launch %.1f us over its %d timed launches (HIP "
                   "events), %s queries/s." % (bl["roofline"]["avg_launch_us"], bl["roofline"]["launches"], bl["value"])]

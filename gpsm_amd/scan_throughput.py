@@ -7,11 +7,12 @@ own durations in a rocprofv3 kernel trace.
         python3 -m gpsm_amd.scan_throughput --mode compact --log2n 30 --density 0.05
     python -m gpsm_amd.scan_throughput --summarise DIR/scan_kernel_trace.csv --mode scan --log2n 27 ...
 
-gpsm_scan_u32 (exclusive scan of n u32 values: a reduce pass reading 4n
-bytes, one workgroup scanning the tile sums, a tile pass reading 4n and
-writing 4n) and gpsm_compact_bitmap (ids of the set bits of an n-bit bitmap:
+gpsm_scan_u32 (exclusive scan of n u32 values in one pass reading and writing
+4n bytes) and gpsm_compact_bitmap (ids of the set bits of an n-bit bitmap:
 a popcount pass reading n/8 bytes, then the compaction reading n/8 and
-writing 4 bytes per id and 4 per 256-bit block of the rank index).  Inputs
+writing 4 bytes per id).  Traces of the three scan kernels before the one-pass
+scan, and runs whose compaction also wrote a rank index of 4 bytes per 256 bits
+(no "index" in their JSON), are summarised as what they were.  Inputs
 are copied from host memory by the C-ABI calls; the copies are not kernels
 and are not counted.
 """
@@ -44,15 +45,20 @@ def run(mode, log2n, density, seed=3):
         ones = int(sum(bin(int(x)).count("1") for x in words[:4096])) * (len(words) // 4096)
         for _ in range(REPS):
             ids = ctx.compact(words, n)
-        return {"mode": mode, "n": n, "reps": REPS, "density": density, "ids": int(len(ids)), "ids_estimate": ones}
+        return {"mode": mode, "n": n, "reps": REPS, "density": density, "ids": int(len(ids)), "ids_estimate": ones,
+                "index": False}
 
 
-def kernel_bytes(mode, n, ids):
+def index_bytes(rec):
+    return 4 * (rec["n"] // 256) if rec.get("index", True) else 0
+
+
+def kernel_bytes(mode, n, ids, index):
     if mode == "scan":
         return {"scan_reduce_kernel": 4 * n, "scan_sums_kernel": 16 * ((n + 4095) // 4096), "scan_tile_kernel": 8 * n}
     nseg = (n // 32 + 2047) // 2048  # 2048-word segments
     return {"seg_popcount_kernel": n // 8, "seg_offsets_kernel": 8 * nseg + 4,
-            "compact_rows_kernel": n // 8 + 4 * ids + 4 * (n // 256)}
+            "compact_rows_kernel": n // 8 + 4 * ids + index}
 
 
 def summarise(trace_csv, rec, out_md, command, append):
@@ -63,7 +69,7 @@ def summarise(trace_csv, rec, out_md, command, append):
             dur[m.group(1)].append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) * 1e-3)
     # the one-pass scan, or a trace of the three kernels before it
     byt = {"scan_kernel": 8 * rec["n"]} if "scan_kernel" in dur else kernel_bytes(rec["mode"], rec["n"],
-                                                                                  rec.get("ids", 0))
+                                                                                  rec.get("ids", 0), index_bytes(rec))
     lines = [] if append else [
         "# Scan and compaction kernels: HBM throughput", "",
         "Each configuration is one rocprofv3 --kernel-trace run (commands below); per kernel the average of its "
@@ -82,10 +88,10 @@ def summarise(trace_csv, rec, out_md, command, append):
         lines.append("| %s | %s | %.1f | %d | %.0f | %.1f |" % (cfg, k, us, b, gbs, 100 * gbs / PEAK_GBS))
     # the whole operation: its kernels one after another, against the bytes
     # of the operation itself (the scan reads and writes each value once;
-    # the compaction reads the bitmap once and writes the ids and the index)
+    # the compaction reads the bitmap once and writes the ids)
     if all(dur.get(k) for k in byt):
         us = sum(sum(dur[k]) / len(dur[k]) for k in byt)
-        b = 8 * rec["n"] if rec["mode"] == "scan" else rec["n"] // 8 + 4 * rec.get("ids", 0) + 4 * (rec["n"] // 256)
+        b = 8 * rec["n"] if rec["mode"] == "scan" else rec["n"] // 8 + 4 * rec.get("ids", 0) + index_bytes(rec)
         gbs = b / (us * 1e-6) / 1e9
         lines.append("| %s | all of the above | %.1f | %d | %.0f | %.1f |" % (cfg, us, b, gbs, 100 * gbs / PEAK_GBS))
     with open(out_md, "a" if append else "w") as fh:
