@@ -378,6 +378,8 @@ struct AggLds {
   unsigned long long s[WAVE], a[WAVE], b[WAVE];
 };
 
+// STATS: with the work counters, whose registers the timed variant keeps free.
+template <bool STATS>
 __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict__ ids,
                                                       const uint32_t* __restrict__ bitmaps,
                                                       const uint32_t* __restrict__ bprefix, uint32_t W,
@@ -403,7 +405,7 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
     const uint32_t len = mine ? offsets[d.off_base + ci + 1] - off : 0u;
     const uint32_t incl = wave_incl_scan(len);
     const uint32_t D = uniform(__shfl(incl, WAVE - 1, WAVE));
-    if (stats) {
+    if (STATS) {
       tl.aggs += mine;
       tl.items += len;
       if (d.mode == AGG_CHAIN) tl.recs += len;
@@ -473,7 +475,7 @@ __global__ void __launch_bounds__(256) cet_agg_kernel(const uint32_t* __restrict
     }
     wave_sync();
   }
-  if (stats) flush_tally(tl, stats);
+  if constexpr (STATS) flush_tally(tl, stats);
 }
 
 // One thread per term: the table by a binary search over the term ranges.
@@ -534,7 +536,7 @@ void launch_cet_aggs(const DevGraph& g, const uint32_t* bitmaps, const uint32_t*
                      uint32_t ndesc, const uint32_t* chunk_base, const uint32_t* offsets, const uint32_t* lists,
                      CetAgg* aggs, uint32_t grid, hipStream_t s, unsigned long long* stats) {
   if (!ndesc) return;
-  hipLaunchKernelGGL(cet_agg_kernel, dim3(grid), dim3(256), 0, s, g.ids, bitmaps, bprefix, g.W, descs, ndesc,
+  hipLaunchKernelGGL(stats ? cet_agg_kernel<true> : cet_agg_kernel<false>, dim3(grid), dim3(256), 0, s, g.ids, bitmaps, bprefix, g.W, descs, ndesc,
                      chunk_base, offsets, lists, aggs, stats);
 }
 
