@@ -551,6 +551,7 @@ int gpsm_graph_csr(const gpsm_graph* g, uint32_t* row_offset, uint32_t* col) {
 int gpsm_graph_free(gpsm_graph* g) {
   if (!g) return GPSM_EINVAL;
   hipSetDevice(g->ctx->device);
+  std::lock_guard<std::mutex> not_captured(g->ctx->capture);
   hipStreamSynchronize(g->ctx->stream);
   free_graph_arrays(g->ctx, g->dg);
   g->directed.release();
@@ -976,7 +977,11 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if (replayed && rc) return rc;
   if (!replayed) {
     bool captured = false;
-    if (o.use_graph && hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) captured = true;
+    std::unique_lock<std::mutex> capturing(c->capture, std::defer_lock);
+    if (o.use_graph) {
+      capturing.lock();
+      captured = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess;
+    }
     launch_fill_u32(bitmaps, 0u, (uint64_t)erows * W, s);
     launch_fill_u32(dptr<uint32_t>(c, B_FNITEMS), 0u, ncounters + 4ull * std::max<uint32_t>(nq, 1), s);
     if (counters) launch_fill_u32(reinterpret_cast<uint32_t*>(fstats), 0u, 2ull * fstat_step * nstat_slots, s);
@@ -1381,7 +1386,11 @@ int run_batch(gpsm_ctx* c, const gpsm_graph* g, uint32_t nq, const gpsm_query* q
   if (replayed_c && rc) return rc;
   if (!replayed_c) {
     bool captured = false;
-    if (o.use_graph && hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) captured = true;
+    std::unique_lock<std::mutex> capturing(c->capture, std::defer_lock);
+    if (o.use_graph) {
+      capturing.lock();
+      captured = hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess;
+    }
     hipEvent_t pa = pbegin(K_CET_COUNT);
     if (!cdesc.empty())
       launch_cet_count(dg, bitmaps, dptr<uint32_t>(c, B_CLIST), dptr<CetDesc>(c, B_CDESC), (uint32_t)cdesc.size(),

@@ -5,6 +5,7 @@
 #include <atomic>
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "gpsm.h"
@@ -229,6 +230,9 @@ struct gpsm_ctx {
   // place when its topology is the same (hipGraphExecUpdate, graph_updates)
   // and is instantiated afresh when it is not (graph_instantiations).
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
+  // held while a batch captures: a graph freed by another thread waits for the
+  // stream, which must not happen in between
+  std::mutex capture;
   std::vector<uint64_t> gsig[2];
   // this device's copy of the allocation-free scan's static scratch array
   // (hipGetSymbolAddress at gpsm_init)

@@ -7,6 +7,7 @@ a graph uploaded once.  There is no CPU path: without a HIP device every call
 raises GpsmError.
 """
 import ctypes as C
+import threading
 import weakref
 from dataclasses import dataclass, field
 
@@ -189,6 +190,7 @@ class ResidentGraph:
     def __init__(self, ctx, g, handle=None):
         self.ctx = ctx
         self.g = g
+        self._freeing = threading.Lock()  # another thread may free it while the context closes
         if handle is None:
             handle = C.c_void_p()
             ro, col, lab = u32(g.row_offset), u32(g.col), u32(g.labels)
@@ -199,9 +201,10 @@ class ResidentGraph:
 
     def free(self):
         # a graph whose context is already closed was freed with it
-        if self.h and self.ctx.h:
-            _lib.lib().gpsm_graph_free(self.h)
-        self.h = None
+        with self._freeing:
+            if self.h and self.ctx.h:
+                _lib.lib().gpsm_graph_free(self.h)
+            self.h = None
 
     def __del__(self):
         try:
