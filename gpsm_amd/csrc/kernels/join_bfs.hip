@@ -494,7 +494,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) b
     pos = first_pos;
     skip = 0;
   }
-  if (lane == 0) cur[0] = {idx, pos, skip};
+  if (lane == 0) cur[0] = {idx, pos, skip, 0};
 
   // short rows: 16 lanes each, four per wave; the next quad's rows load while
   // this one's candidates are tested
@@ -520,9 +520,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) b
       // a reserved slot that holds no row has only its length
       const uint32_t row_plan = r.get(R_PLAN), st = r.get(R_START), row_src = r.get(R_SRC);
       const uint32_t plan = len ? row_plan : 0u, src = len ? row_src : 0u;
-      // rows of a plan over its budget end here, but not while part of a step is
-      // written: skip counts that step's survivors over all four rows
-      if (len && !skip && a.j.budget && a.j.out[a.j.plans[plan].out].aborted) len = 0;
+      // rows of a plan over its budget end here, but where part of a step is
+      // written the step's rows are those it was saved with: skip counts the
+      // survivors of them all
+      if (len && a.j.budget &&
+          (skip ? !((cur[1].rows >> gi) & 1u) : a.j.out[a.j.plans[plan].out].aborted != 0))
+        len = 0;
       const PlanLevel& p = plans[plan];
       const bool final = p.final;
       const uint32_t qid = p.qid;
@@ -541,6 +544,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) b
           if (done < n) {  // this step again later: its last-level rows are not counted yet
             skip = done;
             full = true;
+            const unsigned long long with = __ballot(len != 0);
+            uint32_t rows = 0;
+            for (uint32_t i = 0; i < PER; ++i) rows |= (uint32_t)((with >> (i * GROUP)) & 1u) << i;
+            if (lane == 0) cur[1].rows = rows;
             break;
           }
         }
@@ -572,7 +579,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) b
     skip = 0;
   }
   if (lane == 0) {
-    cur[1] = {idx, pos, skip};
+    cur[1].idx = idx, cur[1].pos = pos, cur[1].skip = skip;
     if (full) atomicAdd(a.pending, 1u);
   }
   if (a.rows_out) close_slots(a, slots);

@@ -317,6 +317,7 @@ uint64_t join_level_words(uint32_t qmax, uint32_t cap);
 constexpr uint32_t BFS_PLANS = 256;
 struct BfsCursor {
   uint32_t idx, pos, skip;
+  uint32_t rows;  // a quad's rows with candidates in the step that skip counts in, a bit each
 };
 struct BfsArgs {
   JoinArgs j;

@@ -50,3 +50,24 @@ def test_budget_passed_while_a_level_waits_for_its_buffer(ctx, a, b):
             (0, r0.count, r0.hash, r0.level_rows, r0.level_work, r0.join_work)
     for r in res[0::2]:
         assert (r.status, r.count, r.hash) == (_lib.EBUDGET, 0, 0)
+
+
+@pytest.mark.parametrize("part", [16, 10, 6, 4, 3, 2])
+def test_budget_passed_at_any_time(ctx, part):
+    """The budget passed earlier or later on the way through the second level:
+    rows are left out before a wave stops in a step as well as after."""
+    wide, narrow = labelled_cycle(1, 2), labelled_cycle(3, 4)
+    qs = [wide, narrow] * 128
+    orders = [[0, 1, 2, 3]] * len(qs)
+    rg = ctx.upload(two_pairs_of_hubs(501, 201))
+    base = rg.match_batch(qs, explicit_orders=orders)
+    w = base[0].level_work
+    budget = w[1] + w[2] + w[3] // part
+    assert base[1].join_work < budget < base[0].join_work
+    for _ in range(5):
+        res = rg.match_batch(qs, explicit_orders=orders, work_budget=budget)
+        for r, r0 in zip(res[1::2], base[1::2]):
+            assert (r.status, r.count, r.hash, r.level_rows, r.level_work, r.join_work) == \
+                (0, r0.count, r0.hash, r0.level_rows, r0.level_work, r0.join_work)
+        for r in res[0::2]:
+            assert (r.status, r.count, r.hash) == (_lib.EBUDGET, 0, 0)
